@@ -72,6 +72,15 @@ enum {
     JSSO_PC_AMG = 1           /* smoothed-aggregation AMG V-cycle on the scaled system
                                  (the default)                                          */
 };
+/* As long as the caller has not called jsso_plan_set_preconditioner (or asked
+ * jsso_plan_amg_reuse to keep a hierarchy), a batched solve with 1 to 4 load cases
+ * may be direct instead: a multifrontal Cholesky of the scaled constrained K in
+ * FP64 (kept until the next jsso_assemble), refined on the FP64 residual to the
+ * same tolerance; plans whose fronts are small enough for it to be the faster way
+ * take it in every batched precision.  h_info->iterations counts its refinement
+ * steps, h_info->levels and dir_launches are 0.  A factorisation that meets a
+ * pivot that is not positive, or a system that it does not bring to the tolerance
+ * or to its attainable accuracy, hands the whole solve to the AMG. */
 
 typedef struct {
     int32_t iterations;   /* CG iterations performed (max over systems)            */

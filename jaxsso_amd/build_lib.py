@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "_lib")
 LIB = os.path.join(OUT, "libjsso_hip.so")
 SOURCES = ["jsso_api.hip", "jsso_element.hip", "jsso_assemble.hip", "jsso_solve.hip", "jsso_amg.hip",
-           "jsso_dense.hip", "jsso_param.hip"]
+           "jsso_dense.hip", "jsso_direct.hip", "jsso_param.hip"]
 ARCH = os.environ.get("JSSO_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -446,6 +446,7 @@ int jsso_plan_destroy(jsso_plan* plan) {
     if (!plan) return JSSO_OK;
     Plan* q = P(plan);
     amg_destroy(q);
+    direct_destroy(q);
     for (auto& row : q->cg_graph)
         for (auto& pair : row)
             for (auto& g : pair)
@@ -567,6 +568,7 @@ int jsso_assemble(jsso_plan* plan, const double* d_crds, const double* d_prop_be
     timing_end(s, ev);
     JSSO_HIP(hipMemcpyAsync(p->d_crds, d_crds, (size_t)p->n_nodes * 3 * sizeof(double), hipMemcpyDeviceToDevice, s));
     p->amg_valid = false;
+    p->direct_valid = false;
     if (d_K_out && p->nnzb) {
         if ((rc = launch_full_blocks(p, s))) return rc;
         JSSO_HIP(hipMemcpyAsync(d_K_out, p->d_K, (size_t)p->nnzb * 36 * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -907,6 +909,7 @@ int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc) {
         return JSSO_EINVAL;
     }
     P(plan)->precond = pc;
+    P(plan)->precond_set = true;
     return JSSO_OK;
 }
 int jsso_plan_amg_reuse(jsso_plan* plan, int32_t mode, int64_t* h_counts) {
@@ -917,6 +920,7 @@ int jsso_plan_amg_reuse(jsso_plan* plan, int32_t mode, int64_t* h_counts) {
     Plan* p = P(plan);
     if (mode >= 0) {
         p->amg_reuse = mode;
+        if (mode > 0) p->precond_set = true;
         if (mode == 2) p->amg_valid = false;   // rebuild at the next solve even without a new assembly
     }
     if (h_counts) {
@@ -955,8 +959,12 @@ int jsso_plan_cg_tuning(jsso_plan* plan, int32_t precision, int32_t nrhs, int32_
     const int ps = precision == JSSO_PREC_MIXED ? PS_F32 : precision == JSSO_PREC_FP64 ? PS_F64 : PS_F32_V64;
     Plan* p = P(plan);
     int32_t& slot = p->precond == JSSO_PC_AMG ? p->amg_wps[ps][nrhs] : p->cg_wps[ps][nrhs];
-    if (set_wps >= 0) slot = set_wps;
-    if (h_wps) *h_wps = slot;
+    int32_t& direct = p->direct_wps[ps][nrhs];   // (a plan without a chosen preconditioner may solve directly)
+    if (set_wps >= 0) {
+        slot = set_wps;
+        if (!p->precond_set) direct = set_wps;
+    }
+    if (h_wps) *h_wps = !p->precond_set && direct ? direct : slot;
     return JSSO_OK;
 }
 

@@ -1,0 +1,1534 @@
+// Sparse direct solve of the batched systems: multifrontal Cholesky of the
+// constrained, block-Jacobi-scaled stiffness on a nested-dissection tree, with
+// refinement on the FP64 residual (the counterpart of the reference's SuperLU
+// solve, JaxSSO/solver.py:176-218).
+//
+// A front is the dense symmetric matrix of a tree node's pivots (k rows) and its
+// border (b rows), k = 6 np, b = 6 nb, held as its lower triangle, row-major:
+//   F11 = L L^T,   L21 = F21 L^-T,   C = F22 - L21 L21^T   (passed to the parent)
+// and kept for the solves are   S = F11^-1 = L^-T L^-1   and   G = L21 L^-1, so
+// that both directions are plain matrix-vector products without a dependence
+// inside a panel:
+//   forward   r2 -= G r1         (children before parents)
+//   backward  x1 = S r1 - G^T x2 (parents before children)
+// Every product runs on the FP64 matrix cores (v_mfma_f64_16x16x4): operands from
+// LDS as [row][k] with a row stride of 2 (mod 4) doubles, so the 16 rows x 2
+// columns a half wavefront reads fall on 32 different bank pairs.
+//
+// Small fronts (panel rows in LDS) are one workgroup each: gather, factor, panel,
+// contribution, all from LDS; only the children's contributions are read and only
+// S, G and the own contribution written.  Larger fronts go in panels of <= 96
+// pivots whose columns are kept in HBM:
+//   k_front_diag   factor of the panel's diagonal block and its inverse, S
+//   k_front_strip  64 rows below it: L21 (in place) and G
+//   k_front_cols   the panel's update of the pivot columns still to come
+//   k_front_cb     after the last panel: C = gathered children - L21 L21^T over
+//                  all pivots at once, so C is written once and never re-read
+// The front is never assembled as a whole: each kernel gathers what it is the
+// first to touch from the children's contributions and the blocks of K.  All
+// fronts of a tree level, over all structures of the plan, go in the same
+// launches.
+#include <cmath>
+#include <cstring>
+#include <map>
+#include <new>
+#include <type_traits>
+
+#include "direct_symbolic.hpp"
+#include "solver_common.hpp"
+#include "solver_kernels.hpp"
+
+namespace jsso {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+constexpr int DW = 96;                    // pivots per panel, at most (16 nodes)
+constexpr int DROWS = 64;                 // edge of an update tile
+constexpr int SROWS = 96;                 // rows of a strip
+constexpr int DLEAF = 12;                 // nodes eliminated whole at the tree's leaves
+constexpr int DLDS_MAX = 156 * 1024;      // dynamic LDS of a small front
+constexpr int DIRECT_MAX_M = 1500;        // largest front (direct_fits)
+constexpr int DIRECT_STEPS = 6;           // refinement steps, at most
+constexpr double DIRECT_FLOOR_FACTOR = 16.0;   // attainable accuracy: 16 eps (||A|| ||x|| + ||b||), as the AMG solve
+constexpr int DKC = 32;                   // pivot columns staged at a time by the tile kernels
+
+struct FrontMeta {
+    int32_t np, nb, node0, level;
+    int32_t child[2], npre, blk0, nblk;   // npre: border nodes that are pivots of the parent
+    int32_t wn, npan;                     // nodes of a panel (the last may have fewer), panels
+    int32_t small, pad;                   // one-workgroup front
+    int64_t fac, mat, pan, vec;           // offsets (doubles): S|G panels, contribution (b x b), pivot columns
+                                          // (m x k, large fronts), vector (x load cases)
+};
+struct StructMeta {
+    int64_t fac, mat, vec;                // bases of the structure
+    int32_t node0, blk0;                  // first node, first block of the CSR
+};
+struct DirectDev {
+    const FrontMeta* fr;
+    const StructMeta* st;
+    const int32_t *nodes, *rel, *blk, *blkrow, *kref;
+    const int2* inv;                      // per entry of `nodes`: the border node it is in each child, or -1
+    const double* A64;
+    double *fac, *mat, *vec;
+    const double* zero;                   // a zero
+    int32_t* bad;                         // per structure: a pivot was not positive
+};
+struct DTask {
+    int32_t front, sys;
+};
+struct DirectReport {
+    int32_t running, stalled, floor, bad;   // systems; structures with a pivot that is not positive
+    double worst;                           // largest relative residual of the best iterates
+};
+
+struct DirectState {
+    std::vector<FrontMeta> fr;
+    std::vector<StructMeta> st;
+    std::vector<std::vector<DTask>> small_tasks, big_tasks;   // per level
+    std::vector<size_t> small_lds;                            // per level: dynamic LDS
+    std::vector<int> small_m, big_m, big_k, big_b, big_w, big_pan;   // per level: largest fronts, most panels
+    std::vector<int64_t> small_off, big_off;                  // first task of the level on the device
+    int n_levels = 0, max_m = 0;
+    size_t fac_n = 0, mat_n = 0, vec_n = 0;
+    double flops = 0.0;
+    DirectDev dev{};
+    DTask* d_tasks = nullptr;
+    double* d_rho = nullptr;
+    DirectReport *d_report = nullptr, *h_report = nullptr;
+    size_t vec_bytes = 0;
+    std::vector<void*> allocs;
+    bool usable = false, factored = false;
+};
+
+// ---------------------------------------------------------------------------
+// device: tiles
+// ---------------------------------------------------------------------------
+// D = A B + D with A 16x4 (lane: row l % 16, column l / 16), B 4x16 (lane: row
+// l / 16, column l % 16), D 16x16 (element i of a lane: row 4 i + l / 16, column
+// l % 16): a D tile is, element by element, the B operand of four further steps.
+__device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return join_halves(lo, hi);
+}
+
+// acc += X_I Y_J^T over n16 tiles of 16 columns; X, Y point at the first row of
+// the row tiles
+__device__ __forceinline__ d4 tile_xyt(const double* X, const double* Y, int ld, int n16, d4 acc, int lane) {
+    const double* x = X + (lane & 15) * ld + (lane >> 4);
+    const double* y = Y + (lane & 15) * ld + (lane >> 4);
+#pragma unroll 4
+    for (int t = 0; t < 4 * n16; ++t) acc = mfma64(x[4 * t], y[4 * t], acc);
+    return acc;
+}
+
+// 1 / sqrt(d): the hardware estimate and one third-order correction
+__device__ __forceinline__ double fast_rsqrt(double d) {
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = fma(-d * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// the values of v in the four lanes r, r + 16, r + 32, r + 48 (every lane gets all)
+__device__ __forceinline__ void all_rows(double v, double (&x)[4]) {
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    // rows (0, 0, 2, 2) and (1, 1, 3, 3), then each split into its halves
+    auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+        auto l2 = __builtin_amdgcn_permlane32_swap(l[o], l[o], false, false);
+        auto h2 = __builtin_amdgcn_permlane32_swap(h[o], h[o], false, false);
+        x[o] = join_halves(l2[0], h2[0]);
+        x[o + 2] = join_halves(l2[1], h2[1]);
+    }
+}
+
+// Cholesky factor L of a 16x16 block (lower triangle in LDS) and its inverse, by
+// one wavefront; the inverse replaces the block (zeros above the diagonal).
+// Lane (r, q) = (l % 16, l / 16) holds A[r][4 i + q], i = 0..3: for a symmetric A
+// that is at once the layout of the matrix core's result and of its first operand,
+// so the update by four columns of L is one instruction, and so is the same step
+// of the forward substitution W <- I that gives the inverse.  Per four columns:
+// every lane collects its row's four entries (all_rows), the 4x4 diagonal block
+// comes by readlane and is factored by all lanes alike.  Against a column at a
+// time with readlane broadcasts (240 of them, 5 us) this took the block to ~1.5 us.
+__device__ __forceinline__ bool factor16(double* D, int ld, int lane) {
+    const int r = lane & 15, q = lane >> 4;
+    d4 A, W;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int c = 4 * i + q;
+        A[i] = r >= c ? D[r * ld + c] : D[c * ld + r];
+        W[i] = c == r ? 1.0 : 0.0;
+    }
+    bool ok = true;
+#pragma unroll 1
+    for (int b = 0; b < 4; ++b) {   // (a loop: unrolled, it doubles the registers)
+        double p[4], w[4], d[4][4];
+        all_rows(b == 0 ? A[0] : b == 1 ? A[1] : b == 2 ? A[2] : A[3], p);
+        all_rows(b == 0 ? W[0] : b == 1 ? W[1] : b == 2 ? W[2] : W[3], w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c <= i; ++c) d[i][c] = lane_value(p[c], 4 * b + i);
+        const double i0 = fast_rsqrt(d[0][0]);
+        const double l10 = d[1][0] * i0, l20 = d[2][0] * i0, l30 = d[3][0] * i0;
+        const double e1 = fma(-l10, l10, d[1][1]), i1 = fast_rsqrt(e1);
+        const double l21 = fma(-l20, l10, d[2][1]) * i1, l31 = fma(-l30, l10, d[3][1]) * i1;
+        const double e2 = fma(-l21, l21, fma(-l20, l20, d[2][2])), i2 = fast_rsqrt(e2);
+        const double l32 = fma(-l31, l21, fma(-l30, l20, d[3][2])) * i2;
+        const double e3 = fma(-l32, l32, fma(-l31, l31, fma(-l30, l30, d[3][3]))), i3 = fast_rsqrt(e3);
+        ok &= d[0][0] > 0.0 && e1 > 0.0 && e2 > 0.0 && e3 > 0.0;
+        p[0] *= i0;
+        p[1] = fma(-p[0], l10, p[1]) * i1;
+        p[2] = fma(-p[1], l21, fma(-p[0], l20, p[2])) * i2;
+        p[3] = fma(-p[2], l32, fma(-p[1], l31, fma(-p[0], l30, p[3]))) * i3;
+        w[0] *= i0;
+        w[1] = fma(-l10, w[0], w[1]) * i1;
+        w[2] = fma(-l21, w[1], fma(-l20, w[0], w[2])) * i2;
+        w[3] = fma(-l32, w[2], fma(-l31, w[1], fma(-l30, w[0], w[3]))) * i3;
+        double l = q == 0 ? p[0] : q == 1 ? p[1] : q == 2 ? p[2] : p[3];
+        const double x = q == 0 ? w[0] : q == 1 ? w[1] : q == 2 ? w[2] : w[3];
+        if (4 * b + q > r) l = 0.0;
+        D[(4 * b + q) * ld + r] = x;   // (its old entries are all in registers)
+        A = mfma64(-l, l, A);
+        W = mfma64(-l, x, W);
+    }
+    return ok;
+}
+
+// F11 (kp x kp in LDS, kp a multiple of 16; lower triangle, zeros above it) -> its
+// inverse factor (whole workgroup).  Block (I, J) of L^-1, I > J, is left at block
+// row J, block column I (as it is, not transposed), the diagonal blocks in place;
+// the lower blocks hold L.  Per block column kb two phases with a barrier each:
+//   B  what column kb - 1 updates: wavefront 0 takes the diagonal block and factors
+//      it, the others the rest of the trailing triangle and the sums
+//      W_IJ = sum_K L_IK Linv_KJ of the rows below
+//   A  L_I = A_I Dinv^T below the block, and row kb of the inverse, -Dinv W_J
+// The factorisation of a 16x16 block (one wavefront, ~2 us of dependent steps) is
+// the chain that bounds this routine; phase B hides the products behind it.
+__device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wave, int nw, int lane) {
+    const int nt = kp >> 4, r = lane & 15, q = lane >> 4;
+    bool ok = true;
+#pragma unroll 1
+    for (int kb = 0; kb < nt; ++kb) {
+        // B of block column j = kb - 1: products X Y (Y as it is or transposed) added to C
+        const int j = kb - 1, n = nt - kb, ntri = kb ? n * (n + 1) / 2 : 0, all = ntri + n * kb;
+#pragma unroll 1
+        for (int e = wave; e < all; e += wave ? nw - 1 : all) {   // (wavefront 0 only takes tile 0)
+            const double *X, *Y;
+            double* C;
+            int ys;
+            double sign;
+            if (e < ntri) {   // A_IJ -= L_I L_J^T
+                int I = 0, J = e;
+                while (J > I) {
+                    J -= I + 1;
+                    ++I;
+                }
+                I += kb;
+                J += kb;
+                X = P + (16 * I + r) * ld + 16 * j + q;
+                Y = P + (16 * J + r) * ld + 16 * j + q;
+                C = P + (16 * I + q) * ld + 16 * J + r;
+                ys = 4;
+                sign = -1.0;
+            } else {   // W_IJ += L_Ij Linv_jJ, kept at block (J, I)
+                const int I = kb + (e - ntri) % n, J = (e - ntri) / n;
+                X = P + (16 * I + r) * ld + 16 * j + q;
+                Y = P + (16 * J + q) * ld + 16 * j + r;
+                C = P + (16 * J + q) * ld + 16 * I + r;
+                ys = 4 * ld;
+                sign = 1.0;
+            }
+            d4 acc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = C[4 * i * ld];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc = mfma64(sign * X[4 * t], Y[t * ys], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
+        }
+        double* D = P + (16 * kb) * ld + 16 * kb;
+        if (wave == 0) ok &= factor16(D, ld, lane);
+        __syncthreads();
+#pragma unroll 1
+        for (int e = wave; e < nt - 1; e += nw) {
+            const bool inv = e < kb;   // row kb of the inverse: -Dinv W; else L_I = A_I Dinv^T
+            double* C = P + (inv ? (16 * e + q) * ld + 16 * kb : (16 * (e + 1) + q) * ld + 16 * kb) + r;
+            const double* X = inv ? D + r * ld + q : P + (16 * (e + 1) + r) * ld + 16 * kb + q;
+            const double* Y = inv ? C : D + r * ld + q;
+            const int ys = inv ? 4 * ld : 4;
+            const double sign = inv ? -1.0 : 1.0;
+            d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc = mfma64(sign * X[4 * t], Y[t * ys], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
+        }
+        __syncthreads();
+    }
+    return ok;
+}
+
+// 16 rows X (in LDS, stride ld) times Linv^T, block column J: sum over K <= J
+__device__ __forceinline__ d4 strip_L(const double* X, const double* P, int ld, int J, int lane) {
+    const int r = lane & 15, q = lane >> 4;
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int K = 0; K <= J; ++K) {
+        const double* x = X + r * ld + 16 * K + q;
+        const double* y = P + (16 * K + r) * ld + 16 * J + q;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc = mfma64(x[4 * t], y[4 * t], acc);
+    }
+    return acc;
+}
+// 16 rows of L21 times Linv, block column J: sum over K >= J
+__device__ __forceinline__ d4 strip_G(const double* X, const double* P, int ld, int nt, int J, int lane) {
+    const int r = lane & 15, q = lane >> 4;
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int K = J; K < nt; ++K) {
+        const double* x = X + r * ld + 16 * K + q;
+        const double* y = P + (16 * J + q) * ld + 16 * K + r;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc = mfma64(x[4 * t], y[4 * t * ld], acc);
+    }
+    return acc;
+}
+__device__ __forceinline__ void store_tile(double* G, int64_t ldg, d4 v, int nrow, int ncol, int lane) {
+    const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (4 * i + q < nrow && r < ncol) G[(4 * i + q) * ldg + r] = v[i];
+}
+
+// S = Linv^T Linv (k x k, row-major) to global memory
+__device__ __forceinline__ void write_S(const double* P, int ld, int kp, int k, double* S, int wave, int nw,
+                                        int lane) {
+    const int nt = kp >> 4, r = lane & 15, q = lane >> 4;
+#pragma unroll 1
+    for (int e = wave; e < nt * (nt + 1) / 2; e += nw) {
+        int I = 0, J = e;
+        while (J > I) {
+            J -= I + 1;
+            ++I;
+        }
+        d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (int K = I; K < nt; ++K)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc = mfma64(P[(16 * I + 4 * t + q) * ld + 16 * K + r], P[(16 * J + 4 * t + q) * ld + 16 * K + r], acc);
+        store_tile(S + (int64_t)16 * I * k + 16 * J, k, acc, k - 16 * I, k - 16 * J, lane);
+        if (I != J) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (16 * I + 4 * i + q < k && 16 * J + r < k)
+                    S[(int64_t)(16 * J + r) * k + 16 * I + 4 * i + q] = acc[i];
+        }
+    }
+}
+
+// entry (row, column) of the block that enters a front as F[6 a + row][6 c + col]
+__device__ __forceinline__ double stored_entry(const DirectDev& d, int32_t kr, int row, int col) {
+    // the triple names the block (column node, row node): kr even, stored as it is
+    const int e = (kr & 1) ? row * 6 + col : col * 6 + row;
+    const int vp = kr >> 1;
+    return d.A64[(int64_t)(vp >> 6) * 36 * ROWS_PER_WG + ((int64_t)(e >> 1) * ROWS_PER_WG + (vp & 63)) * 2 + (e & 1)];
+}
+
+// a front's contribution C (b x b, row-major, lower triangle)
+__device__ __forceinline__ double* contribution(const DirectDev& d, const FrontMeta& f, const StructMeta& s) {
+    return d.mat + s.mat + f.mat;
+}
+
+// The children's part of a front's entries: where each child keeps its C
+struct Gather {
+    const double *C[2], *zero;
+    int ld[2];
+    bool any;
+};
+__device__ __forceinline__ Gather make_gather(const DirectDev& d, const FrontMeta& f, const StructMeta& st) {
+    Gather g;
+    g.zero = d.zero;
+    g.any = f.child[0] >= 0;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        g.C[c] = d.zero;
+        g.ld[c] = 0;
+        if (f.child[c] >= 0) {
+            const FrontMeta& h = d.fr[f.child[c]];
+            g.C[c] = contribution(d, h, st);
+            g.ld[c] = 6 * h.nb;
+        }
+    }
+    return g;
+}
+// entry (row, col) of the front, row >= col; a, b: `inv` of their nodes.  Without
+// branches, so that a thread's loads are all in flight at once (a wavefront that
+// waited for each in turn spent most of its time here): what a child does not hold
+// is read from a word that is zero.
+__device__ __forceinline__ double gathered(const Gather& g, int2 a, int2 b, int rr, int cc, bool on) {
+    const bool x = on && (a.x | b.x) >= 0, y = on && (a.y | b.y) >= 0;
+    const double* p = x ? g.C[0] + (int64_t)(6 * a.x + rr) * g.ld[0] + 6 * b.x + cc : g.zero;
+    const double* q = y ? g.C[1] + (int64_t)(6 * a.y + rr) * g.ld[1] + 6 * b.y + cc : g.zero;
+    return *p + *q;
+}
+// adds the blocks of K with front rows in [r0, r1) and columns in [c0, c1) to a tile
+// in LDS (rows and columns relative to r0, c0; front rows from `split` on are `gap`
+// rows further down); four chains of dependent loads per thread in flight
+__device__ __forceinline__ void add_stored(const DirectDev& d, const FrontMeta& f, const StructMeta& st, int r0,
+                                           int r1, int c0, int c1, int split, int gap, double* T, int ld, int tid,
+                                           int nth) {
+    if (r1 <= r0) return;
+    const int n0 = r0 / 6, n1 = (r1 + 5) / 6, m = f.np + f.nb;
+    const int32_t* br = d.blkrow + f.node0;
+    const int b0 = br[n0], b1 = n1 < m ? br[n1] : f.blk0 + f.nblk;
+    const int all = (b1 - b0) * 36;
+    for (int e0 = tid; e0 < all; e0 += 4 * nth) {
+        double v[4];
+        int at[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = min(e0 + u * nth, all - 1), blk = e / 36, row = e % 36 / 6, col = e % 6;
+            const int32_t* t3 = d.blk + 3 * (b0 + blk);
+            const int R = 6 * t3[1] + row, C = 6 * t3[2] + col;
+            v[u] = stored_entry(d, d.kref[st.blk0 + t3[0]], row, col);
+            at[u] = e0 + u * nth < all && R >= r0 && R < r1 && C >= c0 && C < c1
+                        ? (R - r0 + (R >= split ? gap : 0)) * ld + C - c0 : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (at[u] >= 0) T[at[u]] += v[u];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// device: factorisation
+// ---------------------------------------------------------------------------
+// One small front per workgroup.  Bound by its chain of phases, not by bandwidth or
+// the matrix cores (a leaf is 0.3 MFLOP), so the phases keep many loads in flight
+// and the next level of parallelism is the number of fronts per CU: the panel rows
+// are all that is held in LDS.
+template <int NT>
+__global__ __launch_bounds__(NT) void k_front_small(DirectDev d, const DTask* __restrict__ tasks) {
+    extern __shared__ double P[];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    const StructMeta st = d.st[task.sys];
+    constexpr int nw = NT / 64;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k = 6 * f.np, b = 6 * f.nb;
+    const int kp = (k + 15) & ~15, bp = (b + 15) & ~15, ld = kp + 2;
+    const int nt = kp >> 4, bt = bp >> 4, bs = (bt + 1) >> 1, r = lane & 15, q = lane >> 4;
+    int2* inv = reinterpret_cast<int2*>(P + (kp + bp) * ld);   // of every node, past the end: none
+    const Gather ga = make_gather(d, f, st);
+    for (int e = tid; e < f.np + f.nb + 3; e += NT) inv[e] = e < f.np + f.nb ? d.inv[f.node0 + e] : int2{-1, -1};
+    __syncthreads();
+    // contribution: 32x32 tiles of the lower triangle; the children's entries of a
+    // wavefront's first tile are requested here, to arrive behind the factorisation
+    auto gather_tile = [&](int I, int J, d4 (&t)[2][2]) {
+        const int2* bi = inv + f.np;
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int col = min(32 * J + 16 * v + r, b - 1), cn = col / 6, cc = col - 6 * cn;
+            const int2 ic = bi[cn];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = min(32 * I + 16 * u + 4 * i + q, b - 1), rn = row / 6;
+                    t[u][v][i] = gathered(ga, bi[rn], ic, row - 6 * rn, cc, col <= row);
+                }
+        }
+    };
+    int I = 0, J = wave;
+    while (J > I) {
+        J -= I + 1;
+        ++I;
+    }
+    d4 acc[2][2] = {};
+    if (ga.any && I < bs) gather_tile(I, J, acc);
+    // panel: what the children pass up (rows by wavefront, four in flight), then K
+    for (int c0 = 0; c0 < kp; c0 += 64) {
+        const int col = c0 + lane, cn = min(col, k) / 6, cc = col - 6 * cn;
+        const int2 ic = inv[cn];
+        for (int row0 = wave; row0 < kp + bp; row0 += 4 * nw) {
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int row = row0 + u * nw, R = row < kp ? row : row - kp + k;
+                const bool on = col < k && (row < kp ? row < k && col <= row : row < kp + b);
+                const int rn = on ? R / 6 : 0;
+                v[u] = ga.any ? gathered(ga, inv[rn], ic, R - 6 * rn, cc, on) : 0.0;
+                if (row == col) v[u] += 1.0;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (row0 + u * nw < kp + bp && col < kp) P[(row0 + u * nw) * ld + col] = v[u];
+        }
+    }
+    __syncthreads();
+    add_stored(d, f, st, 0, k + b, 0, k, k, kp - k, P, ld, tid, NT);
+    __syncthreads();
+    const bool ok = invert_factor(P, ld, kp, wave, nw, lane);
+    if (!ok && tid == 0) atomicOr(d.bad + task.sys, 1);
+    double* S = d.fac + st.fac + f.fac;
+    double* G = S + (int64_t)k * k;
+    for (int B = wave; B < bt; B += nw) {
+        double* X = P + (kp + 16 * B) * ld;
+        for (int K = nt - 1; K >= 0; --K) {   // descending: block K needs the blocks up to K as they were
+            const d4 v = strip_L(X, P, ld, K, lane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) X[(4 * i + q) * ld + 16 * K + r] = v[i];
+        }
+        for (int K = 0; K < nt; ++K)
+            store_tile(G + (int64_t)16 * B * k + 16 * K, k, strip_G(X, P, ld, nt, K, lane), b - 16 * B, k - 16 * K,
+                       lane);
+    }
+    write_S(P, ld, kp, k, S, (wave + nw - bt % nw) % nw, nw, lane);   // from the wavefronts with fewer strips
+    __syncthreads();
+    double* Cout = contribution(d, f, st);
+    while (I < bs) {
+        // (rows past the last tile read the tile before: their products are not stored)
+        const int i1 = 2 * I + 1 < bt ? 16 : 0, j1 = 2 * J + 1 < bt ? 16 : 0;
+        const double* x = P + (kp + 32 * I + r) * ld + q;
+        const double* y = P + (kp + 32 * J + r) * ld + q;
+#pragma unroll 4
+        for (int t = 0; t < 4 * nt; ++t) {
+            const double a0 = -x[4 * t], a1 = -x[i1 * ld + 4 * t], b0 = y[4 * t], b1 = y[j1 * ld + 4 * t];
+            acc[0][0] = mfma64(a0, b0, acc[0][0]);
+            acc[0][1] = mfma64(a0, b1, acc[0][1]);
+            acc[1][0] = mfma64(a1, b0, acc[1][0]);
+            acc[1][1] = mfma64(a1, b1, acc[1][1]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = 32 * I + 16 * u + 4 * i + q, col = 32 * J + 16 * v + r;
+                    if (row < b && col <= row) Cout[(int64_t)row * b + col] = acc[u][v][i];
+                }
+        J += nw;
+        while (J > I) {
+            J -= I + 1;
+            ++I;
+        }
+        if (I < bs) {
+            if (ga.any)
+                gather_tile(I, J, acc);
+            else
+                acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = d4{0.0, 0.0, 0.0, 0.0};
+        }
+    }
+}
+
+// offset of panel p's S (w x w, then its G) in a front's factor
+__device__ __forceinline__ int64_t panel_offset(int m, int w, int p) {
+    return (int64_t)p * w * w + (int64_t)p * m * w - (int64_t)w * w * p * (p + 1) / 2;
+}
+
+// diagonal block of panel p (gathered for the first panel): S to the factor, the
+// inverse factor to the block's place in the pivot columns
+__global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const DTask* __restrict__ tasks, int p) {
+    extern __shared__ double P[];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    if (p >= f.npan) return;
+    const StructMeta st = d.st[task.sys];
+    const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kp = (w + 15) & ~15, ld = kp + 2;
+    double* F = d.mat + st.mat + f.pan + (int64_t)c0 * k + c0;
+    const Gather ga = make_gather(d, f, st);
+    __shared__ int2 inv[DW / 6 + 1];
+    if (tid < w / 6) inv[tid] = d.inv[f.node0 + tid];
+    __syncthreads();
+    for (int c1 = 0; c1 < kp; c1 += 64) {
+        const int col = c1 + lane, cn = min(col, w - 1) / 6, cc = col - 6 * cn;
+        const int2 ic = inv[cn];
+        for (int row0 = wave; row0 < kp; row0 += 32) {
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int row = row0 + 8 * u, rn = min(row, w - 1) / 6;
+                const bool on = row < w && col <= row;
+                if (p > 0)
+                    v[u] = *(on ? F + (int64_t)row * k + col : d.zero) + (row == col && row >= w ? 1.0 : 0.0);
+                else
+                    v[u] = (row == col ? 1.0 : 0.0) + gathered(ga, inv[rn], ic, row - 6 * rn, cc, on);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (row0 + 8 * u < kp && col < kp) P[(row0 + 8 * u) * ld + col] = v[u];
+        }
+    }
+    __syncthreads();
+    if (p == 0) add_stored(d, f, st, 0, w, 0, w, w, 0, P, ld, tid, 512);
+    __syncthreads();
+    const bool ok = invert_factor(P, ld, kp, wave, 8, lane);
+    if (!ok && tid == 0) atomicOr(d.bad + task.sys, 1);
+    double* S = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p);
+    write_S(P, ld, kp, w, S, wave, 8, lane);
+    for (int row = wave; row < w; row += 8)
+        for (int col = lane; col <= row; col += 64)
+            F[(int64_t)row * k + col] = P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)];
+}
+
+// 96 rows below panel p's diagonal block: L21 = F21 L^-T (in place) and G = L21 L^-1
+__global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const DTask* __restrict__ tasks, int p) {
+    extern __shared__ double P[];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    if (p >= f.npan) return;
+    const StructMeta st = d.st[task.sys];
+    const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
+    const int r0 = c0 + w + SROWS * blockIdx.y;
+    if (r0 >= m) return;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kp = (w + 15) & ~15, ld = kp + 2, nt = kp >> 4;
+    double* F = d.mat + st.mat + f.pan + c0;   // column c0 of the pivot columns
+    double* X = P + kp * ld;
+    const int nr = min(SROWS, m - r0);
+    const Gather ga = make_gather(d, f, st);
+    __shared__ int2 ir[SROWS / 6 + 2], icol[DW / 6 + 1];
+    const int rn0 = r0 / 6;
+    if (p == 0) {
+        if (tid < SROWS / 6 + 2) ir[tid] = rn0 + tid < f.np + f.nb ? d.inv[f.node0 + rn0 + tid] : int2{-1, -1};
+        if (tid >= 64 && tid < 64 + w / 6) icol[tid - 64] = d.inv[f.node0 + tid - 64];
+        __syncthreads();
+    }
+    for (int c1 = 0; c1 < kp; c1 += 64) {
+        const int col = c1 + lane, cn = min(col, w - 1) / 6, cc = col - 6 * cn;
+        const int2 ic = p == 0 ? icol[cn] : int2{-1, -1};
+        for (int row0 = wave; row0 < SROWS; row0 += 48) {
+            double v[3], y[3];
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const int row = row0 + 16 * u, R = min(r0 + row, m - 1), rn = R / 6;
+                const bool on = row < nr && col < w;
+                if (p > 0)
+                    v[u] = *(on ? F + (int64_t)R * k + col : d.zero);
+                else
+                    v[u] = gathered(ga, ir[rn - rn0], ic, R - 6 * rn, cc, on);
+                y[u] = *(row < w && col <= row ? F + (int64_t)(c0 + row) * k + col : d.zero) +
+                       (row == col && row >= w ? 1.0 : 0.0);
+            }
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const int row = row0 + 16 * u;
+                if (col < kp) X[row * ld + col] = v[u];
+                // block (I, J) of the inverse factor goes to block row J, block column I
+                if (row < kp && col >> 4 <= row >> 4)
+                    P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)] = y[u];
+            }
+        }
+    }
+    __syncthreads();
+    if (p == 0) {
+        add_stored(d, f, st, r0, r0 + nr, 0, w, m, 0, X, ld, tid, 1024);
+        __syncthreads();
+    }
+    // 6 row tiles x nt block columns over 16 wavefronts
+    d4 v[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int e = wave + 16 * u;
+        if (e < 6 * nt) v[u] = strip_L(X + 16 * (e % 6) * ld, P, ld, e / 6, lane);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int e = wave + 16 * u, I = e % 6, J = e / 6;
+        if (e < 6 * nt) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) X[(16 * I + 4 * i + q) * ld + 16 * J + r] = v[u][i];
+            store_tile(F + (int64_t)(r0 + 16 * I) * k + 16 * J, k, v[u], nr - 16 * I, w - 16 * J, lane);
+        }
+    }
+    __syncthreads();
+    double* G = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w + (int64_t)(r0 - c0 - w) * w;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int e = wave + 16 * u, I = e % 6, J = e / 6;
+        if (e < 6 * nt)
+            store_tile(G + (int64_t)16 * I * w + 16 * J, w, strip_G(X + 16 * I * ld, P, ld, nt, J, lane), nr - 16 * I,
+                       w - 16 * J, lane);
+    }
+}
+
+// acc += X_I Y_J^T of a 64x64 tile (wavefront: 32x32 of it) over the pivot columns
+// [c0, c0 + w): rows i0.. and j0.. of the pivot columns F (m rows, row stride k)
+struct TileAcc {
+    d4 a[2][2];
+};
+__device__ __forceinline__ void tile_product(const double* __restrict__ F, int k, int m, int i0, int j0, int c0, int w,
+                                             double* X, double* Y, int tid, TileAcc& t) {
+    constexpr int LD = DKC + 2;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1);
+    // thread: pairs of columns; 16 pairs of a row, 16 rows at a time
+    const int pc = 2 * (tid & 15), pr = tid >> 4;
+    double2 xv[4], yv[4];
+    auto fetch = [&](int k0) {
+        const bool on = k0 + pc < w;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int ri = i0 + pr + 16 * u, rj = j0 + pr + 16 * u;
+            xv[u] = on && ri < m ? *reinterpret_cast<const double2*>(F + (int64_t)ri * k + c0 + k0 + pc)
+                                 : double2{0.0, 0.0};
+            yv[u] = on && rj < m ? *reinterpret_cast<const double2*>(F + (int64_t)rj * k + c0 + k0 + pc)
+                                 : double2{0.0, 0.0};
+        }
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < w; k0 += DKC) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            *reinterpret_cast<double2*>(X + (pr + 16 * u) * LD + pc) = xv[u];
+            *reinterpret_cast<double2*>(Y + (pr + 16 * u) * LD + pc) = yv[u];
+        }
+        __syncthreads();
+        if (k0 + DKC < w) fetch(k0 + DKC);   // the next chunk is on its way during this one's products
+        const double* x = X + (wi + (lane & 15)) * LD + (lane >> 4);
+        const double* y = Y + (wj + (lane & 15)) * LD + (lane >> 4);
+#pragma unroll
+        for (int s = 0; s < DKC / 4; ++s) {
+            const double a0 = x[4 * s], a1 = x[16 * LD + 4 * s], b0 = y[4 * s], b1 = y[16 * LD + 4 * s];
+            t.a[0][0] = mfma64(a0, b0, t.a[0][0]);
+            t.a[0][1] = mfma64(a0, b1, t.a[0][1]);
+            t.a[1][0] = mfma64(a1, b0, t.a[1][0]);
+            t.a[1][1] = mfma64(a1, b1, t.a[1][1]);
+        }
+    }
+}
+
+// panel p's update of the pivot columns after it (64x64 tiles; gathered here for p = 0)
+__global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const DTask* __restrict__ tasks, int p) {
+    __shared__ double sh[2 * DROWS * (DKC + 2)];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    if (p + 1 >= f.npan) return;
+    const StructMeta st = d.st[task.sys];
+    const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = 6 * f.wn, t0 = c0 + w;
+    const int i0 = t0 + DROWS * blockIdx.y, j0 = t0 + DROWS * blockIdx.z;
+    if (i0 >= m || j0 >= k || j0 > i0) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    double* F = d.mat + st.mat + f.pan;
+    TileAcc t = {};
+    tile_product(F, k, m, i0, j0, c0, w, sh, sh + DROWS * (DKC + 2), tid, t);
+    const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1);
+    const Gather ga = make_gather(d, f, st);
+    const int2* inv = d.inv + f.node0;
+    const int i1 = min(m, i0 + DROWS), j1 = min(k, j0 + DROWS);
+    constexpr int LDT = DROWS + 2;
+    static_assert(LDT * DROWS <= 2 * DROWS * (DKC + 2), "tile fits the staging buffers");
+    if (p == 0) {   // the blocks of K that enter this tile
+        __syncthreads();
+        for (int e = tid; e < LDT * DROWS; e += 256) sh[e] = 0.0;
+        __syncthreads();
+        add_stored(d, f, st, i0, i1, j0, j1, m + k, 0, sh, LDT, tid, 256);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = i0 + wi + 16 * a + 4 * i + (lane >> 4), col = j0 + wj + 16 * b + (lane & 15);
+                if (row >= i1 || col >= j1 || col > row) continue;
+                double v;
+                if (p > 0)
+                    v = F[(int64_t)row * k + col];
+                else
+                    v = (row == col ? 1.0 : 0.0) + gathered(ga, inv[row / 6], inv[col / 6], row % 6, col % 6, true) +
+                        sh[(row - i0) * LDT + col - j0];
+                F[(int64_t)row * k + col] = v - t.a[a][b][i];
+            }
+}
+
+// contribution of a large front, 64x64 tiles of the lower triangle
+__global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const DTask* __restrict__ tasks) {
+    __shared__ double sh[2 * DROWS * (DKC + 2)];
+    __shared__ int2 ir[DROWS / 6 + 3], ic[DROWS / 6 + 3];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    const StructMeta st = d.st[task.sys];
+    const int k = 6 * f.np, b = 6 * f.nb, m = k + b, nt = (b + DROWS - 1) / DROWS;
+    const int e = blockIdx.y;
+    if (e >= nt * (nt + 1) / 2) return;
+    int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
+    while (I * (I + 1) / 2 > e) --I;
+    while ((I + 1) * (I + 2) / 2 <= e) ++I;
+    const int J = e - I * (I + 1) / 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
+    const int rn0 = DROWS * I / 6, cn0 = DROWS * J / 6;
+    if (tid < DROWS / 6 + 3) {
+        ir[tid] = rn0 + tid < f.nb ? d.inv[f.node0 + f.np + rn0 + tid] : int2{-1, -1};
+        ic[tid] = cn0 + tid < f.nb ? d.inv[f.node0 + f.np + cn0 + tid] : int2{-1, -1};
+    }
+    __syncthreads();
+    const int wi = DROWS * I + 32 * (wave >> 1), wj = DROWS * J + 32 * (wave & 1);
+    const Gather ga = make_gather(d, f, st);
+    TileAcc t;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+        const int col = wj + 16 * v + r, cn = col / 6;
+        const int2 jc = ic[cn - cn0];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = wi + 16 * u + 4 * i + q, rn = row / 6;
+                t.a[u][v][i] = -gathered(ga, ir[rn - rn0], jc, row - 6 * rn, col - 6 * cn, row < b && col <= row);
+            }
+    }
+    tile_product(d.mat + st.mat + f.pan, k, m, k + DROWS * I, k + DROWS * J, 0, k, sh, sh + DROWS * (DKC + 2), tid, t);
+    double* C = contribution(d, f, st);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = wi + 16 * u + 4 * i + q, col = wj + 16 * v + r;
+                if (row < b && col <= row) C[(int64_t)row * b + col] = -t.a[u][v][i];
+            }
+}
+
+// ---------------------------------------------------------------------------
+// device: solves
+// ---------------------------------------------------------------------------
+// a front's vector v (pivots, then border; [..][NR]): right-hand side of the
+// pivots plus what its children pass up
+template <int NR>
+__device__ __forceinline__ void gather_rhs(const DirectDev& d, const FrontMeta& f, const StructMeta& st,
+                                           const double* __restrict__ r, int l0, int l1, double* dst, int tid,
+                                           int nth) {
+    // node l of the front, l0 <= l < l1
+    const double* cv[2] = {nullptr, nullptr};
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+        if (f.child[c] >= 0) {
+            const FrontMeta& g = d.fr[f.child[c]];
+            cv[c] = d.vec + (st.vec + g.vec + 6 * g.np) * NR;
+        }
+    for (int e = tid; e < (l1 - l0) * 6 * NR; e += nth) {
+        const int l = l0 + e / (6 * NR), q = e % (6 * NR);
+        const int2 a = d.inv[f.node0 + l];
+        double v = l < f.np ? r[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q] : 0.0;
+        if (a.x >= 0) v += cv[0][(int64_t)a.x * 6 * NR + q];
+        if (a.y >= 0) v += cv[1][(int64_t)a.y * 6 * NR + q];
+        dst[e] = v;
+    }
+}
+
+constexpr int FWD_ROWS = 64;   // border rows of a workgroup
+template <int NR>
+__global__ __launch_bounds__(256) void k_solve_fwd(DirectDev d, const DTask* __restrict__ tasks,
+                                                   const int32_t* __restrict__ active,
+                                                   const double* __restrict__ r, int p, int rows) {
+    __shared__ double r1[DW * NR];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    if (p >= f.npan) return;
+    bool any = false;
+#pragma unroll
+    for (int h = 0; h < NR; ++h) any |= active[task.sys * NR + h] != 0;
+    if (!any) return;
+    const StructMeta st = d.st[task.sys];
+    const int mn = f.np + f.nb, m = 6 * mn, p0 = p * f.wn, wn = min(f.wn, f.np - p0), w = 6 * wn, c0 = 6 * p0;
+    const int r0 = c0 + w + rows * blockIdx.y;
+    if (blockIdx.y > 0 && r0 >= m) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    double* v = d.vec + (st.vec + f.vec) * NR;
+    const int r1end = min(m, r0 + rows);
+    if (p == 0) {
+        gather_rhs<NR>(d, f, st, r, 0, wn, r1, tid, 256);
+        gather_rhs<NR>(d, f, st, r, r0 / 6, r1end / 6, v + (int64_t)r0 * NR, tid, 256);
+    } else {
+        for (int e = tid; e < w * NR; e += 256) r1[e] = v[(int64_t)c0 * NR + e];
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (p == 0 && blockIdx.y == 0)
+        for (int e = tid; e < w * NR; e += 256) v[e] = r1[e];
+    const double* G = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w;
+    // 16 rows per wavefront; lane: row l % 16, columns 4 (l / 16) .. + 3 of every 16
+    for (int row0 = r0 + 16 * wave; row0 < r1end; row0 += 64) {
+        const int row = row0 + (lane & 15);
+        const bool on = row < r1end;
+        const double* g = G + (int64_t)((on ? row : r0) - c0 - w) * w;
+        double acc[NR];
+#pragma unroll
+        for (int h = 0; h < NR; ++h) acc[h] = 0.0;
+        for (int j = 4 * (lane >> 4); j < w; j += 16) {
+            const double2 a = *reinterpret_cast<const double2*>(g + j);
+            const double2 c = j + 2 < w ? *reinterpret_cast<const double2*>(g + j + 2) : double2{0.0, 0.0};
+            const int j2 = j + 2 < w ? j + 2 : j;
+#pragma unroll
+            for (int h = 0; h < NR; ++h)
+                acc[h] += a.x * r1[j * NR + h] + a.y * r1[(j + 1) * NR + h] + c.x * r1[j2 * NR + h] +
+                          c.y * r1[(j2 + 1) * NR + h];
+        }
+#pragma unroll
+        for (int h = 0; h < NR; ++h) {
+            acc[h] += __shfl_xor(acc[h], 16);
+            acc[h] += __shfl_xor(acc[h], 32);
+        }
+        if (on && lane < 16) {
+#pragma unroll
+            for (int h = 0; h < NR; ++h) v[(int64_t)row * NR + h] -= acc[h];
+        }
+    }
+}
+
+// x1 = S r1 - G^T x2 for one panel per workgroup; x in node order
+template <int NR>
+__global__ __launch_bounds__(512) void k_solve_bwd(DirectDev d, const DTask* __restrict__ tasks,
+                                                   const int32_t* __restrict__ active, double* __restrict__ x, int p) {
+    extern __shared__ double P[];
+    const DTask task = tasks[blockIdx.x];
+    const FrontMeta f = d.fr[task.front];
+    if (p >= f.npan) return;
+    bool any = false;
+#pragma unroll
+    for (int h = 0; h < NR; ++h) any |= active[task.sys * NR + h] != 0;
+    if (!any) return;
+    const StructMeta st = d.st[task.sys];
+    const int mn = f.np + f.nb, m = 6 * mn, p0 = p * f.wn, wn = min(f.wn, f.np - p0), w = 6 * wn, c0 = 6 * p0;
+    const int tid = threadIdx.x, nth = blockDim.x, nb = m - c0 - w;
+    if (w == 0) return;
+    double* x2 = P;                          // [nb][NR]
+    double* r1 = P + (int64_t)nb * NR;       // [w][NR]
+    const double* v = d.vec + (st.vec + f.vec) * NR + (int64_t)c0 * NR;
+    for (int e = tid; e < nb * NR; e += nth) {
+        const int l = p0 + wn + e / (6 * NR), q = e % (6 * NR);
+        x2[e] = x[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q];
+    }
+    for (int e = tid; e < w * NR; e += nth) r1[e] = v[e];
+    __syncthreads();
+    const double* S = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p);
+    const double* G = S + (int64_t)w * w;
+    // lane pairs of columns; the groups of w / 2 threads share the rows
+    const int hw = w / 2, ng = nth / hw, g = tid / hw, j = 2 * (tid % hw);
+    double acc[2][NR];
+#pragma unroll
+    for (int h = 0; h < NR; ++h) acc[0][h] = acc[1][h] = 0.0;
+    if (g < ng) {
+        for (int i = g; i < w; i += ng) {    // S is symmetric: row i serves as column i
+            const double2 a = *reinterpret_cast<const double2*>(S + (int64_t)i * w + j);
+#pragma unroll
+            for (int h = 0; h < NR; ++h) {
+                acc[0][h] += a.x * r1[i * NR + h];
+                acc[1][h] += a.y * r1[i * NR + h];
+            }
+        }
+#pragma unroll 4
+        for (int i = g; i < nb; i += ng) {
+            const double2 a = *reinterpret_cast<const double2*>(G + (int64_t)i * w + j);
+#pragma unroll
+            for (int h = 0; h < NR; ++h) {
+                acc[0][h] -= a.x * x2[i * NR + h];
+                acc[1][h] -= a.y * x2[i * NR + h];
+            }
+        }
+    }
+    double* red = r1 + w * NR;               // [ng][w][NR]
+    if (g < ng) {
+#pragma unroll
+        for (int h = 0; h < NR; ++h) {
+            red[(int64_t)(g * w + j) * NR + h] = acc[0][h];
+            red[(int64_t)(g * w + j + 1) * NR + h] = acc[1][h];
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < w * NR; e += nth) {
+        double s = 0.0;
+        for (int q = 0; q < ng; ++q) s += red[(int64_t)q * w * NR + e];
+        const int l = p0 + e / (6 * NR), q = e % (6 * NR);
+        x[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q] = s;
+    }
+}
+
+// x64 += z for the systems still running
+template <int NR>
+__global__ __launch_bounds__(SOLVER_WG) void k_direct_add(Slices sl, const int32_t* __restrict__ slice_act,
+                                                          const double* __restrict__ z, double* __restrict__ x) {
+    const int w = slice_of_block(sl);
+    if (w < 0) return;
+    const int mask = slice_act[w];
+    const int64_t R = 6 * (int64_t)sl.row0[w] + threadIdx.x;
+    if (mask == 0 || R >= 6 * (int64_t)sl.row1[w]) return;
+#pragma unroll
+    for (int h = 0; h < NR; ++h)
+        if ((mask >> h) & 1) x[R * NR + h] += z[R * NR + h];
+}
+
+// what the host needs to know after a refinement step
+__global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, const int32_t* __restrict__ status,
+                                                       const double* __restrict__ best,
+                                                       const int32_t* __restrict__ bad, DirectReport* out) {
+    __shared__ int cnt[4];
+    __shared__ double worst[4];
+    const int tid = threadIdx.x;
+    if (tid < 4) cnt[tid] = 0;
+    __syncthreads();
+    int run = 0, stall = 0, floor = 0, nb = 0;
+    double w = 0.0;
+    for (int k = tid; k < nsys; k += 256) {
+        run += status[k] == SYS_RUNNING;
+        stall += status[k] == SYS_STALLED;
+        floor += status[k] == SYS_FLOOR;
+        w = fmax(w, best[k]);
+    }
+    for (int k = tid; k < n_struct; k += 256) nb += bad[k] != 0;
+    if (run) atomicAdd(&cnt[0], run);
+    if (stall) atomicAdd(&cnt[1], stall);
+    if (floor) atomicAdd(&cnt[2], floor);
+    if (nb) atomicAdd(&cnt[3], nb);
+    for (int o = 32; o > 0; o >>= 1) w = fmax(w, __shfl_xor(w, o));
+    if ((tid & 63) == 0) worst[tid >> 6] = w;
+    __syncthreads();
+    if (tid == 0) {
+        out->running = cnt[0];
+        out->stalled = cnt[1];
+        out->floor = cnt[2];
+        out->bad = cnt[3];
+        out->worst = fmax(fmax(worst[0], worst[1]), fmax(worst[2], worst[3]));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+static size_t small_front_lds(int np, int nb) {
+    const int kp = (6 * np + 15) & ~15, bp = (6 * nb + 15) & ~15;
+    return (size_t)(kp + bp) * (kp + 2) * 8 + (size_t)(np + nb + 3) * 8;
+}
+
+// first-fit allocation of the stored fronts of one structure: a front's matrix
+// lives from its own level to its parent's
+struct Arena {
+    std::vector<std::pair<int64_t, int64_t>> holes;   // (offset, size), by offset
+    int64_t top = 0;
+    int64_t take(int64_t n) {
+        if (n == 0) return 0;
+        n = (n + 1) & ~(int64_t)1;
+        for (size_t i = 0; i < holes.size(); ++i)
+            if (holes[i].second >= n) {
+                const int64_t at = holes[i].first;
+                holes[i].first += n;
+                holes[i].second -= n;
+                if (holes[i].second == 0) holes.erase(holes.begin() + i);
+                return at;
+            }
+        const int64_t at = top;
+        top += n;
+        return at;
+    }
+    void give(int64_t at, int64_t n) {
+        n = (n + 1) & ~(int64_t)1;
+        if (n == 0) return;
+        auto it = std::lower_bound(holes.begin(), holes.end(), std::make_pair(at, (int64_t)0));
+        it = holes.insert(it, {at, n});
+        if (it + 1 != holes.end() && it->first + it->second == (it + 1)->first) {
+            it->second += (it + 1)->second;
+            holes.erase(it + 1);
+        }
+        if (it != holes.begin() && (it - 1)->first + (it - 1)->second == it->first) {
+            (it - 1)->second += it->second;
+            holes.erase(it);
+        }
+    }
+};
+
+static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nodes, std::vector<int32_t>& rel,
+                             std::vector<int32_t>& blk, std::vector<int32_t>& blkrow, std::vector<int2>& inv) {
+    const auto& off = pl->h_node_off;
+    struct Cls {
+        int32_t fr0, n_fr, sys;
+        int64_t fac, mat, vec;
+    };
+    std::vector<Cls> cls;
+    std::map<uint64_t, std::vector<int>> by_hash;
+    D.st.resize(pl->n_sys);
+    std::vector<int32_t> lrp, lci, cls_of(pl->n_sys);
+    for (int s = 0; s < pl->n_sys; ++s) {
+        const int32_t n0 = off[s], n = off[s + 1] - n0, b0 = pl->h_rowptr[n0];
+        const int32_t nb = pl->h_rowptr[n0 + n] - b0;
+        uint64_t h = 1469598103934665603ull ^ (uint64_t)n;
+        for (int i = 0; i <= n; ++i) h = (h ^ (uint32_t)(pl->h_rowptr[n0 + i] - b0)) * 1099511628211ull;
+        for (int k = 0; k < nb; ++k) h = (h ^ (uint32_t)(pl->h_colind[b0 + k] - n0)) * 1099511628211ull;
+        int found = -1;
+        for (int c : by_hash[h]) {
+            const int t = cls[c].sys;
+            const int32_t m0 = off[t], c0 = pl->h_rowptr[m0];
+            if (off[t + 1] - m0 != n || pl->h_rowptr[m0 + n] - c0 != nb) continue;
+            bool same = true;
+            for (int i = 0; i <= n && same; ++i) same = pl->h_rowptr[n0 + i] - b0 == pl->h_rowptr[m0 + i] - c0;
+            for (int k = 0; k < nb && same; ++k) same = pl->h_colind[b0 + k] - n0 == pl->h_colind[c0 + k] - m0;
+            if (same) {
+                found = c;
+                break;
+            }
+        }
+        if (found < 0) {
+            lrp.resize(n + 1);
+            lci.resize(nb);
+            for (int i = 0; i <= n; ++i) lrp[i] = pl->h_rowptr[n0 + i] - b0;
+            for (int k = 0; k < nb; ++k) lci[k] = pl->h_colind[b0 + k] - n0;
+            FrontTree T;
+            build_fronts(n, lrp.data(), lci.data(), DLEAF, T);
+            Cls C{(int32_t)D.fr.size(), (int32_t)T.fronts.size(), s, 0, 0, 0};
+            const int32_t node_base = (int32_t)nodes.size(), blk_base = (int32_t)(blk.size() / 3);
+            for (size_t t = 0; t < T.fronts.size(); ++t) {
+                const auto& F = T.fronts[t];
+                FrontMeta M{};
+                M.np = F.np;
+                M.nb = F.nb;
+                M.node0 = node_base + F.node0;
+                M.level = F.level;
+                M.child[0] = M.child[1] = -1;
+                for (int q = T.child_ptr[t]; q < T.child_ptr[t + 1]; ++q) {
+                    if (q - T.child_ptr[t] >= 2) return JSSO_EUNSUPPORTED;
+                    M.child[q - T.child_ptr[t]] = C.fr0 + T.child[q];
+                }
+                M.blk0 = blk_base + F.blk0;
+                M.nblk = F.nblk;
+                const int k = 6 * F.np, b = 6 * F.nb, m = k + b;
+                M.small = k <= DW && small_front_lds(F.np, F.nb) <= DLDS_MAX;
+                M.npan = M.small ? 1 : std::max(1, (k + DW - 1) / DW);
+                M.wn = std::max(1, (F.np + M.npan - 1) / M.npan);
+                M.npan = std::max(1, (F.np + M.wn - 1) / M.wn);
+                M.fac = C.fac;
+                M.vec = C.vec;
+                for (int p = 0, c0 = 0; p < M.npan; ++p) {
+                    const int w = std::min(6 * M.wn, k - c0);
+                    C.fac += (int64_t)w * w + (int64_t)(m - c0 - w) * w;
+                    c0 += w;
+                }
+                C.fac = (C.fac + 1) & ~(int64_t)1;
+                C.vec += m;
+                const double kd = k, bd = b;
+                D.flops += kd * kd * kd + 2 * bd * kd * kd + bd * bd * kd;
+                D.n_levels = std::max(D.n_levels, F.level + 1);
+                D.max_m = std::max(D.max_m, m);
+                D.fr.push_back(M);
+            }
+            // storage: level by level, a child's matrix is free once its parent's level is done
+            std::vector<std::vector<int32_t>> lev;
+            for (int t = 0; t < C.n_fr; ++t) {
+                const int L = D.fr[C.fr0 + t].level;
+                if ((int)lev.size() <= L) lev.resize(L + 1);
+                lev[L].push_back(C.fr0 + t);
+            }
+            Arena A;
+            auto cb = [](const FrontMeta& M) { return (int64_t)36 * M.nb * M.nb; };
+            auto cols = [](const FrontMeta& M) { return M.small ? 0 : (int64_t)36 * (M.np + M.nb) * M.np; };
+            for (auto& L : lev) {
+                for (int t : L) {
+                    D.fr[t].mat = A.take(cb(D.fr[t]));
+                    D.fr[t].pan = A.take(cols(D.fr[t]));
+                }
+                for (int t : L) {
+                    A.give(D.fr[t].pan, cols(D.fr[t]));
+                    for (int c : D.fr[t].child)
+                        if (c >= 0) A.give(D.fr[c].mat, cb(D.fr[c]));
+                }
+            }
+            C.mat = A.top;
+            inv.resize(inv.size() + T.nodes.size(), int2{-1, -1});
+            for (size_t t = 0; t < T.fronts.size(); ++t)
+                for (int c = 0; c < 2; ++c) {
+                    const int ch = D.fr[C.fr0 + t].child[c];
+                    if (ch < 0) continue;
+                    FrontMeta& G = D.fr[ch];
+                    const int32_t* rl = T.rel.data() + T.fronts[ch - C.fr0].node0 + G.np;
+                    for (int l = 0; l < G.nb; ++l) {
+                        int2& a = inv[D.fr[C.fr0 + t].node0 + rl[l]];
+                        (c ? a.y : a.x) = l;
+                        G.npre += rl[l] < D.fr[C.fr0 + t].np;
+                    }
+                }
+            nodes.insert(nodes.end(), T.nodes.begin(), T.nodes.end());
+            rel.insert(rel.end(), T.rel.begin(), T.rel.end());
+            blk.insert(blk.end(), T.blk.begin(), T.blk.end());
+            for (int32_t q : T.blkrow) blkrow.push_back(blk_base + q);
+            found = (int)cls.size();
+            cls.push_back(C);
+            by_hash[h].push_back(found);
+        } else {
+            const Cls& C = cls[found];
+            for (int t = 0; t < C.n_fr; ++t) {
+                const double kd = 6 * D.fr[C.fr0 + t].np, bd = 6 * D.fr[C.fr0 + t].nb;
+                D.flops += kd * kd * kd + 2 * bd * kd * kd + bd * bd * kd;
+            }
+        }
+        cls_of[s] = found;
+        const Cls& C = cls[found];
+        D.st[s] = StructMeta{(int64_t)D.fac_n, (int64_t)D.mat_n, (int64_t)D.vec_n, n0, b0};
+        D.fac_n += C.fac;
+        D.mat_n += C.mat;
+        D.vec_n += C.vec;
+    }
+    D.small_tasks.resize(D.n_levels);
+    D.big_tasks.resize(D.n_levels);
+    D.small_lds.assign(D.n_levels, 0);
+    D.small_m.assign(D.n_levels, 0);
+    D.big_m.assign(D.n_levels, 0);
+    D.big_k.assign(D.n_levels, 0);
+    D.big_b.assign(D.n_levels, 0);
+    D.big_w.assign(D.n_levels, 0);
+    D.big_pan.assign(D.n_levels, 0);
+    for (int s = 0; s < pl->n_sys; ++s) {
+        const Cls& C = cls[cls_of[s]];
+        for (int t = C.fr0; t < C.fr0 + C.n_fr; ++t) {
+            const FrontMeta& M = D.fr[t];
+            if (M.np == 0 && M.nb == 0) continue;   // (joins components: nothing to do)
+            if (M.small) {
+                D.small_tasks[M.level].push_back({t, s});
+                if (M.np) D.small_m[M.level] = std::max(D.small_m[M.level], 6 * (M.np + M.nb));
+                D.small_lds[M.level] = std::max(D.small_lds[M.level], small_front_lds(M.np, M.nb));
+            } else {
+                D.big_tasks[M.level].push_back({t, s});
+                D.big_m[M.level] = std::max(D.big_m[M.level], 6 * (M.np + M.nb));
+                D.big_k[M.level] = std::max(D.big_k[M.level], 6 * M.np);
+                D.big_b[M.level] = std::max(D.big_b[M.level], 6 * M.nb);
+                D.big_w[M.level] = std::max(D.big_w[M.level], 6 * M.wn);
+                D.big_pan[M.level] = std::max(D.big_pan[M.level], M.npan);
+            }
+        }
+    }
+    return JSSO_OK;
+}
+
+template <typename T>
+static int direct_alloc(DirectState& D, T** dst, size_t count) {
+    *dst = nullptr;
+    void* q = nullptr;
+    if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();
+        return JSSO_ENOMEM;
+    }
+    D.allocs.push_back(q);
+    *dst = (T*)q;
+    return JSSO_OK;
+}
+template <typename T>
+static int direct_upload(DirectState& D, const T** dst, const std::vector<T>& src) {
+    T* p = nullptr;
+    int rc = direct_alloc(D, &p, src.size());
+    if (rc) return rc;
+    if (!src.empty()) JSSO_HIP(hipMemcpy(p, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice));
+    *dst = p;
+    return JSSO_OK;
+}
+
+void direct_destroy(Plan* pl) {
+    DirectState* D = pl->direct;
+    if (!D) return;
+    for (void* a : D->allocs) (void)hipFree(a);
+    if (D->dev.vec) (void)hipFree(D->dev.vec);
+    if (D->h_report) (void)hipHostFree(D->h_report);
+    delete D;
+    pl->direct = nullptr;
+}
+
+static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b);
+
+// builds the analysis and its storage; leaves D.usable false where the direct
+// solve is not the better choice or does not fit
+static int direct_build(Plan* pl, DirectState& D) {
+    std::vector<int32_t> nodes, rel, blk, blkrow;
+    std::vector<int2> inv;
+    if (direct_build_host(pl, D, nodes, rel, blk, blkrow, inv) != JSSO_OK) return JSSO_OK;
+    size_t free_b = 0, total_b = 0;
+    JSSO_HIP(hipMemGetInfo(&free_b, &total_b));
+    if (!direct_fits(D, free_b, total_b)) return JSSO_OK;
+    int rc = 0;
+    std::vector<DTask> tasks;
+    for (int L = 0; L < D.n_levels; ++L) {
+        D.small_off.push_back((int64_t)tasks.size());
+        tasks.insert(tasks.end(), D.small_tasks[L].begin(), D.small_tasks[L].end());
+        D.big_off.push_back((int64_t)tasks.size());
+        tasks.insert(tasks.end(), D.big_tasks[L].begin(), D.big_tasks[L].end());
+    }
+    const DTask* dt = nullptr;
+    // ||A||_2 <= 4: with identity diagonal blocks, x^T A x = sum_e x_e^T A_e x_e is at most
+    // (nodes of an element) x sum_e x_e^T diag(A_e) x_e = (nodes of an element) ||x||^2
+    std::vector<double> rho(pl->n_sys, 4.0);
+    const double* dr = nullptr;
+    if ((rc = direct_upload(D, &D.dev.fr, D.fr)) || (rc = direct_upload(D, &D.dev.st, D.st)) ||
+        (rc = direct_upload(D, &D.dev.nodes, nodes)) || (rc = direct_upload(D, &D.dev.rel, rel)) ||
+        (rc = direct_upload(D, &D.dev.inv, inv)) || (rc = direct_upload(D, &D.dev.blk, blk)) || (rc = direct_upload(D, &D.dev.blkrow, blkrow)) ||
+        (rc = direct_upload(D, &D.dev.kref, pl->h_kref)) || (rc = direct_upload(D, &dt, tasks)) ||
+        (rc = direct_upload(D, &dr, rho)) || (rc = direct_alloc(D, &D.d_report, 1)) || (rc = direct_alloc(D, &D.dev.fac, D.fac_n)) ||
+        (rc = direct_alloc(D, &D.dev.mat, D.mat_n)) || (rc = direct_alloc(D, &D.dev.bad, pl->n_sys)) || (rc = direct_upload(D, &D.dev.zero, std::vector<double>(2, 0.0)))) {
+        for (void* a : D.allocs) (void)hipFree(a);
+        D.allocs.clear();
+        return rc == JSSO_ENOMEM ? JSSO_OK : rc;
+    }
+    JSSO_HIP(hipHostMalloc((void**)&D.h_report, sizeof(DirectReport), hipHostMallocDefault));
+    D.d_tasks = const_cast<DTask*>(dt);
+    D.d_rho = const_cast<double*>(dr);
+    D.dev.A64 = pl->d_Ke64;
+    const std::pair<const void*, size_t> lds[] = {
+        {(const void*)k_front_small<1024>, DLDS_MAX}, {(const void*)k_front_small<512>, DLDS_MAX},
+        {(const void*)k_front_small<256>, DLDS_MAX},  {(const void*)k_front_diag, DW * (DW + 2) * 8},
+        {(const void*)k_front_strip, (DW + SROWS) * (DW + 2) * 8},
+        {(const void*)k_solve_bwd<1>, DLDS_MAX},      {(const void*)k_solve_bwd<2>, DLDS_MAX},
+        {(const void*)k_solve_bwd<3>, DLDS_MAX},      {(const void*)k_solve_bwd<4>, DLDS_MAX}};
+    for (const auto& l : lds)
+        JSSO_HIP(hipFuncSetAttribute(l.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.second));
+    D.usable = true;
+    return JSSO_OK;
+}
+
+static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
+    JSSO_HIP(hipMemsetAsync(D.dev.bad, 0, pl->n_sys * sizeof(int32_t), s));
+    static_assert((DW + SROWS) * (DW + 2) * 8 <= DLDS_MAX, "panel LDS");
+    for (int L = 0; L < D.n_levels; ++L) {
+        const size_t ns = D.small_tasks[L].size(), nb = D.big_tasks[L].size();
+        if (ns) {
+            const int th = D.small_lds[L] > 78 * 1024 ? 1024 : D.small_lds[L] > 52 * 1024 ? 512 : 256;
+            const DTask* t = D.d_tasks + D.small_off[L];
+            const size_t lds = D.small_lds[L];
+            if (th == 1024)
+                hipLaunchKernelGGL(k_front_small<1024>, dim3((unsigned)ns), dim3(1024), lds, s, D.dev, t);
+            else if (th == 512)
+                hipLaunchKernelGGL(k_front_small<512>, dim3((unsigned)ns), dim3(512), lds, s, D.dev, t);
+            else
+                hipLaunchKernelGGL(k_front_small<256>, dim3((unsigned)ns), dim3(256), lds, s, D.dev, t);
+        }
+        if (nb) {
+            const DTask* t = D.d_tasks + D.big_off[L];
+            const int m = D.big_m[L], strips = (m + DROWS - 1) / DROWS;
+            const int kw = (D.big_w[L] + 15) & ~15;   // widest panel
+            for (int p = 0; p < D.big_pan[L]; ++p) {
+                hipLaunchKernelGGL(k_front_diag, dim3((unsigned)nb), dim3(512), (size_t)kw * (kw + 2) * 8, s, D.dev, t,
+                                   p);
+                hipLaunchKernelGGL(k_front_strip, dim3((unsigned)nb, (m + SROWS - 1) / SROWS), dim3(1024),
+                                   (size_t)(kw + SROWS) * (kw + 2) * 8, s, D.dev, t, p);
+                if (p + 1 < D.big_pan[L])
+                    hipLaunchKernelGGL(k_front_cols, dim3((unsigned)nb, strips, (D.big_k[L] + DROWS - 1) / DROWS),
+                                       dim3(256), 0, s, D.dev, t, p);
+            }
+            const int bt = (D.big_b[L] + DROWS - 1) / DROWS;
+            if (bt)
+                hipLaunchKernelGGL(k_front_cb, dim3((unsigned)nb, bt * (bt + 1) / 2), dim3(256), 0, s, D.dev, t);
+        }
+    }
+    JSSO_HIP(hipGetLastError());
+    D.factored = true;
+    return JSSO_OK;
+}
+
+// z = M^-1 r (both in node order, [dof][NR])
+template <int NR>
+static void direct_apply(DirectState& D, const int32_t* active, const double* r, double* z, hipStream_t s) {
+    for (int L = 0; L < D.n_levels; ++L)
+        for (int big = 0; big < 2; ++big) {
+            const size_t n = big ? D.big_tasks[L].size() : D.small_tasks[L].size();
+            if (!n) continue;
+            const DTask* t = D.d_tasks + (big ? D.big_off[L] : D.small_off[L]);
+            const int rows = big ? FWD_ROWS * 3 : 8192;   // a multiple of 6
+            const int ny = big ? std::max(1, (D.big_m[L] + rows - 1) / rows) : 1;
+            for (int p = 0; p < (big ? D.big_pan[L] : 1); ++p)
+                hipLaunchKernelGGL((k_solve_fwd<NR>), dim3((unsigned)n, ny), dim3(256), 0, s, D.dev, t, active, r, p,
+                                   rows / 6 * 6);
+        }
+    for (int L = D.n_levels - 1; L >= 0; --L)
+        for (int big = 0; big < 2; ++big) {
+            const size_t n = big ? D.big_tasks[L].size() : D.small_tasks[L].size();
+            if (!n) continue;
+            const DTask* t = D.d_tasks + (big ? D.big_off[L] : D.small_off[L]);
+            const int th = big ? 512 : 256;
+            const int m = big ? D.big_m[L] : D.small_m[L];
+            const size_t lds = ((size_t)m + DW + 2 * th) * NR * 8;
+            for (int p = (big ? D.big_pan[L] : 1) - 1; p >= 0; --p)
+                hipLaunchKernelGGL((k_solve_bwd<NR>), dim3((unsigned)n), dim3(th), lds, s, D.dev, t, active, z, p);
+        }
+}
+
+// Waves per slice (1, 2 or 4) of the residual kernel, timed on the live plan right
+// after the start-up kernels: x is zero, so the residual it writes is the one that
+// is there already.
+template <int NR>
+static int tune_residual(Plan* pl, const Workspace& w, const Slices& sl, double* r, hipStream_t s, int32_t& out) {
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    JSSO_HIP(hipEventCreate(&e0));
+    JSSO_HIP(hipEventCreate(&e1));
+    float best = 0.f;
+    int pick = 1;
+    auto run = [&](auto W, bool first) -> int {
+        constexpr int WP = decltype(W)::value;
+        if constexpr (WpsFits<double, NR, WP>::value) {
+            float ms = 0.f;
+            for (int rep = 0; rep < 4; ++rep) {
+                if (rep == 1) JSSO_HIP(hipEventRecord(e0, s));
+                hipLaunchKernelGGL((k_replace<double, NR, WP>), slice_grid(sl), dim3(64 * WP), 0, s, sl, w.P, w.st,
+                                   (const double*)pl->d_Ke64, (const double*)w.b64, (const double*)w.x64, r);
+            }
+            JSSO_HIP(hipEventRecord(e1, s));
+            JSSO_HIP(hipEventSynchronize(e1));
+            JSSO_HIP(hipEventElapsedTime(&ms, e0, e1));
+            if (first || ms < best) {
+                best = ms;
+                pick = WP;
+            }
+        }
+        return JSSO_OK;
+    };
+    int rc = run(std::integral_constant<int, 1>(), true);
+    if (!rc) rc = run(std::integral_constant<int, 2>(), false);
+    if (!rc) rc = run(std::integral_constant<int, 4>(), false);
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    JSSO_HIP(hipGetLastError());
+    out = pick;
+    return rc;
+}
+
+// u = K^-1 f by the factorisation and refinement; done = false (and nothing said
+// about u) where a pivot is not positive or a system does not reach its tolerance
+// or its attainable accuracy
+template <int NR>
+static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, double tol, int maxit, int slot,
+                      jsso_info* info, hipStream_t s, bool& done) {
+    Workspace w;
+    int rc = get_workspace(pl, NR, w);
+    if (rc) return rc;
+    if (D.vec_bytes < D.vec_n * NR * 8) {
+        if (D.dev.vec) JSSO_HIP(hipFree(D.dev.vec));
+        D.dev.vec = nullptr;
+        D.vec_bytes = 0;
+        if (hipMalloc((void**)&D.dev.vec, D.vec_n * NR * 8) != hipSuccess) {
+            (void)hipGetLastError();
+            return JSSO_OK;
+        }
+        D.vec_bytes = D.vec_n * NR * 8;
+    }
+    const int nsys = pl->n_sys * NR;
+    const Slices sl = make_slices(pl, 0, pl->n_wg);
+    const dim3 g = slice_grid(sl);
+    double* r = (double*)w.r[0];
+    double* z = (double*)w.p;
+    hipLaunchKernelGGL((k_init<double, NR>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f, w.b64,
+                       w.x64, w.xbest, (double*)w.xlo, r, z);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 0, tol, 0, 0,
+                       (const double*)nullptr, 0.0, 0);
+    int32_t& wps = pl->direct_wps[slot][NR];
+    if (wps <= 0 && (rc = tune_residual<NR>(pl, w, sl, r, s, wps))) return rc;
+    if (!D.factored) {
+        std::pair<hipEvent_t, hipEvent_t>* ev = nullptr;
+        timing_begin_slot(s, ev, JSSO_TIMING_SETUP);
+        if ((rc = direct_factor(pl, D, s))) return rc;
+        timing_end(s, ev);
+    }
+    const int64_t nr = 6 * (int64_t)pl->n_nodes;
+    for (int it = 1; it <= std::min(maxit, DIRECT_STEPS); ++it) {
+        direct_apply<NR>(D, w.st.active, r, z, s);
+        hipLaunchKernelGGL((k_direct_add<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.slice_act,
+                           (const double*)z, w.x64);
+        auto residual = [&](auto W) {
+            constexpr int WP = decltype(W)::value;
+            hipLaunchKernelGGL((k_replace<double, NR, WP>), g, dim3(64 * WP), 0, s, sl, w.P, w.st,
+                               (const double*)pl->d_Ke64, (const double*)w.b64, (const double*)w.x64, r);
+        };
+        if (WpsFits<double, NR, 4>::value && wps >= 4)
+            residual(std::integral_constant<int, WpsFits<double, NR, 4>::value ? 4 : 1>());
+        else if (WpsFits<double, NR, 2>::value && wps >= 2)
+            residual(std::integral_constant<int, WpsFits<double, NR, 2>::value ? 2 : 1>());
+        else
+            residual(std::integral_constant<int, 1>());
+        // (a step that gains less than 10% ends a system at once: near its attainable
+        // accuracy as converged there, else as stalled)
+        hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 1, tol, 1, 2,
+                           (const double*)D.d_rho, DIRECT_FLOOR_FACTOR, 0);
+        hipLaunchKernelGGL((k_save<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.save,
+                           (const double*)w.x64, w.xbest);
+        hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys, (const int32_t*)w.st.status,
+                           (const double*)w.st.best, (const int32_t*)D.dev.bad, D.d_report);
+        // (final unless a system is still running)
+        hipLaunchKernelGGL((k_unscale<NR>), dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, pl->n_nodes,
+                           pl->d_Linv, (const double*)w.xbest, u);
+        JSSO_HIP(hipGetLastError());
+        JSSO_HIP(hipMemcpyAsync(D.h_report, D.d_report, sizeof(DirectReport), hipMemcpyDeviceToHost, s));
+        JSSO_HIP(hipStreamSynchronize(s));
+        const DirectReport& R = *D.h_report;
+        if (R.bad || R.stalled) return JSSO_OK;
+        if (R.running) continue;
+        done = true;
+        if (info) {
+            *info = jsso_info{};
+            info->iterations = info->replacements = it;
+            info->converged = info->n_systems = nsys;
+            info->rel_residual = R.worst;
+            info->at_floor = R.floor;
+            info->waves_per_slice = wps;
+        }
+        timing_collect();
+        return JSSO_OK;
+    }
+    return JSSO_OK;
+}
+
+// The direct solve is taken where its fronts stay small: fill and operations grow
+// with the largest front (m rows: m^2 storage, m^3 operations), while the
+// AMG-preconditioned CG grows with the number of nodes.  One shell of n x n quads
+// has m ~ 9 n: measured per solve with its set-up, 40x40 (m = 366) 1.06 against
+// 3.87 ms, 100x100 (m = 912) 2.5 against 3.0 ms, 200x200 (m = 1812) 6.6 against
+// 6.5 ms; batches gain more (64 SIMP shells of 100x100: 35 against 56 ms), since
+// they fill the chip on every tree level.  It needs its storage too: up to an
+// eighth of the card, and half of what is free.
+static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b) {
+    const size_t need = (D.fac_n + D.mat_n) * 8;
+    return D.max_m <= DIRECT_MAX_M && need <= total_b / 8 && need <= free_b / 2;
+}
+
+int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
+                 hipStream_t s, bool& done) {
+    done = false;
+    if (!(nrhs >= 1 && nrhs <= 4)) return JSSO_OK;
+    if (!pl->direct) {
+        pl->direct = new (std::nothrow) DirectState();
+        if (!pl->direct) return JSSO_OK;
+        int rc = JSSO_OK;
+        try {
+            rc = direct_build(pl, *pl->direct);
+        } catch (const std::bad_alloc&) {   // (host memory: the iterative solve needs less)
+            pl->direct->usable = false;
+        }
+        if (rc) {
+            direct_destroy(pl);
+            return rc;
+        }
+    }
+    DirectState& D = *pl->direct;
+    if (!D.usable) return JSSO_OK;
+    if (!pl->direct_valid) D.factored = false;
+    pl->direct_valid = true;
+    switch (nrhs) {
+        case 1: return run_direct<1>(pl, D, f, u, tol, maxit, slot, info, s, done);
+        case 2: return run_direct<2>(pl, D, f, u, tol, maxit, slot, info, s, done);
+        case 3: return run_direct<3>(pl, D, f, u, tol, maxit, slot, info, s, done);
+        default: return run_direct<4>(pl, D, f, u, tol, maxit, slot, info, s, done);
+    }
+}
+
+}  // namespace jsso

@@ -95,6 +95,7 @@ struct CgGraph {
 };
 
 struct AmgState;   // smoothed-aggregation multigrid hierarchy (jsso_amg.hip)
+struct DirectState;   // multifrontal factorisation (jsso_direct.hip)
 
 struct Plan {
     // sizes
@@ -163,6 +164,10 @@ struct Plan {
     double* d_crds = nullptr;     // node coordinates of the current assembly (for the AMG null space)
     // preconditioner of the batched solves (JSSO_PC_*) and the AMG hierarchy
     int32_t precond = JSSO_PC_AMG;
+    bool precond_set = false;     // chosen by the caller (jsso_plan_set_preconditioner, jsso_plan_amg_reuse)
+    DirectState* direct = nullptr;
+    int32_t direct_wps[3][9] = {};   // waves per slice of the direct solve's residual kernel, as amg_wps
+    bool direct_valid = false;    // the factorisation matches the current assembly
     AmgState* amg = nullptr;
     bool amg_valid = false;       // the AMG numeric set-up matches the current assembly
     int32_t amg_reuse = 0;        // jsso_plan_amg_reuse mode
@@ -230,6 +235,9 @@ int launch_defect_residual(Plan* p, const double* K, const double* f, const doub
 int launch_axpy(int64_t n, const double* x, double* y, hipStream_t s);
 int amg_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
               hipStream_t s);
+int direct_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
+                 hipStream_t s, bool& done);
+void direct_destroy(Plan* p);
 int amg_levels(Plan* p, int32_t* h_nodes, int32_t cap, int32_t* h_levels);
 void amg_destroy(Plan* p);
 int dense_solve(Plan* p, const double* K, const double* f, double* u, int nrhs, bool lu, bool transpose,

@@ -977,6 +977,11 @@ int solve_batched(Plan* p, const double* f, double* u, int nrhs, int slot, doubl
                   jsso_info* info, hipStream_t s) {
     int rc = check_status(p, s);
     if (rc) return rc;
+    if (!p->precond_set) {   // the caller left the choice: directly where that is cheaper
+        bool done = false;
+        rc = direct_solve(p, f, u, nrhs, slot, tol, maxit, info, s, done);
+        if (rc || done) return rc;
+    }
     if (p->precond == JSSO_PC_AMG) return amg_solve(p, f, u, nrhs, slot, tol, maxit, info, s);
     if (slot == PS_F32) return dispatch_nr<float, float>(p, f, u, nrhs, tol, maxit, replace_interval(true), info, s);
     if (slot == PS_F32_V64)

@@ -49,6 +49,7 @@ class FEPlan:
         nat.check(L.jsso_plan_sizes(self._h, nat.ptr(sizes)))
         self.nnzb = int(sizes[1])
         self.preconditioner = "amg"   # the library's default
+        self._pc_chosen = False       # by the caller: until then the library may solve directly
         self.last_info = None
         self._assembled_key = None
 
@@ -117,6 +118,7 @@ class FEPlan:
             raise ValueError(f"unknown preconditioner {name!r} ({sorted(PRECONDITIONERS)})")
         nat.check(nat.load_library().jsso_plan_set_preconditioner(self._h, PRECONDITIONERS[name]))
         self.preconditioner = name
+        self._pc_chosen = True
 
     def element_tuning(self, set_epw: int = -1) -> int:
         """MITC-4 elements per workgroup of the assembly kernel (4, 8 or 16): 0 until
@@ -149,7 +151,7 @@ class FEPlan:
         """Solve K u = f (K^T u = f with ``transpose``; u = 0 at supports).  f: (ndof,)
         or (ndof, nrhs) FP64 on the device."""
         L = nat.lib()
-        if preconditioner is not None and preconditioner != self.preconditioner:
+        if preconditioner is not None and (preconditioner != self.preconditioner or not self._pc_chosen):
             self.set_preconditioner(preconditioner)
         f = _dev64(f)
         vec = f.dim() == 1
