@@ -225,7 +225,11 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
  * (same arguments and results as jsso_solve; a symmetric plan is solved as by
  * jsso_solve).
  *   <- the custom VJP's solve with K_aug^T  JaxSSO/solver.py:236
- * Non-symmetric plans (both entry points): the dense LU (jsso_dense_solve) up to
+ * Non-symmetric plans (both entry points): without members parallel to global Y,
+ * and where the direct solve is taken (see JSSO_PC_AMG), refinement with the
+ * factorisation of S = (K + K^T)/2 to the attainable accuracy (at least tol;
+ * h_info->iterations and replacements count its steps).  Otherwise, and where that
+ * does not converge, the dense LU (jsso_dense_solve) up to
  * 16 384 DOF or when members parallel to global Y are present; above that a
  * defect correction: r = f - K u (K^T u), S du = r with S = (K + K^T)/2 (the
  * assembly writes S into the solver copies of such a plan; inner batched solve
@@ -236,7 +240,7 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
 int jsso_solve_transpose(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs, int32_t precision,
                          double tol, int32_t maxit, jsso_info* h_info, void* stream);
 /* Route of non-symmetric plans: mode 0 automatic (above), 1 always the dense LU,
- * 2 always the defect correction (JSSO_EUNSUPPORTED with members parallel to
+ * 2 always a correction with S (direct or iterative) (JSSO_EUNSUPPORTED with members parallel to
  * global Y, whose transformation, element.py:92-94, leaves S indefinite);
  * -1 only reads it.  *h_mode (may be NULL) receives the mode in force. */
 int jsso_plan_nonsymmetric_route(jsso_plan* plan, int32_t mode, int32_t* h_mode);

@@ -579,20 +579,32 @@ int jsso_assemble(jsso_plan* plan, const double* d_crds, const double* d_prop_be
 
 // K u = f (or K^T u = f) for a plan whose K is not symmetric.  The reference
 // factorises K_aug (and K_aug^T for the adjoint) with SuperLU
-// (solver.py:195-209,236).  Here: the dense LU (jsso_dense_solve) up to
-// NONSYM_DENSE_MAX_DOF DOF or with members parallel to global Y; otherwise a
-// defect correction preconditioned by the batched solver on the symmetric part
-// S = (K + K^T)/2 (which the assembly writes into the solver copies of such a
-// plan):  r = f - op(K) u;  S du = r (inner AMG-CG, relative tolerance 1e-3);
-// u += du, until max ||r|| / ||f|| <= tol over the systems.  It converges when
-// the spectral radius of I - S^-1 K is below 1: 0.04-0.14 for MITC-4 shells with
-// kx_mod/ky_mod from 1.2/0.8 to 2/0.5; the transformation of Y-parallel members
-// leaves S indefinite, so those plans stay on the dense LU.
+// (solver.py:195-209,236).  Here, in this order:
+//  - refinement with the factorisation of the symmetric part S = (K + K^T)/2 (which
+//    the assembly writes into the solver copies of such a plan), to the attainable
+//    accuracy, where the direct solve is taken at all (direct_defect) and no member
+//    is parallel to global Y;
+//  - the dense LU (jsso_dense_solve) up to NONSYM_DENSE_MAX_DOF DOF or with members
+//    parallel to global Y;
+//  - a defect correction preconditioned by the batched solver on S:
+//    r = f - op(K) u;  S du = r (inner AMG-CG, relative tolerance 1e-3);  u += du,
+//    until max ||r|| / ||f|| <= tol over the systems.
+// Both corrections converge when the spectral radius of I - S^-1 K is below 1:
+// 0.04-0.14 for MITC-4 shells with kx_mod/ky_mod from 1.2/0.8 to 2/0.5; the
+// transformation of Y-parallel members leaves S indefinite, so those plans stay on
+// the dense LU.  One evaluation of a 20x20 shell (2 646 DOF, kx/ky 1.2/0.8; state
+// and adjoint) took 100 ms by the LU (a launch per column and pivot search) and takes
+// 3.4 ms by the refinement.
 static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs, int precision, double tol,
                               int maxit, jsso_info* h_info, bool transpose, hipStream_t s, int32_t status) {
     int rc = launch_full_blocks(p, s);
     if (rc) return rc;
     const int64_t ndof = 6 * (int64_t)p->n_nodes;
+    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set) {
+        bool done = false;
+        rc = direct_defect(p, p->d_K, d_f, d_u, nrhs, transpose, tol, maxit, h_info, s, done);
+        if (rc || done) return rc;
+    }
     const bool dense = p->nonsym_route == 1 ||
                        (p->nonsym_route == 0 && ((status & STATUS_Y_BEAM) || ndof <= NONSYM_DENSE_MAX_DOF));
     if (dense) {

@@ -49,6 +49,7 @@ constexpr int DLEAF = 12;                 // nodes eliminated whole at the tree'
 constexpr int DLDS_MAX = 156 * 1024;      // dynamic LDS of a small front
 constexpr int DIRECT_MAX_M = 1500;        // largest front (direct_fits)
 constexpr int DIRECT_STEPS = 6;           // refinement steps, at most
+constexpr int DEFECT_STEPS = 40;          // of a K that is not symmetric
 constexpr double DIRECT_FLOOR_FACTOR = 16.0;   // attainable accuracy: 16 eps (||A|| ||x|| + ||b||), as the AMG solve
 constexpr int DKC = 32;                   // pivot columns staged at a time by the tile kernels
 
@@ -1014,6 +1015,124 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
 }
 
 // ---------------------------------------------------------------------------
+// device: refinement with a K that is not symmetric (the factorisation is of its
+// symmetric part)
+// ---------------------------------------------------------------------------
+// r = f - op(K) u on the free DOFs, scaled to L^-1 r for the factorisation; per-slice
+// partial sums of <r, r>.  Thread = scalar row of the slice, a row's blocks in column
+// order; op(K) = K^T reads column rr of the block at the transposed position.
+template <int NR>
+__global__ __launch_bounds__(SOLVER_WG) void k_defect(Slices sl, Partials P, SysState st,
+                                                      const int32_t* __restrict__ rowptr,
+                                                      const int32_t* __restrict__ colind,
+                                                      const int32_t* __restrict__ tpos,
+                                                      const uint8_t* __restrict__ fixed,
+                                                      const double* __restrict__ K, const double* __restrict__ Linv,
+                                                      const double* __restrict__ f, const double* __restrict__ u,
+                                                      double* __restrict__ rs) {
+    __shared__ double lds[NWAVES * NR], rl[SOLVER_WG][NR];
+    const int w = slice_of_block(sl);
+    if (w < 0 || st.slice_act[w] == 0) return;
+    const int tid = threadIdx.x;
+    const int64_t R = 6 * (int64_t)sl.row0[w] + tid;
+    const bool on = R < 6 * (int64_t)sl.row1[w];
+    double v[NR];
+#pragma unroll
+    for (int h = 0; h < NR; ++h) v[h] = 0.0;
+    const int i = (int)(R / 6), rr = (int)(R % 6);
+    if (on && !fixed[R]) {
+        double acc[NR];
+#pragma unroll
+        for (int h = 0; h < NR; ++h) acc[h] = 0.0;
+        for (int k = rowptr[i]; k < rowptr[i + 1]; ++k) {
+            const int64_t j = colind[k];
+            const double* b = tpos ? K + (int64_t)tpos[k] * 36 + rr : K + (int64_t)k * 36 + rr * 6;
+            const int step = tpos ? 6 : 1;
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+#pragma unroll
+                for (int h = 0; h < NR; ++h) acc[h] += b[c * step] * u[(6 * j + c) * NR + h];
+        }
+#pragma unroll
+        for (int h = 0; h < NR; ++h) v[h] = f[R * NR + h] - acc[h];
+    }
+#pragma unroll
+    for (int h = 0; h < NR; ++h) rl[tid][h] = v[h];
+    __syncthreads();
+    if (on) {
+#pragma unroll
+        for (int h = 0; h < NR; ++h) {
+            double s = 0.0;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) s += Linv[(int64_t)i * 36 + rr * 6 + c] * rl[tid - rr + c][h];
+            rs[R * NR + h] = s;
+            v[h] *= v[h];
+        }
+    }
+    write_partials<NR, NWAVES>(v, lds, P.t, w);
+}
+
+// A system ends where its residual ||r|| / ||f|| no longer halves: at its attainable
+// accuracy if that is within tol, else without convergence.  One wavefront per
+// structure; step 0 takes ||f|| from u = 0.
+template <int NR>
+__global__ __launch_bounds__(64) void k_defect_decide(Slices sl, Partials P, SysState st, int step, double tol) {
+    const int sys = blockIdx.x, lane = threadIdx.x;
+    const int s0 = sl.sys_off[sys], s1 = sl.sys_off[sys + 1];
+    double t[NR];
+#pragma unroll
+    for (int h = 0; h < NR; ++h) t[h] = 0.0;
+    for (int w = s0 + lane; w < s1; w += 64)
+#pragma unroll
+        for (int h = 0; h < NR; ++h) t[h] += P.t[(int64_t)w * NR + h];
+    int mask = 0;
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+        const double rr = wave_sum(t[h]);
+        const int k = sys * NR + h;
+        if (!st.active[k]) continue;
+        const double ff = step == 0 ? rr : st.bnorm2[k], prev = st.relres[k];
+        const double rel = step == 0 ? (rr > 0.0 ? 1.0 : 0.0) : sqrt(rr / ff);
+        int active = rel > 0.0 ? 1 : 0, status = active ? SYS_RUNNING : SYS_CONVERGED;
+        if (step > 0 && active && !(rel <= 0.5 * prev)) {
+            active = 0;
+            status = rel <= tol ? SYS_CONVERGED : SYS_STALLED;
+        }
+        if (lane == 0) {
+            if (step == 0) st.bnorm2[k] = ff;
+            st.relres[k] = rel;
+            st.best[k] = rel;
+            st.active[k] = active;
+            st.status[k] = status;
+        }
+        mask |= active << h;
+    }
+    for (int w = s0 + lane; w < s1; w += 64) st.slice_act[w] = mask;
+}
+
+// u += L^-T z for the systems still running
+template <int NR>
+__global__ __launch_bounds__(SOLVER_WG) void k_defect_add(Slices sl, const int32_t* __restrict__ slice_act,
+                                                          const double* __restrict__ Linv,
+                                                          const double* __restrict__ z, double* __restrict__ u) {
+    const int w = slice_of_block(sl);
+    if (w < 0) return;
+    const int mask = slice_act[w];
+    const int64_t R = 6 * (int64_t)sl.row0[w] + threadIdx.x;
+    if (mask == 0 || R >= 6 * (int64_t)sl.row1[w]) return;
+    const int64_t i = R / 6;
+    const int r = (int)(R % 6);
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+        if (!((mask >> h) & 1)) continue;
+        double s = 0.0;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) s += Linv[i * 36 + c * 6 + r] * z[(6 * i + c) * NR + h];
+        u[R * NR + h] += s;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
 static size_t small_front_lds(int np, int nb) {
@@ -1365,6 +1484,31 @@ static void direct_apply(DirectState& D, const int32_t* active, const double* r,
         }
 }
 
+static int direct_vectors(DirectState& D, int nrhs, bool& have) {
+    const size_t need = D.vec_n * nrhs * 8;
+    have = true;
+    if (D.vec_bytes >= need) return JSSO_OK;
+    if (D.dev.vec) JSSO_HIP(hipFree(D.dev.vec));
+    D.dev.vec = nullptr;
+    D.vec_bytes = 0;
+    if (hipMalloc((void**)&D.dev.vec, need) != hipSuccess) {
+        (void)hipGetLastError();
+        have = false;
+        return JSSO_OK;
+    }
+    D.vec_bytes = need;
+    return JSSO_OK;
+}
+
+static int ensure_factor(Plan* pl, DirectState& D, hipStream_t s) {
+    if (D.factored) return JSSO_OK;
+    std::pair<hipEvent_t, hipEvent_t>* ev = nullptr;
+    timing_begin_slot(s, ev, JSSO_TIMING_SETUP);
+    const int rc = direct_factor(pl, D, s);
+    timing_end(s, ev);
+    return rc;
+}
+
 // Waves per slice (1, 2 or 4) of the residual kernel, timed on the live plan right
 // after the start-up kernels: x is zero, so the residual it writes is the one that
 // is there already.
@@ -1413,16 +1557,8 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
     Workspace w;
     int rc = get_workspace(pl, NR, w);
     if (rc) return rc;
-    if (D.vec_bytes < D.vec_n * NR * 8) {
-        if (D.dev.vec) JSSO_HIP(hipFree(D.dev.vec));
-        D.dev.vec = nullptr;
-        D.vec_bytes = 0;
-        if (hipMalloc((void**)&D.dev.vec, D.vec_n * NR * 8) != hipSuccess) {
-            (void)hipGetLastError();
-            return JSSO_OK;
-        }
-        D.vec_bytes = D.vec_n * NR * 8;
-    }
+    bool have = false;
+    if ((rc = direct_vectors(D, NR, have)) || !have) return rc;
     const int nsys = pl->n_sys * NR;
     const Slices sl = make_slices(pl, 0, pl->n_wg);
     const dim3 g = slice_grid(sl);
@@ -1434,12 +1570,7 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
                        (const double*)nullptr, 0.0, 0);
     int32_t& wps = pl->direct_wps[slot][NR];
     if (wps <= 0 && (rc = tune_residual<NR>(pl, w, sl, r, s, wps))) return rc;
-    if (!D.factored) {
-        std::pair<hipEvent_t, hipEvent_t>* ev = nullptr;
-        timing_begin_slot(s, ev, JSSO_TIMING_SETUP);
-        if ((rc = direct_factor(pl, D, s))) return rc;
-        timing_end(s, ev);
-    }
+    if ((rc = ensure_factor(pl, D, s))) return rc;
     const int64_t nr = 6 * (int64_t)pl->n_nodes;
     for (int it = 1; it <= std::min(maxit, DIRECT_STEPS); ++it) {
         direct_apply<NR>(D, w.st.active, r, z, s);
@@ -1501,9 +1632,9 @@ static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b) {
     return D.max_m <= DIRECT_MAX_M && need <= total_b / 8 && need <= free_b / 2;
 }
 
-int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
-                 hipStream_t s, bool& done) {
-    done = false;
+// the plan's analysis, built at its first use; nullptr where the direct solve is not taken
+static int direct_state(Plan* pl, int nrhs, DirectState** out) {
+    *out = nullptr;
     if (!(nrhs >= 1 && nrhs <= 4)) return JSSO_OK;
     if (!pl->direct) {
         pl->direct = new (std::nothrow) DirectState();
@@ -1523,11 +1654,91 @@ int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, doubl
     if (!D.usable) return JSSO_OK;
     if (!pl->direct_valid) D.factored = false;
     pl->direct_valid = true;
+    *out = &D;
+    return JSSO_OK;
+}
+
+int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
+                 hipStream_t s, bool& done) {
+    done = false;
+    DirectState* D = nullptr;
+    int rc = direct_state(pl, nrhs, &D);
+    if (rc || !D) return rc;
     switch (nrhs) {
-        case 1: return run_direct<1>(pl, D, f, u, tol, maxit, slot, info, s, done);
-        case 2: return run_direct<2>(pl, D, f, u, tol, maxit, slot, info, s, done);
-        case 3: return run_direct<3>(pl, D, f, u, tol, maxit, slot, info, s, done);
-        default: return run_direct<4>(pl, D, f, u, tol, maxit, slot, info, s, done);
+        case 1: return run_direct<1>(pl, *D, f, u, tol, maxit, slot, info, s, done);
+        case 2: return run_direct<2>(pl, *D, f, u, tol, maxit, slot, info, s, done);
+        case 3: return run_direct<3>(pl, *D, f, u, tol, maxit, slot, info, s, done);
+        default: return run_direct<4>(pl, *D, f, u, tol, maxit, slot, info, s, done);
+    }
+}
+
+template <int NR>
+static int run_defect(Plan* pl, DirectState& D, const double* K, const double* f, double* u, bool transpose,
+                      double tol, int maxit, jsso_info* info, hipStream_t s, bool& done) {
+    Workspace w;
+    int rc = get_workspace(pl, NR, w);
+    if (rc) return rc;
+    bool have = false;
+    if ((rc = direct_vectors(D, NR, have)) || !have) return rc;
+    const int nsys = pl->n_sys * NR;
+    const Slices sl = make_slices(pl, 0, pl->n_wg);
+    const dim3 g = slice_grid(sl);
+    double *r = (double*)w.r[0], *z = (double*)w.p;
+    // activity from L^-1 f
+    hipLaunchKernelGGL((k_init<double, NR>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f, w.b64,
+                       w.x64, w.xbest, (double*)w.xlo, r, z);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 0, tol, 0, 0,
+                       (const double*)nullptr, 0.0, 0);
+    JSSO_HIP(hipMemsetAsync(u, 0, 6 * (size_t)pl->n_nodes * NR * sizeof(double), s));
+    if ((rc = ensure_factor(pl, D, s))) return rc;
+    const int most = std::min(maxit, DEFECT_STEPS);
+    for (int it = 0; it <= most; ++it) {
+        hipLaunchKernelGGL((k_defect<NR>), g, dim3(SOLVER_WG), 0, s, sl, w.P, w.st, pl->d_rowptr, pl->d_colind,
+                           transpose ? (const int32_t*)pl->d_tpos : (const int32_t*)nullptr, pl->d_fixed, K,
+                           pl->d_Linv, f, (const double*)u, r);
+        hipLaunchKernelGGL((k_defect_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, it, tol);
+        // (the host looks from the fourth step on, at every second one: a gain of 30 a
+        // step, the best seen, needs five)
+        if (it == most || (it >= 4 && it % 2 == 0)) {
+            hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys,
+                               (const int32_t*)w.st.status, (const double*)w.st.best, (const int32_t*)D.dev.bad,
+                               D.d_report);
+            JSSO_HIP(hipGetLastError());
+            JSSO_HIP(hipMemcpyAsync(D.h_report, D.d_report, sizeof(DirectReport), hipMemcpyDeviceToHost, s));
+            JSSO_HIP(hipStreamSynchronize(s));
+            const DirectReport& R = *D.h_report;
+            if (R.bad || R.stalled) return JSSO_OK;
+            if (!R.running) {
+                done = true;
+                if (info) {
+                    *info = jsso_info{};
+                    info->iterations = info->replacements = it;
+                    info->converged = info->n_systems = nsys;
+                    info->rel_residual = R.worst;
+                }
+                return JSSO_OK;
+            }
+        }
+        direct_apply<NR>(D, w.st.active, r, z, s);
+        hipLaunchKernelGGL((k_defect_add<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.slice_act,
+                           pl->d_Linv, (const double*)z, u);
+    }
+    return JSSO_OK;
+}
+
+// op(K) u = f for a K that is not symmetric (block CSR values K), by refinement with
+// the factorisation of S = (K + K^T) / 2; done = false where it does not converge
+int direct_defect(Plan* pl, const double* K, const double* f, double* u, int nrhs, bool transpose, double tol,
+                  int maxit, jsso_info* info, hipStream_t s, bool& done) {
+    done = false;
+    DirectState* D = nullptr;
+    int rc = direct_state(pl, nrhs, &D);
+    if (rc || !D) return rc;
+    switch (nrhs) {
+        case 1: return run_defect<1>(pl, *D, K, f, u, transpose, tol, maxit, info, s, done);
+        case 2: return run_defect<2>(pl, *D, K, f, u, transpose, tol, maxit, info, s, done);
+        case 3: return run_defect<3>(pl, *D, K, f, u, transpose, tol, maxit, info, s, done);
+        default: return run_defect<4>(pl, *D, K, f, u, transpose, tol, maxit, info, s, done);
     }
 }
 

@@ -237,6 +237,8 @@ int amg_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double to
               hipStream_t s);
 int direct_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
                  hipStream_t s, bool& done);
+int direct_defect(Plan* p, const double* K, const double* f, double* u, int nrhs, bool transpose, double tol,
+                  int maxit, jsso_info* info, hipStream_t s, bool& done);
 void direct_destroy(Plan* p);
 int amg_levels(Plan* p, int32_t* h_nodes, int32_t cap, int32_t* h_levels);
 void amg_destroy(Plan* p);

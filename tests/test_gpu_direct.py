@@ -123,3 +123,41 @@ def test_direct_solve_repeats_itself_and_hands_over_what_it_does_not_take():
     b.plan.amg_reuse(2)
     u1 = b.solve()
     assert b.plan.last_info["levels"] > 0 and rel(u1.cpu().numpy(), u0.cpu().numpy()) < 1e-8
+
+
+def orthotropic(n, kx, ky):
+    st = wl.shell_pinned_edges(n, 0.3 * n, 0.05 * n, design=3)
+    st.prop_quads[:, 3], st.prop_quads[:, 4] = kx, ky
+    return st
+
+
+@pytest.mark.parametrize("nrhs", [1, 3])
+@pytest.mark.parametrize("kx,ky", [(1.2, 0.8), (2.0, 0.5), (0.3, 3.0)])
+def test_orthotropic_batch_by_refinement_with_the_symmetric_part(kx, ky, nrhs):
+    """K and K^T solves of shells of two sizes (several load cases, a structure without
+    load) against the oracle's refined direct solves; the dense LU agrees."""
+    designs = [orthotropic(6, kx, ky), orthotropic(17, kx, ky), orthotropic(9, kx, ky)]
+    designs[2].nodal_loads[:] = 0.0
+    rng = np.random.default_rng(5)
+    for st in designs[:2]:
+        st.extra_loads = [st.nodal_loads * rng.uniform(0.0, 2.0, st.ndof) for _ in range(nrhs - 1)]
+    b = StructureBatch(designs, n_cases=nrhs)
+    b.assemble()
+    assert not b.plan.symmetric()
+    f = b.f[:, 0].contiguous() if nrhs == 1 else b.f
+    got = {t: b.plan.solve(f, transpose=t) for t in (False, True)}
+    info = b.plan.last_info
+    assert info["converged"] == info["n_systems"] == 3 * nrhs, info
+    b.plan.nonsymmetric_route(1)
+    for t in (False, True):
+        dense = b.plan.solve(f, transpose=t)
+        assert b.plan.last_info["iterations"] == 0
+        assert rel(got[t].cpu().numpy(), dense.cpu().numpy()) < 1e-9
+        u = got[t].cpu().numpy().reshape(-1, nrhs)
+        for i, st in enumerate(designs):
+            K = system.assemble_K(st.crds, st.cnct_beamcols, st.prop_beamcols, st.cnct_quads, st.prop_quads)
+            o = 6 * int(b.node_off[i])
+            for c, fc in enumerate(st.load_cases()[:nrhs]):
+                v = u[o:o + st.ndof, c]
+                ref = osolve.solve_reduced(K.T.tocsr() if t else K, st.known_id, fc)
+                assert rel(v, ref) < 1e-9 if fc.any() else not v.any(), (t, i, c)
