@@ -209,7 +209,9 @@ int jsso_spmv_k(jsso_plan* plan, const double* d_K, const double* d_x, double* d
  * Cholesky, or, when the plan's last assembly makes K non-symmetric (members
  * parallel to global Y, element.py:92-94; quads with kx_mod != ky_mod and nu != 0,
  * whose Cm is not symmetric, element.py:852-875), by a blocked LU with partial pivoting --
- * then triangular solves.  transpose != 0 solves Kc^T u = f (the adjoint system).
+ * then triangular solves.  For the plan's own symmetric assembly (d_K NULL) with
+ * 1 to 4 load cases, where the direct solve is taken (see JSSO_PC_AMG), its
+ * factorisation serves instead, refined to the attainable accuracy.  transpose != 0 solves Kc^T u = f (the adjoint system).
  * d_K as for jsso_spmv_k (NULL = the plan's current assembly); d_f, d_u:
  * (6*n_nodes) x nrhs, nrhs <= 64.  Needs 8 N^2 bytes of device memory (N =
  * 6*n_nodes rounded up to a multiple of 64).  Returns JSSO_ESINGULAR for a

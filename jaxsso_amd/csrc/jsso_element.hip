@@ -522,7 +522,7 @@ __device__ __forceinline__ double load_lam(const double* u, const double* lam, d
 // those by D the outer products of the local forces k u', k l' with lam, u, and the
 // chain through the direction cosines C = d / L ends in the node coordinates.  Dual
 // numbers through all 144 entries of k per direction (12 threads an element) took
-// 4.8 ms for 256 gridshells (233k beams) x 4 load cases; this takes 48 us.
+// 4.8 ms for 256 gridshells (228k beams) x 4 load cases; this takes 48 us.
 __device__ __forceinline__ void beam_force(const double v[12], double a, double t, double z1, double z2, double z3,
                                            double y1, double y2, double y3, double w[12]) {
     const double dz = v[1] - v[7], sz = v[5] + v[11], dy = v[2] - v[8], sy = v[4] + v[10];

@@ -161,3 +161,19 @@ def test_orthotropic_batch_by_refinement_with_the_symmetric_part(kx, ky, nrhs):
                 v = u[o:o + st.ndof, c]
                 ref = osolve.solve_reduced(K.T.tocsr() if t else K, st.known_id, fc)
                 assert rel(v, ref) < 1e-9 if fc.any() else not v.any(), (t, i, c)
+
+
+@pytest.mark.parametrize("m", [1, 4, 5])
+def test_dense_solve_of_the_plans_own_assembly(m):
+    """plan.dense_solve without K values (1 to 4 right-hand sides through the direct
+    factorisation, more through the dense one) against the dense factorisation of the
+    exported K and the oracle."""
+    st = wl.notebook_barrel()
+    plan = FEPlan([0, st.n_node], st.cnct_beamcols, st.cnct_quads, st.known_id)
+    K = plan.assemble(torch.tensor(st.crds), None, torch.tensor(st.prop_quads), export_K=True)
+    F = np.random.default_rng(3).normal(size=(st.ndof, m))
+    f = torch.tensor(F[:, 0] if m == 1 else F, device="cuda")
+    u, v = plan.dense_solve(f), plan.dense_solve(f, K=K)
+    assert rel(u.cpu().numpy(), v.cpu().numpy()) < 1e-9
+    ref = oracle_u(st, F)
+    assert rel(u.cpu().numpy().reshape(-1, m), ref) < 1e-9
