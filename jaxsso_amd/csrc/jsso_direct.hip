@@ -45,38 +45,42 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int DW = 96;                    // pivots per panel, at most (16 nodes)
 constexpr int DROWS = 64;                 // edge of an update tile
 constexpr int SROWS = 96;                 // rows of a strip
-constexpr int DLEAF = 12;                 // nodes eliminated whole at the tree's leaves
+constexpr int DLEAF = 10;                 // nodes eliminated whole at the tree's leaves (5 to 12: within 3%)
 constexpr int DLDS_MAX = 156 * 1024;      // dynamic LDS of a small front
-constexpr int DIRECT_MAX_M = 1500;        // largest front (direct_fits)
+constexpr int DIRECT_MAX_M = 2300;        // largest front (direct_fits)
+static_assert((DIRECT_MAX_M + 2 * 1024) * 4 * 8 <= DLDS_MAX, "LDS of the backward solve with 4 load cases");
 constexpr int DIRECT_STEPS = 6;           // refinement steps, at most
 constexpr int DEFECT_STEPS = 40;          // of a K that is not symmetric
 constexpr double DIRECT_FLOOR_FACTOR = 16.0;   // attainable accuracy: 16 eps (||A|| ||x|| + ||b||), as the AMG solve
+constexpr int STRIP_TILES = 3;            // 16x16 tiles of a strip that a wavefront holds
 constexpr int DKC = 32;                   // pivot columns staged at a time by the tile kernels
 
+// host: a front of a connectivity pattern; offsets within one structure's storage
 struct FrontMeta {
     int32_t np, nb, node0, level;
-    int32_t child[2], npre, blk0, nblk;   // npre: border nodes that are pivots of the parent
+    int32_t child[2], blk0, nblk;
     int32_t wn, npan;                     // nodes of a panel (the last may have fewer), panels
-    int32_t small, pad;                   // one-workgroup front
-    int64_t fac, mat, pan, vec;           // offsets (doubles): S|G panels, contribution (b x b), pivot columns
+    bool small;                           // one-workgroup front
+    int64_t fac, mat, pan, vec;           // (doubles) S|G panels, contribution (b x b), pivot columns
                                           // (m x k, large fronts), vector (x load cases)
 };
-struct StructMeta {
-    int64_t fac, mat, vec;                // bases of the structure
-    int32_t node0, blk0;                  // first node, first block of the CSR
+// A front of a structure as the kernels take it: everything a workgroup needs in
+// one read (following front -> children -> structure by dependent loads cost each of
+// the ~100 kernels of a solve 2 us).
+struct FrontTask {
+    int32_t np, nb, wn, npan;
+    int32_t node0, blk0, nblk, kref0;     // first entry in nodes / inv / blkrow, stored blocks, their base in kref
+    int32_t sys, gnode0, cb[2];           // structure, its first node, border nodes of the children (0: none)
+    int64_t mat, pan, fac, vec;           // offsets (doubles; vec: x load cases)
+    int64_t cmat[2], cvec[2];             // the children's contributions and border vectors
 };
 struct DirectDev {
-    const FrontMeta* fr;
-    const StructMeta* st;
-    const int32_t *nodes, *rel, *blk, *blkrow, *kref;
+    const int32_t *nodes, *blk, *blkrow, *kref;
     const int2* inv;                      // per entry of `nodes`: the border node it is in each child, or -1
     const double* A64;
     double *fac, *mat, *vec;
     const double* zero;                   // a zero
     int32_t* bad;                         // per structure: a pivot was not positive
-};
-struct DTask {
-    int32_t front, sys;
 };
 struct DirectReport {
     int32_t running, stalled, floor, bad;   // systems; structures with a pivot that is not positive
@@ -84,17 +88,19 @@ struct DirectReport {
 };
 
 struct DirectState {
-    std::vector<FrontMeta> fr;
-    std::vector<StructMeta> st;
-    std::vector<std::vector<DTask>> small_tasks, big_tasks;   // per level
-    std::vector<size_t> small_lds;                            // per level: dynamic LDS
+    std::vector<std::vector<FrontTask>> small_tasks, big_tasks;   // per level
+    struct Bucket {               // small fronts of a level that need alike much LDS
+        size_t lds = 0, off = 0, n = 0;
+        int threads = 0;
+    };
+    std::vector<std::vector<Bucket>> buckets;                        // per level
     std::vector<int> small_m, big_m, big_k, big_b, big_w, big_pan;   // per level: largest fronts, most panels
-    std::vector<int64_t> small_off, big_off;                  // first task of the level on the device
+    std::vector<size_t> small_n, big_n, small_off, big_off;          // tasks of the level, first on the device
     int n_levels = 0, max_m = 0;
     size_t fac_n = 0, mat_n = 0, vec_n = 0;
     double flops = 0.0;
     DirectDev dev{};
-    DTask* d_tasks = nullptr;
+    const FrontTask* d_tasks = nullptr;
     double* d_rho = nullptr;
     DirectReport *d_report = nullptr, *h_report = nullptr;
     size_t vec_bytes = 0;
@@ -135,50 +141,33 @@ __device__ __forceinline__ double fast_rsqrt(double d) {
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// the values of v in the four lanes r, r + 16, r + 32, r + 48 (every lane gets all)
-__device__ __forceinline__ void all_rows(double v, double (&x)[4]) {
-    const long long b = __double_as_longlong(v);
-    const int lo = (int)b, hi = (int)(b >> 32);
-    // rows (0, 0, 2, 2) and (1, 1, 3, 3), then each split into its halves
-    auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-    auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-#pragma unroll
-    for (int o = 0; o < 2; ++o) {
-        auto l2 = __builtin_amdgcn_permlane32_swap(l[o], l[o], false, false);
-        auto h2 = __builtin_amdgcn_permlane32_swap(h[o], h[o], false, false);
-        x[o] = join_halves(l2[0], h2[0]);
-        x[o + 2] = join_halves(l2[1], h2[1]);
-    }
-}
-
-// Cholesky factor L of a 16x16 block (lower triangle in LDS) and its inverse, by
-// one wavefront; the inverse replaces the block (zeros above the diagonal).
+// Cholesky factor L of a symmetric 16x16 block A and its inverse, by one wavefront;
+// the inverse goes to D (LDS, zeros above the diagonal).
 // Lane (r, q) = (l % 16, l / 16) holds A[r][4 i + q], i = 0..3: for a symmetric A
-// that is at once the layout of the matrix core's result and of its first operand,
-// so the update by four columns of L is one instruction, and so is the same step
-// of the forward substitution W <- I that gives the inverse.  Per four columns:
-// every lane collects its row's four entries (all_rows), the 4x4 diagonal block
-// comes by readlane and is factored by all lanes alike.  Against a column at a
-// time with readlane broadcasts (240 of them, 5 us) this took the block to ~1.5 us.
-__device__ __forceinline__ bool factor16(double* D, int ld, int lane) {
+// that is at once the layout of the matrix core's result, of its first operand and,
+// read as A[4 i + q][r], of its second.  Per four columns, with T the inverse factor
+// of their 4x4 diagonal block (fetched by readlane, factored by all lanes alike),
+//   l = A[:, 4 columns] T^T,  A -= l l^T,   x = T W[4 rows, :],  W -= l x   (W <- I)
+// are four matrix instructions, x the four rows of the inverse.  Bound by its chain
+// of dependent steps (four reciprocal roots per four columns): 4 700 cycles with the
+// products by lane-wise arithmetic and readlane, 3 300 so.
+__device__ __forceinline__ bool factor16(d4 A, double* D, int ld, int lane) {
     const int r = lane & 15, q = lane >> 4;
-    d4 A, W;
+    d4 W;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int c = 4 * i + q;
-        A[i] = r >= c ? D[r * ld + c] : D[c * ld + r];
-        W[i] = c == r ? 1.0 : 0.0;
-    }
+    for (int i = 0; i < 4; ++i) W[i] = 4 * i + q == r ? 1.0 : 0.0;
     bool ok = true;
-#pragma unroll 1
-    for (int b = 0; b < 4; ++b) {   // (a loop: unrolled, it doubles the registers)
-        double p[4], w[4], d[4][4];
-        all_rows(b == 0 ? A[0] : b == 1 ? A[1] : b == 2 ? A[2] : A[3], p);
-        all_rows(b == 0 ? W[0] : b == 1 ? W[1] : b == 2 ? W[2] : W[3], w);
+    auto is = [&](int i, int c) { return r == i && q == c ? 1.0 : 0.0; };
+    const double m0 = is(0, 0), m10 = is(1, 0), m1 = is(1, 1), m20 = is(2, 0), m21 = is(2, 1), m2 = is(2, 2),
+                 m30 = is(3, 0), m31 = is(3, 1), m32 = is(3, 2), m3 = is(3, 3);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int b = 0; b < 4; ++b) {
+        const double a = A[b], w = W[b];
+        double d[4][4];
 #pragma unroll
-            for (int c = 0; c <= i; ++c) d[i][c] = lane_value(p[c], 4 * b + i);
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int i = c; i < 4; ++i) d[i][c] = lane_value(a, 16 * c + 4 * b + i);
         const double i0 = fast_rsqrt(d[0][0]);
         const double l10 = d[1][0] * i0, l20 = d[2][0] * i0, l30 = d[3][0] * i0;
         const double e1 = fma(-l10, l10, d[1][1]), i1 = fast_rsqrt(e1);
@@ -187,20 +176,22 @@ __device__ __forceinline__ bool factor16(double* D, int ld, int lane) {
         const double l32 = fma(-l31, l21, fma(-l30, l20, d[3][2])) * i2;
         const double e3 = fma(-l32, l32, fma(-l31, l31, fma(-l30, l30, d[3][3]))), i3 = fast_rsqrt(e3);
         ok &= d[0][0] > 0.0 && e1 > 0.0 && e2 > 0.0 && e3 > 0.0;
-        p[0] *= i0;
-        p[1] = fma(-p[0], l10, p[1]) * i1;
-        p[2] = fma(-p[1], l21, fma(-p[0], l20, p[2])) * i2;
-        p[3] = fma(-p[2], l32, fma(-p[1], l31, fma(-p[0], l30, p[3]))) * i3;
-        w[0] *= i0;
-        w[1] = fma(-l10, w[0], w[1]) * i1;
-        w[2] = fma(-l21, w[1], fma(-l20, w[0], w[2])) * i2;
-        w[3] = fma(-l32, w[2], fma(-l31, w[1], fma(-l30, w[0], w[3]))) * i3;
-        double l = q == 0 ? p[0] : q == 1 ? p[1] : q == 2 ? p[2] : p[3];
-        const double x = q == 0 ? w[0] : q == 1 ? w[1] : q == 2 ? w[2] : w[3];
-        if (4 * b + q > r) l = 0.0;
-        D[(4 * b + q) * ld + r] = x;   // (its old entries are all in registers)
-        A = mfma64(-l, l, A);
-        W = mfma64(-l, x, W);
+        const double t10 = -l10 * i0 * i1, t21 = -l21 * i1 * i2, t32 = -l32 * i2 * i3;
+        const double t20 = -fma(l21, t10, l20 * i0) * i2, t31 = -fma(l32, t21, l31 * i1) * i3;
+        const double t30 = -fma(l32, t20, fma(l31, t10, l30 * i0)) * i3;
+        // T[r][q] for r < 4, zero elsewhere (by masks: selects became branches)
+        double T = m0 * i0;
+        T = fma(m10, t10, fma(m1, i1, T));
+        T = fma(m21, t21, fma(m20, t20, fma(m2, i2, T)));
+        T = fma(m3, i3, fma(m32, t32, fma(m31, t31, fma(m30, t30, T))));
+        const d4 zero = {0.0, 0.0, 0.0, 0.0};
+        const d4 lt = mfma64(T, a, zero), xt = mfma64(T, w, zero);   // element 0: rows q of the 4 x 16 results
+        const double l = 4 * b + q > r ? 0.0 : lt[0], x = xt[0];
+        D[(4 * b + q) * ld + r] = x;
+        if (b < 3) {
+            A = mfma64(-l, l, A);
+            W = mfma64(-l, x, W);
+        }
     }
     return ok;
 }
@@ -213,7 +204,7 @@ __device__ __forceinline__ bool factor16(double* D, int ld, int lane) {
 //      it, the others the rest of the trailing triangle and the sums
 //      W_IJ = sum_K L_IK Linv_KJ of the rows below
 //   A  L_I = A_I Dinv^T below the block, and row kb of the inverse, -Dinv W_J
-// The factorisation of a 16x16 block (one wavefront, ~2 us of dependent steps) is
+// The factorisation of a 16x16 block (one wavefront, ~1.5 us of dependent steps) is
 // the chain that bounds this routine; phase B hides the products behind it.
 __device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wave, int nw, int lane) {
     const int nt = kp >> 4, r = lane & 15, q = lane >> 4;
@@ -223,7 +214,7 @@ __device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wav
         // B of block column j = kb - 1: products X Y (Y as it is or transposed) added to C
         const int j = kb - 1, n = nt - kb, ntri = kb ? n * (n + 1) / 2 : 0, all = ntri + n * kb;
 #pragma unroll 1
-        for (int e = wave; e < all; e += wave ? nw - 1 : all) {   // (wavefront 0 only takes tile 0)
+        for (int e = wave ? wave : all; e < all; e += nw - 1) {   // (tile 0 is wavefront 0's)
             const double *X, *Y;
             double* C;
             int ys;
@@ -258,7 +249,20 @@ __device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wav
             for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
         }
         double* D = P + (16 * kb) * ld + 16 * kb;
-        if (wave == 0) ok &= factor16(D, ld, lane);
+        if (wave == 0) {
+            d4 A;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = 4 * i + q;
+                A[i] = r >= c ? D[r * ld + c] : D[c * ld + r];
+            }
+            if (kb > 0) {
+                const double* X = P + (16 * kb + r) * ld + 16 * j + q;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) A = mfma64(-X[4 * t], X[4 * t], A);
+            }
+            ok &= factor16(A, D, ld, lane);
+        }
         __syncthreads();
 #pragma unroll 1
         for (int e = wave; e < nt - 1; e += nw) {
@@ -345,32 +349,40 @@ __device__ __forceinline__ double stored_entry(const DirectDev& d, int32_t kr, i
     return d.A64[(int64_t)(vp >> 6) * 36 * ROWS_PER_WG + ((int64_t)(e >> 1) * ROWS_PER_WG + (vp & 63)) * 2 + (e & 1)];
 }
 
-// a front's contribution C (b x b, row-major, lower triangle)
-__device__ __forceinline__ double* contribution(const DirectDev& d, const FrontMeta& f, const StructMeta& s) {
-    return d.mat + s.mat + f.mat;
-}
-
-// The children's part of a front's entries: where each child keeps its C
+// The children's part of a front's entries: where each child keeps its contribution
+// C (b x b, row-major, lower triangle)
 struct Gather {
     const double *C[2], *zero;
     int ld[2];
     bool any;
 };
-__device__ __forceinline__ Gather make_gather(const DirectDev& d, const FrontMeta& f, const StructMeta& st) {
+__device__ __forceinline__ Gather make_gather(const DirectDev& d, const FrontTask& f) {
     Gather g;
     g.zero = d.zero;
-    g.any = f.child[0] >= 0;
+    g.any = f.cb[0] > 0 || f.cb[1] > 0;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-        g.C[c] = d.zero;
-        g.ld[c] = 0;
-        if (f.child[c] >= 0) {
-            const FrontMeta& h = d.fr[f.child[c]];
-            g.C[c] = contribution(d, h, st);
-            g.ld[c] = 6 * h.nb;
-        }
+        g.C[c] = d.mat + f.cmat[c];
+        g.ld[c] = 6 * f.cb[c];
     }
     return g;
+}
+// (task, part) of a workgroup of a launch over `parts` parts of n tasks.  Many tasks:
+// all parts of a task one after the other on one XCD, whose L2 then holds what they
+// share; few: spread over the chip.
+struct Where {
+    int task, part;
+};
+__device__ __forceinline__ Where locate(int n, int parts) {
+    const int b = blockIdx.x;
+    if (n >= 64) {
+        const int q = b >> 3, t = q / parts;
+        return {8 * t + (b & 7), q - t * parts};
+    }
+    return {b % n, b / n};
+}
+static dim3 part_grid(size_t n, int parts) {
+    return dim3((unsigned)((n >= 64 ? 8 * ((n + 7) / 8) : n) * parts));
 }
 // entry (row, col) of the front, row >= col; a, b: `inv` of their nodes.  Without
 // branches, so that a thread's loads are all in flight at once (a wavefront that
@@ -385,7 +397,7 @@ __device__ __forceinline__ double gathered(const Gather& g, int2 a, int2 b, int 
 // adds the blocks of K with front rows in [r0, r1) and columns in [c0, c1) to a tile
 // in LDS (rows and columns relative to r0, c0; front rows from `split` on are `gap`
 // rows further down); four chains of dependent loads per thread in flight
-__device__ __forceinline__ void add_stored(const DirectDev& d, const FrontMeta& f, const StructMeta& st, int r0,
+__device__ __forceinline__ void add_stored(const DirectDev& d, const FrontTask& f, int r0,
                                            int r1, int c0, int c1, int split, int gap, double* T, int ld, int tid,
                                            int nth) {
     if (r1 <= r0) return;
@@ -401,7 +413,7 @@ __device__ __forceinline__ void add_stored(const DirectDev& d, const FrontMeta& 
             const int e = min(e0 + u * nth, all - 1), blk = e / 36, row = e % 36 / 6, col = e % 6;
             const int32_t* t3 = d.blk + 3 * (b0 + blk);
             const int R = 6 * t3[1] + row, C = 6 * t3[2] + col;
-            v[u] = stored_entry(d, d.kref[st.blk0 + t3[0]], row, col);
+            v[u] = stored_entry(d, d.kref[f.kref0 + t3[0]], row, col);
             at[u] = e0 + u * nth < all && R >= r0 && R < r1 && C >= c0 && C < c1
                         ? (R - r0 + (R >= split ? gap : 0)) * ld + C - c0 : -1;
         }
@@ -414,16 +426,15 @@ __device__ __forceinline__ void add_stored(const DirectDev& d, const FrontMeta& 
 // ---------------------------------------------------------------------------
 // device: factorisation
 // ---------------------------------------------------------------------------
-// One small front per workgroup.  Bound by its chain of phases, not by bandwidth or
-// the matrix cores (a leaf is 0.3 MFLOP), so the phases keep many loads in flight
-// and the next level of parallelism is the number of fronts per CU: the panel rows
-// are all that is held in LDS.
+// One small front per workgroup.  Bound by its chain of phases (a leaf of 12 nodes
+// on a full chip, us: blocks of K 5, factor 12, strips 9, contribution 7), so every
+// phase keeps many loads in flight and spreads over all wavefronts; the children's
+// entries of a wavefront's first contribution tile are requested before the
+// factorisation and arrive behind it.  Only the panel rows are held in LDS.
 template <int NT>
-__global__ __launch_bounds__(NT) void k_front_small(DirectDev d, const DTask* __restrict__ tasks) {
+__global__ __launch_bounds__(NT, NT == 1024 ? 4 : NT == 512 ? 4 : 3) void k_front_small(DirectDev d, const FrontTask* __restrict__ tasks) {
     extern __shared__ double P[];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
-    const StructMeta st = d.st[task.sys];
+    const FrontTask f = tasks[blockIdx.x];
     constexpr int nw = NT / 64;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -431,11 +442,7 @@ __global__ __launch_bounds__(NT) void k_front_small(DirectDev d, const DTask* __
     const int kp = (k + 15) & ~15, bp = (b + 15) & ~15, ld = kp + 2;
     const int nt = kp >> 4, bt = bp >> 4, bs = (bt + 1) >> 1, r = lane & 15, q = lane >> 4;
     int2* inv = reinterpret_cast<int2*>(P + (kp + bp) * ld);   // of every node, past the end: none
-    const Gather ga = make_gather(d, f, st);
-    for (int e = tid; e < f.np + f.nb + 3; e += NT) inv[e] = e < f.np + f.nb ? d.inv[f.node0 + e] : int2{-1, -1};
-    __syncthreads();
-    // contribution: 32x32 tiles of the lower triangle; the children's entries of a
-    // wavefront's first tile are requested here, to arrive behind the factorisation
+    const Gather ga = make_gather(d, f);
     auto gather_tile = [&](int I, int J, d4 (&t)[2][2]) {
         const int2* bi = inv + f.np;
 #pragma unroll
@@ -451,60 +458,87 @@ __global__ __launch_bounds__(NT) void k_front_small(DirectDev d, const DTask* __
                 }
         }
     };
+    // contribution: 32x32 tiles of the lower triangle
     int I = 0, J = wave;
     while (J > I) {
         J -= I + 1;
         ++I;
     }
     d4 acc[2][2] = {};
-    if (ga.any && I < bs) gather_tile(I, J, acc);
-    // panel: what the children pass up (rows by wavefront, four in flight), then K
-    for (int c0 = 0; c0 < kp; c0 += 64) {
-        const int col = c0 + lane, cn = min(col, k) / 6, cc = col - 6 * cn;
-        const int2 ic = inv[cn];
-        for (int row0 = wave; row0 < kp + bp; row0 += 4 * nw) {
+    // panel: what the children pass up, by 4 rows x 16 columns per wavefront, four at a
+    // time; the identity on the diagonal
+    if (ga.any) {
+        for (int e = tid; e < f.np + f.nb + 3; e += NT) inv[e] = e < f.np + f.nb ? d.inv[f.node0 + e] : int2{-1, -1};
+        __syncthreads();
+        if (I < bs) gather_tile(I, J, acc);
+        const int items = ((kp + bp) >> 2) * nt;
+        for (int e0 = wave; e0 < items; e0 += 4 * nw) {
             double v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int row = row0 + u * nw, R = row < kp ? row : row - kp + k;
+                const int e = min(e0 + u * nw, items - 1), g = e / nt, K = e - g * nt;
+                const int row = 4 * g + q, col = 16 * K + r, R = row < kp ? row : row - kp + k;
                 const bool on = col < k && (row < kp ? row < k && col <= row : row < kp + b);
-                const int rn = on ? R / 6 : 0;
-                v[u] = ga.any ? gathered(ga, inv[rn], ic, R - 6 * rn, cc, on) : 0.0;
-                if (row == col) v[u] += 1.0;
+                const int rn = on ? R / 6 : 0, cn = on ? col / 6 : 0;
+                v[u] = gathered(ga, inv[rn], inv[cn], R - 6 * rn, col - 6 * cn, on) + (row == col ? 1.0 : 0.0);
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (row0 + u * nw < kp + bp && col < kp) P[(row0 + u * nw) * ld + col] = v[u];
+            for (int u = 0; u < 4; ++u) {   // (the last item again where there are fewer)
+                const int e = min(e0 + u * nw, items - 1), g = e / nt, K = e - g * nt;
+                P[(4 * g + q) * ld + 16 * K + r] = v[u];
+            }
         }
+    } else {
+        for (int e = 2 * tid; e < (kp + bp) * ld; e += 2 * NT)
+            *reinterpret_cast<double2*>(P + e) = double2{0.0, 0.0};
+        __syncthreads();
+        for (int e = tid; e < kp; e += NT) P[e * ld + e] = 1.0;
     }
     __syncthreads();
-    add_stored(d, f, st, 0, k + b, 0, k, k, kp - k, P, ld, tid, NT);
+    add_stored(d, f, 0, k + b, 0, k, k, kp - k, P, ld, tid, NT);
     __syncthreads();
     const bool ok = invert_factor(P, ld, kp, wave, nw, lane);
-    if (!ok && tid == 0) atomicOr(d.bad + task.sys, 1);
-    double* S = d.fac + st.fac + f.fac;
+    if (!ok && tid == 0) atomicOr(d.bad + f.sys, 1);
+    double* S = d.fac + f.fac;
     double* G = S + (int64_t)k * k;
-    for (int B = wave; B < bt; B += nw) {
-        double* X = P + (kp + 16 * B) * ld;
-        for (int K = nt - 1; K >= 0; --K) {   // descending: block K needs the blocks up to K as they were
-            const d4 v = strip_L(X, P, ld, K, lane);
+    // strips, tile by tile: L21 (kept in registers until every wavefront has read F21),
+    // then G = L21 L^-1; as many rounds as 16 x 16 tiles per wavefront need
+    for (int e0 = 0; e0 < bt * nt; e0 += STRIP_TILES * nw) {
+        // (rows of one round are whole: a round takes all columns of its row tiles)
+        const int rows = min(bt - e0 / nt, STRIP_TILES * nw / nt), n = rows * nt, row0 = e0 / nt;
+        d4 v[STRIP_TILES];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) X[(4 * i + q) * ld + 16 * K + r] = v[i];
+        for (int u = 0; u < STRIP_TILES; ++u) {
+            const int e = wave + nw * u;
+            if (e < n) v[u] = strip_L(P + (kp + 16 * (row0 + e % rows)) * ld, P, ld, nt - 1 - e / rows, lane);
         }
-        for (int K = 0; K < nt; ++K)
-            store_tile(G + (int64_t)16 * B * k + 16 * K, k, strip_G(X, P, ld, nt, K, lane), b - 16 * B, k - 16 * K,
-                       lane);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < STRIP_TILES; ++u) {
+            const int e = wave + nw * u, B = row0 + e % rows, K = nt - 1 - e / rows;
+            if (e < n) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) P[(kp + 16 * B + 4 * i + q) * ld + 16 * K + r] = v[u][i];
+            }
+        }
+        __syncthreads();
+        for (int e = wave; e < n; e += nw) {
+            const int B = row0 + e % rows, K = e / rows;
+            store_tile(G + (int64_t)16 * B * k + 16 * K, k, strip_G(P + (kp + 16 * B) * ld, P, ld, nt, K, lane),
+                       b - 16 * B, k - 16 * K, lane);
+        }
+        e0 += n - STRIP_TILES * nw;
     }
-    write_S(P, ld, kp, k, S, (wave + nw - bt % nw) % nw, nw, lane);   // from the wavefronts with fewer strips
-    __syncthreads();
-    double* Cout = contribution(d, f, st);
+    write_S(P, ld, kp, k, S, nw - 1 - wave, nw, lane);
+    double* Cout = d.mat + f.mat;
+    const int k4 = (k + 3) >> 2;
     while (I < bs) {
         // (rows past the last tile read the tile before: their products are not stored)
         const int i1 = 2 * I + 1 < bt ? 16 : 0, j1 = 2 * J + 1 < bt ? 16 : 0;
         const double* x = P + (kp + 32 * I + r) * ld + q;
         const double* y = P + (kp + 32 * J + r) * ld + q;
 #pragma unroll 4
-        for (int t = 0; t < 4 * nt; ++t) {
+        for (int t = 0; t < k4; ++t) {
             const double a0 = -x[4 * t], a1 = -x[i1 * ld + 4 * t], b0 = y[4 * t], b1 = y[j1 * ld + 4 * t];
             acc[0][0] = mfma64(a0, b0, acc[0][0]);
             acc[0][1] = mfma64(a0, b1, acc[0][1]);
@@ -541,18 +575,16 @@ __device__ __forceinline__ int64_t panel_offset(int m, int w, int p) {
 
 // diagonal block of panel p (gathered for the first panel): S to the factor, the
 // inverse factor to the block's place in the pivot columns
-__global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const DTask* __restrict__ tasks, int p) {
+__global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const FrontTask* __restrict__ tasks, int p) {
     extern __shared__ double P[];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
+    const FrontTask f = tasks[blockIdx.x];
     if (p >= f.npan) return;
-    const StructMeta st = d.st[task.sys];
     const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kp = (w + 15) & ~15, ld = kp + 2;
-    double* F = d.mat + st.mat + f.pan + (int64_t)c0 * k + c0;
-    const Gather ga = make_gather(d, f, st);
+    double* F = d.mat + f.pan + (int64_t)c0 * k + c0;
+    const Gather ga = make_gather(d, f);
     __shared__ int2 inv[DW / 6 + 1];
     if (tid < w / 6) inv[tid] = d.inv[f.node0 + tid];
     __syncthreads();
@@ -576,34 +608,34 @@ __global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const DTask* __
         }
     }
     __syncthreads();
-    if (p == 0) add_stored(d, f, st, 0, w, 0, w, w, 0, P, ld, tid, 512);
+    if (p == 0) add_stored(d, f, 0, w, 0, w, w, 0, P, ld, tid, 512);
     __syncthreads();
     const bool ok = invert_factor(P, ld, kp, wave, 8, lane);
-    if (!ok && tid == 0) atomicOr(d.bad + task.sys, 1);
-    double* S = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p);
+    if (!ok && tid == 0) atomicOr(d.bad + f.sys, 1);
+    double* S = d.fac + f.fac + panel_offset(m, 6 * f.wn, p);
     write_S(P, ld, kp, w, S, wave, 8, lane);
     for (int row = wave; row < w; row += 8)
         for (int col = lane; col <= row; col += 64)
             F[(int64_t)row * k + col] = P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)];
 }
 
-// 96 rows below panel p's diagonal block: L21 = F21 L^-T (in place) and G = L21 L^-1
-__global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const DTask* __restrict__ tasks, int p) {
+// `rows` (<= 96) rows below panel p's diagonal block: L21 = F21 L^-T (in place) and G = L21 L^-1
+__global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const FrontTask* __restrict__ tasks, int p, int n, int parts, int rows) {
     extern __shared__ double P[];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
+    const Where at = locate(n, parts);
+    if (at.task >= n) return;
+    const FrontTask f = tasks[at.task];
     if (p >= f.npan) return;
-    const StructMeta st = d.st[task.sys];
     const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
-    const int r0 = c0 + w + SROWS * blockIdx.y;
+    const int r0 = c0 + w + rows * at.part;
     if (r0 >= m) return;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kp = (w + 15) & ~15, ld = kp + 2, nt = kp >> 4;
-    double* F = d.mat + st.mat + f.pan + c0;   // column c0 of the pivot columns
+    double* F = d.mat + f.pan + c0;   // column c0 of the pivot columns
     double* X = P + kp * ld;
-    const int nr = min(SROWS, m - r0);
-    const Gather ga = make_gather(d, f, st);
+    const int nr = min(rows, m - r0), rt = rows >> 4;
+    const Gather ga = make_gather(d, f);
     __shared__ int2 ir[SROWS / 6 + 2], icol[DW / 6 + 1];
     const int rn0 = r0 / 6;
     if (p == 0) {
@@ -614,7 +646,7 @@ __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const DTask* 
     for (int c1 = 0; c1 < kp; c1 += 64) {
         const int col = c1 + lane, cn = min(col, w - 1) / 6, cc = col - 6 * cn;
         const int2 ic = p == 0 ? icol[cn] : int2{-1, -1};
-        for (int row0 = wave; row0 < SROWS; row0 += 48) {
+        for (int row0 = wave; row0 < max(rows, kp); row0 += 48) {
             double v[3], y[3];
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
@@ -630,7 +662,7 @@ __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const DTask* 
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
                 const int row = row0 + 16 * u;
-                if (col < kp) X[row * ld + col] = v[u];
+                if (col < kp && row < rows) X[row * ld + col] = v[u];
                 // block (I, J) of the inverse factor goes to block row J, block column I
                 if (row < kp && col >> 4 <= row >> 4)
                     P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)] = y[u];
@@ -639,32 +671,32 @@ __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const DTask* 
     }
     __syncthreads();
     if (p == 0) {
-        add_stored(d, f, st, r0, r0 + nr, 0, w, m, 0, X, ld, tid, 1024);
+        add_stored(d, f, r0, r0 + nr, 0, w, m, 0, X, ld, tid, 1024);
         __syncthreads();
     }
-    // 6 row tiles x nt block columns over 16 wavefronts
+    // rt row tiles x nt block columns over 16 wavefronts
     d4 v[3];
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
         const int e = wave + 16 * u;
-        if (e < 6 * nt) v[u] = strip_L(X + 16 * (e % 6) * ld, P, ld, e / 6, lane);
+        if (e < rt * nt) v[u] = strip_L(X + 16 * (e % rt) * ld, P, ld, e / rt, lane);
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
-        const int e = wave + 16 * u, I = e % 6, J = e / 6;
-        if (e < 6 * nt) {
+        const int e = wave + 16 * u, I = e % rt, J = e / rt;
+        if (e < rt * nt) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) X[(16 * I + 4 * i + q) * ld + 16 * J + r] = v[u][i];
             store_tile(F + (int64_t)(r0 + 16 * I) * k + 16 * J, k, v[u], nr - 16 * I, w - 16 * J, lane);
         }
     }
     __syncthreads();
-    double* G = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w + (int64_t)(r0 - c0 - w) * w;
+    double* G = d.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w + (int64_t)(r0 - c0 - w) * w;
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
-        const int e = wave + 16 * u, I = e % 6, J = e / 6;
-        if (e < 6 * nt)
+        const int e = wave + 16 * u, I = e % rt, J = e / rt;
+        if (e < rt * nt)
             store_tile(G + (int64_t)16 * I * w + 16 * J, w, strip_G(X + 16 * I * ld, P, ld, nt, J, lane), nr - 16 * I,
                        w - 16 * J, lane);
     }
@@ -706,33 +738,40 @@ __device__ __forceinline__ void tile_product(const double* __restrict__ F, int k
         if (k0 + DKC < w) fetch(k0 + DKC);   // the next chunk is on its way during this one's products
         const double* x = X + (wi + (lane & 15)) * LD + (lane >> 4);
         const double* y = Y + (wj + (lane & 15)) * LD + (lane >> 4);
-#pragma unroll
-        for (int s = 0; s < DKC / 4; ++s) {
+        auto step = [&](int s) {
             const double a0 = x[4 * s], a1 = x[16 * LD + 4 * s], b0 = y[4 * s], b1 = y[16 * LD + 4 * s];
             t.a[0][0] = mfma64(a0, b0, t.a[0][0]);
             t.a[0][1] = mfma64(a0, b1, t.a[0][1]);
             t.a[1][0] = mfma64(a1, b0, t.a[1][0]);
             t.a[1][1] = mfma64(a1, b1, t.a[1][1]);
+        };
+        if (k0 + DKC <= w) {
+#pragma unroll
+            for (int s = 0; s < DKC / 4; ++s) step(s);
+        } else {
+#pragma unroll 2
+            for (int s = 0; s < (w - k0 + 3) >> 2; ++s) step(s);
         }
     }
 }
 
 // panel p's update of the pivot columns after it (64x64 tiles; gathered here for p = 0)
-__global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const DTask* __restrict__ tasks, int p) {
+__global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const FrontTask* __restrict__ tasks, int p, int n, int parts) {
     __shared__ double sh[2 * DROWS * (DKC + 2)];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
+    const Where at = locate(n, parts);
+    if (at.task >= n) return;
+    const FrontTask f = tasks[at.task];
     if (p + 1 >= f.npan) return;
-    const StructMeta st = d.st[task.sys];
     const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = 6 * f.wn, t0 = c0 + w;
-    const int i0 = t0 + DROWS * blockIdx.y, j0 = t0 + DROWS * blockIdx.z;
-    if (i0 >= m || j0 >= k || j0 > i0) return;
+    const int nc = (k - t0 + DROWS - 1) / DROWS;   // tile columns; part -> (row, column), columns of a row together
+    const int i0 = t0 + DROWS * (at.part / nc), j0 = t0 + DROWS * (at.part % nc);
+    if (i0 >= m || j0 > i0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double* F = d.mat + st.mat + f.pan;
+    double* F = d.mat + f.pan;
     TileAcc t = {};
     tile_product(F, k, m, i0, j0, c0, w, sh, sh + DROWS * (DKC + 2), tid, t);
     const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1);
-    const Gather ga = make_gather(d, f, st);
+    const Gather ga = make_gather(d, f);
     const int2* inv = d.inv + f.node0;
     const int i1 = min(m, i0 + DROWS), j1 = min(k, j0 + DROWS);
     constexpr int LDT = DROWS + 2;
@@ -741,7 +780,7 @@ __global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const DTask* __
         __syncthreads();
         for (int e = tid; e < LDT * DROWS; e += 256) sh[e] = 0.0;
         __syncthreads();
-        add_stored(d, f, st, i0, i1, j0, j1, m + k, 0, sh, LDT, tid, 256);
+        add_stored(d, f, i0, i1, j0, j1, m + k, 0, sh, LDT, tid, 256);
         __syncthreads();
     }
 #pragma unroll
@@ -763,14 +802,14 @@ __global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const DTask* __
 }
 
 // contribution of a large front, 64x64 tiles of the lower triangle
-__global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const DTask* __restrict__ tasks) {
+__global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const FrontTask* __restrict__ tasks, int n, int parts) {
     __shared__ double sh[2 * DROWS * (DKC + 2)];
     __shared__ int2 ir[DROWS / 6 + 3], ic[DROWS / 6 + 3];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
-    const StructMeta st = d.st[task.sys];
+    const Where at = locate(n, parts);
+    if (at.task >= n) return;
+    const FrontTask f = tasks[at.task];
     const int k = 6 * f.np, b = 6 * f.nb, m = k + b, nt = (b + DROWS - 1) / DROWS;
-    const int e = blockIdx.y;
+    const int e = at.part;
     if (e >= nt * (nt + 1) / 2) return;
     int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
     while (I * (I + 1) / 2 > e) --I;
@@ -784,7 +823,7 @@ __global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const DTask* __re
     }
     __syncthreads();
     const int wi = DROWS * I + 32 * (wave >> 1), wj = DROWS * J + 32 * (wave & 1);
-    const Gather ga = make_gather(d, f, st);
+    const Gather ga = make_gather(d, f);
     TileAcc t;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
@@ -798,8 +837,8 @@ __global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const DTask* __re
                 t.a[u][v][i] = -gathered(ga, ir[rn - rn0], jc, row - 6 * rn, col - 6 * cn, row < b && col <= row);
             }
     }
-    tile_product(d.mat + st.mat + f.pan, k, m, k + DROWS * I, k + DROWS * J, 0, k, sh, sh + DROWS * (DKC + 2), tid, t);
-    double* C = contribution(d, f, st);
+    tile_product(d.mat + f.pan, k, m, k + DROWS * I, k + DROWS * J, 0, k, sh, sh + DROWS * (DKC + 2), tid, t);
+    double* C = d.mat + f.mat;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -815,76 +854,85 @@ __global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const DTask* __re
 // device: solves
 // ---------------------------------------------------------------------------
 // a front's vector v (pivots, then border; [..][NR]): right-hand side of the
-// pivots plus what its children pass up
+// pivots plus what its children pass up; nodes l0 <= l < l1
 template <int NR>
-__device__ __forceinline__ void gather_rhs(const DirectDev& d, const FrontMeta& f, const StructMeta& st,
-                                           const double* __restrict__ r, int l0, int l1, double* dst, int tid,
-                                           int nth) {
-    // node l of the front, l0 <= l < l1
-    const double* cv[2] = {nullptr, nullptr};
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-        if (f.child[c] >= 0) {
-            const FrontMeta& g = d.fr[f.child[c]];
-            cv[c] = d.vec + (st.vec + g.vec + 6 * g.np) * NR;
-        }
+__device__ __forceinline__ void gather_rhs(const DirectDev& d, const FrontTask& f, const double* __restrict__ r,
+                                           int l0, int l1, double* dst, int tid, int nth) {
+    const double *v0 = d.vec + f.cvec[0] * NR, *v1 = d.vec + f.cvec[1] * NR;
     for (int e = tid; e < (l1 - l0) * 6 * NR; e += nth) {
         const int l = l0 + e / (6 * NR), q = e % (6 * NR);
         const int2 a = d.inv[f.node0 + l];
-        double v = l < f.np ? r[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q] : 0.0;
-        if (a.x >= 0) v += cv[0][(int64_t)a.x * 6 * NR + q];
-        if (a.y >= 0) v += cv[1][(int64_t)a.y * 6 * NR + q];
-        dst[e] = v;
+        const double* pr = l < f.np ? r + ((int64_t)f.gnode0 + d.nodes[f.node0 + l]) * 6 * NR + q : d.zero;
+        const double* p0 = a.x >= 0 ? v0 + a.x * 6 * NR + q : d.zero;
+        const double* p1 = a.y >= 0 ? v1 + a.y * 6 * NR + q : d.zero;
+        dst[e] = *pr + *p0 + *p1;
     }
 }
-
-constexpr int FWD_ROWS = 64;   // border rows of a workgroup
 template <int NR>
-__global__ __launch_bounds__(256) void k_solve_fwd(DirectDev d, const DTask* __restrict__ tasks,
-                                                   const int32_t* __restrict__ active,
-                                                   const double* __restrict__ r, int p, int rows) {
-    __shared__ double r1[DW * NR];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
-    if (p >= f.npan) return;
+__device__ __forceinline__ bool any_active(const int32_t* __restrict__ active, int sys) {
     bool any = false;
 #pragma unroll
-    for (int h = 0; h < NR; ++h) any |= active[task.sys * NR + h] != 0;
-    if (!any) return;
-    const StructMeta st = d.st[task.sys];
+    for (int h = 0; h < NR; ++h) any |= active[sys * NR + h] != 0;
+    return any;
+}
+
+// r2 -= G r1 for one panel of every front, `rows` rows below it per workgroup; the
+// first panel gathers the vector.  Bound by the reads of G (each once).
+template <int NR>
+__global__ __launch_bounds__(256) void k_solve_fwd(DirectDev d, const FrontTask* __restrict__ tasks,
+                                                   const int32_t* __restrict__ active,
+                                                   const double* __restrict__ r, int p, int n, int parts, int rows) {
+    __shared__ double r1[DW * NR];
+    const Where at = locate(n, parts);
+    if (at.task >= n) return;
+    const FrontTask f = tasks[at.task];
+    if (p >= f.npan || !any_active<NR>(active, f.sys)) return;
     const int mn = f.np + f.nb, m = 6 * mn, p0 = p * f.wn, wn = min(f.wn, f.np - p0), w = 6 * wn, c0 = 6 * p0;
-    const int r0 = c0 + w + rows * blockIdx.y;
-    if (blockIdx.y > 0 && r0 >= m) return;
+    const int r0 = c0 + w + rows * at.part;
+    if (at.part > 0 && r0 >= m) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double* v = d.vec + (st.vec + f.vec) * NR;
+    double* v = d.vec + f.vec * NR;
     const int r1end = min(m, r0 + rows);
     if (p == 0) {
-        gather_rhs<NR>(d, f, st, r, 0, wn, r1, tid, 256);
-        gather_rhs<NR>(d, f, st, r, r0 / 6, r1end / 6, v + (int64_t)r0 * NR, tid, 256);
+        gather_rhs<NR>(d, f, r, 0, wn, r1, tid, 256);
+        gather_rhs<NR>(d, f, r, r0 / 6, r1end / 6, v + (int64_t)r0 * NR, tid, 256);
     } else {
         for (int e = tid; e < w * NR; e += 256) r1[e] = v[(int64_t)c0 * NR + e];
     }
     __threadfence_block();
     __syncthreads();
-    if (p == 0 && blockIdx.y == 0)
+    if (p == 0 && at.part == 0)
         for (int e = tid; e < w * NR; e += 256) v[e] = r1[e];
-    const double* G = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w;
-    // 16 rows per wavefront; lane: row l % 16, columns 4 (l / 16) .. + 3 of every 16
+    const double* G = d.fac + f.fac + panel_offset(m, 6 * f.wn, p) + (int64_t)w * w;
+    // 16 rows per wavefront; lane: row l % 16, columns 4 (l / 16) .. + 3 of every 16, all
+    // loads of a row in flight
     for (int row0 = r0 + 16 * wave; row0 < r1end; row0 += 64) {
-        const int row = row0 + (lane & 15);
+        const int row = row0 + (lane & 15), j0 = 4 * (lane >> 4);
         const bool on = row < r1end;
         const double* g = G + (int64_t)((on ? row : r0) - c0 - w) * w;
         double acc[NR];
 #pragma unroll
         for (int h = 0; h < NR; ++h) acc[h] = 0.0;
-        for (int j = 4 * (lane >> 4); j < w; j += 16) {
-            const double2 a = *reinterpret_cast<const double2*>(g + j);
-            const double2 c = j + 2 < w ? *reinterpret_cast<const double2*>(g + j + 2) : double2{0.0, 0.0};
-            const int j2 = j + 2 < w ? j + 2 : j;
+        constexpr int T = NR == 1 ? DW / 16 : 2;   // (more load cases: fewer loads ahead, or registers run out)
+#pragma unroll 1
+        for (int t0 = 0; 16 * t0 < w; t0 += T) {
+            double2 a[T][2];
 #pragma unroll
-            for (int h = 0; h < NR; ++h)
-                acc[h] += a.x * r1[j * NR + h] + a.y * r1[(j + 1) * NR + h] + c.x * r1[j2 * NR + h] +
-                          c.y * r1[(j2 + 1) * NR + h];
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int j = j0 + 16 * (t0 + t) + 2 * u;
+                    a[t][u] = *reinterpret_cast<const double2*>(j < w ? g + j : d.zero);
+                }
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int j = min(j0 + 16 * (t0 + t) + 2 * u, w - 2);
+#pragma unroll
+                    for (int h = 0; h < NR; ++h)
+                        acc[h] += a[t][u].x * r1[j * NR + h] + a[t][u].y * r1[(j + 1) * NR + h];
+                }
         }
 #pragma unroll
         for (int h = 0; h < NR; ++h) {
@@ -899,70 +947,60 @@ __global__ __launch_bounds__(256) void k_solve_fwd(DirectDev d, const DTask* __r
 }
 
 // x1 = S r1 - G^T x2 for one panel per workgroup; x in node order
-template <int NR>
-__global__ __launch_bounds__(512) void k_solve_bwd(DirectDev d, const DTask* __restrict__ tasks,
-                                                   const int32_t* __restrict__ active, double* __restrict__ x, int p) {
+template <int NR, int NT>
+__global__ __launch_bounds__(NT) void k_solve_bwd(DirectDev d, const FrontTask* __restrict__ tasks,
+                                                  const int32_t* __restrict__ active, double* __restrict__ x, int p) {
     extern __shared__ double P[];
-    const DTask task = tasks[blockIdx.x];
-    const FrontMeta f = d.fr[task.front];
-    if (p >= f.npan) return;
-    bool any = false;
-#pragma unroll
-    for (int h = 0; h < NR; ++h) any |= active[task.sys * NR + h] != 0;
-    if (!any) return;
-    const StructMeta st = d.st[task.sys];
+    const FrontTask f = tasks[blockIdx.x];
+    if (p >= f.npan || f.np == 0 || !any_active<NR>(active, f.sys)) return;
     const int mn = f.np + f.nb, m = 6 * mn, p0 = p * f.wn, wn = min(f.wn, f.np - p0), w = 6 * wn, c0 = 6 * p0;
-    const int tid = threadIdx.x, nth = blockDim.x, nb = m - c0 - w;
-    if (w == 0) return;
-    double* x2 = P;                          // [nb][NR]
-    double* r1 = P + (int64_t)nb * NR;       // [w][NR]
-    const double* v = d.vec + (st.vec + f.vec) * NR + (int64_t)c0 * NR;
-    for (int e = tid; e < nb * NR; e += nth) {
-        const int l = p0 + wn + e / (6 * NR), q = e % (6 * NR);
-        x2[e] = x[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q];
+    const int tid = threadIdx.x, nb = m - c0 - w;
+    double* r1 = P;                          // [w][NR], then x2 [nb][NR]: one vector for the rows of S and -G
+    const double* v = d.vec + f.vec * NR + (int64_t)c0 * NR;
+    for (int e = tid; e < (w + nb) * NR; e += NT) {
+        const int l = p0 + e / (6 * NR), q = e % (6 * NR);
+        r1[e] = e < w * NR ? v[e] : -x[((int64_t)f.gnode0 + d.nodes[f.node0 + l]) * 6 * NR + q];
     }
-    for (int e = tid; e < w * NR; e += nth) r1[e] = v[e];
     __syncthreads();
-    const double* S = d.fac + st.fac + f.fac + panel_offset(m, 6 * f.wn, p);
-    const double* G = S + (int64_t)w * w;
-    // lane pairs of columns; the groups of w / 2 threads share the rows
-    const int hw = w / 2, ng = nth / hw, g = tid / hw, j = 2 * (tid % hw);
+    const double* S = d.fac + f.fac + panel_offset(m, 6 * f.wn, p);   // w rows of S (symmetric), then G's
+    // lane pairs of columns; the groups of w / 2 threads share the rows, eight in flight
+    const int hw = w / 2, ng = NT / hw, g = tid / hw, j = 2 * (tid - g * hw);
     double acc[2][NR];
 #pragma unroll
     for (int h = 0; h < NR; ++h) acc[0][h] = acc[1][h] = 0.0;
     if (g < ng) {
-        for (int i = g; i < w; i += ng) {    // S is symmetric: row i serves as column i
-            const double2 a = *reinterpret_cast<const double2*>(S + (int64_t)i * w + j);
+        for (int i0 = g; i0 < w + nb; i0 += 8 * ng) {
+            double2 a[8];
 #pragma unroll
-            for (int h = 0; h < NR; ++h) {
-                acc[0][h] += a.x * r1[i * NR + h];
-                acc[1][h] += a.y * r1[i * NR + h];
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + u * ng;
+                a[u] = *reinterpret_cast<const double2*>(i < w + nb ? S + (int64_t)i * w + j : d.zero);
             }
-        }
-#pragma unroll 4
-        for (int i = g; i < nb; i += ng) {
-            const double2 a = *reinterpret_cast<const double2*>(G + (int64_t)i * w + j);
 #pragma unroll
-            for (int h = 0; h < NR; ++h) {
-                acc[0][h] -= a.x * x2[i * NR + h];
-                acc[1][h] -= a.y * x2[i * NR + h];
+            for (int u = 0; u < 8; ++u) {
+                const int i = min(i0 + u * ng, w + nb - 1);
+#pragma unroll
+                for (int h = 0; h < NR; ++h) {
+                    acc[0][h] += a[u].x * r1[i * NR + h];
+                    acc[1][h] += a[u].y * r1[i * NR + h];
+                }
             }
         }
     }
-    double* red = r1 + w * NR;               // [ng][w][NR]
+    double* red = r1 + (w + nb) * NR;        // [ng][w][NR]
     if (g < ng) {
 #pragma unroll
         for (int h = 0; h < NR; ++h) {
-            red[(int64_t)(g * w + j) * NR + h] = acc[0][h];
-            red[(int64_t)(g * w + j + 1) * NR + h] = acc[1][h];
+            red[(g * w + j) * NR + h] = acc[0][h];
+            red[(g * w + j + 1) * NR + h] = acc[1][h];
         }
     }
     __syncthreads();
-    for (int e = tid; e < w * NR; e += nth) {
+    for (int e = tid; e < w * NR; e += NT) {
         double s = 0.0;
-        for (int q = 0; q < ng; ++q) s += red[(int64_t)q * w * NR + e];
+        for (int q = 0; q < ng; ++q) s += red[q * w * NR + e];
         const int l = p0 + e / (6 * NR), q = e % (6 * NR);
-        x[((int64_t)st.node0 + d.nodes[f.node0 + l]) * 6 * NR + q] = s;
+        x[((int64_t)f.gnode0 + d.nodes[f.node0 + l]) * 6 * NR + q] = s;
     }
 }
 
@@ -1176,8 +1214,8 @@ struct Arena {
     }
 };
 
-static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nodes, std::vector<int32_t>& rel,
-                             std::vector<int32_t>& blk, std::vector<int32_t>& blkrow, std::vector<int2>& inv) {
+static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nodes, std::vector<int32_t>& blk,
+                             std::vector<int32_t>& blkrow, std::vector<int2>& inv) {
     const auto& off = pl->h_node_off;
     struct Cls {
         int32_t fr0, n_fr, sys;
@@ -1185,7 +1223,11 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
     };
     std::vector<Cls> cls;
     std::map<uint64_t, std::vector<int>> by_hash;
-    D.st.resize(pl->n_sys);
+    std::vector<FrontMeta> fr;
+    struct Base {
+        int64_t fac, mat, vec;
+    };
+    std::vector<Base> base(pl->n_sys);
     std::vector<int32_t> lrp, lci, cls_of(pl->n_sys);
     for (int s = 0; s < pl->n_sys; ++s) {
         const int32_t n0 = off[s], n = off[s + 1] - n0, b0 = pl->h_rowptr[n0];
@@ -1213,7 +1255,7 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
             for (int k = 0; k < nb; ++k) lci[k] = pl->h_colind[b0 + k] - n0;
             FrontTree T;
             build_fronts(n, lrp.data(), lci.data(), DLEAF, T);
-            Cls C{(int32_t)D.fr.size(), (int32_t)T.fronts.size(), s, 0, 0, 0};
+            Cls C{(int32_t)fr.size(), (int32_t)T.fronts.size(), s, 0, 0, 0};
             const int32_t node_base = (int32_t)nodes.size(), blk_base = (int32_t)(blk.size() / 3);
             for (size_t t = 0; t < T.fronts.size(); ++t) {
                 const auto& F = T.fronts[t];
@@ -1247,12 +1289,12 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
                 D.flops += kd * kd * kd + 2 * bd * kd * kd + bd * bd * kd;
                 D.n_levels = std::max(D.n_levels, F.level + 1);
                 D.max_m = std::max(D.max_m, m);
-                D.fr.push_back(M);
+                fr.push_back(M);
             }
             // storage: level by level, a child's matrix is free once its parent's level is done
             std::vector<std::vector<int32_t>> lev;
             for (int t = 0; t < C.n_fr; ++t) {
-                const int L = D.fr[C.fr0 + t].level;
+                const int L = fr[C.fr0 + t].level;
                 if ((int)lev.size() <= L) lev.resize(L + 1);
                 lev[L].push_back(C.fr0 + t);
             }
@@ -1261,31 +1303,29 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
             auto cols = [](const FrontMeta& M) { return M.small ? 0 : (int64_t)36 * (M.np + M.nb) * M.np; };
             for (auto& L : lev) {
                 for (int t : L) {
-                    D.fr[t].mat = A.take(cb(D.fr[t]));
-                    D.fr[t].pan = A.take(cols(D.fr[t]));
+                    fr[t].mat = A.take(cb(fr[t]));
+                    fr[t].pan = A.take(cols(fr[t]));
                 }
                 for (int t : L) {
-                    A.give(D.fr[t].pan, cols(D.fr[t]));
-                    for (int c : D.fr[t].child)
-                        if (c >= 0) A.give(D.fr[c].mat, cb(D.fr[c]));
+                    A.give(fr[t].pan, cols(fr[t]));
+                    for (int c : fr[t].child)
+                        if (c >= 0) A.give(fr[c].mat, cb(fr[c]));
                 }
             }
             C.mat = A.top;
             inv.resize(inv.size() + T.nodes.size(), int2{-1, -1});
             for (size_t t = 0; t < T.fronts.size(); ++t)
                 for (int c = 0; c < 2; ++c) {
-                    const int ch = D.fr[C.fr0 + t].child[c];
+                    const int ch = fr[C.fr0 + t].child[c];
                     if (ch < 0) continue;
-                    FrontMeta& G = D.fr[ch];
+                    const FrontMeta& G = fr[ch];
                     const int32_t* rl = T.rel.data() + T.fronts[ch - C.fr0].node0 + G.np;
                     for (int l = 0; l < G.nb; ++l) {
-                        int2& a = inv[D.fr[C.fr0 + t].node0 + rl[l]];
+                        int2& a = inv[fr[C.fr0 + t].node0 + rl[l]];
                         (c ? a.y : a.x) = l;
-                        G.npre += rl[l] < D.fr[C.fr0 + t].np;
                     }
                 }
             nodes.insert(nodes.end(), T.nodes.begin(), T.nodes.end());
-            rel.insert(rel.end(), T.rel.begin(), T.rel.end());
             blk.insert(blk.end(), T.blk.begin(), T.blk.end());
             for (int32_t q : T.blkrow) blkrow.push_back(blk_base + q);
             found = (int)cls.size();
@@ -1294,20 +1334,19 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
         } else {
             const Cls& C = cls[found];
             for (int t = 0; t < C.n_fr; ++t) {
-                const double kd = 6 * D.fr[C.fr0 + t].np, bd = 6 * D.fr[C.fr0 + t].nb;
+                const double kd = 6 * fr[C.fr0 + t].np, bd = 6 * fr[C.fr0 + t].nb;
                 D.flops += kd * kd * kd + 2 * bd * kd * kd + bd * bd * kd;
             }
         }
         cls_of[s] = found;
         const Cls& C = cls[found];
-        D.st[s] = StructMeta{(int64_t)D.fac_n, (int64_t)D.mat_n, (int64_t)D.vec_n, n0, b0};
+        base[s] = Base{(int64_t)D.fac_n, (int64_t)D.mat_n, (int64_t)D.vec_n};
         D.fac_n += C.fac;
         D.mat_n += C.mat;
         D.vec_n += C.vec;
     }
     D.small_tasks.resize(D.n_levels);
     D.big_tasks.resize(D.n_levels);
-    D.small_lds.assign(D.n_levels, 0);
     D.small_m.assign(D.n_levels, 0);
     D.big_m.assign(D.n_levels, 0);
     D.big_k.assign(D.n_levels, 0);
@@ -1317,14 +1356,23 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
     for (int s = 0; s < pl->n_sys; ++s) {
         const Cls& C = cls[cls_of[s]];
         for (int t = C.fr0; t < C.fr0 + C.n_fr; ++t) {
-            const FrontMeta& M = D.fr[t];
+            const FrontMeta& M = fr[t];
             if (M.np == 0 && M.nb == 0) continue;   // (joins components: nothing to do)
+            const Base& B = base[s];
+            FrontTask T{M.np, M.nb, M.wn, M.npan, M.node0, M.blk0, M.nblk, pl->h_rowptr[off[s]], s, off[s], {0, 0},
+                        B.mat + M.mat, B.mat + M.pan, B.fac + M.fac, B.vec + M.vec, {0, 0}, {0, 0}};
+            for (int c = 0; c < 2; ++c)
+                if (M.child[c] >= 0) {
+                    const FrontMeta& G = fr[M.child[c]];
+                    T.cb[c] = G.nb;
+                    T.cmat[c] = B.mat + G.mat;
+                    T.cvec[c] = B.vec + G.vec + 6 * G.np;
+                }
             if (M.small) {
-                D.small_tasks[M.level].push_back({t, s});
+                D.small_tasks[M.level].push_back(T);
                 if (M.np) D.small_m[M.level] = std::max(D.small_m[M.level], 6 * (M.np + M.nb));
-                D.small_lds[M.level] = std::max(D.small_lds[M.level], small_front_lds(M.np, M.nb));
             } else {
-                D.big_tasks[M.level].push_back({t, s});
+                D.big_tasks[M.level].push_back(T);
                 D.big_m[M.level] = std::max(D.big_m[M.level], 6 * (M.np + M.nb));
                 D.big_k[M.level] = std::max(D.big_k[M.level], 6 * M.np);
                 D.big_b[M.level] = std::max(D.big_b[M.level], 6 * M.nb);
@@ -1373,45 +1421,67 @@ static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b);
 // builds the analysis and its storage; leaves D.usable false where the direct
 // solve is not the better choice or does not fit
 static int direct_build(Plan* pl, DirectState& D) {
-    std::vector<int32_t> nodes, rel, blk, blkrow;
+    std::vector<int32_t> nodes, blk, blkrow;
     std::vector<int2> inv;
-    if (direct_build_host(pl, D, nodes, rel, blk, blkrow, inv) != JSSO_OK) return JSSO_OK;
+    if (direct_build_host(pl, D, nodes, blk, blkrow, inv) != JSSO_OK) return JSSO_OK;
     size_t free_b = 0, total_b = 0;
     JSSO_HIP(hipMemGetInfo(&free_b, &total_b));
     if (!direct_fits(D, free_b, total_b)) return JSSO_OK;
     int rc = 0;
-    std::vector<DTask> tasks;
+    std::vector<FrontTask> tasks;
+    D.buckets.resize(D.n_levels);
     for (int L = 0; L < D.n_levels; ++L) {
-        D.small_off.push_back((int64_t)tasks.size());
+        // small fronts by the LDS they need: 3, 2 or 1 workgroups per CU, of as many
+        // threads as then fill it.  Fewer fronts than CUs go in one launch.
+        auto& st = D.small_tasks[L];
+        auto lds = [](const FrontTask& t) { return small_front_lds(t.np, t.nb); };
+        std::stable_sort(st.begin(), st.end(),
+                         [&](const FrontTask& x, const FrontTask& y) { return lds(x) > lds(y); });
+        constexpr size_t limit[3] = {78 * 1024, 52 * 1024, 0};
+        for (size_t i = 0; i < st.size();) {
+            const size_t need = lds(st[i]);
+            const int c = need > limit[0] ? 0 : need > limit[1] ? 1 : 2;
+            size_t j = st.size();
+            if (st.size() > 512)
+                for (j = i; j < st.size() && lds(st[j]) > limit[c];) ++j;
+            D.buckets[L].push_back({need, tasks.size() + i, j - i, 1024 >> c});
+            i = j;
+        }
+        D.small_off.push_back(tasks.size());
+        D.small_n.push_back(D.small_tasks[L].size());
         tasks.insert(tasks.end(), D.small_tasks[L].begin(), D.small_tasks[L].end());
-        D.big_off.push_back((int64_t)tasks.size());
+        D.big_off.push_back(tasks.size());
+        D.big_n.push_back(D.big_tasks[L].size());
         tasks.insert(tasks.end(), D.big_tasks[L].begin(), D.big_tasks[L].end());
     }
-    const DTask* dt = nullptr;
+    D.small_tasks.clear();
+    D.big_tasks.clear();
     // ||A||_2 <= 4: with identity diagonal blocks, x^T A x = sum_e x_e^T A_e x_e is at most
     // (nodes of an element) x sum_e x_e^T diag(A_e) x_e = (nodes of an element) ||x||^2
     std::vector<double> rho(pl->n_sys, 4.0);
     const double* dr = nullptr;
-    if ((rc = direct_upload(D, &D.dev.fr, D.fr)) || (rc = direct_upload(D, &D.dev.st, D.st)) ||
-        (rc = direct_upload(D, &D.dev.nodes, nodes)) || (rc = direct_upload(D, &D.dev.rel, rel)) ||
-        (rc = direct_upload(D, &D.dev.inv, inv)) || (rc = direct_upload(D, &D.dev.blk, blk)) || (rc = direct_upload(D, &D.dev.blkrow, blkrow)) ||
-        (rc = direct_upload(D, &D.dev.kref, pl->h_kref)) || (rc = direct_upload(D, &dt, tasks)) ||
-        (rc = direct_upload(D, &dr, rho)) || (rc = direct_alloc(D, &D.d_report, 1)) || (rc = direct_alloc(D, &D.dev.fac, D.fac_n)) ||
-        (rc = direct_alloc(D, &D.dev.mat, D.mat_n)) || (rc = direct_alloc(D, &D.dev.bad, pl->n_sys)) || (rc = direct_upload(D, &D.dev.zero, std::vector<double>(2, 0.0)))) {
+    if ((rc = direct_upload(D, &D.dev.nodes, nodes)) || (rc = direct_upload(D, &D.dev.inv, inv)) ||
+        (rc = direct_upload(D, &D.dev.blk, blk)) || (rc = direct_upload(D, &D.dev.blkrow, blkrow)) ||
+        (rc = direct_upload(D, &D.dev.kref, pl->h_kref)) || (rc = direct_upload(D, &D.d_tasks, tasks)) ||
+        (rc = direct_upload(D, &dr, rho)) || (rc = direct_alloc(D, &D.d_report, 1)) ||
+        (rc = direct_alloc(D, &D.dev.fac, D.fac_n)) || (rc = direct_alloc(D, &D.dev.mat, D.mat_n)) ||
+        (rc = direct_alloc(D, &D.dev.bad, pl->n_sys)) ||
+        (rc = direct_upload(D, &D.dev.zero, std::vector<double>(2, 0.0)))) {
         for (void* a : D.allocs) (void)hipFree(a);
         D.allocs.clear();
         return rc == JSSO_ENOMEM ? JSSO_OK : rc;
     }
     JSSO_HIP(hipHostMalloc((void**)&D.h_report, sizeof(DirectReport), hipHostMallocDefault));
-    D.d_tasks = const_cast<DTask*>(dt);
     D.d_rho = const_cast<double*>(dr);
     D.dev.A64 = pl->d_Ke64;
     const std::pair<const void*, size_t> lds[] = {
         {(const void*)k_front_small<1024>, DLDS_MAX}, {(const void*)k_front_small<512>, DLDS_MAX},
         {(const void*)k_front_small<256>, DLDS_MAX},  {(const void*)k_front_diag, DW * (DW + 2) * 8},
         {(const void*)k_front_strip, (DW + SROWS) * (DW + 2) * 8},
-        {(const void*)k_solve_bwd<1>, DLDS_MAX},      {(const void*)k_solve_bwd<2>, DLDS_MAX},
-        {(const void*)k_solve_bwd<3>, DLDS_MAX},      {(const void*)k_solve_bwd<4>, DLDS_MAX}};
+        {(const void*)k_solve_bwd<1, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<1, 1024>, DLDS_MAX},
+        {(const void*)k_solve_bwd<2, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<2, 1024>, DLDS_MAX},
+        {(const void*)k_solve_bwd<3, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<3, 1024>, DLDS_MAX},
+        {(const void*)k_solve_bwd<4, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<4, 1024>, DLDS_MAX}};
     for (const auto& l : lds)
         JSSO_HIP(hipFuncSetAttribute(l.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.second));
     D.usable = true;
@@ -1422,34 +1492,35 @@ static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
     JSSO_HIP(hipMemsetAsync(D.dev.bad, 0, pl->n_sys * sizeof(int32_t), s));
     static_assert((DW + SROWS) * (DW + 2) * 8 <= DLDS_MAX, "panel LDS");
     for (int L = 0; L < D.n_levels; ++L) {
-        const size_t ns = D.small_tasks[L].size(), nb = D.big_tasks[L].size();
-        if (ns) {
-            const int th = D.small_lds[L] > 78 * 1024 ? 1024 : D.small_lds[L] > 52 * 1024 ? 512 : 256;
-            const DTask* t = D.d_tasks + D.small_off[L];
-            const size_t lds = D.small_lds[L];
-            if (th == 1024)
-                hipLaunchKernelGGL(k_front_small<1024>, dim3((unsigned)ns), dim3(1024), lds, s, D.dev, t);
-            else if (th == 512)
-                hipLaunchKernelGGL(k_front_small<512>, dim3((unsigned)ns), dim3(512), lds, s, D.dev, t);
+        for (const auto& B : D.buckets[L]) {
+            const FrontTask* t = D.d_tasks + B.off;
+            const dim3 g((unsigned)B.n);
+            if (B.threads == 1024)
+                hipLaunchKernelGGL(k_front_small<1024>, g, dim3(1024), B.lds, s, D.dev, t);
+            else if (B.threads == 512)
+                hipLaunchKernelGGL(k_front_small<512>, g, dim3(512), B.lds, s, D.dev, t);
             else
-                hipLaunchKernelGGL(k_front_small<256>, dim3((unsigned)ns), dim3(256), lds, s, D.dev, t);
+                hipLaunchKernelGGL(k_front_small<256>, g, dim3(256), B.lds, s, D.dev, t);
         }
+        const int nb = (int)D.big_n[L];
         if (nb) {
-            const DTask* t = D.d_tasks + D.big_off[L];
-            const int m = D.big_m[L], strips = (m + DROWS - 1) / DROWS;
-            const int kw = (D.big_w[L] + 15) & ~15;   // widest panel
+            const FrontTask* t = D.d_tasks + D.big_off[L];
+            const int m = D.big_m[L], kw = (D.big_w[L] + 15) & ~15;   // largest front, widest panel
+            // strips of 96 rows, or of 32 while that leaves CUs without work
+            const int rows = (int64_t)nb * ((m + SROWS - 1) / SROWS) >= 512 ? SROWS : 32;
             for (int p = 0; p < D.big_pan[L]; ++p) {
-                hipLaunchKernelGGL(k_front_diag, dim3((unsigned)nb), dim3(512), (size_t)kw * (kw + 2) * 8, s, D.dev, t,
-                                   p);
-                hipLaunchKernelGGL(k_front_strip, dim3((unsigned)nb, (m + SROWS - 1) / SROWS), dim3(1024),
-                                   (size_t)(kw + SROWS) * (kw + 2) * 8, s, D.dev, t, p);
-                if (p + 1 < D.big_pan[L])
-                    hipLaunchKernelGGL(k_front_cols, dim3((unsigned)nb, strips, (D.big_k[L] + DROWS - 1) / DROWS),
-                                       dim3(256), 0, s, D.dev, t, p);
+                hipLaunchKernelGGL(k_front_diag, dim3(nb), dim3(512), (size_t)kw * (kw + 2) * 8, s, D.dev, t, p);
+                const int strips = (m + rows - 1) / rows;
+                hipLaunchKernelGGL(k_front_strip, part_grid(nb, strips), dim3(1024),
+                                   (size_t)(kw + rows) * (kw + 2) * 8, s, D.dev, t, p, nb, strips, rows);
+                if (p + 1 < D.big_pan[L]) {
+                    const int tiles = ((m + DROWS - 1) / DROWS) * ((D.big_k[L] + DROWS - 1) / DROWS);
+                    hipLaunchKernelGGL(k_front_cols, part_grid(nb, tiles), dim3(256), 0, s, D.dev, t, p, nb, tiles);
+                }
             }
-            const int bt = (D.big_b[L] + DROWS - 1) / DROWS;
+            const int bt = (D.big_b[L] + DROWS - 1) / DROWS, tiles = bt * (bt + 1) / 2;
             if (bt)
-                hipLaunchKernelGGL(k_front_cb, dim3((unsigned)nb, bt * (bt + 1) / 2), dim3(256), 0, s, D.dev, t);
+                hipLaunchKernelGGL(k_front_cb, part_grid(nb, tiles), dim3(256), 0, s, D.dev, t, nb, tiles);
         }
     }
     JSSO_HIP(hipGetLastError());
@@ -1460,28 +1531,29 @@ static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
 // z = M^-1 r (both in node order, [dof][NR])
 template <int NR>
 static void direct_apply(DirectState& D, const int32_t* active, const double* r, double* z, hipStream_t s) {
-    for (int L = 0; L < D.n_levels; ++L)
-        for (int big = 0; big < 2; ++big) {
-            const size_t n = big ? D.big_tasks[L].size() : D.small_tasks[L].size();
-            if (!n) continue;
-            const DTask* t = D.d_tasks + (big ? D.big_off[L] : D.small_off[L]);
-            const int rows = big ? FWD_ROWS * 3 : 8192;   // a multiple of 6
-            const int ny = big ? std::max(1, (D.big_m[L] + rows - 1) / rows) : 1;
-            for (int p = 0; p < (big ? D.big_pan[L] : 1); ++p)
-                hipLaunchKernelGGL((k_solve_fwd<NR>), dim3((unsigned)n, ny), dim3(256), 0, s, D.dev, t, active, r, p,
-                                   rows / 6 * 6);
-        }
-    for (int L = D.n_levels - 1; L >= 0; --L)
-        for (int big = 0; big < 2; ++big) {
-            const size_t n = big ? D.big_tasks[L].size() : D.small_tasks[L].size();
-            if (!n) continue;
-            const DTask* t = D.d_tasks + (big ? D.big_off[L] : D.small_off[L]);
-            const int th = big ? 512 : 256;
-            const int m = big ? D.big_m[L] : D.small_m[L];
-            const size_t lds = ((size_t)m + DW + 2 * th) * NR * 8;
-            for (int p = (big ? D.big_pan[L] : 1) - 1; p >= 0; --p)
-                hipLaunchKernelGGL((k_solve_bwd<NR>), dim3((unsigned)n), dim3(th), lds, s, D.dev, t, active, z, p);
-        }
+    for (int L = 0; L < D.n_levels; ++L) {
+        if (D.small_n[L])
+            hipLaunchKernelGGL((k_solve_fwd<NR>), part_grid(D.small_n[L], 1), dim3(256), 0, s, D.dev,
+                               D.d_tasks + D.small_off[L], active, r, 0, (int)D.small_n[L], 1, 1 << 20);
+        const int nb = (int)D.big_n[L];
+        if (!nb) continue;
+        const int rows = nb * ((D.big_m[L] + 191) / 192) >= 512 ? 192 : 48;   // (multiples of 6)
+        const int parts = (D.big_m[L] + rows - 1) / rows;
+        for (int p = 0; p < D.big_pan[L]; ++p)
+            hipLaunchKernelGGL((k_solve_fwd<NR>), part_grid(nb, parts), dim3(256), 0, s, D.dev,
+                               D.d_tasks + D.big_off[L], active, r, p, nb, parts, rows);
+    }
+    for (int L = D.n_levels - 1; L >= 0; --L) {
+        const int nb = (int)D.big_n[L];
+        for (int p = D.big_pan[L] - 1; nb && p >= 0; --p)
+            hipLaunchKernelGGL((k_solve_bwd<NR, 1024>), dim3(nb), dim3(1024),
+                               ((size_t)D.big_m[L] + 2 * 1024) * NR * 8, s, D.dev, D.d_tasks + D.big_off[L], active, z,
+                               p);
+        if (D.small_n[L])
+            hipLaunchKernelGGL((k_solve_bwd<NR, 256>), dim3((unsigned)D.small_n[L]), dim3(256),
+                               ((size_t)D.small_m[L] + 2 * 256) * NR * 8, s, D.dev, D.d_tasks + D.small_off[L], active,
+                               z, 0);
+    }
 }
 
 static int direct_vectors(DirectState& D, int nrhs, bool& have) {
@@ -1622,11 +1694,12 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
 // The direct solve is taken where its fronts stay small: fill and operations grow
 // with the largest front (m rows: m^2 storage, m^3 operations), while the
 // AMG-preconditioned CG grows with the number of nodes.  One shell of n x n quads
-// has m ~ 9 n: measured per solve with its set-up, 40x40 (m = 366) 1.06 against
-// 3.87 ms, 100x100 (m = 912) 2.5 against 3.0 ms, 200x200 (m = 1812) 6.6 against
-// 6.5 ms; batches gain more (64 SIMP shells of 100x100: 35 against 56 ms), since
-// they fill the chip on every tree level.  It needs its storage too: up to an
-// eighth of the card, and half of what is free.
+// has m ~ 9 n: assembly and solve of one smooth shell, ms direct / AMG: 40x40
+// (m = 366) 0.86 / 3.85, 100x100 2.1 / 3.1, 200x200 5.7 / 6.5, 250x250 (m = 2256)
+// 8.1 / 8.1, 300x300 12.0 / 9.1.  Designs that take the CG more iterations gain more
+// (a 200x200 SIMP shell 7.8 / 21), and so do batches, which fill the chip on every
+// tree level (64 SIMP shells of 100x100: 33 / 59).  It needs its storage too: up to
+// an eighth of the card, and half of what is free.
 static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b) {
     const size_t need = (D.fac_n + D.mat_n) * 8;
     return D.max_m <= DIRECT_MAX_M && need <= total_b / 8 && need <= free_b / 2;
