@@ -122,6 +122,10 @@ class SSO_model:
             ep = np.asarray(self.eleparameters_props, dtype=np.int64)
             bc = torch.as_tensor(self.parameters_bc, device=dev)
             qd = torch.as_tensor(self.parameters_quads, device=dev)
+            # (all element parameters of one type: their values need no selection, whose
+            # backward would sort the indices)
+            bc = None if len(self.parameters_bc) == len(et) else bc
+            qd = None if len(self.parameters_quads) == len(et) else qd
             self._index_cache = (dev, tags, xyz,
                                  torch.as_tensor(et[self.parameters_bc], device=dev),
                                  torch.as_tensor(ep[self.parameters_bc], device=dev), bc,
@@ -129,21 +133,23 @@ class SSO_model:
                                  torch.as_tensor(ep[self.parameters_quads], device=dev), qd)
         return self._index_cache
 
-    def node_params_crds(self, nodeparameter_values):
+    def node_params_crds(self, nodeparameter_values, crds=None):
         v = _to_dev(nodeparameter_values)
         ix = self._indices(v.device)
-        crds = torch.as_tensor(self.model.crds, dtype=torch.float64, device=v.device)
+        if crds is None:
+            crds = torch.as_tensor(self.model.crds, dtype=torch.float64, device=v.device)
         return crds.index_put((ix[1], ix[2]), v)
 
-    def ele_params_props(self, eleparameter_values):
+    def ele_params_props(self, eleparameter_values, pb=None, pq=None):
         v = _to_dev(eleparameter_values)
         ix = self._indices(v.device)
-        pb = torch.as_tensor(self.model.prop_beamcols, dtype=torch.float64, device=v.device)
-        pq = torch.as_tensor(self.model.prop_quads, dtype=torch.float64, device=v.device)
+        if pb is None or pq is None:
+            pb = torch.as_tensor(self.model.prop_beamcols, dtype=torch.float64, device=v.device)
+            pq = torch.as_tensor(self.model.prop_quads, dtype=torch.float64, device=v.device)
         if len(self.parameters_bc):
-            pb = pb.index_put((ix[3], ix[4]), v[ix[5]])
+            pb = pb.index_put((ix[3], ix[4]), v if ix[5] is None else v[ix[5]])
         if len(self.parameters_quads):
-            pq = pq.index_put((ix[6], ix[7]), v[ix[8]])
+            pq = pq.index_put((ix[6], ix[7]), v if ix[8] is None else v[ix[8]])
         return pb, pq
 
     def set_node_filter(self, B):
@@ -176,19 +182,15 @@ class SSO_model:
 
     def _inputs(self, parameter_values):
         p = _to_dev(parameter_values)
+        m = self.model
+        crds, pb, pq, f = _upload(p.device, m.crds, m.prop_beamcols, m.prop_quads, m.nodal_loads)
         if self.n_node_params > 0:
             v = p[:self.n_node_params]
             if self._node_filter is not None:
                 v = self._node_filter(v)
-            crds = self.node_params_crds(v)
-        else:
-            crds = torch.as_tensor(self.model.crds, dtype=torch.float64, device=p.device)
+            crds = self.node_params_crds(v, crds)
         if self.n_ele_params > 0:
-            pb, pq = self.ele_params_props(p[self.n_node_params:])
-        else:
-            pb = torch.as_tensor(self.model.prop_beamcols, dtype=torch.float64, device=p.device)
-            pq = torch.as_tensor(self.model.prop_quads, dtype=torch.float64, device=p.device)
-        f = torch.as_tensor(self.model.nodal_loads, dtype=torch.float64, device=p.device)
+            pb, pq = self.ele_params_props(p[self.n_node_params:], pb, pq)
         return crds, pb, pq, f
 
     def _opts(self, which_solver, enforce_scipy_sparse):
@@ -257,7 +259,24 @@ class SSO_model:
         p = _to_dev(self.parameter_values).clone().requires_grad_(True)
         val = self.helper_params_to_objective(p, which_solver, enforce_scipy_sparse)
         (g,) = torch.autograd.grad(val, p)
-        return float(val.detach()), g.detach().cpu().numpy()
+        out = torch.cat([val.detach().reshape(1).to(g), g.detach()]).cpu()   # one copy back
+        return float(out[0]), out[1:].numpy()
+
+
+def _upload(dev, *arrays):
+    """Host arrays as FP64 tensors on ``dev``, in one copy from pinned memory (a pageable
+    copy per array waits for each in turn).  Every array starts on a 128-byte boundary.
+    Tensors that a caller put into the model are taken as they are."""
+    if any(isinstance(a, torch.Tensor) for a in arrays):
+        return [torch.as_tensor(a, dtype=torch.float64, device=dev) for a in arrays]
+    arrays = [np.asarray(a, dtype=np.float64) for a in arrays]
+    at = np.cumsum([0] + [-(-a.size // 16) * 16 for a in arrays])
+    host = torch.empty(int(at[-1]), dtype=torch.float64, pin_memory=True)
+    view = host.numpy()
+    for o, a in zip(at, arrays):
+        view[o:o + a.size] = a.ravel()
+    all_ = host.to(dev, non_blocking=True)
+    return [all_[o:o + a.size].view(a.shape) for o, a in zip(at.tolist(), arrays)]
 
 
 def _to_host(x):

@@ -57,8 +57,8 @@ class _Displacement(torch.autograd.Function):
     @staticmethod
     def forward(ctx, crds, prop_beam, prop_quad, f, plan: FEPlan, opts: SolveOptions):
         plan.assemble(crds, prop_beam, prop_quad)
+        ctx.plan, ctx.opts, ctx.assembly_id = plan, opts, plan.assembly_id
         u = _solve(plan, f, opts)
-        ctx.plan, ctx.opts = plan, opts
         ctx.save_for_backward(crds, prop_beam, prop_quad, u)
         return u
 
@@ -66,7 +66,9 @@ class _Displacement(torch.autograd.Function):
     def backward(ctx, u_bar):
         crds, pb, pq, u = ctx.saved_tensors
         plan, opts = ctx.plan, ctx.opts
-        plan.ensure_assembled(crds, pb, pq)  # the plan may have been re-assembled since forward
+        # the plan may have been re-assembled since forward; otherwise its K and its factors are
+        # those of the saved tensors (which autograd refuses to hand out once they were changed)
+        ctx.assembly_id = plan.ensure_assembled(crds, pb, pq, ctx.assembly_id)
         lam = _solve(plan, u_bar.contiguous(), opts, transpose=True)
         need = ctx.needs_input_grad
         dc, db, dq = _grads(plan, crds, pb, pq, u, lam, 0.0, need)
@@ -78,8 +80,8 @@ class _Compliance(torch.autograd.Function):
     @staticmethod
     def forward(ctx, crds, prop_beam, prop_quad, f, plan: FEPlan, opts: SolveOptions):
         plan.assemble(crds, prop_beam, prop_quad)
+        ctx.plan, ctx.opts, ctx.assembly_id = plan, opts, plan.assembly_id
         u = _solve(plan, f, opts)
-        ctx.plan, ctx.opts = plan, opts
         ctx.save_for_backward(crds, prop_beam, prop_quad, u, f)
         C = 0.5 * (f * u).sum(0) if f.dim() == 2 else 0.5 * torch.dot(f, u)
         ctx.mark_non_differentiable(u)
@@ -90,7 +92,9 @@ class _Compliance(torch.autograd.Function):
         crds, pb, pq, u, f = ctx.saved_tensors
         plan = ctx.plan
         need = ctx.needs_input_grad
-        plan.ensure_assembled(crds, pb, pq)  # the plan may have been re-assembled since forward
+        # the plan may have been re-assembled since forward; otherwise its K and its factors are
+        # those of the saved tensors (which autograd refuses to hand out once they were changed)
+        ctx.assembly_id = plan.ensure_assembled(crds, pb, pq, ctx.assembly_id)
         if plan.symmetric():
             dc, db, dq = _grads(plan, crds, pb, pq, u, None, 0.5, need, weight=C_bar)
             f_bar = (u * C_bar) if need[3] else None   # dC/df = K^-1 f = u

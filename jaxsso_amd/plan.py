@@ -51,7 +51,7 @@ class FEPlan:
         self.preconditioner = "amg"   # the library's default
         self._pc_chosen = False       # by the caller: until then the library may solve directly
         self.last_info = None
-        self._assembled_key = None
+        self.assembly_id = 0          # counts the assemblies: names the one the plan holds
 
     def __del__(self):
         h = getattr(self, "_h", None)
@@ -77,15 +77,16 @@ class FEPlan:
         pq = _dev64(prop_quad) if self.n_quad else None
         assert crds.shape == (self.n_nodes, 3)
         Kout = torch.empty((self.nnzb, 6, 6), dtype=torch.float64, device=crds.device) if export_K else None
+        self.assembly_id += 1         # before the call: one that fails leaves no earlier K either
         nat.check(L.jsso_assemble(self._h, nat.ptr(crds), nat.ptr(pb), nat.ptr(pq), nat.ptr(Kout), nat.stream_ptr()))
-        self._keep = (crds, pb, pq)
         return Kout
 
-    def ensure_assembled(self, crds, prop_beam, prop_quad):
-        """Assemble unless the plan's current assembly was made from these very tensors."""
-        k = getattr(self, "_keep", None)
-        if k is None or k[0] is not crds or k[1] is not prop_beam or k[2] is not prop_quad:
+    def ensure_assembled(self, crds, prop_beam, prop_quad, assembly_id):
+        """Assemble again unless the plan still holds assembly ``assembly_id`` (the caller
+        answers for it being that of these inputs).  Returns the id it holds now."""
+        if self.assembly_id != assembly_id:
             self.assemble(crds, prop_beam, prop_quad)
+        return self.assembly_id
 
     def symmetric(self) -> bool:
         """False when the last assembly holds beam-columns parallel to global Y (the
