@@ -2,7 +2,7 @@
 // kernels.  Element math lives in element_math.hpp.
 #include <mutex>
 
-#include "element_math.hpp"
+#include "quad_adjoint.hpp"
 #include "jsso_internal.hpp"
 
 namespace jsso {
@@ -505,7 +505,7 @@ int launch_quad_gauss(int32_t n, const double* xy, const double* props, double r
 
 // ---------------------------------------------------------------------------
 // Adjoint of the element energy phi = -lam_e^T K_e u_e.  Beams: in closed form.
-// Quads: dual numbers seeded on an input, whose tangent is dphi/dp (adj_quad_*).
+// Quads: in reverse mode, a Gauss point per lane.
 // Beam directions: 6 coordinates, then E,G,Iy,Iz,J,A.
 // Quad directions: 12 coordinates, then t,E,nu,kx_mod,ky_mod.
 // gbuf[(elem_dir) * nrhs + rhs] receives dphi/dp (coordinate directions);
@@ -638,127 +638,155 @@ __global__ __launch_bounds__(256) void adj_beam_kernel(int32_t n, const int32_t*
     }
 }
 
-// Quad adjoint for load case `rhs`.  phi = lambda_e^T K_e u_e depends on the
-// coordinates only through the frame R and the in-plane coordinates xy
-// (element_math.hpp), so it is differentiated in three kernels that each run
-// uniform wavefronts:
-//   adj_quad_fwd:     forward mode in one free in-plane coordinate (k < 6: dphi/dxy
-//                     into the element's gbuf slot k) or one property (k >= 6:
-//                     dprop), with R and the local nodal values plain doubles;
-//   adj_quad_frame:   dphi/dR by reverse mode (gbuf slots 6..14);
-//   adj_quad_combine: thread (element, coordinate p) applies the frame's Jacobian
-//                     column dc_p (forward mode through quad_frame) to those 15
-//                     partials and overwrites slot p.
-// The result equals forward mode through the whole element per coordinate (to
-// rounding) at about half the work, and without the dual frame and nodal values
-// that made that form spill.
-__device__ constexpr int QA_XY_FREE[6] = {0, 1, 2, 3, 6, 7};   // xy[4] = xy[5] = 0: node 3 is the origin
-constexpr int QA_FWD = 11;                                      // 6 in-plane coordinates + 5 properties
-constexpr int QA_E = 32;                                        // elements per combine workgroup
-
-__device__ __forceinline__ void quad_geometry(int64_t e, const int32_t* __restrict__ cnct,
-                                              const double* __restrict__ crds, int nd[4], V3<double> R[3],
-                                              double xy[8]) {
-    double c[12];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        nd[a] = cnct[4 * e + a];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) c[3 * a + q] = crds[3 * nd[a] + q];
+// Quads: four lanes per (element, load case).  Lane g loads and rotates node g and
+// works Gauss point g in reverse mode (quad_adjoint.hpp); quad permutations add the
+// four points' sums, and lane g ends with the derivative by node g and by property g
+// (the fifth goes with lane 0).  Bound by FP64 arithmetic, with two waves a SIMD to
+// cover its latency: for that the nodes' local values, the frame and the constants
+// stay in LDS until a phase reads them (held in registers they allow one wave, and
+// 66 us instead of 52).  The four lanes share an element because one lane for all four
+// points would leave the chip idle on small plans.  Forward mode in 11 directions,
+// each re-reading and re-rotating the nodes at every Gauss point, took 0.73 ms for 16
+// shells of 100 x 100 (160k elements); this takes 52 us.
+// SELF: lambda = lam_scale u, so phi is lam_scale times the energy of u alone.
+__device__ __forceinline__ double quad_lane(double v, int a) {   // a constant after unrolling
+    const long long x = __double_as_longlong(v);
+    int lo = (int)x, hi = (int)(x >> 32);
+    switch (a) {
+        case 0: lo = __builtin_amdgcn_mov_dpp(lo, 0x00, 15, 15, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x00, 15, 15, true); break;
+        case 1: lo = __builtin_amdgcn_mov_dpp(lo, 0x55, 15, 15, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x55, 15, 15, true); break;
+        case 2: lo = __builtin_amdgcn_mov_dpp(lo, 0xAA, 15, 15, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xAA, 15, 15, true); break;
+        default: lo = __builtin_amdgcn_mov_dpp(lo, 0xFF, 15, 15, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xFF, 15, 15, true); break;
     }
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+__device__ __forceinline__ double quad_total(double v) {   // sum over the four lanes, the same in each
+    long long x = __double_as_longlong(v);
+    int lo = __builtin_amdgcn_mov_dpp((int)x, 0xB1, 15, 15, true);          // lanes 1 0 3 2
+    int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), 0xB1, 15, 15, true);
+    v += __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    x = __double_as_longlong(v);
+    lo = __builtin_amdgcn_mov_dpp((int)x, 0x4E, 15, 15, true);              // lanes 2 3 0 1
+    hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), 0x4E, 15, 15, true);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+template <bool SELF>
+__global__ __launch_bounds__(256, 2) void adj_quad_kernel(int32_t n, int32_t n_beam, const int32_t* __restrict__ cnct,
+                                                       const double* __restrict__ crds,
+                                                       const double* __restrict__ props,
+                                                       const double* __restrict__ u,
+                                                       const double* __restrict__ lam, double lam_scale, int nrhs,
+                                                       double* __restrict__ gbuf, double* __restrict__ dprop) {
+    struct Shared {
+        QuadTurn turn;
+        QuadConsts q;
+        QuadAxes x;
+        double v[SELF ? 1 : 2][6][4];   // local values of u, lambda: component, node
+        double pad;   // an odd number of doubles apart: a wave's elements start in different banks
+    };
+    __shared__ Shared shared[64];   // kept here until it is used: it frees 80 registers
+    Shared& sh = shared[threadIdx.x >> 2];
+    const int64_t item = (xcd_wg() * 256 + threadIdx.x) >> 2;
+    if (item >= (int64_t)n * nrhs) return;   // all four lanes of an item, or none
+    const int g = threadIdx.x & 3;
+    const int64_t e = nrhs == 1 ? item : item / nrhs;
+    const int rhs = (int)(item - e * nrhs);
+    const int64_t nd = cnct[4 * e + g];
+    double own[3], c[12], xy[8], ul[6], ll[6];
+    V3<double> R[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) own[k] = crds[3 * nd + k];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const int64_t gi = (6 * nd + k) * nrhs + rhs;
+        ul[k] = u[gi];
+        ll[k] = SELF ? 0.0 : lam[gi];
+    }
+    const double* pr = props + 5 * e;
+    QuadConsts q;
+    quad_consts(pr[0], pr[1], pr[2], pr[3], pr[4], q);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) c[3 * a + k] = quad_lane(own[k], a);
     quad_frame<double>(c, R, xy);
-}
-
-__device__ __forceinline__ int64_t quad_slot(int32_t n_beam, int64_t e, int slot, int nrhs, int rhs) {
-    return ((int64_t)n_beam * BDIR + e * QDIR + slot) * nrhs + rhs;
-}
-
-__global__ __launch_bounds__(256) void adj_quad_fwd(int32_t n, int32_t n_beam, const int32_t* __restrict__ cnct,
-                                                    const double* __restrict__ crds,
-                                                    const double* __restrict__ props, const double* __restrict__ u,
-                                                    const double* __restrict__ lam, double lam_scale, int nrhs,
-                                                    int rhs, double* __restrict__ gbuf,
-                                                    double* __restrict__ dprop) {
-    // workgroup g: direction g % QA_FWD of the 256 elements of chunk g / QA_FWD, so
-    // that the 11 workgroups of a chunk (one XCD, in sequence) share its inputs in L2
-    const int64_t g = xcd_wg();
-    const int k = (int)(g % QA_FWD);
-    const int64_t e = (g / QA_FWD) * 256 + threadIdx.x;
-    if (e >= n) return;
-    int nd[4];
-    V3<double> R[3];
-    double xy[8];
-    quad_geometry(e, cnct, crds, nd, R, xy);
-    const double* pr = props + 5 * e;
-    if (k < 6) {
-        Dual xd[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) xd[i] = Dual(xy[i], i == QA_XY_FREE[k] ? 1.0 : 0.0);
-        gbuf[quad_slot(n_beam, e, k, nrhs, rhs)] =
-            quad_phi<Dual, double>(R, xd, pr[0], pr[1], pr[2], pr[3], pr[4], nd, u, lam, lam_scale, nrhs, rhs).d;
-    } else {
-        Dual m[5];
-#pragma unroll
-        for (int i = 0; i < 5; ++i) m[i] = Dual(pr[i], i == k - 6 ? 1.0 : 0.0);
-        const double d =
-            quad_phi<double, Dual>(R, xy, m[0], m[1], m[2], m[3], m[4], nd, u, lam, lam_scale, nrhs, rhs).d;
-        if (dprop) dprop[(e * 5 + (k - 6)) * nrhs + rhs] = -d;
+    {
+        QuadTurn f;
+        quad_turn(c, R, xy, f);
+        sh.turn = f;   // the four lanes write the same
     }
-}
-
-__global__ __launch_bounds__(256) void adj_quad_frame(int32_t n, int32_t n_beam, const int32_t* __restrict__ cnct,
-                                                      const double* __restrict__ crds,
-                                                      const double* __restrict__ props,
-                                                      const double* __restrict__ u, const double* __restrict__ lam,
-                                                      double lam_scale, int nrhs, int rhs,
-                                                      double* __restrict__ gbuf) {
-    const int64_t e = xcd_wg() * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    int nd[4];
-    V3<double> R[3];
-    double xy[8];
-    quad_geometry(e, cnct, crds, nd, R, xy);
-    const double* pr = props + 5 * e;
-    double dR[3][3];
-    quad_frame_adjoint(R, xy, pr[0], pr[1], pr[2], pr[3], pr[4], nd, u, lam, lam_scale, nrhs, rhs, dR);
+    auto rotate = [&](double v[6]) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+        for (int h = 0; h < 6; h += 3) {
+            const double x = v[h], y = v[h + 1], z = v[h + 2];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) gbuf[quad_slot(n_beam, e, 6 + 3 * i + j, nrhs, rhs)] = dR[i][j];
-}
-
-__global__ __launch_bounds__(12 * QA_E) void adj_quad_combine(int32_t n, int32_t n_beam,
-                                                              const int32_t* __restrict__ cnct,
-                                                              const double* __restrict__ crds, int nrhs, int rhs,
-                                                              double* __restrict__ gbuf) {
-    __shared__ double part[QA_E][15];   // dphi/dxy (6 free entries), dphi/dR (9)
-    const int tid = threadIdx.x;
-    const int64_t e0 = xcd_wg() * QA_E;
-    for (int v = tid; v < QA_E * 15; v += blockDim.x) {
-        const int el = v / 15, q = v % 15;
-        if (e0 + el < n) part[el][q] = gbuf[quad_slot(n_beam, e0 + el, q, nrhs, rhs)];
+            for (int i = 0; i < 3; ++i) v[h + i] = R[i].x * x + R[i].y * y + R[i].z * z;
+        }
+    };
+    rotate(ul);
+    if (!SELF) rotate(ll);
+    const double(&lv)[6] = SELF ? ul : ll;
+    QuadPoint P;
+    QuadAxes x;
+    quad_axes(xy, x);
+    sh.x = x;
+    sh.q = q;
+    quad_point(xy, x, (g == 0 || g == 3) ? GP : -GP, g < 2 ? GP : -GP, P);   // gauss_r, gauss_s
+    quad_phase();
+    QuadBars b = {};
+    double krz, en[3];
+    {
+        double diag[8], w[8];
+        quad_point_diag(P, q, diag);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) diag[i] = quad_total(diag[i]);
+        quad_drill_weights(diag, quad_total(ul[5] * lv[5]), krz, w);
+        quad_phase();
+        quad_drill_bars(P, q, w, b, en);
     }
-    __syncthreads();   // every partial is read before any slot is overwritten
-    const int el = tid % QA_E, p = tid / QA_E;   // coordinate p = 3 * node + component
-    const int64_t e = e0 + el;
-    if (e >= n) return;
-    Dual c[12];
+    quad_phase();
+    double o[13];
+    const double d0 = krz * (lv[5] * ul[3] + ul[5] * lv[3]), d1 = krz * (lv[5] * ul[4] + ul[5] * lv[4]);
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int node = cnct[4 * e + a];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) c[3 * a + q] = Dual(crds[3 * node + q], 3 * a + q == p ? 1.0 : 0.0);
+    for (int j = 0; j < 6; ++j) {
+        sh.v[0][j][g] = ul[j];
+        if (!SELF) sh.v[1][j][g] = ll[j];
     }
-    V3<Dual> Rd[3];
-    Dual xyd[8];
-    quad_frame<Dual>(c, Rd, xyd);
-    double sum = 0.0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // written by lanes of the same wave
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    auto sums = [&](int f, QuadSums& s) {
+        keep_loads_here();
+        const double(*v)[4] = sh.v[SELF ? 0 : f];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) sum += part[el][q] * xyd[QA_XY_FREE[q]].d;
+        for (int j = 0; j < 6; ++j) quad_sums(P, j, v[j][0], v[j][1], v[j][2], v[j][3], s);
+    };
+    keep_loads_here();
+    quad_phase();
+    const double W = quad_point_adjoint(P, sh.q, sums, b, en, o);
+    keep_loads_here();
+    quad_phase();
+    quad_point_xy(P, sh.x, b, W, o);
+    quad_phase();
+    o[6] -= d0;   // drilling, the lane's own node
+    o[7] -= d1;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-        sum += part[el][6 + 3 * i] * Rd[i].x.d + part[el][7 + 3 * i] * Rd[i].y.d + part[el][8 + 3 * i] * Rd[i].z.d;
-    gbuf[quad_slot(n_beam, e, p, nrhs, rhs)] = -sum;
+    for (int i = 0; i < 13; ++i) o[i] = quad_total(o[i]);
+    const double sg = SELF ? -lam_scale : -1.0;
+    double d[3];
+    keep_loads_here();
+    const QuadTurn f = sh.turn;
+    quad_node_adjoint(f, o, g, d);
+    double* out = gbuf + ((int64_t)n_beam * BDIR + e * QDIR + 3 * g) * nrhs + rhs;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) out[(int64_t)k * nrhs] = sg * d[k];
+    if (dprop) {
+        double* dp = dprop + 5 * e * nrhs + rhs;
+        dp[(int64_t)g * nrhs] = sg * (g == 0 ? o[8] : g == 1 ? o[9] : g == 2 ? o[10] : o[11]);
+        if (g == 0) dp[(int64_t)4 * nrhs] = sg * o[12];
+    }
 }
 
 // node gradient: sum of the coordinate derivatives of the elements incident to
@@ -788,16 +816,13 @@ int launch_adjoint(Plan* p, const double* crds, const double* prop_beam, const d
         JSSO_HIP(hipGetLastError());
     }
     if (p->n_quad > 0) {
-        const int nq = p->n_quad;
-        for (int rhs = 0; rhs < nrhs; ++rhs) {
-            hipLaunchKernelGGL(adj_quad_fwd, xcd_grid((int64_t)QA_FWD * ((nq + 255) / 256)), dim3(256), 0, s,
-                               nq, p->n_beam, p->d_cnct_quad, crds, prop_quad, u, lam, lam_scale, nrhs, rhs, gbuf,
-                               dprop_quad);
-            hipLaunchKernelGGL(adj_quad_frame, xcd_grid((nq + 255) / 256), dim3(256), 0, s, nq, p->n_beam,
-                               p->d_cnct_quad, crds, prop_quad, u, lam, lam_scale, nrhs, rhs, gbuf);
-            hipLaunchKernelGGL(adj_quad_combine, xcd_grid((nq + QA_E - 1) / QA_E), dim3(12 * QA_E), 0, s,
-                               nq, p->n_beam, p->d_cnct_quad, crds, nrhs, rhs, gbuf);
-        }
+        const dim3 grid = xcd_grid((4 * (int64_t)p->n_quad * nrhs + 255) / 256);
+        if (lam)
+            hipLaunchKernelGGL(adj_quad_kernel<false>, grid, dim3(256), 0, s, p->n_quad, p->n_beam, p->d_cnct_quad,
+                               crds, prop_quad, u, lam, lam_scale, nrhs, gbuf, dprop_quad);
+        else
+            hipLaunchKernelGGL(adj_quad_kernel<true>, grid, dim3(256), 0, s, p->n_quad, p->n_beam, p->d_cnct_quad,
+                               crds, prop_quad, u, lam, lam_scale, nrhs, gbuf, dprop_quad);
         JSSO_HIP(hipGetLastError());
     }
     return JSSO_OK;
