@@ -378,7 +378,9 @@ static int ensure_device(Plan* p) {
         (rc = upload(p, &p->d_ell_src, p->h_ell_src)) || (rc = upload(p, &p->d_tpos, p->h_tpos)))
         return rc;
     const size_t n = p->n_nodes;
-    if ((rc = dalloc(p, &p->d_ke, (size_t)p->n_contrib * 36)) || (rc = dalloc(p, &p->d_K, (size_t)p->nnzb * 36)) ||
+    // (at least one element block: the gathers read block 0 where a node has fewer than they read at once)
+    if ((rc = dalloc(p, &p->d_ke, (size_t)std::max<int64_t>(p->n_contrib, 1) * 36)) ||
+         (rc = dalloc(p, &p->d_K, (size_t)p->nnzb * 36)) ||
         (rc = dalloc(p, &p->d_Kc, (size_t)p->nnzb * 36)) || (rc = dalloc(p, &p->d_Linv, n * 36)) ||
         (rc = dalloc(p, &p->d_Minv, n * 36)) || (rc = dalloc(p, &p->d_status, 1)) ||
         (rc = dalloc(p, &p->d_Ke64, (size_t)p->ell_slots * 36)) || (rc = dalloc(p, &p->d_Ke32, (size_t)p->ell_slots * 36)) ||
@@ -563,16 +565,12 @@ int jsso_assemble(jsso_plan* plan, const double* d_crds, const double* d_prop_be
     if (rc) return rc;
     timing_end(s, ev);
     timing_begin_slot(s, ev, JSSO_TIMING_GATHER);
-    rc = launch_assemble(p, s);
+    rc = launch_assemble(p, d_crds, s);
     if (rc) return rc;
     timing_end(s, ev);
-    JSSO_HIP(hipMemcpyAsync(p->d_crds, d_crds, (size_t)p->n_nodes * 3 * sizeof(double), hipMemcpyDeviceToDevice, s));
     p->amg_valid = false;
     p->direct_valid = false;
-    if (d_K_out && p->nnzb) {
-        if ((rc = launch_full_blocks(p, s))) return rc;
-        JSSO_HIP(hipMemcpyAsync(d_K_out, p->d_K, (size_t)p->nnzb * 36 * sizeof(double), hipMemcpyDeviceToDevice, s));
-    }
+    if (d_K_out && (rc = launch_export_blocks(p, d_K_out, s))) return rc;
     p->assembled = true;
     return JSSO_OK;
 }

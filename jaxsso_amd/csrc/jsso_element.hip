@@ -91,7 +91,9 @@ __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* _
 // per element, QK_LOCAL row-major 24x24 of k_m + k_b before the rotation
 // (Quad.element_K_quad_local, element.py:1086-1095).  EPW elements per
 // workgroup (4, 8 or 16: 64, 128 or 256 threads), chosen per plan by timing on
-// the live assembly (tune_ke_quad).
+// the live assembly (tune_ke_quad).  QK_BLOCKS is bound by its stores: a wave's 64
+// blocks are one contiguous 18 KB, which go out through LDS in whole lines.  A lane
+// storing its own 288 bytes took 79 us for 40k elements (184 MB); this takes KE_US us.
 // ---------------------------------------------------------------------------
 enum { QK_BLOCKS = 0, QK_GLOBAL = 1, QK_LOCAL = 2 };
 
@@ -110,11 +112,15 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
                                                            const double* __restrict__ crds_nodes,
                                                            const double* __restrict__ props,
                                                            double* __restrict__ ke, int32_t* status = nullptr) {
-    __shared__ QuadTile sh[EPW];
+    // one wave's part: the tiles of its four elements, then (QK_BLOCKS) its 64 blocks on
+    // their way out, a lane's 36 values an odd stride apart
+    constexpr int TILE = sizeof(QuadTile) / sizeof(double), OUT = 37;
+    constexpr int WAVE_LDS = MODE == QK_BLOCKS ? 64 * OUT : 4 * TILE;
+    __shared__ double lds[EPW / 4][WAVE_LDS];
     const int le = threadIdx.x >> 4, lane = threadIdx.x & 15;
     const int e = blockIdx.x * EPW + le;
     const bool valid = e < n;
-    QuadTile& T = sh[le];
+    QuadTile& T = *(QuadTile*)&lds[le >> 2][(le & 3) * TILE];
     if (valid && lane < 4) {
         double c[12];
         if (cnct) {
@@ -173,7 +179,7 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
         T.diag[lane] = acc;
     }
     __syncthreads();
-    if (!valid) return;
+    if (MODE != QK_BLOCKS && !valid) return;   // (there the wave stores together)
     const int a = lane >> 2, b = lane & 3;
     double cb, cs, Cm[3][3];
     quad_plate_consts<double>(T.t, T.E, T.nu, cb, cs);
@@ -254,15 +260,27 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
             for (int j = 0; j < 3; ++j)
                 out[3 * p + i][3 * q + j] = R[0][i] * tmp[0][j] + R[1][i] * tmp[1][j] + R[2][i] * tmp[2][j];
     }
+    if (MODE == QK_BLOCKS) {
+        double* st = lds[le >> 2];
+        const int wl = threadIdx.x & 63;
+        __syncthreads();   // the tiles have been read
+#pragma unroll
+        for (int q = 0; q < 36; ++q) st[wl * OUT + q] = out[q / 6][q % 6];
+        __syncthreads();
+        const int64_t e0 = (int64_t)blockIdx.x * EPW + (threadIdx.x >> 6) * 4;
+        const int count = (int)(n - e0 < 4 ? n - e0 : 4) * 16 * 18;   // pairs of values (none past the end)
+        double2* dst = (double2*)(ke + e0 * 16 * 36);
+#pragma unroll 6
+        for (int i = wl; i < count; i += 64) {
+            const double* v = st + (i / 18) * OUT + 2 * (i % 18);
+            dst[i] = make_double2(v[0], v[1]);
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 6; ++i)
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-            if (MODE == QK_BLOCKS)
-                ke[((int64_t)e * 16 + lane) * 36 + i * 6 + j] = out[i][j];
-            else
-                ke[(int64_t)e * 576 + (6 * a + i) * 24 + 6 * b + j] = out[i][j];
-        }
+        for (int j = 0; j < 6; ++j) ke[(int64_t)e * 576 + (6 * a + i) * 24 + 6 * b + j] = out[i][j];
 }
 
 int launch_ke_beam(int32_t n, const double* crds_e, const int32_t* cnct, const double* crds_nodes,

@@ -207,7 +207,8 @@ int launch_quad_local(int32_t n, const double* crds, const double* props, double
                       double* kl, hipStream_t s);
 int launch_quad_gauss(int32_t n, const double* xy, const double* props, double r, double s_, double* J, double* Bk,
                       double* Bg, double* Bm, double* Cb, double* Cs, double* Cm, hipStream_t s);
-int launch_assemble(Plan* p, hipStream_t s);
+int launch_assemble(Plan* p, const double* crds, hipStream_t s);   // also keeps crds in d_crds
+int launch_export_blocks(Plan* p, double* K, hipStream_t s);
 int launch_csr_spmv(int32_t n_rows, const int32_t* rowptr, const int32_t* colind, const double* vals,
                     const double* x, const double* c, double* y, hipStream_t s);
 int launch_full_blocks(Plan* p, hipStream_t s);
