@@ -24,7 +24,7 @@ namespace jsso {
 // entries fastest, so that every access is whole lines.  W = 2 needs 16-byte aligned
 // K.  KC: also the constrained Kc (plain path).  A 200 x 200 shell (361k blocks,
 // 104 MB of K) took 151 us with a thread per entry and both outputs, and 40 us more to
-// copy K to the caller; this takes GATHER_US us, straight into the caller's buffer.
+// copy K to the caller; this takes 62 us, straight into the caller's buffer.
 constexpr int GATHER_BLOCKS = 128;
 constexpr int MAX_CONTRIB = 2;   // element blocks per off-diagonal block read without a loop (2 on a quad mesh)
 
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(int64_t nnzb, const 
 // is not positive definite.  64 nodes per workgroup: all threads gather the blocks
 // (entry fastest) into LDS, the first wave factorises a node per lane, all threads
 // write.  A lane per node reading and writing its own 36-value rows took 37 us for
-// 40k nodes (a 200 x 200 shell); this takes DIAG_US us, bound by the chain of one
+// 40k nodes (a 200 x 200 shell); this takes 20 us, bound by the chain of one
 // factorisation and by two rounds of memory latency.  The coordinates that the plan
 // keeps are copied here as well: a copy of its own costs a launch.
 constexpr int DIAG_NODES = 64;
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void diag_factor_kernel(int32_t n_nodes, const
     __syncthreads();
     if (t < nn) {
         const int64_t i = i0 + t;
-        double A[6][6], L[6][6], Li[6][6], B[36], il[6];
+        double A[6][6], L[6][6], Li[6][6], B[36];
 #pragma unroll
         for (int q = 0; q < 36; ++q) B[q] = tile[t][q];
         bool fx[6];
@@ -199,25 +199,25 @@ __global__ __launch_bounds__(256) void diag_factor_kernel(int32_t n_nodes, const
             for (int k = 0; k < j; ++k) d -= L[j][k] * L[j][k];
             if (!(d > 0.0)) { ok = false; d = 1.0; }
             const double ljj = sqrt(d);
-            il[j] = 1.0 / ljj;
+            L[j][j] = ljj;
 #pragma unroll
             for (int r = j + 1; r < 6; ++r) {
                 double s = A[r][j];
 #pragma unroll
                 for (int k = 0; k < j; ++k) s -= L[r][k] * L[j][k];
-                L[r][j] = s * il[j];
+                L[r][j] = s / ljj;
             }
         }
         // inverse of the lower-triangular factor
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            Li[j][j] = il[j];
+            Li[j][j] = 1.0 / L[j][j];
 #pragma unroll
             for (int r = j + 1; r < 6; ++r) {
                 double s = 0.0;
 #pragma unroll
                 for (int k = j; k < r; ++k) s -= L[r][k] * Li[k][j];
-                Li[r][j] = s * il[r];
+                Li[r][j] = s / L[r][r];
             }
         }
 #pragma unroll
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void diag_factor_kernel(int32_t n_nodes, const
 //   phase 3: Ks goes back through LDS and out in the value-slot layout (16-byte
 //            groups of entries, lanes interleaved per group), whole lines at a time.
 //            Stored from phase 2 entry by entry, 160k blocks (a 200 x 200 shell) took
-//            71 us; this takes ELL_US us.
+//            71 us; this takes 62 us.
 constexpr int ASM_WG = 256;
 
 struct alignas(8) Half4 {
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(ASM_WG) void ell_assemble_kernel(
     // element-local blocks of the same elements
     const bool sym_part = (*status & STATUS_NONSYM) != 0;
     __shared__ double tile[P][37];
-    __shared__ double li[P][37], lj[P][37];
+    __shared__ double li[P][21], lj[P][21];   // lower triangles, row by row
     __shared__ int32_t cidx[P][MAX_CONTRIB], cstart[P], ccount[P], rowi[P], colj[P];
     __shared__ uint8_t rfix[P][6], cfix[P][6];
     const int64_t slot = blockIdx.x;
@@ -306,15 +306,19 @@ __global__ __launch_bounds__(ASM_WG) void ell_assemble_kernel(
     }
     __syncthreads();
     constexpr int NPAIR = P * 36 / ASM_WG;   // 9
-    double v[NPAIR][MAX_CONTRIB], lv[NPAIR][2];
+    double v[NPAIR][MAX_CONTRIB];
 #pragma unroll
     for (int it = 0; it < NPAIR; ++it) {
         const int u = t + it * ASM_WG;
         const int p = u / 36, q = u % 36;
 #pragma unroll
         for (int c = 0; c < MAX_CONTRIB; ++c) v[it][c] = ke[(int64_t)cidx[p][c] * 36 + q];
-        lv[it][0] = Linv[(int64_t)rowi[p] * 36 + q];
-        lv[it][1] = Linv[(int64_t)colj[p] * 36 + q];
+    }
+    for (int u = t; u < P * 21; u += ASM_WG) {
+        const int p = u / 21, q = u % 21;
+        const int r = (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15), at = 6 * r + q - r * (r + 1) / 2;
+        li[p][q] = Linv[(int64_t)rowi[p] * 36 + at];
+        lj[p][q] = Linv[(int64_t)colj[p] * 36 + at];
     }
 #pragma unroll
     for (int it = 0; it < NPAIR; ++it) {
@@ -345,8 +349,6 @@ __global__ __launch_bounds__(ASM_WG) void ell_assemble_kernel(
             sum = 0.5 * (sum + st);
         }
         tile[p][q] = (n > 0 && !(rfix[p][q / 6] | cfix[p][q % 6])) ? sum : 0.0;
-        li[p][q] = lv[it][0];
-        lj[p][q] = lv[it][1];
     }
     __syncthreads();
     const int wave = t >> 6, lane = t & 63;
@@ -362,14 +364,14 @@ __global__ __launch_bounds__(ASM_WG) void ell_assemble_kernel(
             double s = 0.0;
 #pragma unroll
             for (int k2 = 0; k2 < 6; ++k2)
-                if (k2 <= c) s += tile[lane][r * 6 + k2] * lj[lane][c * 6 + k2];
+                if (k2 <= c) s += tile[lane][r * 6 + k2] * lj[lane][c * (c + 1) / 2 + k2];
             Tc[r] = s;
         }
 #pragma unroll
         for (int r = 0; r < 6; ++r) {
             double s = 0.0;
 #pragma unroll
-            for (int k2 = 0; k2 <= r; ++k2) s += li[lane][r * 6 + k2] * Tc[k2];
+            for (int k2 = 0; k2 <= r; ++k2) s += li[lane][r * (r + 1) / 2 + k2] * Tc[k2];
             Ks[h][r] = ccount[lane] ? s : 0.0;   // padding (or an empty block): zero
         }
     }

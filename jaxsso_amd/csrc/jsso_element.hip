@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* _
 // workgroup (4, 8 or 16: 64, 128 or 256 threads), chosen per plan by timing on
 // the live assembly (tune_ke_quad).  QK_BLOCKS is bound by its stores: a wave's 64
 // blocks are one contiguous 18 KB, which go out through LDS in whole lines.  A lane
-// storing its own 288 bytes took 79 us for 40k elements (184 MB); this takes KE_US us.
+// storing its own 288 bytes took 79 us for 40k elements (184 MB); this takes 53 us.
 // ---------------------------------------------------------------------------
 enum { QK_BLOCKS = 0, QK_GLOBAL = 1, QK_LOCAL = 2 };
 
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
                                                            double* __restrict__ ke, int32_t* status = nullptr) {
     // one wave's part: the tiles of its four elements, then (QK_BLOCKS) its 64 blocks on
     // their way out, a lane's 36 values an odd stride apart
-    constexpr int TILE = sizeof(QuadTile) / sizeof(double), OUT = 37;
+    constexpr int TILE = sizeof(QuadTile) / sizeof(double), OUT = 19;
     constexpr int WAVE_LDS = MODE == QK_BLOCKS ? 64 * OUT : 4 * TILE;
     __shared__ double lds[EPW / 4][WAVE_LDS];
     const int le = threadIdx.x >> 4, lane = threadIdx.x & 15;
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
     quad_plate_consts<double>(T.t, T.E, T.nu, cb, cs);
     quad_cm<double>(T.E, T.nu, T.kx, T.ky, Cm);
     double mem[2][2] = {{0, 0}, {0, 0}}, ben[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll
+#pragma unroll 1
     for (int g = 0; g < 4; ++g) {
         const double dJ = T.detJ[g];
         const double ha0 = T.dH[g][a], ha1 = T.dH[g][4 + a], hb0 = T.dH[g][b], hb1 = T.dH[g][4 + b];
@@ -263,17 +263,21 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
     if (MODE == QK_BLOCKS) {
         double* st = lds[le >> 2];
         const int wl = threadIdx.x & 63;
-        __syncthreads();   // the tiles have been read
-#pragma unroll
-        for (int q = 0; q < 36; ++q) st[wl * OUT + q] = out[q / 6][q % 6];
-        __syncthreads();
         const int64_t e0 = (int64_t)blockIdx.x * EPW + (threadIdx.x >> 6) * 4;
-        const int count = (int)(n - e0 < 4 ? n - e0 : 4) * 16 * 18;   // pairs of values (none past the end)
+        const int count = (int)(n - e0 < 4 ? n - e0 : 4) * 16 * 9;   // pairs of values (none past the end)
         double2* dst = (double2*)(ke + e0 * 16 * 36);
-#pragma unroll 6
-        for (int i = wl; i < count; i += 64) {
-            const double* v = st + (i / 18) * OUT + 2 * (i % 18);
-            dst[i] = make_double2(v[0], v[1]);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            __syncthreads();   // the tiles, or the first half, have been read
+#pragma unroll
+            for (int q = 0; q < 18; ++q) st[wl * OUT + q] = out[3 * half + q / 6][q % 6];
+            __syncthreads();
+#pragma unroll 3
+            for (int i = wl; i < count; i += 64) {
+                const int blk = i / 9, k = i % 9;
+                const double* v = st + blk * OUT + 2 * k;
+                dst[blk * 18 + 9 * half + k] = make_double2(v[0], v[1]);
+            }
         }
         return;
     }
