@@ -19,9 +19,10 @@
 // contribution, all from LDS; only the children's contributions are read and only
 // S, G and the own contribution written.  Larger fronts go in panels of <= 96
 // pivots whose columns are kept in HBM:
-//   k_front_diag   factor of the panel's diagonal block and its inverse, S
-//   k_front_strip  64 rows below it: L21 (in place) and G
-//   k_front_cols   the panel's update of the pivot columns still to come
+//   k_front_diag   inverse factor of a panel's diagonal block
+//   k_front_strip  the rows below a panel's diagonal block: L21 (in place) and G; S
+//   k_front_cols   the panel's update of the pivot columns still to come, with the
+//                  inverse factor of the next panel's diagonal block
 //   k_front_cb     after the last panel: C = gathered children - L21 L21^T over
 //                  all pivots at once, so C is written once and never re-read
 // The front is never assembled as a whole: each kernel gathers what it is the
@@ -52,6 +53,9 @@ static_assert((DIRECT_MAX_M + 2 * 1024) * 4 * 8 <= DLDS_MAX, "LDS of the backwar
 constexpr int DIRECT_STEPS = 6;           // refinement steps, at most
 constexpr int DEFECT_STEPS = 40;          // of a K that is not symmetric
 constexpr double DIRECT_FLOOR_FACTOR = 16.0;   // attainable accuracy: 16 eps (||A|| ||x|| + ||b||), as the AMG solve
+constexpr int HEAD_FRONTS = 64;           // below: k_front_cols factors the next panel's block itself (64
+                                          // designs of 100 x 100: 34.3 ms with it, 33.7 without)
+constexpr int BWD_PARTS = 8;              // workgroups per panel of the backward solve, at most
 constexpr int STRIP_TILES = 3;            // 16x16 tiles of a strip that a wavefront holds
 constexpr int DKC = 32;                   // pivot columns staged at a time by the tile kernels
 
@@ -373,16 +377,17 @@ __device__ __forceinline__ Gather make_gather(const DirectDev& d, const FrontTas
 struct Where {
     int task, part;
 };
-__device__ __forceinline__ Where locate(int n, int parts) {
-    const int b = blockIdx.x;
+__device__ __forceinline__ Where locate(int n, int parts, int b) {
     if (n >= 64) {
         const int q = b >> 3, t = q / parts;
         return {8 * t + (b & 7), q - t * parts};
     }
     return {b % n, b / n};
 }
+__device__ __forceinline__ Where locate(int n, int parts) { return locate(n, parts, (int)blockIdx.x); }
+__host__ __device__ inline int task_slots(int n) { return n >= 64 ? 8 * ((n + 7) / 8) : n; }
 static dim3 part_grid(size_t n, int parts) {
-    return dim3((unsigned)((n >= 64 ? 8 * ((n + 7) / 8) : n) * parts));
+    return dim3((unsigned)(task_slots((int)n) * parts));
 }
 // entry (row, col) of the front, row >= col; a, b: `inv` of their nodes.  Without
 // branches, so that a thread's loads are all in flight at once (a wavefront that
@@ -573,13 +578,23 @@ __device__ __forceinline__ int64_t panel_offset(int m, int w, int p) {
     return (int64_t)p * w * w + (int64_t)p * m * w - (int64_t)w * w * p * (p + 1) / 2;
 }
 
-// diagonal block of panel p (gathered for the first panel): S to the factor, the
-// inverse factor to the block's place in the pivot columns
+// The inverse factor of a diagonal block: from the block in P (whole workgroup) to the
+// block's place in the pivot columns.
+__device__ __forceinline__ void factor_block(const DirectDev& d, const FrontTask& f, double* P, int ld, int kp, int w,
+                                             double* F, int k, int wave, int lane) {
+    const bool ok = invert_factor(P, ld, kp, wave, 8, lane);
+    if (!ok && wave == 0 && lane == 0) atomicOr(d.bad + f.sys, 1);
+    for (int row = wave; row < w; row += 8)
+        for (int col = lane; col <= row; col += 64)
+            F[(int64_t)row * k + col] = P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)];
+}
+
+// diagonal block of panel p (gathered for the first panel), factored
 __global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const FrontTask* __restrict__ tasks, int p) {
     extern __shared__ double P[];
     const FrontTask f = tasks[blockIdx.x];
     if (p >= f.npan) return;
-    const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
+    const int k = 6 * f.np, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kp = (w + 15) & ~15, ld = kp + 2;
@@ -610,16 +625,11 @@ __global__ __launch_bounds__(512) void k_front_diag(DirectDev d, const FrontTask
     __syncthreads();
     if (p == 0) add_stored(d, f, 0, w, 0, w, w, 0, P, ld, tid, 512);
     __syncthreads();
-    const bool ok = invert_factor(P, ld, kp, wave, 8, lane);
-    if (!ok && tid == 0) atomicOr(d.bad + f.sys, 1);
-    double* S = d.fac + f.fac + panel_offset(m, 6 * f.wn, p);
-    write_S(P, ld, kp, w, S, wave, 8, lane);
-    for (int row = wave; row < w; row += 8)
-        for (int col = lane; col <= row; col += 64)
-            F[(int64_t)row * k + col] = P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)];
+    factor_block(d, f, P, ld, kp, w, F, k, wave, lane);
 }
 
-// `rows` (<= 96) rows below panel p's diagonal block: L21 = F21 L^-T (in place) and G = L21 L^-1
+// `rows` (<= 96) rows below panel p's diagonal block: L21 = F21 L^-T (in place) and G = L21 L^-1;
+// the last part: S = L^-T L^-1, which nothing waits for
 __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const FrontTask* __restrict__ tasks, int p, int n, int parts, int rows) {
     extern __shared__ double P[];
     const Where at = locate(n, parts);
@@ -628,11 +638,32 @@ __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const FrontTa
     if (p >= f.npan) return;
     const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = min(6 * f.wn, k - c0);
     const int r0 = c0 + w + rows * at.part;
-    if (r0 >= m) return;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kp = (w + 15) & ~15, ld = kp + 2, nt = kp >> 4;
     double* F = d.mat + f.pan + c0;   // column c0 of the pivot columns
+    if (at.part == parts - 1) {
+        static_assert(DW <= 96, "six rows a wavefront");
+        for (int col = lane; col < kp; col += 64) {
+            double y[6];
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+                const int row = wave + 16 * u;
+                y[u] = *(row < w && col <= row ? F + (int64_t)(c0 + row) * k + col : d.zero) +
+                       (row == col && row >= w ? 1.0 : 0.0);
+            }
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+                const int row = wave + 16 * u;
+                if (row < kp && col >> 4 <= row >> 4)
+                    P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)] = y[u];
+            }
+        }
+        __syncthreads();
+        write_S(P, ld, kp, w, d.fac + f.fac + panel_offset(m, 6 * f.wn, p), wave, 16, lane);
+        return;
+    }
+    if (r0 >= m) return;
     double* X = P + kp * ld;
     const int nr = min(rows, m - r0), rt = rows >> 4;
     const Gather ga = make_gather(d, f);
@@ -755,25 +786,122 @@ __device__ __forceinline__ void tile_product(const double* __restrict__ F, int k
     }
 }
 
-// panel p's update of the pivot columns after it (64x64 tiles; gathered here for p = 0)
-__global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const FrontTask* __restrict__ tasks, int p, int n, int parts) {
-    __shared__ double sh[2 * DROWS * (DKC + 2)];
-    const Where at = locate(n, parts);
+// The next panel's diagonal block: panel p's update of it (gathered here for p = 0) and
+// its inverse factor, by one workgroup of 512 threads.
+__device__ __forceinline__ void next_block(const DirectDev& d, const FrontTask& f, int p, double* P, int tid) {
+    const int k = 6 * f.np, c0 = 6 * p * f.wn, w = 6 * f.wn, c1 = c0 + w, w1 = min(w, k - c1);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, q = lane >> 4;
+    const int ldx = ((w + 15) & ~15) + 2, kp = (w1 + 15) & ~15, ld = kp + 2, nt = kp >> 4;
+    double* F = d.mat + f.pan + (int64_t)c1 * k;   // rows of the next panel
+    __shared__ int2 inv[DW / 6 + 1];
+    if (p == 0) {
+        if (tid < w1 / 6) inv[tid] = d.inv[f.node0 + c1 / 6 + tid];
+        __syncthreads();
+    }
+    // a wavefront's tiles of the lower triangle in the matrix core's layout, and the
+    // panel's columns of these rows: all on their way together
+    constexpr int MT = (DW / 16 * (DW / 16 + 1) / 2 + 7) / 8;
+    const Gather ga = make_gather(d, f);
+    d4 t[MT];
+    int ti[MT], tj[MT];
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+        int I = 0, J = wave + 8 * u;
+        while (J > I) {
+            J -= I + 1;
+            ++I;
+        }
+        ti[u] = I;
+        tj[u] = J;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = 16 * I + 4 * i + q, col = 16 * J + r;
+            const bool on = row < w1 && col <= row;
+            if (p > 0) {
+                t[u][i] = *(on ? F + (int64_t)row * k + c1 + col : d.zero) + (row == col && row >= w1 ? 1.0 : 0.0);
+            } else {
+                const int rn = min(row, w1 - 1) / 6, cn = min(col, w1 - 1) / 6;
+                t[u][i] = (row == col ? 1.0 : 0.0) + gathered(ga, inv[rn], inv[cn], row - 6 * rn, col - 6 * cn, on);
+            }
+        }
+    }
+    static_assert(DW <= 96, "12 rows a wavefront, 48 pairs of columns");
+#pragma unroll
+    for (int u0 = 0; u0 < 12; u0 += 6) {
+        double2 x[6];
+#pragma unroll
+        for (int u = 0; u < 6; ++u) {
+            const int row = wave + 8 * (u0 + u);
+            x[u] = *reinterpret_cast<const double2*>(row < w1 && 2 * lane < w ? F + (int64_t)row * k + c0 + 2 * lane
+                                                                              : d.zero);
+        }
+#pragma unroll
+        for (int u = 0; u < 6; ++u)
+            if (wave + 8 * (u0 + u) < kp && 2 * lane < ldx - 2)
+                *reinterpret_cast<double2*>(P + (wave + 8 * (u0 + u)) * ldx + 2 * lane) = x[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+        if (ti[u] >= nt) continue;
+        const double *X = P + (16 * ti[u] + r) * ldx + q, *Y = P + (16 * tj[u] + r) * ldx + q;
+#pragma unroll 4
+        for (int c = 0; c < (w + 3) >> 2; ++c) t[u] = mfma64(-X[4 * c], Y[4 * c], t[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+        if (ti[u] >= nt) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            P[(16 * ti[u] + 4 * i + q) * ld + 16 * tj[u] + r] = t[u][i];
+            if (ti[u] != tj[u]) P[(16 * tj[u] + 4 * i + q) * ld + 16 * ti[u] + r] = 0.0;
+        }
+    }
+    __syncthreads();
+    if (p == 0) {
+        add_stored(d, f, c1, c1 + w1, c1, c1 + w1, 6 * (f.np + f.nb) + k, 0, P, ld, tid, 512);
+        __syncthreads();
+    }
+    factor_block(d, f, P, ld, kp, w1, F + c1, k, wave, lane);
+}
+
+// Panel p's update of the pivot columns after it.  The first workgroups take the next
+// panel's diagonal block, one per front, and factor it: the chain of the panels, which
+// the update of the rest (`parts` pairs of 64x64 tiles a front; gathered here for
+// p = 0) runs beside.  Factored in a
+// launch of its own after the update, a panel took 65 us, so 57 (200 x 200 shell, 58
+// panels in sequence).  Launches of many fronts fill the chip without it, and do so
+// better with a tile per workgroup (HEAD_FRONTS).
+template <bool HEAD>
+__global__ __launch_bounds__(HEAD ? 512 : 256, HEAD ? 4 : 1) void k_front_cols(DirectDev d, const FrontTask* __restrict__ tasks, int p, int n, int parts) {
+    extern __shared__ double P[];
+    const int heads = HEAD ? task_slots(n) : 0, b = blockIdx.x;
+    const Where at = b < heads ? Where{b, 0} : locate(n, parts, b - heads);
     if (at.task >= n) return;
     const FrontTask f = tasks[at.task];
     if (p + 1 >= f.npan) return;
+    if (b < heads) {
+        next_block(d, f, p, P, threadIdx.x);
+        return;
+    }
     const int k = 6 * f.np, m = k + 6 * f.nb, c0 = 6 * p * f.wn, w = 6 * f.wn, t0 = c0 + w;
-    const int nc = (k - t0 + DROWS - 1) / DROWS;   // tile columns; part -> (row, column), columns of a row together
-    const int i0 = t0 + DROWS * (at.part / nc), j0 = t0 + DROWS * (at.part % nc);
-    if (i0 >= m || j0 > i0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int w1 = HEAD ? min(w, k - t0) : 0;      // rows and columns that the head takes
+    const int nc = (k - t0 + DROWS - 1) / DROWS;   // tile columns; tile -> (row, column), columns of a row together
+    const int half = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    const int first = (HEAD ? 2 : 1) * at.part;
+    if (t0 + DROWS * (first / nc) >= m) return;
+    const int i0 = t0 + DROWS * ((first + half) / nc), j0 = t0 + DROWS * ((first + half) % nc);
+    const bool on = i0 < m && j0 <= i0 && (i0 - t0 + DROWS > w1 || j0 - t0 + DROWS > w1);
+    if (!HEAD && !on) return;
+    double* sh = P + half * 2 * DROWS * (DKC + 2);
     double* F = d.mat + f.pan;
     TileAcc t = {};
-    tile_product(F, k, m, i0, j0, c0, w, sh, sh + DROWS * (DKC + 2), tid, t);
+    tile_product(F, k, on ? m : 0, i0, j0, c0, w, sh, sh + DROWS * (DKC + 2), tid, t);
     const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1);
     const Gather ga = make_gather(d, f);
     const int2* inv = d.inv + f.node0;
-    const int i1 = min(m, i0 + DROWS), j1 = min(k, j0 + DROWS);
+    const int i1 = on ? min(m, i0 + DROWS) : i0, j1 = min(k, j0 + DROWS);
     constexpr int LDT = DROWS + 2;
     static_assert(LDT * DROWS <= 2 * DROWS * (DKC + 2), "tile fits the staging buffers");
     if (p == 0) {   // the blocks of K that enter this tile
@@ -790,7 +918,7 @@ __global__ __launch_bounds__(256) void k_front_cols(DirectDev d, const FrontTask
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = i0 + wi + 16 * a + 4 * i + (lane >> 4), col = j0 + wj + 16 * b + (lane & 15);
-                if (row >= i1 || col >= j1 || col > row) continue;
+                if (row >= i1 || col >= j1 || col > row || (row - t0 < w1 && col - t0 < w1)) continue;
                 double v;
                 if (p > 0)
                     v = F[(int64_t)row * k + col];
@@ -946,12 +1074,17 @@ __global__ __launch_bounds__(256) void k_solve_fwd(DirectDev d, const FrontTask*
     }
 }
 
-// x1 = S r1 - G^T x2 for one panel per workgroup; x in node order
+// x1 = S r1 - G^T x2 for one panel of every front, its columns over `parts` workgroups;
+// x in node order.  Bound by the reads of S and G, each once: a workgroup alone with the
+// panel of a large front (2 300 rows of 96) took 13 us, eight take 8.
 template <int NR, int NT>
 __global__ __launch_bounds__(NT) void k_solve_bwd(DirectDev d, const FrontTask* __restrict__ tasks,
-                                                  const int32_t* __restrict__ active, double* __restrict__ x, int p) {
+                                                  const int32_t* __restrict__ active, double* __restrict__ x, int p,
+                                                  int n, int parts) {
     extern __shared__ double P[];
-    const FrontTask f = tasks[blockIdx.x];
+    const Where at = locate(n, parts);
+    if (at.task >= n) return;
+    const FrontTask f = tasks[at.task];
     if (p >= f.npan || f.np == 0 || !any_active<NR>(active, f.sys)) return;
     const int mn = f.np + f.nb, m = 6 * mn, p0 = p * f.wn, wn = min(f.wn, f.np - p0), w = 6 * wn, c0 = 6 * p0;
     const int tid = threadIdx.x, nb = m - c0 - w;
@@ -963,8 +1096,10 @@ __global__ __launch_bounds__(NT) void k_solve_bwd(DirectDev d, const FrontTask* 
     }
     __syncthreads();
     const double* S = d.fac + f.fac + panel_offset(m, 6 * f.wn, p);   // w rows of S (symmetric), then G's
-    // lane pairs of columns; the groups of w / 2 threads share the rows, eight in flight
-    const int hw = w / 2, ng = NT / hw, g = tid / hw, j = 2 * (tid - g * hw);
+    // lane pairs of columns, this part's from j0 on; groups of hw threads share the rows, eight in flight
+    const int h0 = w / 2 * at.part / parts, hw = w / 2 * (at.part + 1) / parts - h0, j0 = 2 * h0, wj = 2 * hw;
+    if (hw == 0) return;
+    const int ng = NT / hw, g = tid / hw, j = 2 * (tid - g * hw);
     double acc[2][NR];
 #pragma unroll
     for (int h = 0; h < NR; ++h) acc[0][h] = acc[1][h] = 0.0;
@@ -974,7 +1109,7 @@ __global__ __launch_bounds__(NT) void k_solve_bwd(DirectDev d, const FrontTask* 
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int i = i0 + u * ng;
-                a[u] = *reinterpret_cast<const double2*>(i < w + nb ? S + (int64_t)i * w + j : d.zero);
+                a[u] = *reinterpret_cast<const double2*>(i < w + nb ? S + (int64_t)i * w + j0 + j : d.zero);
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
@@ -987,19 +1122,27 @@ __global__ __launch_bounds__(NT) void k_solve_bwd(DirectDev d, const FrontTask* 
             }
         }
     }
-    double* red = r1 + (w + nb) * NR;        // [ng][w][NR]
+    double* red = r1 + (w + nb) * NR;        // [ng][wj][NR]
     if (g < ng) {
 #pragma unroll
         for (int h = 0; h < NR; ++h) {
-            red[(g * w + j) * NR + h] = acc[0][h];
-            red[(g * w + j + 1) * NR + h] = acc[1][h];
+            red[(g * wj + j) * NR + h] = acc[0][h];
+            red[(g * wj + j + 1) * NR + h] = acc[1][h];
         }
     }
     __syncthreads();
-    for (int e = tid; e < w * NR; e += NT) {
+    // sums over the groups: eight partial sums each, then those
+    for (int e = tid; e < 8 * wj * NR; e += NT) {
+        const int c = e % (wj * NR), q0 = e / (wj * NR);
         double s = 0.0;
-        for (int q = 0; q < ng; ++q) s += red[q * w * NR + e];
-        const int l = p0 + e / (6 * NR), q = e % (6 * NR);
+        for (int q = q0; q < ng; q += 8) s += red[q * wj * NR + c];
+        if (q0 < ng) red[e] = s;   // (its own first term's place)
+    }
+    __syncthreads();
+    for (int e = tid; e < wj * NR; e += NT) {
+        double s = 0.0;
+        for (int q = 0; q < min(8, ng); ++q) s += red[q * wj * NR + e];
+        const int c = j0 * NR + e, l = p0 + c / (6 * NR), q = c % (6 * NR);
         x[((int64_t)f.gnode0 + d.nodes[f.node0 + l]) * 6 * NR + q] = s;
     }
 }
@@ -1477,7 +1620,7 @@ static int direct_build(Plan* pl, DirectState& D) {
     const std::pair<const void*, size_t> lds[] = {
         {(const void*)k_front_small<1024>, DLDS_MAX}, {(const void*)k_front_small<512>, DLDS_MAX},
         {(const void*)k_front_small<256>, DLDS_MAX},  {(const void*)k_front_diag, DW * (DW + 2) * 8},
-        {(const void*)k_front_strip, (DW + SROWS) * (DW + 2) * 8},
+        {(const void*)k_front_strip, (DW + SROWS) * (DW + 2) * 8}, {(const void*)k_front_cols<true>, DW * (DW + 2) * 8},
         {(const void*)k_solve_bwd<1, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<1, 1024>, DLDS_MAX},
         {(const void*)k_solve_bwd<2, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<2, 1024>, DLDS_MAX},
         {(const void*)k_solve_bwd<3, 256>, DLDS_MAX}, {(const void*)k_solve_bwd<3, 1024>, DLDS_MAX},
@@ -1508,14 +1651,22 @@ static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
             const int m = D.big_m[L], kw = (D.big_w[L] + 15) & ~15;   // largest front, widest panel
             // strips of 96 rows, or of 32 while that leaves CUs without work
             const int rows = (int64_t)nb * ((m + SROWS - 1) / SROWS) >= 512 ? SROWS : 32;
+            const bool head = nb < HEAD_FRONTS;
+            const size_t block = (size_t)kw * (kw + 2) * 8, tile = (size_t)2 * DROWS * (DKC + 2) * 8;
             for (int p = 0; p < D.big_pan[L]; ++p) {
-                hipLaunchKernelGGL(k_front_diag, dim3(nb), dim3(512), (size_t)kw * (kw + 2) * 8, s, D.dev, t, p);
-                const int strips = (m + rows - 1) / rows;
+                if (p == 0 || !head) hipLaunchKernelGGL(k_front_diag, dim3(nb), dim3(512), block, s, D.dev, t, p);
+                const int strips = (m + rows - 1) / rows + 1;
                 hipLaunchKernelGGL(k_front_strip, part_grid(nb, strips), dim3(1024),
                                    (size_t)(kw + rows) * (kw + 2) * 8, s, D.dev, t, p, nb, strips, rows);
                 if (p + 1 < D.big_pan[L]) {
                     const int tiles = ((m + DROWS - 1) / DROWS) * ((D.big_k[L] + DROWS - 1) / DROWS);
-                    hipLaunchKernelGGL(k_front_cols, part_grid(nb, tiles), dim3(256), 0, s, D.dev, t, p, nb, tiles);
+                    const int parts = (tiles + 1) / 2;
+                    if (head)
+                        hipLaunchKernelGGL(k_front_cols<true>, part_grid(nb, parts + 1), dim3(512),
+                                           std::max(block, 2 * tile), s, D.dev, t, p, nb, parts);
+                    else
+                        hipLaunchKernelGGL(k_front_cols<false>, part_grid(nb, tiles), dim3(256), tile, s, D.dev, t, p,
+                                           nb, tiles);
                 }
             }
             const int bt = (D.big_b[L] + DROWS - 1) / DROWS, tiles = bt * (bt + 1) / 2;
@@ -1545,14 +1696,16 @@ static void direct_apply(DirectState& D, const int32_t* active, const double* r,
     }
     for (int L = D.n_levels - 1; L >= 0; --L) {
         const int nb = (int)D.big_n[L];
+        // columns in parts while that leaves CUs without work
+        const int cols = nb ? std::max(1, std::min(BWD_PARTS, 256 / nb)) : 1;
         for (int p = D.big_pan[L] - 1; nb && p >= 0; --p)
-            hipLaunchKernelGGL((k_solve_bwd<NR, 1024>), dim3(nb), dim3(1024),
+            hipLaunchKernelGGL((k_solve_bwd<NR, 1024>), part_grid(nb, cols), dim3(1024),
                                ((size_t)D.big_m[L] + 2 * 1024) * NR * 8, s, D.dev, D.d_tasks + D.big_off[L], active, z,
-                               p);
+                               p, nb, cols);
         if (D.small_n[L])
-            hipLaunchKernelGGL((k_solve_bwd<NR, 256>), dim3((unsigned)D.small_n[L]), dim3(256),
+            hipLaunchKernelGGL((k_solve_bwd<NR, 256>), part_grid(D.small_n[L], 1), dim3(256),
                                ((size_t)D.small_m[L] + 2 * 256) * NR * 8, s, D.dev, D.d_tasks + D.small_off[L], active,
-                               z, 0);
+                               z, 0, (int)D.small_n[L], 1);
     }
 }
 

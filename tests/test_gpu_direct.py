@@ -177,3 +177,23 @@ def test_dense_solve_of_the_plans_own_assembly(m):
     assert rel(u.cpu().numpy(), v.cpu().numpy()) < 1e-9
     ref = oracle_u(st, F)
     assert rel(u.cpu().numpy().reshape(-1, m), ref) < 1e-9
+
+
+@pytest.mark.parametrize("copies", [1, 3, 64])
+def test_fronts_in_panels_of_few_and_of_many_structures(copies):
+    """40 x 40 shells, whose upper fronts go in panels: few structures (the update of a panel
+    factors the next panel's block, a panel's columns are solved for in parts) and 64 of them
+    (launches of their own), against the oracle."""
+    designs = []
+    for i in range(copies):
+        st = wl.shell_pinned_edges(40, 10.0, 1.5, design=4)
+        st.crds[st.design_nodes, 2] += np.random.default_rng(i).normal(0.0, 0.01, len(st.design_nodes))
+        designs.append(st)
+    b = StructureBatch(designs)
+    print(f"direct panels x {copies}", flush=True)
+    u = b.solve().cpu().numpy().ravel()
+    info = b.plan.last_info
+    assert info["converged"] == copies and info["levels"] == 0, info
+    for i in {0, copies // 2, copies - 1}:
+        o, st = 6 * int(b.node_off[i]), designs[i]
+        assert rel(u[o:o + st.ndof], oracle_u(st, st.nodal_loads)) < 1e-8, (i, info)
