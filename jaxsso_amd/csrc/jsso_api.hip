@@ -553,7 +553,7 @@ int jsso_assemble(jsso_plan* plan, const double* d_crds, const double* d_prop_be
     hipStream_t s = (hipStream_t)stream;
     int rc0 = ensure_device(p);
     if (rc0) return rc0;
-    JSSO_HIP(hipMemsetAsync(p->d_status, 0, sizeof(int32_t), s));
+    if ((rc0 = launch_clear_status(p, s))) return rc0;
     p->status_cache = -1;
     std::pair<hipEvent_t, hipEvent_t>* ev = nullptr;
     timing_begin_slot(s, ev, JSSO_TIMING_ELEMENT);
@@ -602,7 +602,10 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
     int rc = launch_full_blocks(p, s);
     if (rc) return rc;
     const int64_t ndof = 6 * (int64_t)p->n_nodes;
-    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set) {
+    // (it sets u to zero first and reads f again at every step: not for f inside u)
+    const size_t bytes = (size_t)ndof * nrhs * sizeof(double);
+    const bool apart = (const char*)d_f + bytes <= (const char*)d_u || (const char*)d_u + bytes <= (const char*)d_f;
+    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set && apart) {
         bool done = false;
         rc = direct_defect(p, p->d_K, d_f, d_u, nrhs, transpose, tol, maxit, h_info, s, done);
         if (rc || done) return rc;
@@ -697,17 +700,20 @@ int jsso_solve(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs, in
     }
     int rc = ensure_device(p);
     if (rc) return rc;
+    const int slot = precision == JSSO_PREC_FP64 ? PS_F64 : precision == JSSO_PREC_MIXED ? PS_F32 : PS_F32_V64;
+    bool tried = false;
+    if (precision != JSSO_PREC_PLAIN && !p->precond_set && expect_symmetric(p)) {
+        bool done = false;
+        rc = direct_solve(p, d_f, d_u, nrhs, slot, tol, maxit, h_info, s, done);
+        if (rc || done) return rc;
+        tried = true;
+    }
     int32_t status = 0;
     if ((rc = assembly_status(p, s, &status))) return rc;
     if (status & STATUS_NONSYM) return solve_nonsymmetric(p, d_f, d_u, nrhs, precision, tol, maxit, h_info, false, s,
                                                            status);
-    switch (precision) {
-        case JSSO_PREC_FP64: return solve_batched(p, d_f, d_u, nrhs, PS_F64, tol, maxit, h_info, s);
-        case JSSO_PREC_MIXED: return solve_batched(p, d_f, d_u, nrhs, PS_F32, tol, maxit, h_info, s);
-        case JSSO_PREC_MIXED_V64: return solve_batched(p, d_f, d_u, nrhs, PS_F32_V64, tol, maxit, h_info, s);
-        case JSSO_PREC_PLAIN: return solve_plain(p, d_f, d_u, nrhs, tol, maxit, h_info, s);
-        default: set_error("unknown precision %d", precision); return JSSO_EINVAL;
-    }
+    if (precision == JSSO_PREC_PLAIN) return solve_plain(p, d_f, d_u, nrhs, tol, maxit, h_info, s);
+    return solve_batched(p, d_f, d_u, nrhs, slot, tol, maxit, h_info, s, tried);
 }
 
 int jsso_solve_transpose(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs, int32_t precision,
@@ -873,6 +879,13 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
     int rc = ensure_device(p);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
+    bool tried = false;
+    if (!d_K && expect_symmetric(p)) {
+        bool done = false;
+        rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, nullptr, s, done);
+        if (rc || done) return rc;
+        tried = true;
+    }
     int32_t status = 0;
     if (p->assembled && (rc = assembly_status(p, s, &status))) return rc;
     if (!d_K) {
@@ -884,7 +897,7 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
         // (19x19 barrel vault, 2 400 DOF, evaluation with gradient: 8.9 ms dense, 1.2
         // ms so), refined to its attainable accuracy; what it does not take or finish (a
         // pivot that is not positive) is left to the dense factorisation and its errors
-        if (!(status & (STATUS_NONSYM | 1))) {
+        if (!tried && !(status & (STATUS_NONSYM | 1))) {
             bool done = false;
             rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, nullptr, s, done);
             if (rc || done) return rc;

@@ -426,6 +426,14 @@ int launch_export_blocks(Plan* p, double* K, hipStream_t s) {
     return JSSO_OK;
 }
 
+__global__ void clear_status_kernel(int32_t* status) { *status = 0; }
+
+int launch_clear_status(Plan* p, hipStream_t s) {
+    hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(1), 0, s, p->d_status);
+    JSSO_HIP(hipGetLastError());
+    return JSSO_OK;
+}
+
 int launch_assemble(Plan* p, const double* crds, hipStream_t s) {
     JSSO_REQUIRE(p->on_device, JSSO_EINVAL, "plan not uploaded to the device");
     p->full_valid = false;

@@ -89,6 +89,8 @@ struct DirectDev {
 struct DirectReport {
     int32_t running, stalled, floor, bad;   // systems; structures with a pivot that is not positive
     double worst;                           // largest relative residual of the best iterates
+    int32_t flags;                          // the assembly's (d_status)
+    int32_t final;                          // every system done, on a K that this solve is for
 };
 
 struct DirectState {
@@ -106,7 +108,7 @@ struct DirectState {
     DirectDev dev{};
     const FrontTask* d_tasks = nullptr;
     double* d_rho = nullptr;
-    DirectReport *d_report = nullptr, *h_report = nullptr;
+    DirectReport *d_report = nullptr, *h_report = nullptr, *host_report = nullptr;   // host_report: h_report for the device
     size_t vec_bytes = 0;
     std::vector<void*> allocs;
     bool usable = false, factored = false;
@@ -1164,7 +1166,9 @@ __global__ __launch_bounds__(SOLVER_WG) void k_direct_add(Slices sl, const int32
 // what the host needs to know after a refinement step
 __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, const int32_t* __restrict__ status,
                                                        const double* __restrict__ best,
-                                                       const int32_t* __restrict__ bad, DirectReport* out) {
+                                                       const int32_t* __restrict__ bad,
+                                                       const int32_t* __restrict__ flags, DirectReport* out,
+                                                       DirectReport* host) {
     __shared__ int cnt[4];
     __shared__ double worst[4];
     const int tid = threadIdx.x;
@@ -1187,12 +1191,54 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
     if ((tid & 63) == 0) worst[tid >> 6] = w;
     __syncthreads();
     if (tid == 0) {
-        out->running = cnt[0];
-        out->stalled = cnt[1];
-        out->floor = cnt[2];
-        out->bad = cnt[3];
-        out->worst = fmax(fmax(worst[0], worst[1]), fmax(worst[2], worst[3]));
+        DirectReport v;
+        v.running = cnt[0];
+        v.stalled = cnt[1];
+        v.floor = cnt[2];
+        v.bad = cnt[3];
+        v.worst = fmax(fmax(worst[0], worst[1]), fmax(worst[2], worst[3]));
+        v.flags = *flags;
+        v.final = !(v.running | v.stalled | v.bad | (v.flags & (STATUS_NONSYM | 1)));
+        *out = v;
+        *host = v;   // pinned: no copy of its own
     }
+}
+
+// After a step's report: u = L^-T x of the best iterates where that is the end (u is
+// not touched before: it may be f itself, which another route then still needs), else
+// the iterates that have become the best are kept.
+template <int NR>
+__global__ __launch_bounds__(SOLVER_WG) void k_direct_finish(Slices sl, const int32_t* __restrict__ save,
+                                                             const DirectReport* __restrict__ report,
+                                                             const double* __restrict__ Linv,
+                                                             const double* __restrict__ x64,
+                                                             double* __restrict__ xbest, double* __restrict__ u) {
+    const int w = slice_of_block(sl);
+    if (w < 0) return;
+    const int sys = sl.sys[w];
+    const int64_t R = 6 * (int64_t)sl.row0[w] + threadIdx.x;
+    const bool end = report->final != 0;
+    if (R >= 6 * (int64_t)sl.row1[w] || (!end && report->running == 0)) return;
+    const int64_t i = R / 6;
+    const int r = (int)(R % 6);
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+        const bool now = save[sys * NR + h] != 0;
+        if (end) {
+            const double* x = now ? x64 : xbest;
+            double v = 0.0;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) v += Linv[i * 36 + c * 6 + r] * x[(6 * i + c) * NR + h];
+            u[R * NR + h] = v;
+        } else if (now) {
+            xbest[R * NR + h] = x64[R * NR + h];
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_direct_clear(int n, int32_t* __restrict__ bad) {
+    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (i < n) bad[i] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1615,6 +1661,7 @@ static int direct_build(Plan* pl, DirectState& D) {
         return rc == JSSO_ENOMEM ? JSSO_OK : rc;
     }
     JSSO_HIP(hipHostMalloc((void**)&D.h_report, sizeof(DirectReport), hipHostMallocDefault));
+    JSSO_HIP(hipHostGetDevicePointer((void**)&D.host_report, D.h_report, 0));
     D.d_rho = const_cast<double*>(dr);
     D.dev.A64 = pl->d_Ke64;
     const std::pair<const void*, size_t> lds[] = {
@@ -1632,7 +1679,7 @@ static int direct_build(Plan* pl, DirectState& D) {
 }
 
 static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
-    JSSO_HIP(hipMemsetAsync(D.dev.bad, 0, pl->n_sys * sizeof(int32_t), s));
+    hipLaunchKernelGGL(k_direct_clear, dim3((unsigned)((pl->n_sys + 255) / 256)), dim3(256), 0, s, pl->n_sys, D.dev.bad);
     static_assert((DW + SROWS) * (DW + 2) * 8 <= DLDS_MAX, "panel LDS");
     for (int L = 0; L < D.n_levels; ++L) {
         for (const auto& B : D.buckets[L]) {
@@ -1796,11 +1843,11 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
     int32_t& wps = pl->direct_wps[slot][NR];
     if (wps <= 0 && (rc = tune_residual<NR>(pl, w, sl, r, s, wps))) return rc;
     if ((rc = ensure_factor(pl, D, s))) return rc;
-    const int64_t nr = 6 * (int64_t)pl->n_nodes;
     for (int it = 1; it <= std::min(maxit, DIRECT_STEPS); ++it) {
-        direct_apply<NR>(D, w.st.active, r, z, s);
-        hipLaunchKernelGGL((k_direct_add<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.slice_act,
-                           (const double*)z, w.x64);
+        direct_apply<NR>(D, w.st.active, r, it == 1 ? w.x64 : z, s);   // (x is zero before)
+        if (it > 1)
+            hipLaunchKernelGGL((k_direct_add<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.slice_act,
+                               (const double*)z, w.x64);
         auto residual = [&](auto W) {
             constexpr int WP = decltype(W)::value;
             hipLaunchKernelGGL((k_replace<double, NR, WP>), g, dim3(64 * WP), 0, s, sl, w.P, w.st,
@@ -1816,19 +1863,17 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
         // accuracy as converged there, else as stalled)
         hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 1, tol, 1, 2,
                            (const double*)D.d_rho, DIRECT_FLOOR_FACTOR, 0);
-        hipLaunchKernelGGL((k_save<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.save,
-                           (const double*)w.x64, w.xbest);
         hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys, (const int32_t*)w.st.status,
-                           (const double*)w.st.best, (const int32_t*)D.dev.bad, D.d_report);
-        // (final unless a system is still running)
-        hipLaunchKernelGGL((k_unscale<NR>), dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, pl->n_nodes,
-                           pl->d_Linv, (const double*)w.xbest, u);
+                           (const double*)w.st.best, (const int32_t*)D.dev.bad, (const int32_t*)pl->d_status,
+                           D.d_report, D.host_report);
+        hipLaunchKernelGGL((k_direct_finish<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.save,
+                           (const DirectReport*)D.d_report, pl->d_Linv, (const double*)w.x64, w.xbest, u);
         JSSO_HIP(hipGetLastError());
-        JSSO_HIP(hipMemcpyAsync(D.h_report, D.d_report, sizeof(DirectReport), hipMemcpyDeviceToHost, s));
         JSSO_HIP(hipStreamSynchronize(s));
         const DirectReport& R = *D.h_report;
-        if (R.bad || R.stalled) return JSSO_OK;
-        if (R.running) continue;
+        pl->status_cache = pl->status_last = R.flags;
+        if (R.running && !R.bad && !R.stalled && !(R.flags & (STATUS_NONSYM | 1))) continue;
+        if (!R.final) return JSSO_OK;
         done = true;
         if (info) {
             *info = jsso_info{};
@@ -1928,9 +1973,8 @@ static int run_defect(Plan* pl, DirectState& D, const double* K, const double* f
         if (it == most || (it >= 4 && it % 2 == 0)) {
             hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys,
                                (const int32_t*)w.st.status, (const double*)w.st.best, (const int32_t*)D.dev.bad,
-                               D.d_report);
+                               (const int32_t*)pl->d_status, D.d_report, D.host_report);
             JSSO_HIP(hipGetLastError());
-            JSSO_HIP(hipMemcpyAsync(D.h_report, D.d_report, sizeof(DirectReport), hipMemcpyDeviceToHost, s));
             JSSO_HIP(hipStreamSynchronize(s));
             const DirectReport& R = *D.h_report;
             if (R.bad || R.stalled) return JSSO_OK;

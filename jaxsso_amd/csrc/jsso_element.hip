@@ -7,11 +7,37 @@
 
 namespace jsso {
 
+// A wavefront's 64 element blocks (a lane's 6x6 each, consecutive in memory from dst on;
+// the first n of them are stored) through LDS in whole lines, a half of each block at a
+// time; st: 64 * OUT doubles of the wavefront, free once the workgroup gets here.
+constexpr int OUT = 19;   // odd: the lanes' values start in different banks
+__device__ __forceinline__ void store_blocks(const double (&out)[6][6], double* st, double* dst, int n) {
+    const int wl = threadIdx.x & 63;
+    double2* to = (double2*)dst;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 18; ++q) st[wl * OUT + q] = out[3 * half + q / 6][q % 6];
+        __syncthreads();
+#pragma unroll 3
+        for (int i = wl; i < 9 * n; i += 64) {
+            const int blk = i / 9, k = i % 9;
+            const double* v = st + blk * OUT + 2 * k;
+            to[blk * 18 + 9 * half + k] = make_double2(v[0], v[1]);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Beam-column stiffness: one thread per (element, node pair a, b).
 // Ke_ab = blockdiag(D^-1, D^-1) K_loc,ab blockdiag(D, D)  (solve(T,K)@T,
 // element.py:130-139); D^-1 = D^T for the orthogonal general branch.
 // BLOCKS: output [e][a][b][6x6] (assembly), else row-major 12x12 per element.
+// The entries of K_loc are formed once and placed by the signs of their node pair:
+// looked up entry by entry (36 switches with their divisions) and stored by lane, 220
+// beams took 19 us; this takes 5 us, and 62 us for 228k (256 gridshells, 263 MB), bound
+// by its stores.
 // ---------------------------------------------------------------------------
 template <bool BLOCKS>
 __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* __restrict__ crds_e,
@@ -21,7 +47,7 @@ __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* _
                                                       double* __restrict__ ke, int32_t* flags,
                                                       int32_t* status) {
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int e = tid >> 2;
+    const int e = BLOCKS ? min(tid >> 2, n - 1) : tid >> 2;   // (there the wave stores together)
     if (e >= n) return;
     const int a = (tid >> 1) & 1, b = tid & 1;
     double c[6];
@@ -50,16 +76,27 @@ __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* _
     }
     if (flags && a == 0 && b == 0) flags[e] = special ? 1 : 0;
     if (status && special && a == 0 && b == 0) atomicOr(status, STATUS_NONSYM | STATUS_Y_BEAM);
+    // K_loc (beam_kloc's entries): axial, torsion; per bending plane the coefficients of
+    // w w, w theta, theta theta of one node, theta theta of two
+    const double ax = A * E / L, to = G * Jt / L;
+    const double z12 = 12.0 * E * Iz / (L * L * L), z6 = 6.0 * E * Iz / (L * L), zr = (a == b ? 4.0 : 2.0) * E * Iz / L;
+    const double y12 = 12.0 * E * Iy / (L * L * L), y6 = 6.0 * E * Iy / (L * L), yr = (a == b ? 4.0 : 2.0) * E * Iy / L;
+    const bool same = a == b;
     double out[6][6];
 #pragma unroll
     for (int pq = 0; pq < 4; ++pq) {
         const int p = pq >> 1, q = pq & 1;  // translation / rotation sub-blocks
-        double S[3][3], tmp[3][3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                S[i][j] = beam_kloc<double>(6 * a + 3 * p + i, 6 * b + 3 * q + j, L, E, G, Iy, Iz, Jt, A);
+        double S[3][3] = {}, tmp[3][3];
+        if (p == q) {
+            S[0][0] = p ? (same ? to : -to) : (same ? ax : -ax);
+            S[1][1] = p ? yr : (same ? z12 : -z12);
+            S[2][2] = p ? zr : (same ? y12 : -y12);
+        } else {
+            const bool first = (p ? b : a) == 0;   // the translation's node
+            const double sz = first ? z6 : -z6, sy = first ? -y6 : y6;
+            S[1][2] = p ? sy : sz;
+            S[2][1] = p ? sz : sy;
+        }
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -71,15 +108,16 @@ __global__ __launch_bounds__(256) void ke_beam_kernel(int32_t n, const double* _
             for (int j = 0; j < 3; ++j)
                 out[3 * p + i][3 * q + j] = Di[i][0] * tmp[0][j] + Di[i][1] * tmp[1][j] + Di[i][2] * tmp[2][j];
     }
+    if (BLOCKS) {
+        __shared__ double lds[4][64 * OUT];
+        const int b0 = blockIdx.x * 256 + (threadIdx.x & ~63);   // the wave's first block
+        store_blocks(out, lds[threadIdx.x >> 6], ke + (int64_t)b0 * 36, min(64, 4 * n - b0));
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 6; ++i)
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-            if (BLOCKS)
-                ke[((int64_t)e * 4 + a * 2 + b) * 36 + i * 6 + j] = out[i][j];
-            else
-                ke[(int64_t)e * 144 + (6 * a + i) * 12 + 6 * b + j] = out[i][j];
-        }
+        for (int j = 0; j < 6; ++j) ke[(int64_t)e * 144 + (6 * a + i) * 12 + 6 * b + j] = out[i][j];
 }
 
 // ---------------------------------------------------------------------------
@@ -114,7 +152,7 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
                                                            double* __restrict__ ke, int32_t* status = nullptr) {
     // one wave's part: the tiles of its four elements, then (QK_BLOCKS) its 64 blocks on
     // their way out, a lane's 36 values an odd stride apart
-    constexpr int TILE = sizeof(QuadTile) / sizeof(double), OUT = 19;
+    constexpr int TILE = sizeof(QuadTile) / sizeof(double);
     constexpr int WAVE_LDS = MODE == QK_BLOCKS ? 64 * OUT : 4 * TILE;
     __shared__ double lds[EPW / 4][WAVE_LDS];
     const int le = threadIdx.x >> 4, lane = threadIdx.x & 15;
@@ -261,24 +299,8 @@ __global__ __launch_bounds__(16 * EPW) void ke_quad_kernel(int32_t n, const doub
                 out[3 * p + i][3 * q + j] = R[0][i] * tmp[0][j] + R[1][i] * tmp[1][j] + R[2][i] * tmp[2][j];
     }
     if (MODE == QK_BLOCKS) {
-        double* st = lds[le >> 2];
-        const int wl = threadIdx.x & 63;
         const int64_t e0 = (int64_t)blockIdx.x * EPW + (threadIdx.x >> 6) * 4;
-        const int count = (int)(n - e0 < 4 ? n - e0 : 4) * 16 * 9;   // pairs of values (none past the end)
-        double2* dst = (double2*)(ke + e0 * 16 * 36);
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            __syncthreads();   // the tiles, or the first half, have been read
-#pragma unroll
-            for (int q = 0; q < 18; ++q) st[wl * OUT + q] = out[3 * half + q / 6][q % 6];
-            __syncthreads();
-#pragma unroll 3
-            for (int i = wl; i < count; i += 64) {
-                const int blk = i / 9, k = i % 9;
-                const double* v = st + blk * OUT + 2 * k;
-                dst[blk * 18 + 9 * half + k] = make_double2(v[0], v[1]);
-            }
-        }
+        store_blocks(out, lds[le >> 2], ke + e0 * 16 * 36, (int)(n - e0 < 4 ? n - e0 : 4) * 16);
         return;
     }
 #pragma unroll

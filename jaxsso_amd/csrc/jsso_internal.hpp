@@ -159,6 +159,7 @@ struct Plan {
     int32_t nonsym_route = 0;     // non-symmetric K: 0 auto, 1 dense LU, 2 defect correction
     bool sym_part_solve = false;  // set while the defect correction solves with the symmetric part
     int32_t status_cache = -1;    // host copy of *d_status once read after an assembly (-1: not read)
+    int32_t status_last = -1;     // the flags read last, of this assembly or an earlier one
     bool assembled = false;
     bool full_valid = false;      // d_K / d_Kc hold the current assembly
     double* d_crds = nullptr;     // node coordinates of the current assembly (for the AMG null space)
@@ -209,6 +210,7 @@ int launch_quad_gauss(int32_t n, const double* xy, const double* props, double r
                       double* Bg, double* Bm, double* Cb, double* Cs, double* Cm, hipStream_t s);
 int launch_assemble(Plan* p, const double* crds, hipStream_t s);   // also keeps crds in d_crds
 int launch_export_blocks(Plan* p, double* K, hipStream_t s);
+int launch_clear_status(Plan* p, hipStream_t s);
 int launch_csr_spmv(int32_t n_rows, const int32_t* rowptr, const int32_t* colind, const double* vals,
                     const double* x, const double* c, double* y, hipStream_t s);
 int launch_full_blocks(Plan* p, hipStream_t s);
@@ -218,8 +220,9 @@ int launch_adjoint(Plan* p, const double* crds, const double* prop_beam, const d
 int launch_gather_grad(Plan* p, const double* gbuf, int nrhs, double* dcrds, hipStream_t s);
 int noalloc_scratch(double** ptr, size_t* bytes);
 int launch_spmv_full(Plan* p, const double* K, const double* x, double* y, hipStream_t s);
+// direct_tried: direct_solve has been asked already and did not take or finish it
 int solve_batched(Plan* p, const double* f, double* u, int nrhs, int slot, double tol,
-                  int maxit, jsso_info* info, hipStream_t s);
+                  int maxit, jsso_info* info, hipStream_t s, bool direct_tried = false);
 int timing_enable(int every);
 int timing_read(int slot, double* avg_ms, int64_t* samples, int reset);
 void timing_begin(hipStream_t s, std::pair<hipEvent_t, hipEvent_t>*& ev);
@@ -246,6 +249,7 @@ void amg_destroy(Plan* p);
 int dense_solve(Plan* p, const double* K, const double* f, double* u, int nrhs, bool lu, bool transpose,
                 hipStream_t s);
 int assembly_status(Plan* p, hipStream_t s, int32_t* status);
+bool expect_symmetric(const Plan* p);
 int solve_plain(Plan* p, const double* f, double* u, int nrhs, double tol, int maxit,
                 jsso_info* info, hipStream_t s);
 

@@ -4,10 +4,13 @@ single-front structures, one-workgroup fronts of every padding, fronts in panels
 several components, both element types, 1 to 4 load cases, uneven batches."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from jaxsso_amd import _native as nat
 from jaxsso_amd import workloads as wl
 from jaxsso_amd.batch import StructureBatch
 from jaxsso_amd.plan import FEPlan
@@ -197,3 +200,33 @@ def test_fronts_in_panels_of_few_and_of_many_structures(copies):
     for i in {0, copies // 2, copies - 1}:
         o, st = 6 * int(b.node_off[i]), designs[i]
         assert rel(u[o:o + st.ndof], oracle_u(st, st.nodal_loads)) < 1e-8, (i, info)
+
+
+@pytest.mark.parametrize("kinds", ["sym sym ortho sym ortho ortho", "ortho sym sym", "sym bad sym"])
+def test_assemblies_that_change_kind_on_one_plan(kinds):
+    """The direct solve starts before the assembly's flags are known where the last ones
+    allowed it: K that is or is not symmetric, or has a diagonal block that is not positive
+    definite, in any order on one plan, also with the result over the right-hand side."""
+    st = orthotropic(9, 1.0, 1.0)
+    plan = FEPlan([0, st.n_node], st.cnct_beamcols, st.cnct_quads, st.known_id)
+    f = torch.tensor(st.nodal_loads, device="cuda")
+    for kind in kinds.split():
+        print(f"direct flags {kind}", flush=True)
+        pq = st.prop_quads.copy()
+        pq[:, 3:] = (1.5, 0.6) if kind == "ortho" else (1.0, 1.0)
+        if kind == "bad":
+            pq[:, 1] *= -1.0
+        plan.assemble(torch.tensor(st.crds), None, torch.tensor(pq))
+        if kind == "bad":
+            with pytest.raises(RuntimeError):
+                plan.solve(f)
+            continue
+        u = plan.solve(f).cpu().numpy()
+        K = system.assemble_K(st.crds, st.cnct_beamcols, st.prop_beamcols, st.cnct_quads, pq)
+        assert rel(u, osolve.solve_reduced(K, st.known_id, st.nodal_loads)) < 1e-8, kind
+        # in place, and again with the flags unread
+        plan.assemble(torch.tensor(st.crds), None, torch.tensor(pq))
+        v, info = f.clone(), nat.Info()
+        nat.check(nat.lib().jsso_solve(plan._h, nat.ptr(v), nat.ptr(v), 1, nat.PREC["fp64"], 1e-12, 1000,
+                                       ctypes.byref(info), nat.stream_ptr()), allow_not_converged=True)
+        assert rel(v.cpu().numpy(), u) < 1e-8, kind
