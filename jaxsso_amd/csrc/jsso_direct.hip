@@ -206,12 +206,16 @@ __device__ __forceinline__ bool factor16(d4 A, double* D, int ld, int lane) {
 // inverse factor (whole workgroup).  Block (I, J) of L^-1, I > J, is left at block
 // row J, block column I (as it is, not transposed), the diagonal blocks in place;
 // the lower blocks hold L.  Per block column kb two phases with a barrier each:
-//   B  what column kb - 1 updates: wavefront 0 takes the diagonal block and factors
-//      it, the others the rest of the trailing triangle and the sums
+//   B  wavefront 0 factors the diagonal block; the others take what column kb - 1
+//      updates: the rest of the trailing triangle and the sums
 //      W_IJ = sum_K L_IK Linv_KJ of the rows below
-//   A  L_I = A_I Dinv^T below the block, and row kb of the inverse, -Dinv W_J
+//   A  wavefront 0: L = A Dinv^T of the next block row and with it the next diagonal
+//      block, from its registers; the others: the L below, and row kb of the inverse,
+//      -Dinv W_J
 // The factorisation of a 16x16 block (one wavefront, ~1.5 us of dependent steps) is
-// the chain that bounds this routine; phase B hides the products behind it.
+// the chain that bounds this routine (96 columns: 14 us); phase B hides the products
+// behind it.  With the next diagonal block updated in a phase of its own, a 200 x 200
+// shell took 4.99 ms, so 4.92.
 __device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wave, int nw, int lane) {
     const int nt = kp >> 4, r = lane & 15, q = lane >> 4;
     bool ok = true;
@@ -255,34 +259,49 @@ __device__ __forceinline__ bool invert_factor(double* P, int ld, int kp, int wav
             for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
         }
         double* D = P + (16 * kb) * ld + 16 * kb;
-        if (wave == 0) {
+        auto lower = [&](const double* T) {
             d4 A;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int c = 4 * i + q;
-                A[i] = r >= c ? D[r * ld + c] : D[c * ld + r];
+                A[i] = r >= c ? T[r * ld + c] : T[c * ld + r];
             }
-            if (kb > 0) {
-                const double* X = P + (16 * kb + r) * ld + 16 * j + q;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) A = mfma64(-X[4 * t], X[4 * t], A);
-            }
-            ok &= factor16(A, D, ld, lane);
-        }
+            return A;
+        };
+        if (wave == 0) ok &= factor16(lower(D), D, ld, lane);
         __syncthreads();
+        if (wave == 0) {
+            if (kb + 1 < nt) {
+                // M = L^T = Dinv A^T: element i of a lane is L[r][4 i + q], both operands of L L^T
+                double* N = P + (16 * (kb + 1) + r) * ld + 16 * kb + q;
+                double* T = D + 16 * ld + 16;   // the next diagonal block
+                d4 A = lower(T);
+                d4 M = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) M = mfma64(D[r * ld + 4 * t + q], N[4 * t], M);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) N[4 * i] = M[i];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) A = mfma64(-M[t], M[t], A);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) T[r * ld + 4 * i + q] = A[i];   // (held on to, it costs the others registers)
+            }
+        } else {
 #pragma unroll 1
-        for (int e = wave; e < nt - 1; e += nw) {
-            const bool inv = e < kb;   // row kb of the inverse: -Dinv W; else L_I = A_I Dinv^T
-            double* C = P + (inv ? (16 * e + q) * ld + 16 * kb : (16 * (e + 1) + q) * ld + 16 * kb) + r;
-            const double* X = inv ? D + r * ld + q : P + (16 * (e + 1) + r) * ld + 16 * kb + q;
-            const double* Y = inv ? C : D + r * ld + q;
-            const int ys = inv ? 4 * ld : 4;
-            const double sign = inv ? -1.0 : 1.0;
-            d4 acc = {0.0, 0.0, 0.0, 0.0};
+            for (int e0 = wave - 1; e0 < nt - 1 - (kb + 1 < nt); e0 += nw - 1) {
+                const int e = e0 + (kb + 1 < nt && e0 >= kb);   // (the next block row is wavefront 0's)
+                const bool inv = e < kb;   // row kb of the inverse: -Dinv W; else L_I = A_I Dinv^T
+                double* C = P + (inv ? (16 * e + q) * ld + 16 * kb : (16 * (e + 1) + q) * ld + 16 * kb) + r;
+                const double* X = inv ? D + r * ld + q : P + (16 * (e + 1) + r) * ld + 16 * kb + q;
+                const double* Y = inv ? C : D + r * ld + q;
+                const int ys = inv ? 4 * ld : 4;
+                const double sign = inv ? -1.0 : 1.0;
+                d4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc = mfma64(sign * X[4 * t], Y[t * ys], acc);
+                for (int t = 0; t < 4; ++t) acc = mfma64(sign * X[4 * t], Y[t * ys], acc);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
+                for (int i = 0; i < 4; ++i) C[4 * i * ld] = acc[i];
+            }
         }
         __syncthreads();
     }
@@ -676,31 +695,45 @@ __global__ __launch_bounds__(1024) void k_front_strip(DirectDev d, const FrontTa
         if (tid >= 64 && tid < 64 + w / 6) icol[tid - 64] = d.inv[f.node0 + tid - 64];
         __syncthreads();
     }
-    for (int c1 = 0; c1 < kp; c1 += 64) {
-        const int col = c1 + lane, cn = min(col, w - 1) / 6, cc = col - 6 * cn;
-        const int2 ic = p == 0 ? icol[cn] : int2{-1, -1};
-        for (int row0 = wave; row0 < max(rows, kp); row0 += 48) {
-            double v[3], y[3];
+    // lane: two columns; wavefront: rows wave, wave + 16, ..; U of them in flight
+    const int col = 2 * lane, cn = min(col, w - 1) / 6, cc = col - 6 * cn;
+    auto load = [&](auto count, int u0, auto entry) {
+        constexpr int U = decltype(count)::value;
+        double2 v[U], y[U];
 #pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const int row = row0 + 16 * u, R = min(r0 + row, m - 1), rn = R / 6;
-                const bool on = row < nr && col < w;
-                if (p > 0)
-                    v[u] = *(on ? F + (int64_t)R * k + col : d.zero);
-                else
-                    v[u] = gathered(ga, ir[rn - rn0], ic, R - 6 * rn, cc, on);
-                y[u] = *(row < w && col <= row ? F + (int64_t)(c0 + row) * k + col : d.zero) +
-                       (row == col && row >= w ? 1.0 : 0.0);
-            }
+        for (int u = 0; u < U; ++u) {
+            const int row = wave + 16 * (u0 + u);
+            v[u] = entry(min(r0 + row, m - 1), row < nr && col < w);
+            y[u] = *reinterpret_cast<const double2*>(row < w && col <= row ? F + (int64_t)(c0 + row) * k + col : d.zero);
+        }
 #pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const int row = row0 + 16 * u;
-                if (col < kp && row < rows) X[row * ld + col] = v[u];
-                // block (I, J) of the inverse factor goes to block row J, block column I
-                if (row < kp && col >> 4 <= row >> 4)
-                    P[(16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)] = y[u];
+        for (int u = 0; u < U; ++u) {
+            const int row = wave + 16 * (u0 + u);
+            if (col < kp && row < rows) *reinterpret_cast<double2*>(X + row * ld + col) = v[u];
+            // block (I, J) of the inverse factor goes to block row J, block column I; zeros
+            // above its diagonal, ones on the padding's
+            if (row < kp && col >> 4 <= row >> 4) {
+                double2 z;
+                z.x = col <= row && row < w ? y[u].x : row == col ? 1.0 : 0.0;
+                z.y = col + 1 <= row && row < w ? y[u].y : row == col + 1 && row >= w ? 1.0 : 0.0;
+                *reinterpret_cast<double2*>(P + (16 * (col >> 4) + (row & 15)) * ld + 16 * (row >> 4) + (col & 15)) = z;
             }
         }
+    };
+    static_assert(DW <= 96 && SROWS <= 96, "six rows a wavefront, 48 pairs of columns");
+    if (p > 0) {
+        load(std::integral_constant<int, 6>(), 0, [&](int R, bool on) {
+            return *reinterpret_cast<const double2*>(on ? F + (int64_t)R * k + col : d.zero);
+        });
+    } else {
+        const int2 ic = icol[cn];
+        auto entry = [&](int R, bool on) {
+            const int rn = R / 6;
+            const int2 jr = ir[rn - rn0];
+            return make_double2(gathered(ga, jr, ic, R - 6 * rn, cc, on), gathered(ga, jr, ic, R - 6 * rn, cc + 1, on));
+        };
+        load(std::integral_constant<int, 3>(), 0, entry);
+        load(std::integral_constant<int, 3>(), 3, entry);
     }
     __syncthreads();
     if (p == 0) {
@@ -815,17 +848,24 @@ __device__ __forceinline__ void next_block(const DirectDev& d, const FrontTask& 
         }
         ti[u] = I;
         tj[u] = J;
+    }
+    if (p > 0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 16 * I + 4 * i + q, col = 16 * J + r;
-            const bool on = row < w1 && col <= row;
-            if (p > 0) {
-                t[u][i] = *(on ? F + (int64_t)row * k + c1 + col : d.zero) + (row == col && row >= w1 ? 1.0 : 0.0);
-            } else {
-                const int rn = min(row, w1 - 1) / 6, cn = min(col, w1 - 1) / 6;
-                t[u][i] = (row == col ? 1.0 : 0.0) + gathered(ga, inv[rn], inv[cn], row - 6 * rn, col - 6 * cn, on);
+        for (int u = 0; u < MT; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = 16 * ti[u] + 4 * i + q, col = 16 * tj[u] + r;
+                t[u][i] = *(row < w1 && col <= row ? F + (int64_t)row * k + c1 + col : d.zero);
             }
-        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = 16 * ti[u] + 4 * i + q, col = 16 * tj[u] + r;
+                const int rn = min(row, w1 - 1) / 6, cn = min(col, w1 - 1) / 6;
+                t[u][i] = gathered(ga, inv[rn], inv[cn], row - 6 * rn, col - 6 * cn, row < w1 && col <= row);
+            }
     }
     static_assert(DW <= 96, "12 rows a wavefront, 48 pairs of columns");
 #pragma unroll
@@ -843,20 +883,24 @@ __device__ __forceinline__ void next_block(const DirectDev& d, const FrontTask& 
                 *reinterpret_cast<double2*>(P + (wave + 8 * (u0 + u)) * ldx + 2 * lane) = x[u];
     }
     __syncthreads();
+    const double *X[MT], *Y[MT];   // (a tile past the last: any, unused)
 #pragma unroll
     for (int u = 0; u < MT; ++u) {
-        if (ti[u] >= nt) continue;
-        const double *X = P + (16 * ti[u] + r) * ldx + q, *Y = P + (16 * tj[u] + r) * ldx + q;
-#pragma unroll 4
-        for (int c = 0; c < (w + 3) >> 2; ++c) t[u] = mfma64(-X[4 * c], Y[4 * c], t[u]);
+        X[u] = P + (16 * min(ti[u], nt - 1) + r) * ldx + q;
+        Y[u] = P + (16 * min(tj[u], nt - 1) + r) * ldx + q;
     }
+#pragma unroll 2
+    for (int c = 0; c < (w + 3) >> 2; ++c)   // the tiles in turn: their chains overlap
+#pragma unroll
+        for (int u = 0; u < MT; ++u) t[u] = mfma64(-X[u][4 * c], Y[u][4 * c], t[u]);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < MT; ++u) {
         if (ti[u] >= nt) continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            P[(16 * ti[u] + 4 * i + q) * ld + 16 * tj[u] + r] = t[u][i];
+            const int row = 16 * ti[u] + 4 * i + q, col = 16 * tj[u] + r;
+            P[row * ld + col] = t[u][i] + (row == col && (p == 0 || row >= w1) ? 1.0 : 0.0);
             if (ti[u] != tj[u]) P[(16 * tj[u] + 4 * i + q) * ld + 16 * ti[u] + r] = 0.0;
         }
     }
