@@ -975,8 +975,11 @@ __global__ __launch_bounds__(HEAD ? 512 : 256, HEAD ? 4 : 1) void k_front_cols(D
             }
 }
 
-// contribution of a large front, 64x64 tiles of the lower triangle
-__global__ __launch_bounds__(256) void k_front_cb(DirectDev d, const FrontTask* __restrict__ tasks, int n, int parts) {
+// contribution of a large front, 64x64 tiles of the lower triangle; bound by the FP64
+// matrix cores' rate and by the latency of the gathers before them, which three waves a
+// SIMD cover best (64 designs of 100 x 100: 32.4 ms an evaluation with the two that
+// unbounded registers leave, 31.7 with three, 33.3 with four, which spill)
+__global__ __launch_bounds__(256, 3) void k_front_cb(DirectDev d, const FrontTask* __restrict__ tasks, int n, int parts) {
     __shared__ double sh[2 * DROWS * (DKC + 2)];
     __shared__ int2 ir[DROWS / 6 + 3], ic[DROWS / 6 + 3];
     const Where at = locate(n, parts);
