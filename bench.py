@@ -13,8 +13,10 @@ coordinates) and dC/d(element properties), with dC/drho by the chain rule
 through E.  Inputs are resident on the GPU before timing starts.
 
 The JSON line carries:
-* ``roofline``: the solve's dominant kernel (k_pcg_dir, the CG direction and
-  product), algorithmic bytes per launch over its mean duration from HIP
+* ``roofline``: the direct solve's factorisation (all k_front_* launches of a
+  step, from HIP events; operations of the fronts' factors, S and G over the
+  FP64 matrix peak), or, where the iterative solve runs, its dominant kernel
+  (k_pcg_dir, the CG direction and product), algorithmic bytes per launch over its mean duration from HIP
   events on the solver stream, sampled inside the timed steps: every other
   iteration chunk is launched eagerly with its k_pcg_dir launches bracketed,
   and the samples of chunks that began with all designs still iterating (so
@@ -168,6 +170,17 @@ def simp_headline(args, L, nat):
                 "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
                 "traffic_source": tsrc, "avg_launch_us": avg_ms * 1e3, "sampled_launches": nsamp,
                 "alg_bytes_per_launch": int(alg)}
+    ff = "simp64_shell100_fp64_flops.txt"
+    if info["dir_launches"] == 0:   # the direct solve (no CG launches): its factorisation is the largest part
+        kname = "direct_factorisation"
+        fl = _measured_flops(ff, kname)
+        ms = t["setup"][0]
+        achieved = fl * args.designs / 64 / (ms * 1e-3) / 1e12 if fl and ms > 0 else None
+        roofline = {"kernel": "k_front_* (direct factorisation)", "bound": "fp64 matrix", "achieved": achieved,
+                    "peak": FP64_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
+                    "frac": achieved / FP64_VECTOR_PEAK_TFLOPS if achieved else None, "traffic": None,
+                    "traffic_source": None, "avg_launch_us": ms * 1e3, "sampled_launches": t["setup"][1],
+                    "alg_flops": fl, "flops_source": f"profiles/{ff}" if fl else None}
     eb, gb = _asm_bytes(b.plan)
     (te, ne), (tg, ng) = t["element"], t["gather"]
     assembly = {"element_kernels_us": te * 1e3, "element_alg_bytes": eb,
@@ -178,14 +191,14 @@ def simp_headline(args, L, nat):
                 "assembly_frac_of_hbm": (eb + gb) / ((te + tg) * 1e-3) / 1e9 / HBM_PEAK_GBS if te + tg > 0 else None,
                 "elements_per_s": b.plan.n_quad / ((te + tg) * 1e-3) if te + tg > 0 else None,
                 "samples": ne}
-    phases = {"element_ms": te, "gather_ms": tg, "amg_setup_ms": t["setup"][0], "adjoint_ms": t["adjoint"][0]}
+    # (setup: the AMG hierarchy, or the factorisation of the direct solve)
+    phases = {"element_ms": te, "gather_ms": tg,
+              "amg_setup_ms" if info["dir_launches"] else "factor_ms": t["setup"][0], "adjoint_ms": t["adjoint"][0]}
     # FP64 rate of the element kernel and of the quad adjoint (operation counts
     # from the committed rocprofv3 SQ_INSTS_VALU_*_F64 summary of this workload)
-    ff = "simp64_shell100_fp64_flops.txt"
     ke_name = f"ke_quad_kernel<0, {b.plan.element_tuning()}>"
     fe = _measured_flops(ff, ke_name)
-    fa = [_measured_flops(ff, k) for k in ("adj_quad_fwd", "adj_quad_frame", "adj_quad_combine")]
-    fa = sum(fa) if all(x is not None for x in fa) else None
+    fa = _measured_flops(ff, "adj_quad_kernel<true>")
     compute = {"fp64_vector_peak_TFLOPs": FP64_VECTOR_PEAK_TFLOPS, "source": f"profiles/{ff}" if fe else None,
                "element_kernel": ke_name, "element_flops_per_launch": fe,
                "element_TFLOPs": fe / (te * 1e-3) / 1e12 if fe and te > 0 else None,
@@ -364,7 +377,7 @@ def simp_loop(args, L, nat, n_steps=8, step=0.05):
     Cs = {}
     for keep in (False, True):
         rho = rho0.clone()
-        b.plan.amg_reuse(0)
+        b.plan.amg_reuse(2 if keep else 0)
         b.prop_quad[:, 1] = rho ** 3 * 30e9
         b.compliance_and_gradient(precision="fp64", tol=args.tol)        # warm-up on the start design
         policy = AmgKeepPolicy(b.plan) if keep else None
@@ -484,6 +497,8 @@ def trace_summary(trace_dir, bench_log):
     for name, (n, us) in sorted(stats.items(), key=lambda kv: -kv[1][1])[:30]:
         short = re.sub(r"\s+", " ", name)[:120]
         print(f"{us / 1e3:10.2f} {n:7d} {us / n:9.2f}  {short}")
+    if "alg_bytes_per_launch" not in out["roofline"]:
+        return   # the direct solve: no iterations to average over
     d = [(s1 - s0) / 1e3 for s0, s1, name in rows if name.startswith(f"void jsso::{kname}")]
     log = out["solve_log"]["solves"]
     # the live tuner's timing launches (first solve on the plan, before its own
@@ -547,7 +562,7 @@ def flops_summary(pmc_dir, bench_log):
         agg.setdefault(d["name"], []).append(fl)
     print("# FP64 lane operations per launch (64 x (ADD + MUL + TRANS + 2 FMA) wave instructions)")
     for name in sorted(agg):
-        if name.startswith("void jsso::ke_quad_kernel") or name.startswith("jsso::adj_quad"):
+        if name.startswith("void jsso::ke_quad_kernel") or name.startswith("void jsso::adj_quad"):
             v = agg[name]
             print(f"flops_per_launch {name.replace('void jsso::', '').replace('jsso::', '')}: {int(sum(v) / len(v))}"
                   f"  # {len(v)} launches")
@@ -736,7 +751,8 @@ def main():
                                "corners + mid-edge nodes pinned, -1.5 kN/node; compliance + gradient w.r.t. "
                                "node coordinates and rho (through E) per design",
                    "batch": args.designs, "tol": args.tol, "precision": args.precision,
-                   "preconditioner": "smoothed-aggregation AMG V-cycle (FP32 / FP16)",
+                   "preconditioner": "smoothed-aggregation AMG V-cycle (FP32 / FP16)" if h["info"]["dir_launches"]
+                                     else "none: multifrontal Cholesky (FP64), refined to tol",
                    "cg_iterations": h["iters"][-1], "parallelism": "batched structures, 1 GPU"},
         "roofline": h["roofline"],
         "cpu_baseline": cpu,

@@ -3,7 +3,7 @@
 ``displacement(plan, crds, prop_beam, prop_quad, f)`` returns u = K^-1 f and
 backpropagates like the reference's custom VJP (``JaxSSO/solver.py:221-250``):
 lam = K^-T u_bar (a second solve), then for every input p
-    p_bar = -lam^T (dK/dp) u     (hand-written forward-mode adjoint kernel)
+    p_bar = -lam^T (dK/dp) u     (hand-written adjoint kernels)
 and f_bar = lam.
 
 ``compliance(plan, ...)`` returns C = 1/2 f.u (``JaxSSO/SSO_model.py:297-301``);
@@ -17,9 +17,8 @@ from .plan import DEFAULT_MAXIT, DEFAULT_TOL, FEPlan
 
 
 class SolveOptions:
-    """How the state solves run: ``method`` "sparse" (the GPU CG solver, with
-    ``precision`` / ``tol`` / ``maxit``) or "dense" (the dense FP64 Cholesky of
-    ``jsso_dense_solve``)."""
+    """How the state solves run: ``method`` "sparse" (the direct or CG solver, with
+    ``precision`` / ``tol`` / ``maxit``) or "dense" (``jsso_dense_solve``)."""
 
     def __init__(self, precision="fp64", tol=DEFAULT_TOL, maxit=DEFAULT_MAXIT, method="sparse"):
         if method not in ("sparse", "dense"):

@@ -390,6 +390,9 @@ JDEV void quad_local_vals(const V3<double> R[3], const double* u, const double* 
     }
 }
 
+// The two functions below are the split form that the host checks compare with forward
+// mode through the whole element; the GPU's adjoint is quad_adjoint.hpp.
+//
 // phi with the frame and the nodal values fixed; TX is the type of xy, TM that
 // of the properties (Dual for the one direction being differentiated).
 template <typename TX, typename TM>

@@ -1,4 +1,4 @@
-// Element stiffness kernels (beam-column, MITC-4) and the forward-mode adjoint
+// Element stiffness kernels (beam-column, MITC-4) and the adjoint
 // kernels.  Element math lives in element_math.hpp.
 #include <mutex>
 

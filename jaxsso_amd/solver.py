@@ -3,12 +3,14 @@
 The reference offers a dense LU (``jax_dense_solve``, solver.py:75-93), a GPU
 sparse direct solve (``jax_sparse_solve``, :102-168) and a host SuperLU through
 ``pure_callback`` (``sci_sparse_solve``, :176-250), each on the Lagrange-
-augmented system.  Here every sparse solve is the GPU conjugate-gradient solver
-of ``libjsso_hip.so`` (block-Jacobi scaled; FP64 by default, or FP32
-recurrences with FP64 reliable updates when ``precision="mixed"`` -- faster on
-shells, but slender beam chains need a tighter tolerance in that mode), and the
-dense solve is an FP64 blocked Cholesky of the constrained system on the GPU.  All return ``u_aug = [u; mu]`` with the
-Lagrange multipliers ``mu = f_c - (K u)_c`` (support reactions), as the
+augmented system.  Here every sparse solve is the GPU solver of
+``libjsso_hip.so`` (block-Jacobi scaled): an FP64 multifrontal Cholesky
+factorisation with refinement, or, where that does not fit or a preconditioner
+was chosen, conjugate gradients (FP64 by default, or FP32 recurrences with FP64
+reliable updates when ``precision="mixed"``).  The dense solve of a plan's own
+symmetric assembly uses the same factorisation, refined to its floor; otherwise
+it is an FP64 blocked Cholesky or LU on the GPU.  All return ``u_aug = [u; mu]``
+with the Lagrange multipliers ``mu = f_c - (K u)_c`` (support reactions), as the
 reference's augmented solve does.
 """
 from __future__ import annotations
