@@ -1940,11 +1940,11 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
 // with the largest front (m rows: m^2 storage, m^3 operations), while the
 // AMG-preconditioned CG grows with the number of nodes.  One shell of n x n quads
 // has m ~ 9 n: assembly and solve of one smooth shell, ms direct / AMG: 40x40
-// (m = 366) 0.86 / 3.85, 100x100 2.1 / 3.1, 200x200 5.7 / 6.5, 250x250 (m = 2256)
-// 8.1 / 8.1, 300x300 12.0 / 9.1.  Designs that take the CG more iterations gain more
-// (a 200x200 SIMP shell 7.8 / 21), and so do batches, which fill the chip on every
-// tree level (64 SIMP shells of 100x100: 33 / 59).  It needs its storage too: up to
-// an eighth of the card, and half of what is free.
+// (m = 366) 0.79 / 1.9, 100x100 1.8 / 3.2, 200x200 4.8 / 6.7, 250x250 (m = 2256)
+// 6.7 / 8.4, 300x300 10.2 / 9.4.  Designs that take the CG more iterations gain more,
+// and so do batches, which fill the chip on every tree level (64 SIMP shells of
+// 100x100, with gradients: 31.6 / 62).  It needs its storage too: up to an eighth of
+// the card, and half of what is free.
 static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b) {
     const size_t need = (D.fac_n + D.mat_n) * 8;
     return D.max_m <= DIRECT_MAX_M && need <= total_b / 8 && need <= free_b / 2;
