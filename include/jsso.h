@@ -163,7 +163,11 @@ int jsso_assemble(jsso_plan* plan, const double* d_crds, const double* d_prop_be
                   const double* d_prop_quad, double* d_K_out, void* stream);
 
 /* Solve K u = f with u = 0 at constrained DOFs, for nrhs load cases per structure.
- * d_f, d_u: (6*n_nodes) x nrhs.  tol: on the block-Jacobi-scaled residual. */
+ * d_f, d_u: (6*n_nodes) x nrhs.  tol: on the block-Jacobi-scaled residual.
+ * A structure and load case whose load holds a NaN or an infinity at a free DOF has a u
+ * that is not finite either (wholly NaN by the direct solve, at the least at the loaded
+ * nodes by an iterative one) and is not counted in h_info->converged; the others are not
+ * affected. */
 int jsso_solve(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs,
                int32_t precision, double tol, int32_t maxit, jsso_info* h_info,
                void* stream);
@@ -211,7 +215,9 @@ int jsso_spmv_k(jsso_plan* plan, const double* d_K, const double* d_x, double* d
  * whose Cm is not symmetric, element.py:852-875), by a blocked LU with partial pivoting --
  * then triangular solves.  For the plan's own symmetric assembly (d_K NULL) with
  * 1 to 4 load cases, where the direct solve is taken (see JSSO_PC_AMG), its
- * factorisation serves instead, refined to the attainable accuracy.  transpose != 0 solves Kc^T u = f (the adjoint system).
+ * factorisation serves instead, refined to the attainable accuracy (a load whose squares
+ * leave the range of FP64 is left to the dense one; for one that is not finite u is NaN, and
+ * the call succeeds).  transpose != 0 solves Kc^T u = f (the adjoint system).
  * d_K as for jsso_spmv_k (NULL = the plan's current assembly); d_f, d_u:
  * (6*n_nodes) x nrhs, nrhs <= 64.  Needs 8 N^2 bytes of device memory (N =
  * 6*n_nodes rounded up to a multiple of 64).  Returns JSSO_ESINGULAR for a

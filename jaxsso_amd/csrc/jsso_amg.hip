@@ -2871,8 +2871,8 @@ static void amg_replace(Plan* pl, AmgState& A, const Workspace& w, const AmgBufs
     constexpr int RW = WpsFits<double, NR, 4>::value ? 4 : 1;
     hipLaunchKernelGGL((k_replace<VT, NR, RW>), g, dim3(64 * RW), 0, s, sl, w.P, w.st, (const double*)pl->d_Ke64,
                        (const double*)w.b64, (const double*)w.x64, bf.r[k & 1]);
-    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 1, tol, steps,
-                       AMG_STALL_WINDOW, (const double*)A.dev[0].d_rho, AMG_FLOOR_FACTOR, AMG_FLOOR_WINDOW);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, DECIDE_STEP, tol,
+                       steps, AMG_STALL_WINDOW, (const double*)A.dev[0].d_rho, AMG_FLOOR_FACTOR, AMG_FLOOR_WINDOW);
     hipLaunchKernelGGL((k_save<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.save, (const double*)w.x64,
                        w.xbest);
     wps_dispatch<VT, NR>(A.wps0, [&](auto W) {
@@ -3002,8 +3002,8 @@ static int run_amg(Plan* pl, const double* f, double* u, double tol, int maxit, 
     JSSO_HIP(hipMemsetAsync(w.P.cg[0], 0, 2 * 4 * (size_t)pl->n_wg * NR * sizeof(double), s));
     hipLaunchKernelGGL((k_init<VT, NR>), gridS, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f, w.b64,
                        w.x64, w.xbest, bf.xlo, bf.r[0], bf.p[0]);
-    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 0, tol, 0, 0,
-                       (const double*)nullptr, 0.0, 0);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, DECIDE_START, tol,
+                       0, 0, (const double*)nullptr, 0.0, 0);
     int32_t& wsel = pl->amg_wps[prec_slot<MT, VT>()][NR];
     if (wsel <= 0 && (rc = tune_amg_wps<MT, VT, NR>(pl, A, w, bf, A0, s, wsel))) return rc;
     A.wps0 = wsel;

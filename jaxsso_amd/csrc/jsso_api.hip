@@ -644,7 +644,7 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
     std::vector<double> rr(nsys), ff(nsys);
     const int slot = precision == JSSO_PREC_MIXED ? PS_F32 : precision == JSSO_PREC_MIXED_V64 ? PS_F32_V64 : PS_F64;
     JSSO_HIP(hipMemsetAsync(d_u, 0, vb, s));
-    int inner_its = 0, outer = 0, conv = 0;
+    int inner_its = 0, outer = 0, conv = 0, lost = 0;   // lost: systems whose load is not finite
     double relmax = 0.0, prev = 0.0;
     for (;; ++outer) {
         if ((rc = launch_defect_residual(p, p->d_K, d_f, d_u, nrhs, transpose, r, s))) return rc;
@@ -653,13 +653,18 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
         JSSO_HIP(hipStreamSynchronize(s));
         if (outer == 0) ff = rr;   // u = 0: r = f on the free DOFs
         relmax = 0.0;
-        conv = 0;
+        conv = lost = 0;
         for (int k = 0; k < nsys; ++k) {
+            if (!std::isfinite(ff[k])) {
+                ++lost;
+                continue;
+            }
             const double rel = ff[k] > 0.0 ? std::sqrt(std::max(rr[k], 0.0) / ff[k]) : 0.0;
             relmax = std::max(relmax, rel);
             conv += rel <= tol ? 1 : 0;
         }
-        if (conv == nsys || inner_its >= maxit || !std::isfinite(relmax)) break;
+        // (at least one correction where a load is not finite: it takes that into u)
+        if ((conv + lost == nsys && (lost == 0 || outer > 0)) || inner_its >= maxit || !std::isfinite(relmax)) break;
         // (a step that gains less than 10%: the attainable accuracy, or no convergence)
         if (outer >= 2 && relmax > 0.9 * prev) break;
         prev = relmax;
@@ -704,7 +709,7 @@ int jsso_solve(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs, in
     bool tried = false;
     if (precision != JSSO_PREC_PLAIN && !p->precond_set && expect_symmetric(p)) {
         bool done = false;
-        rc = direct_solve(p, d_f, d_u, nrhs, slot, tol, maxit, h_info, s, done);
+        rc = direct_solve(p, d_f, d_u, nrhs, slot, tol, maxit, false, h_info, s, done);
         if (rc || done) return rc;
         tried = true;
     }
@@ -882,8 +887,8 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
     bool tried = false;
     if (!d_K && expect_symmetric(p)) {
         bool done = false;
-        rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, nullptr, s, done);
-        if (rc || done) return rc;
+        rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, true, nullptr, s, done);
+        if (rc || done) return std::min(rc, 0);   // (a NaN in f is no error: u is NaN too)
         tried = true;
     }
     int32_t status = 0;
@@ -899,8 +904,8 @@ int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, doub
         // pivot that is not positive) is left to the dense factorisation and its errors
         if (!tried && !(status & (STATUS_NONSYM | 1))) {
             bool done = false;
-            rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, nullptr, s, done);
-            if (rc || done) return rc;
+            rc = direct_solve(p, d_f, d_u, nrhs, PS_F64, DENSE_TOL, INT32_MAX, true, nullptr, s, done);
+            if (rc || done) return std::min(rc, 0);
         }
         if ((rc = launch_full_blocks(p, s))) return rc;
         d_K = p->d_K;

@@ -91,6 +91,7 @@ struct DirectReport {
     double worst;                           // largest relative residual of the best iterates
     int32_t flags;                          // the assembly's (d_status)
     int32_t final;                          // every system done, on a K that this solve is for
+    int32_t not_finite;                     // systems whose load is not finite (done: so is u)
 };
 
 struct DirectState {
@@ -1216,17 +1217,18 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
                                                        const int32_t* __restrict__ bad,
                                                        const int32_t* __restrict__ flags, DirectReport* out,
                                                        DirectReport* host) {
-    __shared__ int cnt[4];
+    __shared__ int cnt[5];
     __shared__ double worst[4];
     const int tid = threadIdx.x;
-    if (tid < 4) cnt[tid] = 0;
+    if (tid < 5) cnt[tid] = 0;
     __syncthreads();
-    int run = 0, stall = 0, floor = 0, nb = 0;
+    int run = 0, stall = 0, floor = 0, nb = 0, load = 0;
     double w = 0.0;
     for (int k = tid; k < nsys; k += 256) {
         run += status[k] == SYS_RUNNING;
         stall += status[k] == SYS_STALLED;
         floor += status[k] == SYS_FLOOR;
+        load += status[k] == SYS_LOAD;
         w = fmax(w, best[k]);
     }
     for (int k = tid; k < n_struct; k += 256) nb += bad[k] != 0;
@@ -1234,6 +1236,7 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
     if (stall) atomicAdd(&cnt[1], stall);
     if (floor) atomicAdd(&cnt[2], floor);
     if (nb) atomicAdd(&cnt[3], nb);
+    if (load) atomicAdd(&cnt[4], load);
     for (int o = 32; o > 0; o >>= 1) w = fmax(w, __shfl_xor(w, o));
     if ((tid & 63) == 0) worst[tid >> 6] = w;
     __syncthreads();
@@ -1243,6 +1246,7 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
         v.stalled = cnt[1];
         v.floor = cnt[2];
         v.bad = cnt[3];
+        v.not_finite = cnt[4];
         v.worst = fmax(fmax(worst[0], worst[1]), fmax(worst[2], worst[3]));
         v.flags = *flags;
         v.final = !(v.running | v.stalled | v.bad | (v.flags & (STATUS_NONSYM | 1)));
@@ -1252,10 +1256,11 @@ __global__ __launch_bounds__(256) void k_direct_report(int nsys, int n_struct, c
 }
 
 // After a step's report: u = L^-T x of the best iterates where that is the end (u is
-// not touched before: it may be f itself, which another route then still needs), else
-// the iterates that have become the best are kept.
+// not touched before: it may be f itself, which another route then still needs), NaN
+// for a load that is not finite; else the iterates that have become the best are kept.
 template <int NR>
 __global__ __launch_bounds__(SOLVER_WG) void k_direct_finish(Slices sl, const int32_t* __restrict__ save,
+                                                             const int32_t* __restrict__ status,
                                                              const DirectReport* __restrict__ report,
                                                              const double* __restrict__ Linv,
                                                              const double* __restrict__ x64,
@@ -1276,7 +1281,7 @@ __global__ __launch_bounds__(SOLVER_WG) void k_direct_finish(Slices sl, const in
             double v = 0.0;
 #pragma unroll
             for (int c = 0; c < 6; ++c) v += Linv[i * 36 + c * 6 + r] * x[(6 * i + c) * NR + h];
-            u[R * NR + h] = v;
+            u[R * NR + h] = status[sys * NR + h] == SYS_LOAD ? __builtin_nan("") : v;
         } else if (now) {
             xbest[R * NR + h] = x64[R * NR + h];
         }
@@ -1347,8 +1352,8 @@ __global__ __launch_bounds__(SOLVER_WG) void k_defect(Slices sl, Partials P, Sys
 }
 
 // A system ends where its residual ||r|| / ||f|| no longer halves: at its attainable
-// accuracy if that is within tol, else without convergence.  One wavefront per
-// structure; step 0 takes ||f|| from u = 0.
+// accuracy if that is within tol, else without convergence, as does a load whose squares
+// leave the range of FP64.  One wavefront per structure; step 0 takes ||f|| from u = 0.
 template <int NR>
 __global__ __launch_bounds__(64) void k_defect_decide(Slices sl, Partials P, SysState st, int step, double tol) {
     const int sys = blockIdx.x, lane = threadIdx.x;
@@ -1366,9 +1371,9 @@ __global__ __launch_bounds__(64) void k_defect_decide(Slices sl, Partials P, Sys
         const int k = sys * NR + h;
         if (!st.active[k]) continue;
         const double ff = step == 0 ? rr : st.bnorm2[k], prev = st.relres[k];
-        const double rel = step == 0 ? (rr > 0.0 ? 1.0 : 0.0) : sqrt(rr / ff);
-        int active = rel > 0.0 ? 1 : 0, status = active ? SYS_RUNNING : SYS_CONVERGED;
-        if (step > 0 && active && !(rel <= 0.5 * prev)) {
+        const double rel = step == 0 ? 1.0 : sqrt(rr / ff);
+        int active = 1, status = SYS_RUNNING;
+        if (step == 0 ? !(rr >= LOAD2_MIN && rr <= LOAD2_MAX) : rel == 0.0 || !(rel <= 0.5 * prev)) {
             active = 0;
             status = rel <= tol ? SYS_CONVERGED : SYS_STALLED;
         }
@@ -1382,6 +1387,19 @@ __global__ __launch_bounds__(64) void k_defect_decide(Slices sl, Partials P, Sys
         mask |= active << h;
     }
     for (int w = s0 + lane; w < s1; w += 64) st.slice_act[w] = mask;
+}
+
+// u = 0, NaN for a load that is not finite
+template <int NR>
+__global__ __launch_bounds__(SOLVER_WG) void k_defect_start(Slices sl, const int32_t* __restrict__ status,
+                                                            double* __restrict__ u) {
+    const int w = slice_of_block(sl);
+    if (w < 0) return;
+    const int sys = sl.sys[w];
+    const int64_t R = 6 * (int64_t)sl.row0[w] + threadIdx.x;
+    if (R >= 6 * (int64_t)sl.row1[w]) return;
+#pragma unroll
+    for (int h = 0; h < NR; ++h) u[R * NR + h] = status[sys * NR + h] == SYS_LOAD ? __builtin_nan("") : 0.0;
 }
 
 // u += L^-T z for the systems still running
@@ -1869,10 +1887,12 @@ static int tune_residual(Plan* pl, const Workspace& w, const Slices& sl, double*
 
 // u = K^-1 f by the factorisation and refinement; done = false (and nothing said
 // about u) where a pivot is not positive or a system does not reach its tolerance
-// or its attainable accuracy
+// or its attainable accuracy (strict: or whose load's squares leave the range of FP64).
+// A structure and load case whose load is not finite gets NaN and is not counted as
+// converged (JSSO_NOT_CONVERGED).
 template <int NR>
 static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, double tol, int maxit, int slot,
-                      jsso_info* info, hipStream_t s, bool& done) {
+                      bool strict, jsso_info* info, hipStream_t s, bool& done) {
     Workspace w;
     int rc = get_workspace(pl, NR, w);
     if (rc) return rc;
@@ -1883,10 +1903,10 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
     const dim3 g = slice_grid(sl);
     double* r = (double*)w.r[0];
     double* z = (double*)w.p;
-    hipLaunchKernelGGL((k_init<double, NR>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f, w.b64,
-                       w.x64, w.xbest, (double*)w.xlo, r, z);
-    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 0, tol, 0, 0,
-                       (const double*)nullptr, 0.0, 0);
+    hipLaunchKernelGGL((k_init<double, NR, true>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f,
+                       w.b64, w.x64, w.xbest, (double*)w.xlo, r, z);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys,
+                       strict ? DECIDE_START_STRICT : DECIDE_START, tol, 0, 0, (const double*)nullptr, 0.0, 0);
     int32_t& wps = pl->direct_wps[slot][NR];
     if (wps <= 0 && (rc = tune_residual<NR>(pl, w, sl, r, s, wps))) return rc;
     if ((rc = ensure_factor(pl, D, s))) return rc;
@@ -1908,13 +1928,13 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
             residual(std::integral_constant<int, 1>());
         // (a step that gains less than 10% ends a system at once: near its attainable
         // accuracy as converged there, else as stalled)
-        hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 1, tol, 1, 2,
-                           (const double*)D.d_rho, DIRECT_FLOOR_FACTOR, 0);
+        hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, DECIDE_STEP, tol,
+                           1, 2, (const double*)D.d_rho, DIRECT_FLOOR_FACTOR, 0);
         hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys, (const int32_t*)w.st.status,
                            (const double*)w.st.best, (const int32_t*)D.dev.bad, (const int32_t*)pl->d_status,
                            D.d_report, D.host_report);
         hipLaunchKernelGGL((k_direct_finish<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.save,
-                           (const DirectReport*)D.d_report, pl->d_Linv, (const double*)w.x64, w.xbest, u);
+                           (const int32_t*)w.st.status, (const DirectReport*)D.d_report, pl->d_Linv, (const double*)w.x64, w.xbest, u);
         JSSO_HIP(hipGetLastError());
         JSSO_HIP(hipStreamSynchronize(s));
         const DirectReport& R = *D.h_report;
@@ -1925,13 +1945,14 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
         if (info) {
             *info = jsso_info{};
             info->iterations = info->replacements = it;
-            info->converged = info->n_systems = nsys;
+            info->converged = nsys - R.not_finite;
+            info->n_systems = nsys;
             info->rel_residual = R.worst;
             info->at_floor = R.floor;
             info->waves_per_slice = wps;
         }
         timing_collect();
-        return JSSO_OK;
+        return R.not_finite ? JSSO_NOT_CONVERGED : JSSO_OK;
     }
     return JSSO_OK;
 }
@@ -1976,17 +1997,17 @@ static int direct_state(Plan* pl, int nrhs, DirectState** out) {
     return JSSO_OK;
 }
 
-int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
-                 hipStream_t s, bool& done) {
+int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, bool strict,
+                 jsso_info* info, hipStream_t s, bool& done) {
     done = false;
     DirectState* D = nullptr;
     int rc = direct_state(pl, nrhs, &D);
     if (rc || !D) return rc;
     switch (nrhs) {
-        case 1: return run_direct<1>(pl, *D, f, u, tol, maxit, slot, info, s, done);
-        case 2: return run_direct<2>(pl, *D, f, u, tol, maxit, slot, info, s, done);
-        case 3: return run_direct<3>(pl, *D, f, u, tol, maxit, slot, info, s, done);
-        default: return run_direct<4>(pl, *D, f, u, tol, maxit, slot, info, s, done);
+        case 1: return run_direct<1>(pl, *D, f, u, tol, maxit, slot, strict, info, s, done);
+        case 2: return run_direct<2>(pl, *D, f, u, tol, maxit, slot, strict, info, s, done);
+        case 3: return run_direct<3>(pl, *D, f, u, tol, maxit, slot, strict, info, s, done);
+        default: return run_direct<4>(pl, *D, f, u, tol, maxit, slot, strict, info, s, done);
     }
 }
 
@@ -2003,11 +2024,11 @@ static int run_defect(Plan* pl, DirectState& D, const double* K, const double* f
     const dim3 g = slice_grid(sl);
     double *r = (double*)w.r[0], *z = (double*)w.p;
     // activity from L^-1 f
-    hipLaunchKernelGGL((k_init<double, NR>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f, w.b64,
-                       w.x64, w.xbest, (double*)w.xlo, r, z);
-    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, 0, tol, 0, 0,
-                       (const double*)nullptr, 0.0, 0);
-    JSSO_HIP(hipMemsetAsync(u, 0, 6 * (size_t)pl->n_nodes * NR * sizeof(double), s));
+    hipLaunchKernelGGL((k_init<double, NR, true>), g, dim3(SOLVER_WG), 0, s, sl, w.P, pl->d_fixed, pl->d_Linv, f,
+                       w.b64, w.x64, w.xbest, (double*)w.xlo, r, z);
+    hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys,
+                       DECIDE_START_STRICT, tol, 0, 0, (const double*)nullptr, 0.0, 0);
+    hipLaunchKernelGGL((k_defect_start<NR>), g, dim3(SOLVER_WG), 0, s, sl, (const int32_t*)w.st.status, u);
     if ((rc = ensure_factor(pl, D, s))) return rc;
     const int most = std::min(maxit, DEFECT_STEPS);
     for (int it = 0; it <= most; ++it) {
@@ -2030,10 +2051,11 @@ static int run_defect(Plan* pl, DirectState& D, const double* K, const double* f
                 if (info) {
                     *info = jsso_info{};
                     info->iterations = info->replacements = it;
-                    info->converged = info->n_systems = nsys;
+                    info->converged = nsys - R.not_finite;
+                    info->n_systems = nsys;
                     info->rel_residual = R.worst;
                 }
-                return JSSO_OK;
+                return R.not_finite ? JSSO_NOT_CONVERGED : JSSO_OK;
             }
         }
         direct_apply<NR>(D, w.st.active, r, z, s);

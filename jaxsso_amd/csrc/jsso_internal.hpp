@@ -239,8 +239,10 @@ int launch_defect_residual(Plan* p, const double* K, const double* f, const doub
 int launch_axpy(int64_t n, const double* x, double* y, hipStream_t s);
 int amg_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
               hipStream_t s);
-int direct_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, jsso_info* info,
-                 hipStream_t s, bool& done);
+// strict: loads whose squares leave the range of FP64 are not taken (a route that knows no
+// norms is behind the call)
+int direct_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double tol, int maxit, bool strict,
+                 jsso_info* info, hipStream_t s, bool& done);
 int direct_defect(Plan* p, const double* K, const double* f, double* u, int nrhs, bool transpose, double tol,
                   int maxit, jsso_info* info, hipStream_t s, bool& done);
 void direct_destroy(Plan* p);

@@ -11,8 +11,14 @@ namespace jsso {
 
 constexpr int NWAVES = SOLVER_WG / 64;
 // SYS_FLOOR: stopped at the attainable accuracy of the FP64 residual (counted as
-// converged, see k_decide)
-enum { SYS_RUNNING = 0, SYS_CONVERGED = 1, SYS_STALLED = 2, SYS_FLOOR = 3 };
+// converged, see k_decide).  SYS_LOAD: the load holds a NaN or an infinity, so u does too.
+enum { SYS_RUNNING = 0, SYS_CONVERGED = 1, SYS_STALLED = 2, SYS_FLOOR = 3, SYS_LOAD = 4 };
+
+// k_decide.  DECIDE_START_STRICT: DECIDE_START for a caller that has a route without norms
+// behind it: a load whose squares leave the range of FP64 (LOAD2_MIN .. LOAD2_MAX bound
+// ||b||^2, with room for residuals 1e-17 times smaller) is SYS_STALLED at once.
+enum { DECIDE_START = 0, DECIDE_STEP = 1, DECIDE_START_STRICT = 2 };
+constexpr double LOAD2_MIN = 1e-270, LOAD2_MAX = 1e300;
 
 // ---------------------------------------------------------------------------
 // slices and reductions

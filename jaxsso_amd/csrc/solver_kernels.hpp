@@ -6,8 +6,11 @@
 
 namespace jsso {
 
-// b = L^-1 f (constrained DOFs zeroed), x = 0, r_0 = b (buffer 0); partials <b,b>.
-template <typename VT, int NR>
+// b = L^-1 f (constrained DOFs zeroed), x = 0, r_0 = b (buffer 0); partials <b,b>, NaN
+// exactly where an entry of b is not finite (xbest, the result of a system that never
+// runs, is then NaN there too).  MARK: <b,b> of a load that is not zero is not zero either,
+// where all its squares underflow.
+template <typename VT, int NR, bool MARK = false>
 __global__ __launch_bounds__(SOLVER_WG) void k_init(Slices sl, Partials P, const uint8_t* __restrict__ fixed,
                                                     const double* __restrict__ Linv, const double* __restrict__ f,
                                                     double* __restrict__ b64, double* __restrict__ x64,
@@ -35,12 +38,14 @@ __global__ __launch_bounds__(SOLVER_WG) void k_init(Slices sl, Partials P, const
             }
             const int64_t o = R * NR + h;
             b64[o] = s;
+            const double zero = s * 0.0;   // NaN for an infinity or a NaN
             x64[o] = 0.0;
-            xbest[o] = 0.0;
+            xbest[o] = zero;
             xlo[o] = VT(0);
             r0[o] = VT(s);
             p[o] = VT(0);
-            vb[h] = s * s;
+            vb[h] = s * s + zero;
+            if (MARK && s != 0.0) vb[h] = fmax(vb[h], 2.2250738585072014e-308) + zero;   // (fmax drops a NaN)
         }
     }
     write_partials<NR, NWAVES>(vb, lds, P.b, w);
@@ -48,7 +53,8 @@ __global__ __launch_bounds__(SOLVER_WG) void k_init(Slices sl, Partials P, const
 
 // One wavefront per structure: convergence bookkeeping of its load cases from
 // the slice partials, and the per-slice activity masks the CG kernels test.
-// mode 0 (after k_init): bnorm2, activity.  mode 1 (after k_replace): true
+// DECIDE_START (after k_init): bnorm2, activity; a load that is not finite ends its
+// system here, unconverged.  DECIDE_STEP (after k_replace): true
 // relative residual, best iterate, stagnation, status, after `steps` more
 // iterations (counted per system, so the kernel can sit in a captured graph).
 // A system whose true residual has not improved by 10% for max(min_window,
@@ -75,7 +81,7 @@ __global__ __launch_bounds__(64) void k_decide(Slices sl, Partials P, SysState s
     for (int w = s0 + lane; w < s1; w += 64) {
 #pragma unroll
         for (int h = 0; h < NR; ++h) {
-            if (mode == 0) {
+            if (mode != DECIDE_STEP) {
                 ta[h] += P.b[(int64_t)w * NR + h];
             } else {
                 ta[h] += P.t[(int64_t)w * NR + h];
@@ -94,19 +100,21 @@ __global__ __launch_bounds__(64) void k_decide(Slices sl, Partials P, SysState s
 #pragma unroll
     for (int h = 0; h < NR; ++h) {
         const int k = sys * NR + h;
-        if (mode == 0) {
+        if (mode != DECIDE_STEP) {
             const double bb = ta[h];
+            const bool in = mode == DECIDE_START || (bb >= LOAD2_MIN && bb <= LOAD2_MAX);
+            const int status = bb == 0.0 ? SYS_CONVERGED : isnan(bb) ? SYS_LOAD : in ? SYS_RUNNING : SYS_STALLED;
             if (lane == 0) {
                 st.bnorm2[k] = bb;
-                st.relres[k] = bb > 0.0 ? 1.0 : 0.0;
-                st.best[k] = bb > 0.0 ? 1.0 : 0.0;
-                st.active[k] = bb > 0.0 ? 1 : 0;
-                st.status[k] = bb > 0.0 ? SYS_RUNNING : SYS_CONVERGED;
+                st.relres[k] = bb == 0.0 ? 0.0 : 1.0;
+                st.best[k] = bb == 0.0 ? 0.0 : 1.0;
+                st.active[k] = status == SYS_RUNNING ? 1 : 0;
+                st.status[k] = status;
                 st.stall[k] = 0;
                 st.save[k] = 0;
                 st.iters[k] = 0;
             }
-            mask |= bb > 0.0 ? 1 << h : 0;
+            mask |= status == SYS_RUNNING ? 1 << h : 0;
             continue;
         }
         if (!st.active[k]) {
