@@ -80,7 +80,13 @@ enum {
  * take it in every batched precision.  h_info->iterations counts its refinement
  * steps, h_info->levels and dir_launches are 0.  A factorisation that meets a
  * pivot that is not positive, or a system that it does not bring to the tolerance
- * or to its attainable accuracy, hands the whole solve to the AMG. */
+ * or to its attainable accuracy, hands the whole solve to the AMG.
+ * Whether a plan solves directly is decided at the first such solve, for the plan's
+ * life: its largest front has at most 2 300 rows (a shell of n x n quads: about 9 n),
+ * and factor and contributions need at most an eighth of the card's memory and half
+ * of what is free at that moment.  The plan then holds them until it is destroyed
+ * (shells of 100 x 100 quads: 212 MB each, so up to about 170 of them in a plan).
+ * jsso_plan_direct_info tells. */
 
 typedef struct {
     int32_t iterations;   /* CG iterations performed (max over systems)            */
@@ -303,6 +309,17 @@ int jsso_plan_element_tuning(jsso_plan* plan, int32_t set_epw, int32_t* h_epw);
  * pattern (host, once) and its numeric operators after each jsso_assemble (device,
  * at the next solve); the plain path always uses block-Jacobi. */
 int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc);
+/* The direct solve of a plan (see JSSO_PC_AMG): h_info (7 entries) receives
+ *   0  whether the plan solves directly: 1 yes, 0 no (its fronts or its memory are past
+ *      the limits), -1 not decided yet (no solve has asked)
+ *   1  rows of its largest front    2  bytes of device memory that it holds (or would)
+ *   3  operations of a factorisation, over all structures (k^3 + 2 k^2 b + k b^2 for a
+ *      front of k pivot and b border rows: factor, solve operators and contribution)
+ *   4  factorisations run   5  solves begun   6  solves that it finished (the others went
+ *      on to the next route)
+ * Entries 1 to 3 are 0 until decided. */
+int jsso_plan_direct_info(jsso_plan* plan, int64_t* h_info);
+
 /* Reuse of the AMG hierarchy across assemblies, for optimisation loops (no
  * counterpart in the reference, which refactorises with SuperLU every time).
  * mode 0 (default): every solve after a jsso_assemble rebuilds the numeric

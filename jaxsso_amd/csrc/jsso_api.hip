@@ -953,6 +953,14 @@ int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc) {
     P(plan)->precond_set = true;
     return JSSO_OK;
 }
+int jsso_plan_direct_info(jsso_plan* plan, int64_t* h_info) {
+    if (!plan || !h_info) {
+        set_error("jsso_plan_direct_info: NULL argument");
+        return JSSO_EINVAL;
+    }
+    direct_info(P(plan), h_info);
+    return JSSO_OK;
+}
 int jsso_plan_amg_reuse(jsso_plan* plan, int32_t mode, int64_t* h_counts) {
     if (!plan || mode < -1 || mode > 2) {
         set_error("invalid AMG reuse mode %d (-1 query, 0 rebuild, 1 keep, 2 rebuild once then keep)", mode);

@@ -113,6 +113,7 @@ struct DirectState {
     size_t vec_bytes = 0;
     std::vector<void*> allocs;
     bool usable = false, factored = false;
+    int64_t factorisations = 0, begun = 0, finished = 0;
 };
 
 // ---------------------------------------------------------------------------
@@ -1788,6 +1789,7 @@ static int direct_factor(Plan* pl, DirectState& D, hipStream_t s) {
     }
     JSSO_HIP(hipGetLastError());
     D.factored = true;
+    ++D.factorisations;
     return JSSO_OK;
 }
 
@@ -1942,6 +1944,7 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
         if (R.running && !R.bad && !R.stalled && !(R.flags & (STATUS_NONSYM | 1))) continue;
         if (!R.final) return JSSO_OK;
         done = true;
+        ++D.finished;
         if (info) {
             *info = jsso_info{};
             info->iterations = info->replacements = it;
@@ -1994,7 +1997,19 @@ static int direct_state(Plan* pl, int nrhs, DirectState** out) {
     if (!pl->direct_valid) D.factored = false;
     pl->direct_valid = true;
     *out = &D;
+    ++D.begun;
     return JSSO_OK;
+}
+
+void direct_info(const Plan* pl, int64_t* out) {
+    const DirectState* D = pl->direct;
+    out[0] = D ? D->usable : -1;
+    out[1] = D ? D->max_m : 0;
+    out[2] = D ? (int64_t)((D->fac_n + D->mat_n) * 8 + D->vec_bytes) : 0;
+    out[3] = D ? (int64_t)D->flops : 0;
+    out[4] = D ? D->factorisations : 0;
+    out[5] = D ? D->begun : 0;
+    out[6] = D ? D->finished : 0;
 }
 
 int direct_solve(Plan* pl, const double* f, double* u, int nrhs, int slot, double tol, int maxit, bool strict,
@@ -2048,6 +2063,7 @@ static int run_defect(Plan* pl, DirectState& D, const double* K, const double* f
             if (R.bad || R.stalled) return JSSO_OK;
             if (!R.running) {
                 done = true;
+                ++D.finished;
                 if (info) {
                     *info = jsso_info{};
                     info->iterations = info->replacements = it;

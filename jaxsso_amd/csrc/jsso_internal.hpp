@@ -246,6 +246,7 @@ int direct_solve(Plan* p, const double* f, double* u, int nrhs, int slot, double
 int direct_defect(Plan* p, const double* K, const double* f, double* u, int nrhs, bool transpose, double tol,
                   int maxit, jsso_info* info, hipStream_t s, bool& done);
 void direct_destroy(Plan* p);
+void direct_info(const Plan* p, int64_t* out);
 int amg_levels(Plan* p, int32_t* h_nodes, int32_t cap, int32_t* h_levels);
 void amg_destroy(Plan* p);
 int dense_solve(Plan* p, const double* K, const double* f, double* u, int nrhs, bool lu, bool transpose,

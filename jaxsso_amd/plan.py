@@ -139,6 +139,17 @@ class FEPlan:
         nat.check(nat.load_library().jsso_plan_amg_reuse(self._h, int(mode), nat.ptr(out)))
         return {"mode": int(out[0]), "full_setups": int(out[1]), "refreshes": int(out[2])}
 
+    def direct_info(self) -> dict:
+        """The direct solve of this plan: whether it is ``taken`` (None until the first solve
+        that asks decides), its largest front, the device memory it holds, the operations of
+        a factorisation, and how many factorisations and solves (begun, finished) it ran."""
+        out = np.zeros(7, np.int64)
+        nat.check(nat.load_library().jsso_plan_direct_info(self._h, nat.ptr(out)))
+        info = dict(zip(("taken", "max_front", "bytes", "operations", "factorisations", "begun", "finished"),
+                        (int(v) for v in out)))
+        info["taken"] = None if info["taken"] < 0 else bool(info["taken"])
+        return info
+
     def amg_levels(self) -> list:
         """Block rows of every level of the plan's AMG hierarchy (built on the host)."""
         nodes = np.zeros(32, np.int32)

@@ -1,0 +1,42 @@
+"""Which calls the direct solve serves, and what of it a plan keeps."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from jaxsso_amd import _native as nat
+from jaxsso_amd import workloads as wl
+from jaxsso_amd.batch import StructureBatch
+from jaxsso_amd.plan import FEPlan
+
+pytestmark = pytest.mark.gpu
+
+
+def shell(n, kx=1.0, ky=1.0):
+    st = wl.shell_pinned_edges(n, 0.3 * n, 0.05 * n, design=3)
+    st.prop_quads[:, 3], st.prop_quads[:, 4] = kx, ky
+    return st
+
+
+def plan_of(st):
+    plan = FEPlan([0, st.n_node], st.cnct_beamcols, st.cnct_quads, st.known_id)
+    plan.assemble(torch.tensor(st.crds), None, torch.tensor(st.prop_quads))
+    return plan
+
+
+def test_a_plan_tells_how_it_solves():
+    one, two = StructureBatch([shell(24)]), StructureBatch([shell(24), shell(24)])
+    assert one.plan.direct_info()["taken"] is None and one.plan.direct_info()["begun"] == 0
+    for _ in range(2):
+        one.solve(), one.solve(assemble=False), two.solve()
+    a, b = one.plan.direct_info(), two.plan.direct_info()
+    print(a, b, flush=True)
+    assert a["taken"] and a["factorisations"] == 2 and a["begun"] == a["finished"] == 4
+    assert 0 < a["max_front"] == b["max_front"] <= 2300 and a["max_front"] % 6 == 0
+    # the two structures of one pattern: twice the operations and the memory
+    assert b["operations"] == 2 * a["operations"] and b["bytes"] == 2 * a["bytes"] > 0
+    large = FEPlan([0, 301 ** 2], np.zeros((0, 2), np.int32), shell(300).cnct_quads, [0, 1, 2])
+    assert large.direct_info()["taken"] is None
