@@ -670,7 +670,9 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
         prev = relmax;
         jsso_info ii{};
         p->sym_part_solve = true;
-        rc = solve_batched(p, r, du, nrhs, slot, std::max(1e-3, tol), maxit - inner_its, &ii, s);
+        // (not the direct solve: it was asked for the whole of this above, and it takes its
+        // results for K itself only)
+        rc = solve_batched(p, r, du, nrhs, slot, std::max(1e-3, tol), maxit - inner_its, &ii, s, true);
         p->sym_part_solve = false;
         if (rc < 0) return rc;
         inner_its += ii.iterations;

@@ -40,3 +40,21 @@ def test_a_plan_tells_how_it_solves():
     assert b["operations"] == 2 * a["operations"] and b["bytes"] == 2 * a["bytes"] > 0
     large = FEPlan([0, 301 ** 2], np.zeros((0, 2), np.int32), shell(300).cnct_quads, [0, 1, 2])
     assert large.direct_info()["taken"] is None
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_the_iterative_correction_runs_its_inner_solver_alone(transpose):
+    """K so far from its symmetric part (spectral radius of I - S^-1 K about 0.65) that the
+    refinement with the factor of S, which wants 0.5, hands over to the iterative correction:
+    the direct solve is not begun again for its inner solves."""
+    plan = plan_of(shell(12, 14.0, 1.0))
+    plan.nonsymmetric_route(2)
+    f = torch.tensor(shell(12).nodal_loads, device="cuda")
+    u = plan.solve(f, transpose=transpose)
+    info, direct = plan.last_info, plan.direct_info()
+    print(info, direct, flush=True)
+    assert info["converged"] == 1 and info["replacements"] > 3 and info["iterations"] > info["replacements"]
+    assert direct["factorisations"] == direct["begun"] == 1 and direct["finished"] == 0
+    plan.nonsymmetric_route(1)
+    dense = plan.solve(f, transpose=transpose)
+    assert float(torch.linalg.norm(u - dense) / torch.linalg.norm(dense)) < 1e-8
