@@ -602,10 +602,33 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
     int rc = launch_full_blocks(p, s);
     if (rc) return rc;
     const int64_t ndof = 6 * (int64_t)p->n_nodes;
-    // (it sets u to zero first and reads f again at every step: not for f inside u)
-    const size_t bytes = (size_t)ndof * nrhs * sizeof(double);
-    const bool apart = (const char*)d_f + bytes <= (const char*)d_u || (const char*)d_u + bytes <= (const char*)d_f;
-    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set && apart) {
+    const int nsys = p->n_sys * nrhs;
+    const size_t vb = (size_t)ndof * nrhs * sizeof(double);
+    // vectors of the iterative correction (r, du, the squares' sums), then a copy of f
+    const size_t work = 2 * vb + 2 * (size_t)nsys * sizeof(double);
+    auto vectors = [&](size_t need) -> int {
+        if (p->ws.size() <= WS_DEFECT_SLOT) p->ws.resize(WS_DEFECT_SLOT + 1);
+        DBuf& g = p->ws[WS_DEFECT_SLOT];
+        if (g.bytes >= need) return JSSO_OK;
+        if (g.p) JSSO_HIP(hipFree(g.p));
+        g.p = nullptr;
+        g.bytes = 0;
+        hipError_t e = hipMalloc(&g.p, need);
+        JSSO_REQUIRE(e == hipSuccess, JSSO_ENOMEM, "defect-correction vectors hipMalloc(%zu): %s", need,
+                     hipGetErrorString(e));
+        g.bytes = need;
+        return JSSO_OK;
+    };
+    // the corrections set u to zero first and read f again at every step: where f lies in u,
+    // they read a copy of it
+    const bool apart = (const char*)d_f + vb <= (const char*)d_u || (const char*)d_u + vb <= (const char*)d_f;
+    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !apart) {
+        if ((rc = vectors(work + vb))) return rc;
+        double* copy = (double*)((char*)p->ws[WS_DEFECT_SLOT].p + work);
+        JSSO_HIP(hipMemcpyAsync(copy, d_f, vb, hipMemcpyDeviceToDevice, s));
+        d_f = copy;
+    }
+    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set) {
         bool done = false;
         rc = direct_defect(p, p->d_K, d_f, d_u, nrhs, transpose, tol, maxit, h_info, s, done);
         if (rc || done) return rc;
@@ -624,21 +647,8 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
     JSSO_REQUIRE(!(status & STATUS_Y_BEAM), JSSO_EUNSUPPORTED,
                  "members parallel to global Y (element.py:92-94) leave the symmetric part of K indefinite: the "
                  "defect correction cannot converge; use the dense route (jsso_plan_nonsymmetric_route 0 or 1)");
-    const int nsys = p->n_sys * nrhs;
-    const size_t vb = (size_t)ndof * nrhs * sizeof(double);
-    const size_t need = 2 * vb + 2 * (size_t)nsys * sizeof(double);
-    if (p->ws.size() <= WS_DEFECT_SLOT) p->ws.resize(WS_DEFECT_SLOT + 1);
-    DBuf& g = p->ws[WS_DEFECT_SLOT];
-    if (g.bytes < need) {
-        if (g.p) JSSO_HIP(hipFree(g.p));
-        g.p = nullptr;
-        g.bytes = 0;
-        hipError_t e = hipMalloc(&g.p, need);
-        JSSO_REQUIRE(e == hipSuccess, JSSO_ENOMEM, "defect-correction vectors hipMalloc(%zu): %s", need,
-                     hipGetErrorString(e));
-        g.bytes = need;
-    }
-    double* r = (double*)g.p;
+    if ((rc = vectors(work))) return rc;   // (a copy of f made above keeps its place: it asked for more)
+    double* r = (double*)p->ws[WS_DEFECT_SLOT].p;
     double* du = r + (size_t)ndof * nrhs;
     double* d_rr = du + (size_t)ndof * nrhs;
     std::vector<double> rr(nsys), ff(nsys);

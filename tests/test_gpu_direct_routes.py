@@ -58,3 +58,29 @@ def test_the_iterative_correction_runs_its_inner_solver_alone(transpose):
     plan.nonsymmetric_route(1)
     dense = plan.solve(f, transpose=transpose)
     assert float(torch.linalg.norm(u - dense) / torch.linalg.norm(dense)) < 1e-8
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("ratio,route", [(1.5, 0), (1.5, 2), (14.0, 2)])
+def test_a_result_over_the_right_hand_side_of_a_non_symmetric_solve(ratio, route, transpose):
+    """u = f in memory, u half over f, and apart: the same u on each route (refinement with the
+    factor of the symmetric part, iterative correction; two load cases)."""
+    st = shell(9, ratio, 1.0)
+    plan = plan_of(st)
+    n = 2 * st.ndof
+    rng = np.random.default_rng(4)
+    f = torch.tensor(st.nodal_loads[:, None] * rng.uniform(0.5, 2.0, (st.ndof, 2)), device="cuda").reshape(-1)
+    plan.nonsymmetric_route(1)
+    ref = plan.solve(f.reshape(-1, 2), transpose=transpose).reshape(-1)
+    plan.nonsymmetric_route(route)
+    entry = nat.lib().jsso_solve_transpose if transpose else nat.lib().jsso_solve
+    for gap in (0, n // 2, -(n // 2), n):
+        info = nat.Info()
+        both = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+        fv, uv = both[n:2 * n], both[n + gap:2 * n + gap]
+        fv.copy_(f)
+        nat.check(entry(plan._h, nat.ptr(fv), nat.ptr(uv), 2, nat.PREC["fp64"], 1e-11, 10000, ctypes.byref(info),
+                        nat.stream_ptr()))
+        print(ratio, route, gap, info.as_dict(), flush=True)
+        assert info.converged == 2 and info.replacements > 0
+        assert float(torch.linalg.norm(uv - ref) / torch.linalg.norm(ref)) < 1e-8, gap
