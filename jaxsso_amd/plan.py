@@ -81,10 +81,11 @@ class FEPlan:
         nat.check(L.jsso_assemble(self._h, nat.ptr(crds), nat.ptr(pb), nat.ptr(pq), nat.ptr(Kout), nat.stream_ptr()))
         return Kout
 
-    def ensure_assembled(self, crds, prop_beam, prop_quad, assembly_id):
+    def ensure_assembled(self, crds, prop_beam, prop_quad, assembly_id=None):
         """Assemble again unless the plan still holds assembly ``assembly_id`` (the caller
-        answers for it being that of these inputs).  Returns the id it holds now."""
-        if self.assembly_id != assembly_id:
+        answers for it being that of these inputs; None: assemble).  Returns the id it holds
+        now."""
+        if assembly_id is None or self.assembly_id != assembly_id:
             self.assemble(crds, prop_beam, prop_quad)
         return self.assembly_id
 

@@ -84,3 +84,18 @@ def test_a_result_over_the_right_hand_side_of_a_non_symmetric_solve(ratio, route
         print(ratio, route, gap, info.as_dict(), flush=True)
         assert info.converged == 2 and info.replacements > 0
         assert float(torch.linalg.norm(uv - ref) / torch.linalg.norm(ref)) < 1e-8, gap
+
+
+def test_ensure_assembled_without_an_assembly_id():
+    """The call with inputs alone makes the plan hold their assembly."""
+    a, b = shell(9), shell(9, 1.5, 1.0)
+    plan = plan_of(a)
+    f = torch.tensor(a.nodal_loads, device="cuda")
+    u = plan.solve(f)
+    first = plan.assembly_id
+    inputs = torch.tensor(a.crds, device="cuda"), None, torch.tensor(a.prop_quads, device="cuda")
+    plan.assemble(torch.tensor(b.crds), None, torch.tensor(b.prop_quads))
+    assert not torch.equal(plan.solve(f), u)
+    now = plan.ensure_assembled(*inputs)
+    assert now == plan.assembly_id > first and torch.equal(plan.solve(f), u)
+    assert plan.ensure_assembled(*inputs, now) == now
