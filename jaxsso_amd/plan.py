@@ -79,6 +79,9 @@ class FEPlan:
         Kout = torch.empty((self.nnzb, 6, 6), dtype=torch.float64, device=crds.device) if export_K else None
         self.assembly_id += 1         # before the call: one that fails leaves no earlier K either
         nat.check(L.jsso_assemble(self._h, nat.ptr(crds), nat.ptr(pb), nat.ptr(pq), nat.ptr(Kout), nat.stream_ptr()))
+        # the kernels may still read these when the caller drops them, on another stream than
+        # the one they were allocated on: their memory is held until the next assembly
+        self._keep = [None if t is None else t.detach() for t in (crds, pb, pq)]
         return Kout
 
     def ensure_assembled(self, crds, prop_beam, prop_quad, assembly_id=None):

@@ -99,3 +99,24 @@ def test_ensure_assembled_without_an_assembly_id():
     now = plan.ensure_assembled(*inputs)
     assert now == plan.assembly_id > first and torch.equal(plan.solve(f), u)
     assert plan.ensure_assembled(*inputs, now) == now
+
+
+def test_a_plan_holds_the_memory_of_the_inputs_that_it_assembles():
+    """Inputs made on the current stream, assembled on another one and dropped: their memory
+    is not handed out while the assembly may still read it."""
+    st = shell(20)
+    plan = plan_of(st)
+    f = torch.tensor(st.nodal_loads, device="cuda")
+    u = plan.solve(f)
+    side = torch.cuda.Stream()
+    crds, pq = torch.tensor(st.crds, device="cuda"), torch.tensor(st.prop_quads, device="cuda")
+    held = {crds.data_ptr(), pq.data_ptr()}
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        plan.assemble(crds, None, pq)
+    shapes = crds.shape, pq.shape
+    del crds, pq
+    new = [torch.zeros(sh, dtype=torch.float64, device="cuda") for sh in shapes for _ in range(4)]
+    assert not held & {t.data_ptr() for t in new}
+    side.synchronize()
+    assert torch.equal(plan.solve(f), u)
