@@ -142,6 +142,10 @@ class SSO_model:
 
     def ele_params_props(self, eleparameter_values, pb=None, pq=None):
         v = _to_dev(eleparameter_values)
+        n = len(self.eleparameters_tags)
+        if v.dim() == 0 or len(v) < n:   # (a single value would be spread over all parameters)
+            raise ValueError(f"{n} element parameters, values of shape {tuple(v.shape)}")
+        v = v if len(v) == n else v[:n]
         ix = self._indices(v.device)
         if pb is None or pq is None:
             pb = torch.as_tensor(self.model.prop_beamcols, dtype=torch.float64, device=v.device)
