@@ -68,12 +68,13 @@ enum {
 
 /* preconditioner of the batched precisions (jsso_plan_set_preconditioner) */
 enum {
+    JSSO_PC_NOT_CHOSEN = -1,  /* takes a choice back                                    */
     JSSO_PC_BLOCK_JACOBI = 0, /* split block-Jacobi scaling                             */
     JSSO_PC_AMG = 1           /* smoothed-aggregation AMG V-cycle on the scaled system
                                  (the default)                                          */
 };
-/* As long as the caller has not called jsso_plan_set_preconditioner (or asked
- * jsso_plan_amg_reuse to keep a hierarchy), a batched solve with 1 to 4 load cases
+/* As long as the caller has chosen no preconditioner (jsso_plan_set_preconditioner;
+ * JSSO_PC_NOT_CHOSEN takes that back) and jsso_plan_amg_reuse is in mode 0, a batched solve with 1 to 4 load cases
  * may be direct instead: a multifrontal Cholesky of the scaled constrained K in
  * FP64 (kept until the next jsso_assemble), refined on the FP64 residual to the
  * same tolerance; plans whose fronts are small enough for it to be the faster way
@@ -307,7 +308,8 @@ int jsso_plan_element_tuning(jsso_plan* plan, int32_t set_epw, int32_t* h_epw);
  * counterpart in the reference, which factorises with SuperLU (JaxSSO/solver.py:
  * 176-218).  JSSO_PC_AMG builds a smoothed-aggregation hierarchy on the plan's
  * pattern (host, once) and its numeric operators after each jsso_assemble (device,
- * at the next solve); the plain path always uses block-Jacobi. */
+ * at the next solve); the plain path always uses block-Jacobi.  A choice holds for
+ * the plan's later solves; JSSO_PC_NOT_CHOSEN is the state of a new plan. */
 int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc);
 /* The direct solve of a plan (see JSSO_PC_AMG): h_info (7 entries) receives
  *   0  whether the plan solves directly: 1 yes, 0 no (its fronts or its memory are past

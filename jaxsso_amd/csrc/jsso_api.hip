@@ -628,7 +628,7 @@ static int solve_nonsymmetric(Plan* p, const double* d_f, double* d_u, int nrhs,
         JSSO_HIP(hipMemcpyAsync(copy, d_f, vb, hipMemcpyDeviceToDevice, s));
         d_f = copy;
     }
-    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && !p->precond_set) {
+    if (p->nonsym_route != 1 && !(status & STATUS_Y_BEAM) && p->may_solve_directly()) {
         bool done = false;
         rc = direct_defect(p, p->d_K, d_f, d_u, nrhs, transpose, tol, maxit, h_info, s, done);
         if (rc || done) return rc;
@@ -719,7 +719,7 @@ int jsso_solve(jsso_plan* plan, const double* d_f, double* d_u, int32_t nrhs, in
     if (rc) return rc;
     const int slot = precision == JSSO_PREC_FP64 ? PS_F64 : precision == JSSO_PREC_MIXED ? PS_F32 : PS_F32_V64;
     bool tried = false;
-    if (precision != JSSO_PREC_PLAIN && !p->precond_set && expect_symmetric(p)) {
+    if (precision != JSSO_PREC_PLAIN && p->may_solve_directly() && expect_symmetric(p)) {
         bool done = false;
         rc = direct_solve(p, d_f, d_u, nrhs, slot, tol, maxit, false, h_info, s, done);
         if (rc || done) return rc;
@@ -957,12 +957,12 @@ int jsso_compliance(jsso_plan* plan, const double* d_f, const double* d_u, int32
 }
 
 int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc) {
-    if (!plan || (pc != JSSO_PC_BLOCK_JACOBI && pc != JSSO_PC_AMG)) {
-        set_error("invalid preconditioner (JSSO_PC_BLOCK_JACOBI or JSSO_PC_AMG)");
+    if (!plan || (pc != JSSO_PC_BLOCK_JACOBI && pc != JSSO_PC_AMG && pc != JSSO_PC_NOT_CHOSEN)) {
+        set_error("invalid preconditioner (JSSO_PC_BLOCK_JACOBI, JSSO_PC_AMG or JSSO_PC_NOT_CHOSEN)");
         return JSSO_EINVAL;
     }
-    P(plan)->precond = pc;
-    P(plan)->precond_set = true;
+    P(plan)->precond_set = pc != JSSO_PC_NOT_CHOSEN;
+    P(plan)->precond = pc == JSSO_PC_NOT_CHOSEN ? JSSO_PC_AMG : pc;
     return JSSO_OK;
 }
 int jsso_plan_direct_info(jsso_plan* plan, int64_t* h_info) {
@@ -981,7 +981,6 @@ int jsso_plan_amg_reuse(jsso_plan* plan, int32_t mode, int64_t* h_counts) {
     Plan* p = P(plan);
     if (mode >= 0) {
         p->amg_reuse = mode;
-        if (mode > 0) p->precond_set = true;
         if (mode == 2) p->amg_valid = false;   // rebuild at the next solve even without a new assembly
     }
     if (h_counts) {
@@ -1023,9 +1022,9 @@ int jsso_plan_cg_tuning(jsso_plan* plan, int32_t precision, int32_t nrhs, int32_
     int32_t& direct = p->direct_wps[ps][nrhs];   // (a plan without a chosen preconditioner may solve directly)
     if (set_wps >= 0) {
         slot = set_wps;
-        if (!p->precond_set) direct = set_wps;
+        if (p->may_solve_directly()) direct = set_wps;
     }
-    if (h_wps) *h_wps = !p->precond_set && direct ? direct : slot;
+    if (h_wps) *h_wps = p->may_solve_directly() && direct ? direct : slot;
     return JSSO_OK;
 }
 

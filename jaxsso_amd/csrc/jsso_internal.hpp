@@ -165,13 +165,15 @@ struct Plan {
     double* d_crds = nullptr;     // node coordinates of the current assembly (for the AMG null space)
     // preconditioner of the batched solves (JSSO_PC_*) and the AMG hierarchy
     int32_t precond = JSSO_PC_AMG;
-    bool precond_set = false;     // chosen by the caller (jsso_plan_set_preconditioner, jsso_plan_amg_reuse)
+    bool precond_set = false;     // chosen by the caller (jsso_plan_set_preconditioner)
     DirectState* direct = nullptr;
     int32_t direct_wps[3][9] = {};   // waves per slice of the direct solve's residual kernel, as amg_wps
     bool direct_valid = false;    // the factorisation matches the current assembly
     AmgState* amg = nullptr;
     bool amg_valid = false;       // the AMG numeric set-up matches the current assembly
     int32_t amg_reuse = 0;        // jsso_plan_amg_reuse mode
+    // the caller left the solver to the plan: no preconditioner chosen, no hierarchy kept
+    bool may_solve_directly() const { return !precond_set && amg_reuse == 0; }
     int64_t amg_full = 0, amg_light = 0;   // numeric set-ups run: full, and refreshes of a kept hierarchy
     // dense direct solve (jsso_dense_solve): N x N factor + right-hand sides, grown on demand
     double* d_dense = nullptr;

@@ -986,7 +986,7 @@ int solve_batched(Plan* p, const double* f, double* u, int nrhs, int slot, doubl
                   jsso_info* info, hipStream_t s, bool direct_tried) {
     int rc = check_status(p, s);
     if (rc) return rc;
-    if (!p->precond_set && !direct_tried) {   // the caller left the choice: directly where that is cheaper
+    if (p->may_solve_directly() && !direct_tried) {   // the caller left the choice: directly where that is cheaper
         bool done = false;
         rc = direct_solve(p, f, u, nrhs, slot, tol, maxit, false, info, s, done);
         if (rc || done) return rc;

@@ -116,14 +116,16 @@ class FEPlan:
         nat.check(nat.lib().jsso_plan_nonsymmetric_route(self._h, int(mode), ctypes.byref(out)))
         return int(out.value)
 
-    def set_preconditioner(self, name: str) -> None:
-        """Preconditioner of the batched precisions: 'amg' (smoothed-aggregation
-        multigrid V-cycle, the default) or 'block_jacobi' (split block-Jacobi scaling)."""
-        if name not in PRECONDITIONERS:
+    def set_preconditioner(self, name: str | None) -> None:
+        """Preconditioner of the batched precisions, for all later solves: 'amg'
+        (smoothed-aggregation multigrid V-cycle) or 'block_jacobi' (split block-Jacobi
+        scaling).  None takes a choice back, as in a new plan: the library solves directly
+        where it can, and by AMG elsewhere."""
+        if name is not None and name not in PRECONDITIONERS:
             raise ValueError(f"unknown preconditioner {name!r} ({sorted(PRECONDITIONERS)})")
-        nat.check(nat.load_library().jsso_plan_set_preconditioner(self._h, PRECONDITIONERS[name]))
-        self.preconditioner = name
-        self._pc_chosen = True
+        nat.check(nat.load_library().jsso_plan_set_preconditioner(self._h, PRECONDITIONERS.get(name, -1)))
+        self.preconditioner = "amg" if name is None else name
+        self._pc_chosen = name is not None
 
     def element_tuning(self, set_epw: int = -1) -> int:
         """MITC-4 elements per workgroup of the assembly kernel (4, 8 or 16): 0 until
@@ -165,10 +167,19 @@ class FEPlan:
               maxit: int = DEFAULT_MAXIT, warn: bool = True, preconditioner: str | None = None,
               transpose: bool = False) -> torch.Tensor:
         """Solve K u = f (K^T u = f with ``transpose``; u = 0 at supports).  f: (ndof,)
-        or (ndof, nrhs) FP64 on the device."""
+        or (ndof, nrhs) FP64 on the device.  ``preconditioner``: as ``set_preconditioner``;
+        the AMG asked for here on a plan that has not chosen serves this call only."""
         L = nat.lib()
-        if preconditioner is not None and (preconditioner != self.preconditioner or not self._pc_chosen):
+        once = preconditioner == self.preconditioner and not self._pc_chosen
+        if preconditioner is not None and (preconditioner != self.preconditioner or once):
             self.set_preconditioner(preconditioner)
+        try:
+            return self._solve(L, f, precision, tol, maxit, warn, transpose)
+        finally:
+            if once:
+                self.set_preconditioner(None)
+
+    def _solve(self, L, f, precision, tol, maxit, warn, transpose):
         f = _dev64(f)
         vec = f.dim() == 1
         f2 = f.reshape(self.ndof, -1).contiguous()
@@ -181,7 +192,7 @@ class FEPlan:
         nat.check(rc, allow_not_converged=True)
         self.last_info = info.as_dict()
         if rc == nat.JSSO_NOT_CONVERGED and warn:
-            warnings.warn(f"CG did not converge: {self.last_info}", RuntimeWarning, stacklevel=2)
+            warnings.warn(f"CG did not converge: {self.last_info}", RuntimeWarning, stacklevel=3)
         return u.reshape(f.shape) if vec else u
 
     def compliance(self, f: torch.Tensor, u: torch.Tensor, scale: float = 0.5) -> torch.Tensor:

@@ -120,3 +120,33 @@ def test_a_plan_holds_the_memory_of_the_inputs_that_it_assembles():
     assert not held & {t.data_ptr() for t in new}
     side.synchronize()
     assert torch.equal(plan.solve(f), u)
+
+
+def test_a_choice_of_the_iterative_solve_can_be_taken_back():
+    """preconditioner="amg" for one call, a kept AMG hierarchy given up, and a chosen
+    preconditioner taken back: the plan solves directly again; a choice that is not taken back
+    stays."""
+    st = shell(12)
+    plan = plan_of(st)
+    f = torch.tensor(st.nodal_loads, device="cuda")
+
+    def direct(**kw):
+        plan.solve(f, **kw)
+        return plan.last_info["levels"] == 0 and plan.last_info["iterations"] <= 6
+
+    assert direct() and not direct(preconditioner="amg") and direct()
+    assert plan.preconditioner == "amg"
+    plan.amg_reuse(2)
+    assert not direct() and not direct(preconditioner="amg") and not direct()
+    plan.amg_reuse(0)
+    assert direct()
+    for name in ("amg", "block_jacobi"):
+        plan.set_preconditioner(name)
+        assert not direct() and not direct(preconditioner=name) and not direct() and plan.preconditioner == name
+        plan.set_preconditioner(None)
+        assert direct()
+    assert not direct(preconditioner="block_jacobi") and not direct() and plan.preconditioner == "block_jacobi"
+    with pytest.raises(ValueError):
+        plan.set_preconditioner("ilu")
+    with pytest.raises(RuntimeError):
+        nat.check(nat.lib().jsso_plan_set_preconditioner(plan._h, 7))
