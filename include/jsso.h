@@ -290,7 +290,8 @@ int jsso_csr_spmv(int32_t n_rows, const int32_t* d_rowptr, const int32_t* d_coli
  * block-Jacobi preconditioner the fused iteration kernel k_cgf, with AMG the
  * level-0 kernels (timed on k_pcg_dir, the direction and CG product).  The
  * choice is kept per preconditioner; this call reads or sets the one of the
- * plan's current preconditioner.  set_wps >= 0 overrides the stored choice
+ * plan's current preconditioner, or, where the plan solves directly, the waves of
+ * its residual kernel (by a rule, not timed: as many as fit).  set_wps >= 0 overrides the stored choice
  * (0 = tune again on the next solve, 1/2/4 = force); h_wps, if not NULL,
  * receives the stored choice (0 = untuned). */
 int jsso_plan_cg_tuning(jsso_plan* plan, int32_t precision, int32_t nrhs, int32_t set_wps,

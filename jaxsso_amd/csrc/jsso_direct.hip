@@ -1848,43 +1848,14 @@ static int ensure_factor(Plan* pl, DirectState& D, hipStream_t s) {
     return rc;
 }
 
-// Waves per slice (1, 2 or 4) of the residual kernel, timed on the live plan right
-// after the start-up kernels: x is zero, so the residual it writes is the one that
-// is there already.
+// Waves per slice of the residual kernel, unless jsso_plan_cg_tuning has set them: as many
+// as fit its registers, 4 with up to two load cases.  A rule and not a timing, so that two
+// plans of one pattern sum in the same order.  Medians in us with 1 / 2 / 4 waves: gridshell
+// of 121 nodes 4.1 / 3.9 / 3.7, 40 x 40 shell 7.3 / 6.1 / 5.6 (two load cases 8.0 / 6.7 /
+// 6.7), 200 x 200 shell 15.5 / 15.9 / 15.3, 64 shells of 100 x 100 237 / 212 / 178.
 template <int NR>
-static int tune_residual(Plan* pl, const Workspace& w, const Slices& sl, double* r, hipStream_t s, int32_t& out) {
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    JSSO_HIP(hipEventCreate(&e0));
-    JSSO_HIP(hipEventCreate(&e1));
-    float best = 0.f;
-    int pick = 1;
-    auto run = [&](auto W, bool first) -> int {
-        constexpr int WP = decltype(W)::value;
-        if constexpr (WpsFits<double, NR, WP>::value) {
-            float ms = 0.f;
-            for (int rep = 0; rep < 4; ++rep) {
-                if (rep == 1) JSSO_HIP(hipEventRecord(e0, s));
-                hipLaunchKernelGGL((k_replace<double, NR, WP>), slice_grid(sl), dim3(64 * WP), 0, s, sl, w.P, w.st,
-                                   (const double*)pl->d_Ke64, (const double*)w.b64, (const double*)w.x64, r);
-            }
-            JSSO_HIP(hipEventRecord(e1, s));
-            JSSO_HIP(hipEventSynchronize(e1));
-            JSSO_HIP(hipEventElapsedTime(&ms, e0, e1));
-            if (first || ms < best) {
-                best = ms;
-                pick = WP;
-            }
-        }
-        return JSSO_OK;
-    };
-    int rc = run(std::integral_constant<int, 1>(), true);
-    if (!rc) rc = run(std::integral_constant<int, 2>(), false);
-    if (!rc) rc = run(std::integral_constant<int, 4>(), false);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    JSSO_HIP(hipGetLastError());
-    out = pick;
-    return rc;
+constexpr int residual_waves() {
+    return WpsFits<double, NR, 4>::value ? 4 : WpsFits<double, NR, 2>::value ? 2 : 1;
 }
 
 // u = K^-1 f by the factorisation and refinement; done = false (and nothing said
@@ -1910,7 +1881,7 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
     hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys,
                        strict ? DECIDE_START_STRICT : DECIDE_START, tol, 0, 0, (const double*)nullptr, 0.0, 0);
     int32_t& wps = pl->direct_wps[slot][NR];
-    if (wps <= 0 && (rc = tune_residual<NR>(pl, w, sl, r, s, wps))) return rc;
+    if (wps <= 0) wps = residual_waves<NR>();
     if ((rc = ensure_factor(pl, D, s))) return rc;
     for (int it = 1; it <= std::min(maxit, DIRECT_STEPS); ++it) {
         direct_apply<NR>(D, w.st.active, r, it == 1 ? w.x64 : z, s);   // (x is zero before)

@@ -150,3 +150,19 @@ def test_a_choice_of_the_iterative_solve_can_be_taken_back():
         plan.set_preconditioner("ilu")
     with pytest.raises(RuntimeError):
         nat.check(nat.lib().jsso_plan_set_preconditioner(plan._h, 7))
+
+
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 4])
+def test_plans_of_one_pattern_give_the_same_bits(nrhs):
+    """The order of the residual's sums is the pattern's, not a timing's: plans made one after
+    the other choose the same waves per slice and return the same bits after two steps."""
+    st = shell(6)
+    f = torch.tensor(np.random.default_rng(3).normal(size=(st.ndof, nrhs)), device="cuda")
+    first = None
+    for _ in range(24):
+        plan = plan_of(st)
+        u = plan.solve(f, tol=1e-16)
+        waves = plan.cg_tuning("fp64", nrhs)
+        assert plan.last_info["iterations"] >= 2 and plan.last_info["waves_per_slice"] == waves
+        first = first or (waves, u)
+        assert waves == first[0] and torch.equal(u, first[1])
