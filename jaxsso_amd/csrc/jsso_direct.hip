@@ -48,7 +48,7 @@ constexpr int DROWS = 64;                 // edge of an update tile
 constexpr int SROWS = 96;                 // rows of a strip
 constexpr int DLEAF = 10;                 // nodes eliminated whole at the tree's leaves (5 to 12: within 3%)
 constexpr int DLDS_MAX = 156 * 1024;      // dynamic LDS of a small front
-constexpr int DIRECT_MAX_M = 2300;        // largest front (direct_fits)
+constexpr int DIRECT_MAX_M = 2300;        // largest front (direct_build)
 static_assert((DIRECT_MAX_M + 2 * 1024) * 4 * 8 <= DLDS_MAX, "LDS of the backward solve with 4 load cases");
 constexpr int DIRECT_STEPS = 6;           // refinement steps, at most
 constexpr int DEFECT_STEPS = 40;          // of a K that is not symmetric
@@ -1469,8 +1469,9 @@ struct Arena {
     }
 };
 
-static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nodes, std::vector<int32_t>& blk,
-                             std::vector<int32_t>& blkrow, std::vector<int2>& inv) {
+// false where the fronts, or the storage of the structures so far, are past the limits
+static bool direct_build_host(Plan* pl, DirectState& D, size_t most_bytes, std::vector<int32_t>& nodes,
+                              std::vector<int32_t>& blk, std::vector<int32_t>& blkrow, std::vector<int2>& inv) {
     const auto& off = pl->h_node_off;
     struct Cls {
         int32_t fr0, n_fr, sys;
@@ -1509,7 +1510,10 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
             for (int i = 0; i <= n; ++i) lrp[i] = pl->h_rowptr[n0 + i] - b0;
             for (int k = 0; k < nb; ++k) lci[k] = pl->h_colind[b0 + k] - n0;
             FrontTree T;
-            build_fronts(n, lrp.data(), lci.data(), DLEAF, T);
+            int32_t largest = 0;
+            const bool fits = build_fronts(n, lrp.data(), lci.data(), DLEAF, T, DIRECT_MAX_M / 6, &largest);
+            D.max_m = std::max(D.max_m, 6 * largest);
+            if (!fits) return false;
             Cls C{(int32_t)fr.size(), (int32_t)T.fronts.size(), s, 0, 0, 0};
             const int32_t node_base = (int32_t)nodes.size(), blk_base = (int32_t)(blk.size() / 3);
             for (size_t t = 0; t < T.fronts.size(); ++t) {
@@ -1521,7 +1525,7 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
                 M.level = F.level;
                 M.child[0] = M.child[1] = -1;
                 for (int q = T.child_ptr[t]; q < T.child_ptr[t + 1]; ++q) {
-                    if (q - T.child_ptr[t] >= 2) return JSSO_EUNSUPPORTED;
+                    if (q - T.child_ptr[t] >= 2) return false;
                     M.child[q - T.child_ptr[t]] = C.fr0 + T.child[q];
                 }
                 M.blk0 = blk_base + F.blk0;
@@ -1543,7 +1547,6 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
                 const double kd = k, bd = b;
                 D.flops += kd * kd * kd + 2 * bd * kd * kd + bd * bd * kd;
                 D.n_levels = std::max(D.n_levels, F.level + 1);
-                D.max_m = std::max(D.max_m, m);
                 fr.push_back(M);
             }
             // storage: level by level, a child's matrix is free once its parent's level is done
@@ -1599,6 +1602,7 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
         D.fac_n += C.fac;
         D.mat_n += C.mat;
         D.vec_n += C.vec;
+        if ((D.fac_n + D.mat_n) * 8 > most_bytes) return false;
     }
     D.small_tasks.resize(D.n_levels);
     D.big_tasks.resize(D.n_levels);
@@ -1636,7 +1640,7 @@ static int direct_build_host(Plan* pl, DirectState& D, std::vector<int32_t>& nod
             }
         }
     }
-    return JSSO_OK;
+    return true;
 }
 
 template <typename T>
@@ -1671,17 +1675,24 @@ void direct_destroy(Plan* pl) {
     pl->direct = nullptr;
 }
 
-static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b);
-
-// builds the analysis and its storage; leaves D.usable false where the direct
-// solve is not the better choice or does not fit
+// Builds the analysis and its storage; leaves D.usable false where the direct solve is
+// not the better choice or does not fit.
+//
+// The direct solve is taken where its fronts stay small: fill and operations grow
+// with the largest front (m rows: m^2 storage, m^3 operations), while the
+// AMG-preconditioned CG grows with the number of nodes.  One shell of n x n quads
+// has m ~ 9 n: assembly and solve of one smooth shell, ms direct / AMG: 40x40
+// (m = 366) 0.79 / 1.9, 100x100 1.8 / 3.2, 200x200 4.8 / 6.7, 250x250 (m = 2256)
+// 6.7 / 8.4, 300x300 10.2 / 9.4.  Designs that take the CG more iterations gain more,
+// and so do batches, which fill the chip on every tree level (64 SIMP shells of
+// 100x100, with gradients: 31.6 / 62).  It needs its storage too: up to an eighth of
+// the card, and half of what is free.
 static int direct_build(Plan* pl, DirectState& D) {
     std::vector<int32_t> nodes, blk, blkrow;
     std::vector<int2> inv;
-    if (direct_build_host(pl, D, nodes, blk, blkrow, inv) != JSSO_OK) return JSSO_OK;
     size_t free_b = 0, total_b = 0;
     JSSO_HIP(hipMemGetInfo(&free_b, &total_b));
-    if (!direct_fits(D, free_b, total_b)) return JSSO_OK;
+    if (!direct_build_host(pl, D, std::min(total_b / 8, free_b / 2), nodes, blk, blkrow, inv)) return JSSO_OK;
     int rc = 0;
     std::vector<FrontTask> tasks;
     D.buckets.resize(D.n_levels);
@@ -1709,8 +1720,8 @@ static int direct_build(Plan* pl, DirectState& D) {
         D.big_n.push_back(D.big_tasks[L].size());
         tasks.insert(tasks.end(), D.big_tasks[L].begin(), D.big_tasks[L].end());
     }
-    D.small_tasks.clear();
-    D.big_tasks.clear();
+    std::vector<std::vector<FrontTask>>().swap(D.small_tasks);
+    std::vector<std::vector<FrontTask>>().swap(D.big_tasks);
     // ||A||_2 <= 4: with identity diagonal blocks, x^T A x = sum_e x_e^T A_e x_e is at most
     // (nodes of an element) x sum_e x_e^T diag(A_e) x_e = (nodes of an element) ||x||^2
     std::vector<double> rho(pl->n_sys, 4.0);
@@ -1929,20 +1940,6 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
         return R.not_finite ? JSSO_NOT_CONVERGED : JSSO_OK;
     }
     return JSSO_OK;
-}
-
-// The direct solve is taken where its fronts stay small: fill and operations grow
-// with the largest front (m rows: m^2 storage, m^3 operations), while the
-// AMG-preconditioned CG grows with the number of nodes.  One shell of n x n quads
-// has m ~ 9 n: assembly and solve of one smooth shell, ms direct / AMG: 40x40
-// (m = 366) 0.79 / 1.9, 100x100 1.8 / 3.2, 200x200 4.8 / 6.7, 250x250 (m = 2256)
-// 6.7 / 8.4, 300x300 10.2 / 9.4.  Designs that take the CG more iterations gain more,
-// and so do batches, which fill the chip on every tree level (64 SIMP shells of
-// 100x100, with gradients: 31.6 / 62).  It needs its storage too: up to an eighth of
-// the card, and half of what is free.
-static bool direct_fits(const DirectState& D, size_t free_b, size_t total_b) {
-    const size_t need = (D.fac_n + D.mat_n) * 8;
-    return D.max_m <= DIRECT_MAX_M && need <= total_b / 8 && need <= free_b / 2;
 }
 
 // the plan's analysis, built at its first use; nullptr where the direct solve is not taken

@@ -166,3 +166,17 @@ def test_plans_of_one_pattern_give_the_same_bits(nrhs):
         assert plan.last_info["iterations"] >= 2 and plan.last_info["waves_per_slice"] == waves
         first = first or (waves, u)
         assert waves == first[0] and torch.equal(u, first[1])
+
+
+def test_a_mesh_past_the_limit_of_the_fronts_takes_the_iterative_route():
+    st = wl.shell_pinned_edges(270, 27.0, 3.0, design=3)
+    plan = plan_of(st)
+    f = torch.tensor(st.nodal_loads, device="cuda")
+    print("270 x 270", flush=True)
+    u = plan.solve(f)
+    info = plan.direct_info()
+    assert info["taken"] is False and info["max_front"] > 2300 and info["begun"] == info["factorisations"] == 0, info
+    assert plan.last_info["levels"] > 0 and plan.last_info["converged"] == 1
+    r = plan.spmv(u) - f
+    r[torch.as_tensor(st.known_id.astype(np.int64), device="cuda")] = 0.0
+    assert float(torch.linalg.norm(r) / torch.linalg.norm(f)) < 1e-6
