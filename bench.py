@@ -6,16 +6,16 @@ designs of 100x100 quads over 15 m x 15 m (10,201 nodes, 10,000 quads, 61,206
 DOF each; 3.92 M DOF in one plan), corners and mid-edge nodes pinned,
 -1.5 kN/node, per-element density rho in [0.01, 1] with E = rho^3 30 GPa,
 thickness 0.12 m, z from 6 Gaussian bumps.  One step evaluates all 64 designs:
-element stiffness and assembly, the AMG numeric set-up, the solve (flexible CG
-preconditioned by the smoothed-aggregation V-cycle, to a 1e-10 scaled
-residual), the compliance in FP64 and the adjoint kernels for dC/d(node
+element stiffness and assembly, the solve (to a 1e-10 scaled residual; by
+default the direct one: multifrontal Cholesky, refined), the compliance in FP64 and the adjoint kernels for dC/d(node
 coordinates) and dC/d(element properties), with dC/drho by the chain rule
 through E.  Inputs are resident on the GPU before timing starts.
 
 The JSON line carries:
 * ``roofline``: the direct solve's factorisation (all k_front_* launches of a
-  step, from HIP events; operations of the fronts' factors, S and G over the
-  FP64 matrix peak), or, where the iterative solve runs, its dominant kernel
+  step, from HIP events; operations of the fronts' factors, solve operators and
+  contributions as the plan counts them, over the FP64 matrix peak; HBM bytes of
+  these launches from the committed counter summary), or, where the iterative solve runs, its dominant kernel
   (k_pcg_dir, the CG direction and product), algorithmic bytes per launch over its mean duration from HIP
   events on the solver stream, sampled inside the timed steps: every other
   iteration chunk is launched eagerly with its k_pcg_dir launches bracketed,
@@ -28,8 +28,10 @@ The JSON line carries:
   separately);
 * errors against the FP64 oracle (committed fixture, designs 0 and 1) and
   against the plain FP64 one-structure-per-launch GPU path;
-* further lines: the 200x200 shell (one structure, 242,406 DOF) with its own
-  roofline, 256 uneven beam gridshells x 4 load cases, the 40x40 shell.
+* the same batch by AMG-CG in every precision (``*_batched``);
+* further lines: the 200x200 shell (one structure, 242,406 DOF; direct, AMG and
+  plain) with the AMG path's roofline, the SIMP batch in an optimisation loop,
+  256 uneven beam gridshells x 4 load cases, the 40x40 shell.
 
 python bench.py [--gpus 1] [--steps K] [--warmup W]
 """
@@ -45,6 +47,7 @@ import numpy as np
 
 HBM_PEAK_GBS = 8000.0
 HERE = os.path.dirname(os.path.abspath(__file__))
+FRONT_KERNELS = "k_front_* (direct factorisation)"
 TIMING_EVERY = 2        # one AMG iteration chunk in 2 runs eagerly with k_pcg_dir bracketed
 
 
@@ -116,6 +119,14 @@ def _assembly_traffic(name, kernels):
     return sum(found[k] for k in kernels) if all(k in found for k in kernels) else None
 
 
+def _route(plan):
+    """How the plan's last solve ran."""
+    i = plan.last_info
+    if i["levels"]:
+        return "AMG-CG"
+    return "direct (FP64 multifrontal Cholesky, refined)" if plan.direct_info()["finished"] else "block-Jacobi CG"
+
+
 def simp_headline(args, L, nat):
     """The SIMP batch: timed steps, roofline, assembly rates, errors."""
     import torch
@@ -172,15 +183,18 @@ def simp_headline(args, L, nat):
                 "alg_bytes_per_launch": int(alg)}
     ff = "simp64_shell100_fp64_flops.txt"
     if info["dir_launches"] == 0:   # the direct solve (no CG launches): its factorisation is the largest part
-        kname = "direct_factorisation"
-        fl = _measured_flops(ff, kname)
+        fl = b.plan.direct_info()["operations"]
         ms = t["setup"][0]
-        achieved = fl * args.designs / 64 / (ms * 1e-3) / 1e12 if fl and ms > 0 else None
-        roofline = {"kernel": "k_front_* (direct factorisation)", "bound": "fp64 matrix", "achieved": achieved,
-                    "peak": FP64_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
-                    "frac": achieved / FP64_VECTOR_PEAK_TFLOPS if achieved else None, "traffic": None,
-                    "traffic_source": None, "avg_launch_us": ms * 1e3, "sampled_launches": t["setup"][1],
-                    "alg_flops": fl, "flops_source": f"profiles/{ff}" if fl else None}
+        achieved = fl / (ms * 1e-3) / 1e12 if ms > 0 else None
+        traffic, tsrc = _measured_traffic(f"simp64_shell100_{args.precision}_traffic.txt", FRONT_KERNELS)
+        if args.designs != 64:   # (the summary is of the 64 designs)
+            traffic, tsrc = None, None
+        roofline = {"kernel": FRONT_KERNELS, "bound": "fp64 matrix", "achieved": achieved,
+                    "peak": FP64_MATRIX_PEAK_TFLOPS, "unit": "TFLOP/s",
+                    "frac": achieved / FP64_MATRIX_PEAK_TFLOPS if achieved else None, "traffic": traffic,
+                    "traffic_source": tsrc, "avg_launch_us": ms * 1e3, "sampled_launches": t["setup"][1],
+                    "alg_flops": fl, "flops_source": "FEPlan.direct_info",
+                    "traffic_GBps": traffic / (ms * 1e-3) / 1e9 if traffic and ms > 0 else None}
     eb, gb = _asm_bytes(b.plan)
     (te, ne), (tg, ng) = t["element"], t["gather"]
     assembly = {"element_kernels_us": te * 1e3, "element_alg_bytes": eb,
@@ -262,18 +276,20 @@ def simp_headline(args, L, nat):
                              "grad_rho": _rel(drn[:sub.plan.n_quad], drp)}}
     out["speedup_vs_plain_fp64"] = value / plain_eps
 
-    # the other batched precisions on the same batch
+    # the iterative solve in every precision on the same batch
+    solve_log_headline = list(solve_log)
+    b.plan.set_preconditioner("amg")
     for other in sorted(SIZES):
-        if other == args.precision:
-            continue
         step(other)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         step(other)
         torch.cuda.synchronize()
-        out[f"{other}_batched"] = {"evals_per_s": args.designs / (time.perf_counter() - t0),
+        out[f"{other}_batched"] = {"route": _route(b.plan), "evals_per_s": args.designs / (time.perf_counter() - t0),
                                    "cg_iterations": b.plan.last_info["iterations"],
                                    "converged": b.plan.last_info["converged"]}
+    b.plan.set_preconditioner(None)
+    out["solve_log"] = solve_log_headline
     return out
 
 
@@ -284,7 +300,7 @@ SHELL200_TOL = 1e-8
 
 def shell200(args, L, nat, profile=False):
     """The 200x200 MITC-4 shell (242,406 DOF) as one structure: evals/s on the
-    AMG path (mixed and FP64) and the plain FP64 path, errors against the
+    default (direct) path, the AMG path (mixed and FP64) and the plain FP64 path, errors against the
     committed FP64 oracle fixture, and the mixed path's k_pcg_dir roofline
     (profile: the mixed path only, with its solve log).  Every path solves to
     the workload's FP64 relative residual of 1e-8 (SHELL200_TOL)."""
@@ -298,12 +314,13 @@ def shell200(args, L, nat, profile=False):
     res = {"workload": "MITC-4 shell 200x200 over 20 m (40,401 nodes, 40,000 quads, 242,406 DOF), edges pinned, "
                        "smooth Fourier thickness; one structure per evaluation", "tol": SHELL200_TOL}
     solve_log = []
-    paths = (("mixed", "mixed", "amg", 10), ("fp64", "fp64", "amg", 5), ("plain", "plain", None, 1))
+    paths = (("mixed", "mixed", "amg", 10), ("fp64", "fp64", "amg", 5), ("direct", "fp64", None, 10),
+             ("plain", "plain", None, 1))
     for key, prec, pc, reps in paths[:1] if profile else paths:
+        b.plan.set_preconditioner(pc)
         if args.wps and key == "mixed":
-            b.plan.set_preconditioner("amg")
             b.plan.cg_tuning(prec, 1, args.wps)
-        b.compliance_and_gradient(precision=prec, tol=SHELL200_TOL, preconditioner=pc)     # warm-up
+        b.compliance_and_gradient(precision=prec, tol=SHELL200_TOL)     # warm-up
         if key == "mixed":
             i = b.plan.last_info
             solve_log.append([i["iterations"], i["dir_launches"], i["full_iterations"]])
@@ -314,7 +331,7 @@ def shell200(args, L, nat, profile=False):
                 _slot(L, nat, name)
         t0 = time.perf_counter()
         for _ in range(reps):
-            C, (dc, _, dq) = b.compliance_and_gradient(precision=prec, tol=SHELL200_TOL, preconditioner=pc)
+            C, (dc, _, dq) = b.compliance_and_gradient(precision=prec, tol=SHELL200_TOL)
             if key == "mixed":
                 i = b.plan.last_info
                 solve_log.append([i["iterations"], i["dir_launches"], i["full_iterations"]])
@@ -322,7 +339,7 @@ def shell200(args, L, nat, profile=False):
         dt = (time.perf_counter() - t0) / reps
         dcn = dc.cpu().numpy().reshape(st.n_node, 3)
         dqn = dq.cpu().numpy().reshape(st.n_quad, 5)
-        res[key] = {"preconditioner": pc or "block_jacobi (plain path)", "evals_per_s": 1.0 / dt,
+        res[key] = {"route": "block-Jacobi CG, plain path" if key == "plain" else _route(b.plan), "evals_per_s": 1.0 / dt,
                     "ms_per_eval": dt * 1e3, "cg_iterations": b.plan.last_info["iterations"],
                     "rel_err_vs_fp64_oracle": {
                         "C": abs(float(C[0, 0]) - fx["C"]) / fx["C"],
@@ -358,12 +375,13 @@ def simp_loop(args, L, nat, n_steps=8, step=0.05):
     """The SIMP batch inside an optimisation loop: every step evaluates the 64
     designs, then moves every element density by a normalised gradient step
     (rho <- clip(rho - step * g / max|g|, 0.01, 1) per design), so each step
-    assembles and solves new designs.  The same sequence runs twice: with the AMG
-    hierarchy rebuilt after every assembly, and with it kept across steps
-    (AmgKeepPolicy: only the level-0 smoothing bound follows each design; a
-    rebuild when the iterations grow by 25%).  Reported: evals/s, iterations per
-    step, AMG set-up ms per step, rebuilds, and the largest relative difference
-    of the compliances of the two runs."""
+    assembles and solves new designs.  The same sequence runs three times: by the
+    plan's own choice (the direct solve), by AMG-CG with the hierarchy rebuilt after
+    every assembly, and with it kept across steps (AmgKeepPolicy: only the level-0
+    smoothing bound follows each design; a rebuild when the iterations grow by 25%).
+    Reported: evals/s, iterations per step, ms per step of the factorisation or of
+    the AMG set-up, rebuilds, and the largest relative difference of the compliances
+    of the runs."""
     import torch
     from jaxsso_amd import workloads as wl
     from jaxsso_amd.batch import StructureBatch
@@ -375,8 +393,10 @@ def simp_loop(args, L, nat, n_steps=8, step=0.05):
     res = {"workload": f"SIMP batch ({nd} x 100x100 shells), {n_steps} normalised-gradient steps on rho "
                        f"(step {step}), FP64"}
     Cs = {}
-    for keep in (False, True):
+    for key in ("direct", "rebuild_every_step", "keep_hierarchy"):
+        keep = key == "keep_hierarchy"
         rho = rho0.clone()
+        b.plan.set_preconditioner(None if key == "direct" else "amg")
         b.plan.amg_reuse(2 if keep else 0)
         b.prop_quad[:, 1] = rho ** 3 * 30e9
         b.compliance_and_gradient(precision="fp64", tol=args.tol)        # warm-up on the start design
@@ -400,13 +420,17 @@ def simp_loop(args, L, nat, n_steps=8, step=0.05):
         dt = time.perf_counter() - t0
         L.jsso_timing_enable(0)
         setup_ms, _ = _slot(L, nat, "setup")
-        Cs[keep] = torch.stack(Cl)
-        key = "keep_hierarchy" if keep else "rebuild_every_step"
-        res[key] = {"evals_per_s": nd * n_steps / dt, "ms_per_step": dt * 1e3 / n_steps, "cg_iterations": iters,
-                    "amg_setup_ms_per_step": setup_ms, "amg": b.plan.amg_reuse(-1),
-                    "rebuilds_triggered": policy.rebuilds if policy else None}
+        Cs[key] = torch.stack(Cl)
+        res[key] = {"route": _route(b.plan), "evals_per_s": nd * n_steps / dt, "ms_per_step": dt * 1e3 / n_steps,
+                    "refinement_steps" if key == "direct" else "cg_iterations": iters,
+                    "factor_ms_per_step" if key == "direct" else "amg_setup_ms_per_step": setup_ms}
+        if key != "direct":
+            res[key].update(amg=b.plan.amg_reuse(-1), rebuilds_triggered=policy.rebuilds if policy else None)
     b.plan.amg_reuse(0)
-    res["max_rel_diff_C"] = float(((Cs[True] - Cs[False]).abs() / Cs[False].abs()).max())
+    b.plan.set_preconditioner(None)
+    ref = Cs["direct"]
+    res["max_rel_diff_C"] = max(float(((c - ref).abs() / ref.abs()).max()) for c in Cs.values())
+    res["speedup_direct_vs_rebuild"] = res["direct"]["evals_per_s"] / res["rebuild_every_step"]["evals_per_s"]
     res["speedup_keep_vs_rebuild"] = res["keep_hierarchy"]["evals_per_s"] / res["rebuild_every_step"]["evals_per_s"]
     return res
 
@@ -432,9 +456,9 @@ def gridshell_batch(args, n_designs=256):
     b = StructureBatch(designs)
     (C, (dc, _, _)), dt = _timed(lambda: b.compliance_and_gradient(precision="mixed", tol=args.tol), reps=3)
     res = {"workload": f"{n_designs} beam gridshells, 8..32 bays (seeded), perimeter pinned, 4 load cases each, "
-                       f"{b.plan.ndof} DOF in one plan", "precision": "mixed", "preconditioner": "amg",
+                       f"{b.plan.ndof} DOF in one plan", "precision": "mixed", "route": _route(b.plan),
            "evals_per_s": n_designs * 4 / dt, "ms_per_step": dt * 1e3,
-           "cg_iterations": b.plan.last_info["iterations"], "converged": b.plan.last_info["converged"]}
+           "iterations": b.plan.last_info["iterations"], "converged": b.plan.last_info["converged"]}
     if not args.no_oracle_check:
         import oracle.gradient as og
         st = designs[0]
@@ -459,8 +483,10 @@ def shell40(args):
     batch = StructureBatch([wl.cfg1(d) for d in range(128)])
     _, dtb = _timed(lambda: batch.compliance_and_gradient(precision="mixed", tol=args.tol), reps=5)
     return {"workload": "MITC-4 shell 40x40 over 10 m (1,681 nodes, 1,600 quads, 10,086 DOF), four fixed corners",
-            "single_evals_per_s": 1.0 / dt1, "single_cg_iterations": one.plan.last_info["iterations"],
-            "batch128_evals_per_s": 128 / dtb, "batch128_cg_iterations": batch.plan.last_info["iterations"]}
+            "single_route": _route(one.plan), "single_evals_per_s": 1.0 / dt1,
+            "single_iterations": one.plan.last_info["iterations"],
+            "batch128_route": _route(batch.plan), "batch128_evals_per_s": 128 / dtb,
+            "batch128_iterations": batch.plan.last_info["iterations"]}
 
 
 def trace_summary(trace_dir, bench_log):
@@ -535,7 +561,7 @@ def trace_summary(trace_dir, bench_log):
               f"{(last[-1][0] - last[0][0]) / 1e6:.2f} ms from its first to its last {kname} launch")
 
 
-FP64_VECTOR_PEAK_TFLOPS = 78.6
+FP64_VECTOR_PEAK_TFLOPS = FP64_MATRIX_PEAK_TFLOPS = 78.6
 FLOP_COUNTERS = ("SQ_INSTS_VALU_ADD_F64", "SQ_INSTS_VALU_MUL_F64", "SQ_INSTS_VALU_FMA_F64", "SQ_INSTS_VALU_TRANS_F64")
 
 
@@ -583,9 +609,11 @@ def traffic_summary(fetch_dir, write_dir, bench_log):
     """HBM bytes per launch of the roofline kernel from two rocprofv3 --pmc runs of
     ``bench.py --profile-run`` (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch),
     each scaled by what the counter reads for the run's 1 GiB device copy; only
-    the launches that processed the whole plan (solve_log) are averaged."""
+    the launches that processed the whole plan (solve_log) are averaged.  With the
+    direct solve: bytes per evaluation of its factorisation and solve kernels."""
     import csv
     import glob
+    import re
     out = None
     with open(bench_log) as fh:
         for line in fh:
@@ -595,6 +623,7 @@ def traffic_summary(fetch_dir, write_dir, bench_log):
     log = out["solve_log"]["solves"]
     res = {}
     asm = {}   # assembly kernels: counter -> name -> values per launch
+    direct = {}   # kernels of the direct solve: counter -> name -> bytes over all launches
     for counter, d in (("FETCH_SIZE", fetch_dir), ("WRITE_SIZE", write_dir)):
         vals, copies = [], []
         for path in sorted(glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True)):
@@ -612,6 +641,10 @@ def traffic_summary(fetch_dir, write_dir, bench_log):
                               "diag_factor_kernel", "ell_assemble_kernel"):
                         if a in name:
                             asm.setdefault(counter, {}).setdefault(a, []).append(v)
+                    m = re.search(r"k_(front|solve)_\w+(<[^>]*>)?", name)
+                    if m:
+                        d = direct.setdefault(counter, {})
+                        d[m.group(0)] = d.get(m.group(0), 0.0) + v
         vals.sort()
         v = [x for _, x in vals]
         extra = len(v) - sum(l for _, l, _ in log)    # the live tuner's launches come first
@@ -634,14 +667,24 @@ def traffic_summary(fetch_dir, write_dir, bench_log):
         print(f"write_bytes_per_launch {kname}: {int(w * wf)}")
         print(f"traffic_bytes_per_launch {kname}: {int(traffic)}")
         print(f"# traffic / algorithmic bytes = {traffic / alg:.3f} over {n} launches")
-        # assembly kernels (every launch covers the whole batch; the element kernel's
-        # three variants are the autotuner's candidates)
-        for a in sorted(asm.get("FETCH_SIZE", {})):
-            fv, wv = asm["FETCH_SIZE"][a], asm.get("WRITE_SIZE", {}).get(a, [])
-            if fv and wv:
-                fb, wb = sum(fv) / len(fv) * ff, sum(wv) / len(wv) * wf
-                print(f"assembly_traffic {a}: fetch {int(fb)} write {int(wb)} total {int(fb + wb)}"
-                      f"  # {len(fv)} launches")
+    if not (ff and wf):
+        return
+    if direct:
+        solves, total = len(log), 0.0
+        for a in sorted(direct.get("FETCH_SIZE", {})):
+            fb = direct["FETCH_SIZE"][a] * ff / solves
+            wb = direct.get("WRITE_SIZE", {}).get(a, 0.0) * wf / solves
+            total += fb + wb if a.startswith("k_front") else 0.0
+            print(f"direct_traffic {a}: fetch {int(fb)} write {int(wb)} total {int(fb + wb)}  # per evaluation")
+        print(f"traffic_bytes_per_launch {FRONT_KERNELS}: {int(total)}")
+    # assembly kernels (every launch covers the whole batch; the element kernel's
+    # three variants are the autotuner's candidates)
+    for a in sorted(asm.get("FETCH_SIZE", {})):
+        fv, wv = asm["FETCH_SIZE"][a], asm.get("WRITE_SIZE", {}).get(a, [])
+        if fv and wv:
+            fb, wb = sum(fv) / len(fv) * ff, sum(wv) / len(wv) * wf
+            print(f"assembly_traffic {a}: fetch {int(fb)} write {int(wb)} total {int(fb + wb)}"
+                  f"  # {len(fv)} launches")
 
 
 def _cpu_model():
