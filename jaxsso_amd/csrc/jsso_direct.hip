@@ -132,16 +132,6 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
     return join_halves(lo, hi);
 }
 
-// acc += X_I Y_J^T over n16 tiles of 16 columns; X, Y point at the first row of
-// the row tiles
-__device__ __forceinline__ d4 tile_xyt(const double* X, const double* Y, int ld, int n16, d4 acc, int lane) {
-    const double* x = X + (lane & 15) * ld + (lane >> 4);
-    const double* y = Y + (lane & 15) * ld + (lane >> 4);
-#pragma unroll 4
-    for (int t = 0; t < 4 * n16; ++t) acc = mfma64(x[4 * t], y[4 * t], acc);
-    return acc;
-}
-
 // 1 / sqrt(d): the hardware estimate and one third-order correction
 __device__ __forceinline__ double fast_rsqrt(double d) {
     const double y = __builtin_amdgcn_rsq(d);
@@ -1910,8 +1900,8 @@ static int run_direct(Plan* pl, DirectState& D, const double* f, double* u, doub
             residual(std::integral_constant<int, WpsFits<double, NR, 2>::value ? 2 : 1>());
         else
             residual(std::integral_constant<int, 1>());
-        // (a step that gains less than 10% ends a system at once: near its attainable
-        // accuracy as converged there, else as stalled)
+        // (a step that gains less than 10% ends a system at its attainable accuracy as
+        // converged there; off it, three steps in a row that gain less end it as stalled)
         hipLaunchKernelGGL((k_decide<NR>), dim3(pl->n_sys), dim3(64), 0, s, sl, w.P, w.st, pl->n_sys, DECIDE_STEP, tol,
                            1, 2, (const double*)D.d_rho, DIRECT_FLOOR_FACTOR, 0);
         hipLaunchKernelGGL(k_direct_report, dim3(1), dim3(256), 0, s, nsys, pl->n_sys, (const int32_t*)w.st.status,
