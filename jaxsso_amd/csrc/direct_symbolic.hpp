@@ -19,11 +19,12 @@
 // the parent's nodes is increasing and a lower triangle maps into a lower
 // triangle.
 //
-// The sets are cut level by level, largest first, so that a pattern whose fronts
-// are past a caller's limit shows at its first few cuts: the front that a set ends
+// Large sets are cut level by level, before all others, so that a pattern whose fronts
+// are past a caller's limit shows at its first few cuts (the others go depth first, while
+// their nodes are in the cache): the front that a set ends
 // in is its separator and the set's own border, both known once it is cut.  (With a
-// limit of 383 nodes, meshes of 300 x 300, 600 x 600 and 1000 x 1000 quads take 25, 75
-// and 320 ms on one core; cut to the end, 0.24, 1.1 and 3.9 s.)
+// limit of 383 nodes, meshes of 300 x 300, 600 x 600 and 1000 x 1000 quads take 23, 65
+// and 215 ms on one core; cut to the end, 0.22, 1.0 and 3.1 s.)
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -65,9 +66,17 @@ public:
         std::vector<Set> sets(1);
         sets[0].nodes.resize(n_);
         for (int i = 0; i < n_; ++i) sets[0].nodes[i] = i;
-        for (size_t t = 0; t < sets.size(); ++t) {   // (part_ of a set's nodes: its number)
+        std::vector<int32_t> large{0}, others;   // sets to come (part_ of a set's nodes: its number)
+        for (size_t next = 0; next < large.size() || !others.empty();) {
+            int32_t t;
+            if (next < large.size()) {
+                t = large[next++];
+            } else {
+                t = others.back();
+                others.pop_back();
+            }
             std::vector<int32_t> side[2], sep;
-            if ((int)sets[t].nodes.size() <= leaf_ || !cut((int32_t)t, sets[t].nodes, side, sep))
+            if ((int)sets[t].nodes.size() <= leaf_ || !cut(t, sets[t].nodes, side, sep))
                 sep = std::move(sets[t].nodes);
             else
                 std::sort(sep.begin(), sep.end());
@@ -78,17 +87,18 @@ public:
                 std::sort(s.begin(), s.end());
                 const int32_t kid = (int32_t)sets.size();
                 for (int v : s) part_[v] = kid;
-                Set next;
-                next.nodes = std::move(s);
+                ((int64_t)s.size() > 4 * (int64_t)max_nodes ? large : others).push_back(kid);
+                Set below;
+                below.nodes = std::move(s);
                 for (const auto* from : {&sets[t].border, &sep})
                     for (int w : *from)
                         for (int k = rp_[w]; k < rp_[w + 1]; ++k)
                             if (part_[ci_[k]] == kid) {
-                                next.border.push_back(w);
+                                below.border.push_back(w);
                                 break;
                             }
                 sets[t].node.kids.push_back(kid);
-                sets.push_back(std::move(next));
+                sets.push_back(std::move(below));
             }
             sets[t].node.own = std::move(sep);
             std::vector<int32_t>().swap(sets[t].nodes);
@@ -233,7 +243,6 @@ private:
         auto& tmp = dist_[3];
         const int reached = bfs(lab, set[0], tmp);
         if (reached < (int)set.size()) {   // several components: no separator needed
-            std::vector<int32_t> order;
             std::vector<std::vector<int32_t>> comp;
             for (int v : set) {
                 if (dist_[2][v] >= 0) continue;

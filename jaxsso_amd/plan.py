@@ -81,7 +81,7 @@ class FEPlan:
         nat.check(L.jsso_assemble(self._h, nat.ptr(crds), nat.ptr(pb), nat.ptr(pq), nat.ptr(Kout), nat.stream_ptr()))
         # the kernels may still read these when the caller drops them, on another stream than
         # the one they were allocated on: their memory is held until the next assembly
-        self._keep = [None if t is None else t.detach() for t in (crds, pb, pq)]
+        self._keep = (crds, pb, pq)
         return Kout
 
     def ensure_assembled(self, crds, prop_beam, prop_quad, assembly_id=None):
