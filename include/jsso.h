@@ -237,8 +237,8 @@ int jsso_spmv_k(jsso_plan* plan, const double* d_K, const double* d_x, double* d
 int jsso_dense_solve(jsso_plan* plan, const double* d_K, const double* d_f, double* d_u, int32_t nrhs,
                      int32_t transpose, void* stream);
 /* K^T u = f with u = 0 at supports: the adjoint system of a non-symmetric plan
- * (same arguments and results as jsso_solve; a symmetric plan is solved as by
- * jsso_solve).
+ * (same arguments and results as jsso_solve, u may lie over f; a symmetric plan is
+ * solved as by jsso_solve).
  *   <- the custom VJP's solve with K_aug^T  JaxSSO/solver.py:236
  * Non-symmetric plans (both entry points): without members parallel to global Y,
  * and where the direct solve is taken (see JSSO_PC_AMG), refinement with the
@@ -320,7 +320,8 @@ int jsso_plan_set_preconditioner(jsso_plan* plan, int32_t pc);
  *      front of k pivot and b border rows: factor, solve operators and contribution)
  *   4  factorisations run   5  solves begun   6  solves that it finished (the others went
  *      on to the next route)
- * Entries 1 to 3 are 0 until decided. */
+ * Entries 1 to 3 are 0 until decided, and what the analysis had counted when it stopped
+ * for a plan past the limits. */
 int jsso_plan_direct_info(jsso_plan* plan, int64_t* h_info);
 
 /* Reuse of the AMG hierarchy across assemblies, for optimisation loops (no

@@ -96,22 +96,23 @@ class FEPlan:
         """False when the last assembly holds beam-columns parallel to global Y (the
         reference's transformation for them is not orthogonal, element.py:92-94) or
         quads with kx_mod != ky_mod (non-symmetric Cm, element.py:852-875): K is not
-        symmetric, solves run on the dense LU path and adjoints need K^T."""
+        symmetric, solves take the routes of ``nonsymmetric_route`` and adjoints need K^T."""
         out = ctypes.c_int32(1)
         nat.check(nat.lib().jsso_plan_symmetric(self._h, ctypes.byref(out), nat.stream_ptr()))
         return bool(out.value)
 
     def solve_transpose(self, f: torch.Tensor, **kw) -> torch.Tensor:
         """K^T u = f (u = 0 at supports): the adjoint solve.  K is symmetric unless
-        the assembly holds members parallel to global Y or orthotropic quads; then
-        ``jsso_solve_transpose`` takes the dense LU of K^T or, for large plans
-        without Y-parallel members, the defect correction (``nonsymmetric_route``)."""
+        the assembly holds members parallel to global Y or orthotropic quads
+        (``nonsymmetric_route``)."""
         return self.solve(f, transpose=True, **kw)
 
     def nonsymmetric_route(self, mode: int = -1) -> int:
-        """How non-symmetric plans are solved: 0 automatic (dense LU up to 16 384
-        DOF or with members parallel to global Y, else defect correction on the
-        symmetric part), 1 dense LU, 2 defect correction; -1 only reads it."""
+        """How non-symmetric plans are solved: 0 automatic (refinement with the factor of
+        the symmetric part where the plan solves directly and no member is parallel to
+        global Y; else the dense LU up to 16 384 DOF or with such members, the iterative
+        correction on the symmetric part above), 1 dense LU, 2 a correction on the
+        symmetric part (by its factor or iterative); -1 only reads it."""
         out = ctypes.c_int32(0)
         nat.check(nat.lib().jsso_plan_nonsymmetric_route(self._h, int(mode), ctypes.byref(out)))
         return int(out.value)
@@ -259,8 +260,9 @@ class FEPlan:
     def dense_solve(self, f: torch.Tensor, K: torch.Tensor | None = None, transpose: bool = False) -> torch.Tensor:
         """u with u = 0 at supports and K_ff u_f = f_f (K_ff^T with ``transpose``), by
         the dense FP64 factorisation of the constrained K on the device
-        (``jsso_dense_solve``: Cholesky, or pivoted LU when the assembly holds
-        members parallel to global Y).  ``K``: block values ((nnzb,6,6)) or None for
+        (``jsso_dense_solve``: Cholesky, or pivoted LU of a K that is not symmetric; up to 4
+        right-hand sides of the plan's own symmetric assembly by the direct solve's
+        factorisation, refined to its floor).  ``K``: block values ((nnzb,6,6)) or None for
         the plan's current assembly; f: (ndof,) or (ndof, m)."""
         L = nat.lib()
         f = _dev64(f)
